@@ -238,8 +238,8 @@ int momoe_swiglu_bwd_saved(const void* ab_save, const void* u_MsumH,
                            int64_t M, int64_t H, int64_t N, int64_t Msum, void* stream);
 
 /* momoe_gs_scatter: Gs_NM[i, idx[r]] = sum_p gs_part[p][r] for every sorted row r of
- * expert i (momoe/momoe.py:699-703 without atomics).  Gs_NM fp32 contiguous [N,M],
- * zero-filled by the caller (:721).
+ * expert i (momoe/momoe.py:699-703 without atomics), zero everywhere else (:721).  Gs_NM fp32
+ * contiguous [N,M]; every element is written.
  */
 int momoe_gs_scatter(const float* gs_part, int64_t nparts, const int32_t* idx_Msum,
                      const int32_t* cumsums_N1, float* Gs_NM,
@@ -322,6 +322,12 @@ int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t gs_stride_
                      const float* p_sel_MN, const float* s_MN, const float* Ng_M, const float* Ks_M,
                      const int32_t* mask_NM, int64_t M, int64_t N, int64_t Ks,
                      void* Glogits_MN, void* stream);
+
+/* momoe_bias_update (momoe/sample_moe.py:65-67): biases_N[i] += rate * sign(c_avg - sizes_N[i]) in
+ * place, fp32; -inf (a shared expert) stays -inf.
+ */
+int momoe_bias_update(const int64_t* sizes_N, float c_avg, float rate, int64_t N, float* biases_N,
+                      void* stream);
 
 #ifdef __cplusplus
 }

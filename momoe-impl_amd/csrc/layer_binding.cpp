@@ -1,0 +1,409 @@
+// The layer's host path: one call per autograd node.  Allocates every output and workspace with
+// torch's caching allocator, enqueues the kernels of libmomoe_hip.so on the current stream and
+// records the autograd nodes.  It is native because a call makes a dozen launches: driven from
+// Python (a wrapper, an allocation or two and a foreign-function call per launch) the host needed
+// 84 us for a forward and 240 us for a training step of any size, longer than the GPU works on a
+// decode call or on a small step.
+//
+// Nothing here synchronises with the device (unless the caller asks for the routing check): every
+// launch is sized from static upper bounds and the routing-dependent tile list lives in device
+// memory.
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/extension.h>
+
+#include <mutex>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/momoe_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ---- launch timing (kernel_timer in _hip.py): an event pair around every library call ---------
+struct TimedCall {
+  const char* name;
+  hipEvent_t begin, end;
+};
+std::mutex g_timing_mutex;
+bool g_timing = false;  // written with no launch in flight; a stale read only skips a record
+std::vector<TimedCall> g_calls;
+
+void timing_start() {
+  std::lock_guard<std::mutex> lock(g_timing_mutex);
+  g_timing = true;
+}
+void timing_stop() {
+  std::lock_guard<std::mutex> lock(g_timing_mutex);
+  g_timing = false;
+}
+// durations in ms of the calls recorded so far; the device must be idle
+std::vector<std::pair<std::string, double>> timing_take() {
+  std::lock_guard<std::mutex> lock(g_timing_mutex);
+  std::vector<std::pair<std::string, double>> out;
+  for (auto& c : g_calls) {
+    float ms = 0.0f;
+    const bool ok = hipEventElapsedTime(&ms, c.begin, c.end) == hipSuccess;
+    (void)hipEventDestroy(c.begin);
+    (void)hipEventDestroy(c.end);
+    if (ok) out.emplace_back(c.name, (double)ms);
+  }
+  g_calls.clear();
+  return out;
+}
+
+template <class Fn, class... Args>
+void call(const char* name, hipStream_t st, Fn fn, Args... args) {
+  int code;
+  if (!g_timing) {
+    code = fn(args..., (void*)st);
+  } else {
+    TimedCall t{name, nullptr, nullptr};
+    const bool ok = hipEventCreate(&t.begin) == hipSuccess && hipEventCreate(&t.end) == hipSuccess &&
+                    hipEventRecord(t.begin, st) == hipSuccess;
+    code = fn(args..., (void*)st);
+    if (ok && hipEventRecord(t.end, st) == hipSuccess) {
+      std::lock_guard<std::mutex> lock(g_timing_mutex);
+      g_calls.push_back(t);
+    }
+  }
+  TORCH_CHECK(code == MOMOE_OK, name, " failed: status ", code, " (", momoe_status_string(code), ")");
+}
+#define MOMOE_CALL(fn, st, ...) call(#fn, st, fn, __VA_ARGS__)
+
+hipStream_t stream_of(const at::Device& dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+Tensor empty_bf16(at::IntArrayRef size, const at::Device& dev) {
+  return at::empty(size, at::TensorOptions().dtype(at::kBFloat16).device(dev));
+}
+Tensor empty_i32(int64_t n, const at::Device& dev) {
+  return at::empty({n}, at::TensorOptions().dtype(at::kInt).device(dev));
+}
+Tensor empty_f32(at::IntArrayRef size, const at::Device& dev) {
+  return at::empty(size, at::TensorOptions().dtype(at::kFloat).device(dev));
+}
+
+// A Python exception of the given type, raised when the binding returns
+[[noreturn]] void throw_python(PyObject* type, const std::string& what) {
+  py::gil_scoped_acquire gil;
+  PyErr_SetString(type, what.c_str());
+  throw py::error_already_set();
+}
+
+// ---- experts -----------------------------------------------------------------------------------
+// What the index build leaves for the rest of the forward and for the backward, in one allocation:
+// [cumsums N+1 | idx Msum | inv Msum | tile table | tile table of the recomputing GEMM], every part
+// on a 16-byte boundary.  The parts are found again from the sizes alone.
+struct Index {
+  int64_t M, N, K, tile_rows;
+  bool with_rc;
+  int64_t off_idx, off_inv, off_table, off_rc, ints;
+  Index(int64_t M_, int64_t N_, int64_t K_, int64_t tile_rows_, bool with_rc_)
+      : M(M_), N(N_), K(K_), tile_rows(tile_rows_), with_rc(with_rc_) {
+    auto up = [](int64_t n) { return (n + 3) & ~(int64_t)3; };
+    off_idx = up(N + 1);
+    off_inv = off_idx + up(M * K);
+    off_table = off_inv + up(M * K);
+    off_rc = off_table + up(momoe_tile_table_ints(M, N, K, (int)tile_rows));
+    ints = off_rc + (with_rc ? up(momoe_tile_table_ints(M, N, K, MOMOE_RECOMPUTE_TILE_ROWS)) : 0);
+  }
+  int32_t* base = nullptr;
+  int32_t* cumsums() const { return base; }
+  int32_t* idx() const { return base + off_idx; }
+  int32_t* inv() const { return base + off_inv; }
+  int32_t* table() const { return base + off_table; }
+  int32_t* table_rc() const { return with_rc ? base + off_rc : nullptr; }
+};
+
+struct Forward {
+  Tensor y, sizes;                     // results
+  Tensor x, W1, W2, s, index, ab_save; // for the backward
+};
+
+Forward experts_forward(const Tensor& x_BSD, const Tensor& Wl1, const Tensor& Wl2, const Tensor& mask_NM,
+                        const Tensor& s_NM, int64_t K, int64_t msave, bool want_rc, int64_t tile_rows,
+                        bool check) {
+  const at::Device dev = Wl1.device();
+  const int64_t B = x_BSD.size(0), S = x_BSD.size(1), D = x_BSD.size(2), M = B * S;
+  const int64_t N = Wl1.size(0), H = Wl1.size(2) / 2, msum = M * K;
+  const c10::DeviceGuard guard(dev);
+  const hipStream_t st = stream_of(dev);
+  Forward f;
+  f.x = x_BSD.reshape({M, D}).to(dev, at::kBFloat16).contiguous();
+  f.W1 = Wl1.to(at::kBFloat16).contiguous();
+  f.W2 = Wl2.to(at::kBFloat16).contiguous();
+  const Tensor mask = mask_NM.to(dev, at::kInt);
+  f.s = s_NM.to(dev, at::kFloat);
+  TORCH_CHECK(mask.dim() == 2 && mask.size(0) == N && mask.size(1) == M, "mask_NM must be [", N, ", ", M, "]");
+  TORCH_CHECK(f.s.dim() == 2 && f.s.size(0) == N && f.s.size(1) == M, "s_NM must be [", N, ", ", M, "]");
+
+  Index ib(M, N, K, tile_rows, want_rc);
+  f.index = empty_i32(ib.ints, dev);
+  ib.base = f.index.data_ptr<int32_t>();
+  f.sizes = at::empty({N}, at::TensorOptions().dtype(at::kLong).device(dev));
+  const int64_t ws_bytes = momoe_index_workspace_bytes(M, N);
+  // only the build itself needs these: its panel counts, the slot of every pair, and the counter
+  // of tokens with another number of experts than K, which starts from zero if it is to be read
+  const Tensor scratch = empty_i32(4 + ((msum + 3) & ~(int64_t)3) + (ws_bytes + 3) / 4, dev);
+  int32_t* violations = scratch.data_ptr<int32_t>();
+  if (check) scratch.narrow(0, 0, 4).zero_();
+  MOMOE_CALL(momoe_index_build, st, mask.data_ptr<int32_t>(), mask.stride(0), mask.stride(1), M, N, K,
+             f.sizes.data_ptr<int64_t>(), ib.cumsums(), ib.idx(), violations + 4, ib.inv(), ib.table(),
+             (int)tile_rows, ib.table_rc(), (void*)(violations + 4 + ((msum + 3) & ~(int64_t)3)), ws_bytes,
+             violations);
+
+  if (msave > 0) f.ab_save = empty_bf16({msave, 2 * H}, dev);
+  Tensor ys;
+  {
+    // h in blocks of 32 hidden columns, [H/32][Msum][32]: the layout the down projection reads
+    const Tensor h = empty_bf16({H / 32, msum, 32}, dev);
+    MOMOE_CALL(momoe_lin1_swiglu_fwd, st, f.x.data_ptr(), f.W1.data_ptr(), ib.idx(), ib.table(), h.data_ptr(),
+               msave > 0 ? f.ab_save.data_ptr() : nullptr, (int64_t)0, msave, M, D, H, N, msum);
+    ys = empty_bf16({msum, D}, dev);
+    MOMOE_CALL(momoe_lin2_scale_fwd, st, h.data_ptr(), f.W2.data_ptr(), f.s.data_ptr<float>(), f.s.stride(0),
+               f.s.stride(1), ib.idx(), ib.table(), ys.data_ptr(), M, D, H, N, msum);
+  }
+  f.y = empty_bf16({B, S, D}, dev);
+  MOMOE_CALL(momoe_combine, st, ys.data_ptr(), ib.inv(), f.y.data_ptr(), M, D, K, msum);
+  if (check) {
+    const int v = scratch.narrow(0, 0, 1).item<int32_t>();
+    TORCH_CHECK(v == 0, "mask_NM: ", v, " tokens do not have exactly K = ", K,
+                " experts (or the mask holds more than M*K pairs)");
+  }
+  if (x_BSD.device() != dev) f.y = f.y.to(x_BSD.device());
+  return f;
+}
+
+struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& W1, const Tensor& W2,
+                               const Tensor& mask, const Tensor& s, int64_t K, int64_t msave, int64_t tile_rows,
+                               bool check) {
+    // the backward's recomputing GEMM walks row tiles of its own height: with the height left to
+    // the library, the index build writes that table too
+    const bool want_rc = msave < x.size(0) * x.size(1) * K && tile_rows == 0;
+    Forward f = experts_forward(x, W1, W2, mask, s, K, msave, want_rc, tile_rows, check);
+    ctx->saved_data["K"] = K;
+    ctx->saved_data["msave"] = msave;
+    ctx->saved_data["tile_rows"] = tile_rows;
+    ctx->saved_data["want_rc"] = want_rc;
+    ctx->save_for_backward({f.x, f.s, f.W1, f.W2, f.index, f.ab_save});
+    ctx->mark_non_differentiable({f.sizes});
+    ctx->set_materialize_grads(false);
+    return {f.y, f.sizes};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &s = saved[1], &W1 = saved[2], &W2 = saved[3], &ab_save = saved[5];
+    const int64_t K = ctx->saved_data["K"].toInt(), msave = ctx->saved_data["msave"].toInt();
+    const int64_t tile_rows = ctx->saved_data["tile_rows"].toInt();
+    const bool need_x = ctx->needs_input_grad(0), need_w1 = ctx->needs_input_grad(1),
+               need_w2 = ctx->needs_input_grad(2), need_s = ctx->needs_input_grad(4);
+    variable_list out(9);
+    if (!grads[0].defined()) return out;
+    const at::Device dev = W1.device(), gdev = grads[0].device();
+    const int64_t B = grads[0].size(0), S = grads[0].size(1), D = grads[0].size(2), M = B * S;
+    const int64_t N = W2.size(0), H = W2.size(1), msum = M * K;
+    const c10::DeviceGuard guard(dev);
+    const hipStream_t st = stream_of(dev);
+    Index ib(M, N, K, tile_rows, ctx->saved_data["want_rc"].toBool());
+    ib.base = saved[4].data_ptr<int32_t>();
+    const Tensor Gy = grads[0].reshape({M, D}).to(dev, at::kBFloat16).contiguous();
+
+    // dL/dh before the gate weight, in sorted order
+    Tensor u = empty_bf16({msum, H}, dev);
+    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table(), u.data_ptr(), M, D, H, N, msum);
+    // SwiGLU backward: rows with saved a|b read them; the others recompute a|b = x.Wl1 and consume
+    // them straight from the GEMM's accumulators.
+    // G_a|G_b in blocks of 32 columns, [2H/32][Msum][32]: the layout dL/dx contracts over
+    const Tensor gz = empty_bf16({2 * H / 32, msum, 32}, dev);
+    // s*h in groups of 32 padded sorted rows, feature-major inside a group: the layout the Wl2
+    // gradient reads fastest
+    Tensor hst = empty_bf16({momoe_padded_rows(msum, N) / 32, H, 32}, dev);
+    const int64_t nparts = (H + MOMOE_GS_BLOCK - 1) / MOMOE_GS_BLOCK;
+    Tensor gs_part = empty_f32({nparts, msum}, dev);
+    if (msave > 0)
+      MOMOE_CALL(momoe_swiglu_bwd_saved, st, ab_save.data_ptr(), u.data_ptr(), s.data_ptr<float>(), s.stride(0),
+                 s.stride(1), ib.idx(), ib.cumsums(), msave, gz.data_ptr(), hst.data_ptr(), H,
+                 gs_part.data_ptr<float>(), nparts, M, H, N, msum);
+    if (msave < msum) {
+      // the recomputing GEMM takes shorter row tiles than the others: its own table, from the
+      // index build, or made here when the tile height was given
+      Tensor own;
+      const int32_t* table_rc = ib.table_rc();
+      if (table_rc == nullptr) {
+        own = empty_i32(momoe_tile_table_ints(M, N, K, MOMOE_RECOMPUTE_TILE_ROWS), dev);
+        MOMOE_CALL(momoe_tile_table_build, st, ib.cumsums(), N, msum, MOMOE_RECOMPUTE_TILE_ROWS,
+                   own.data_ptr<int32_t>());
+        table_rc = own.data_ptr<int32_t>();
+      }
+      MOMOE_CALL(momoe_lin1_swiglu_bwd, st, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc, u.data_ptr(),
+                 s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz.data_ptr(), hst.data_ptr(), H,
+                 gs_part.data_ptr<float>(), M, D, H, N, msum);
+    }
+    u.reset();
+    if (need_s) {
+      out[4] = empty_f32({N, M}, dev);
+      MOMOE_CALL(momoe_gs_scatter, st, gs_part.data_ptr<float>(), nparts, ib.idx(), ib.cumsums(),
+                 out[4].data_ptr<float>(), M, N, msum);
+    }
+    gs_part.reset();
+
+    // scratch for the weight gradients of experts with many rows: what the library can use, but no
+    // more than u occupied (just freed, so the peak does not move)
+    auto workspace = [&](int64_t X, int64_t Y, int64_t& bytes) {
+      bytes = std::min(msum * H * 2, momoe_wgrad_workspace_bytes(N, X, Y, msum));
+      return bytes > 0 ? at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(dev)) : Tensor();
+    };
+    int64_t ws_bytes = 0;
+    if (need_w2) {
+      out[2] = at::empty_like(W2);
+      const Tensor ws = workspace(H, D, ws_bytes);
+      MOMOE_CALL(momoe_wgrad, st, hst.data_ptr(), H, MOMOE_LAYOUT_TRANSPOSED, (const int32_t*)nullptr, Gy.data_ptr(),
+                 D, MOMOE_LAYOUT_ROWS, (const int32_t*)ib.idx(), ib.cumsums(), out[2].data_ptr(), M, N, H, D, msum,
+                 ws.defined() ? ws.data_ptr() : nullptr, ws_bytes);
+    }
+    hst.reset();
+    if (need_w1) {
+      out[1] = at::empty_like(W1);
+      const Tensor ws = workspace(D, 2 * H, ws_bytes);
+      MOMOE_CALL(momoe_wgrad, st, x.data_ptr(), D, MOMOE_LAYOUT_ROWS, (const int32_t*)ib.idx(), gz.data_ptr(), msum,
+                 MOMOE_LAYOUT_KBLOCKED, (const int32_t*)nullptr, ib.cumsums(), out[1].data_ptr(), M, N, D, 2 * H, msum,
+                 ws.defined() ? ws.data_ptr() : nullptr, ws_bytes);
+    }
+    if (need_x) {
+      const Tensor gxs = empty_bf16({msum, D}, dev);
+      MOMOE_CALL(momoe_dgrad_x, st, gz.data_ptr(), W1.data_ptr(), ib.table(), gxs.data_ptr(), M, D, H, N, msum);
+      Tensor Gx = empty_bf16({B, S, D}, dev);
+      MOMOE_CALL(momoe_combine, st, gxs.data_ptr(), ib.inv(), Gx.data_ptr(), M, D, K, msum);
+      out[0] = gdev == dev ? Gx : Gx.to(gdev);
+    }
+    return out;
+  }
+};
+
+std::pair<Tensor, Tensor> experts(const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& mask,
+                                  const Tensor& s, int64_t K, double save_percent, int64_t tile_rows, bool check) {
+  if (W1.device() != W2.device())
+    throw_python(PyExc_AssertionError, "All weights must be on the same device, but got: Wl1_ND2H.device = " +
+                                    W1.device().str() + ", Wl2_NHD.device = " + W2.device().str());
+  TORCH_CHECK(W1.is_cuda(), "MoMoE weights must live on the GPU: there is no CPU compute path");
+  if (x.dim() != 3 || W1.dim() != 3 || W2.dim() != 3 || W1.size(1) != x.size(2) || W2.size(0) != W1.size(0) ||
+      W2.size(1) != W1.size(2) / 2 || W2.size(2) != x.size(2))
+    throw_python(PyExc_AssertionError, "x_BSD [B,S,D], Wl1_ND2H [N,D,2H] and Wl2_NHD [N,H,D] do not fit together");
+  const int64_t msum = x.size(0) * x.size(1) * K;
+  const bool grad = at::GradMode::is_enabled() &&
+                    (x.requires_grad() || W1.requires_grad() || W2.requires_grad() || s.requires_grad());
+  if (!grad) {  // nothing is kept for a backward that cannot happen
+    Forward f = experts_forward(x, W1, W2, mask, s, K, 0, false, tile_rows, check);
+    return {f.y, f.sizes};
+  }
+  // the Wl1 gradient addresses the eight 32-column blocks of a gz tile with 32-bit byte offsets
+  // (momoe_wgrad, k-blocked operand): say so now rather than in the backward
+  TORCH_CHECK(!W1.requires_grad() || 8 * msum * 64 < (1ll << 32),
+              "MoMoE backward supports fewer than 8388608 (token, expert) pairs per call, got ", msum,
+              ": split the batch");
+  const int64_t msave = (int64_t)((double)msum * save_percent / 100.0);  // momoe/momoe.py:251
+  variable_list r = ExpertsFn::apply(x, W1, W2, mask, s, K, msave, tile_rows, check);
+  return {r[0], r[1]};
+}
+
+// ---- router ------------------------------------------------------------------------------------
+struct Routed {
+  Tensor x_MD, mask, s_MN, p_sel, norms;
+};
+Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biases, int64_t N, int64_t K, int64_t Ks) {
+  const at::Device dev = Wg.device();
+  const int64_t D = x_BSD.size(2), M = x_BSD.size(0) * x_BSD.size(1);
+  const c10::DeviceGuard guard(dev);
+  Routed r;
+  r.x_MD = x_BSD.reshape({M, D}).to(dev, at::kBFloat16);
+  const Tensor logits = at::mm(r.x_MD, Wg).contiguous();
+  TORCH_CHECK(logits.size(1) == N, "Wg_DN must have N = ", N, " columns");
+  const Tensor bias = biases.to(dev, at::kFloat).contiguous();
+  TORCH_CHECK(bias.numel() == N, "biases_N must have N = ", N, " elements");
+  r.mask = at::empty({N, M}, at::TensorOptions().dtype(at::kInt).device(dev));
+  r.s_MN = empty_f32({M, N}, dev);
+  r.p_sel = empty_f32({M, N}, dev);
+  r.norms = empty_f32({2, M}, dev);  // per token: sum over the selected, over the shared experts
+  float* norms = r.norms.data_ptr<float>();
+  MOMOE_CALL(momoe_router_fwd, stream_of(dev), logits.data_ptr(), 0, bias.data_ptr<float>(), M, N, K, Ks,
+             r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M);
+  return r;
+}
+
+struct RouterFn : torch::autograd::Function<RouterFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& Wg, const Tensor& biases,
+                               int64_t N, int64_t K, int64_t Ks) {
+    Routed r = router_forward(x, Wg, biases, N, K, Ks);
+    ctx->save_for_backward({r.x_MD, Wg, r.mask, r.p_sel, r.s_MN, r.norms});
+    ctx->saved_data["Ks"] = Ks;
+    ctx->saved_data["shape"] = x.sizes().vec();
+    ctx->mark_non_differentiable({r.mask});
+    ctx->set_materialize_grads(false);
+    return {x, r.mask, r.s_MN.t()};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &Wg = saved[1], &mask = saved[2], &p_sel = saved[3], &s_MN = saved[4], &norms = saved[5];
+    const at::Device dev = Wg.device();
+    const int64_t M = x.size(0), D = x.size(1), N = Wg.size(1);
+    const bool need_x = ctx->needs_input_grad(0), need_wg = ctx->needs_input_grad(1);
+    const c10::DeviceGuard guard(dev);
+    variable_list out(6);
+    const Tensor &G_x_BSD = grads[0], &G_s_NM = grads[2];
+    Tensor G_x;
+    if (G_x_BSD.defined()) G_x = G_x_BSD.reshape({M, D}).to(dev, at::kBFloat16);
+    if (G_s_NM.defined()) {
+      const Tensor G_s = G_s_NM.to(dev, at::kFloat);
+      const Tensor G_logit = empty_bf16({M, N}, dev);
+      const float* nrm = norms.data_ptr<float>();
+      MOMOE_CALL(momoe_router_bwd, stream_of(dev), G_s.data_ptr<float>(), G_s.stride(0), G_s.stride(1),
+                 p_sel.data_ptr<float>(), s_MN.data_ptr<float>(), nrm, nrm + M, mask.data_ptr<int32_t>(), M, N,
+                 ctx->saved_data["Ks"].toInt(), G_logit.data_ptr());
+      if (need_x) G_x = G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
+      if (need_wg) out[1] = at::mm(x.t(), G_logit);
+    } else if (need_wg) {
+      out[1] = at::zeros_like(Wg);
+    }
+    if (need_x && G_x.defined()) out[0] = G_x.reshape(ctx->saved_data["shape"].toIntVector());
+    return out;
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor> router(const Tensor& x, const Tensor& Wg, const Tensor& biases, int64_t N, int64_t K,
+                                          int64_t Ks) {
+  if (Wg.scalar_type() != at::kBFloat16) throw_python(PyExc_AssertionError, "Wg_DN must be of type torch.bfloat16");
+  TORCH_CHECK(Wg.is_cuda(), "TopKRouter weights must live on the GPU: there is no CPU compute path");
+  TORCH_CHECK(x.dim() == 3, "x_BSD must be [B, S, D]");
+  if (!at::GradMode::is_enabled() || !(x.requires_grad() || Wg.requires_grad())) {
+    Routed r = router_forward(x, Wg, biases, N, K, Ks);
+    return {x, r.mask, r.s_MN.t()};
+  }
+  variable_list r = RouterFn::apply(x, Wg, biases, N, K, Ks);
+  return {r[0], r[1], r[2]};
+}
+
+// biases += rate * sign(c_avg - sizes), in place, in fp32
+void bias_update(Tensor biases, const Tensor& sizes, double c_avg, double rate) {
+  const c10::DeviceGuard guard(biases.device());
+  MOMOE_CALL(momoe_bias_update, stream_of(biases.device()), sizes.data_ptr<int64_t>(), (float)c_avg, (float)rate,
+             biases.numel(), biases.data_ptr<float>());
+  biases.unsafeGetTensorImpl()->bump_version();
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_layer, m) {
+  m.def("experts", &experts, py::call_guard<py::gil_scoped_release>());
+  m.def("router", &router, py::call_guard<py::gil_scoped_release>());
+  m.def("bias_update", &bias_update, py::call_guard<py::gil_scoped_release>());
+  m.def("timing_start", &timing_start);
+  m.def("timing_stop", &timing_stop);
+  m.def("timing_take", &timing_take);
+}

@@ -252,6 +252,15 @@ __global__ __launch_bounds__(kRouterThreads) void router_bwd_kernel(RouterBwdArg
   }
 }
 
+// biases += rate * sign(c_avg - sizes): the auxiliary-loss-free balancing step
+__global__ __launch_bounds__(256) void bias_update_kernel(const int64_t* __restrict__ sizes, float c_avg,
+                                                          float rate, int N, float* __restrict__ biases) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= N) return;
+  const float d = c_avg - (float)sizes[i];
+  biases[i] += rate * (d > 0.0f ? 1.0f : d < 0.0f ? -1.0f : 0.0f);
+}
+
 }  // namespace
 }  // namespace momoe
 
@@ -292,5 +301,13 @@ extern "C" int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t
   else if (N <= 128) router_bwd_kernel<32, 2><<<grid32, kRouterThreads, 0, st>>>(a);
   else if (N <= 256) router_bwd_kernel<32, 4><<<grid32, kRouterThreads, 0, st>>>(a);
   else router_bwd_kernel<16, 8><<<(unsigned)cdiv64(M, 16), kRouterThreads, 0, st>>>(a);
+  return launch_status();
+}
+
+extern "C" int momoe_bias_update(const int64_t* sizes_N, float c_avg, float rate, int64_t N,
+                                 float* biases_N, void* stream) {
+  if (!sizes_N || !biases_N || N <= 0) return MOMOE_ERR_BAD_ARG;
+  if (N >= (1ll << 31) - 256) return MOMOE_ERR_UNSUPPORTED;
+  bias_update_kernel<<<(unsigned)cdiv64(N, 256), 256, 0, (hipStream_t)stream>>>(sizes_N, c_avg, rate, (int)N, biases_N);
   return launch_status();
 }

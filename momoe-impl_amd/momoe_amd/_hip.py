@@ -1,4 +1,6 @@
-"""ctypes binding of libmomoe_hip.so (the C ABI declared in include/momoe_hip.h).
+"""ctypes binding of libmomoe_hip.so (the C ABI declared in include/momoe_hip.h), entry point by
+entry point.  The modules do not go through it: their host path is `_layer`, the native extension
+built from csrc/layer_binding.cpp.
 
 The library is the only compute path: if it is missing or fails to load, importing
 this module raises, and every wrapper raises RuntimeError on a non-zero status.
@@ -24,6 +26,8 @@ if not os.path.exists(LIB_PATH):
         "(there is no fallback compute path)")
 
 _lib = ctypes.CDLL(LIB_PATH)
+
+from . import _layer  # noqa: E402  (after the library it is linked against)
 
 _p = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -60,6 +64,7 @@ _SIGNATURES = {
                            _i64, _p, _i64, _p]),
     "momoe_router_fwd": (_int, [_p, _int, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]),
     "momoe_router_bwd": (_int, [_p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "momoe_bias_update": (_int, [_p, ctypes.c_float, ctypes.c_float, _i64, _p, _p]),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
@@ -74,27 +79,23 @@ def status_string(code):
     return _lib.momoe_status_string(int(code)).decode()
 
 
-_TIMINGS = None  # list of (entry point, start event, end event) while kernel_timer() is active
-
-
 class kernel_timer:
-    """Context manager: record a HIP event pair around every C-ABI call made inside it
-    (on torch's current stream).  `durations_ms()` synchronises and returns
+    """Context manager: record a HIP event pair around every library call the modules make inside
+    it (on torch's current stream).  `durations_ms()` returns
     [(entry point, milliseconds), ...] in call order."""
 
     def __enter__(self):
-        global _TIMINGS
-        self.records = _TIMINGS = []
+        _layer.timing_start()
         return self
 
     def __exit__(self, *exc):
-        global _TIMINGS
-        _TIMINGS = None
+        _layer.timing_stop()
+        torch.cuda.synchronize()
+        self.records = _layer.timing_take()
         return False
 
     def durations_ms(self):
-        torch.cuda.synchronize()
-        return [(name, a.elapsed_time(b)) for name, a, b in self.records]
+        return self.records
 
 
 class clock_trace:
@@ -165,16 +166,7 @@ def hbm_stream_probe(weights_NKC, launches=5):
 
 
 def _call(name, *args):
-    fn = getattr(_lib, name)
-    if _TIMINGS is None:
-        code = fn(*args)
-    else:
-        a = torch.cuda.Event(enable_timing=True)
-        b = torch.cuda.Event(enable_timing=True)
-        a.record()
-        code = fn(*args)
-        b.record()
-        _TIMINGS.append((name, a, b))
+    code = getattr(_lib, name)(*args)
     if code != 0:
         raise RuntimeError(f"{name} failed: status {code} ({status_string(code)})")
 

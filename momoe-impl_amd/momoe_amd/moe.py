@@ -6,6 +6,7 @@ Parameter names match the reference so state dicts interchange:
 import torch
 import torch.nn as nn
 
+from . import _layer
 from .experts import MoMoE
 from .router import TopKRouter
 
@@ -39,5 +40,9 @@ class MoE(nn.Module):
         # under-loaded experts become easier to select, over-loaded ones harder
         B, S, _ = x_BSD.shape
         c_avg = B * S * (self.K - self.Ks) / (self.N - self.Ks)
-        self.biases_N += self.bias_update_rate * torch.sign(c_avg - sizes_N.to(self.biases_N.device))
+        b = self.biases_N
+        if b.dtype == torch.float32 and b.is_contiguous() and b.device == sizes_N.device and not b.requires_grad:
+            _layer.bias_update(b, sizes_N, c_avg, self.bias_update_rate)
+        else:
+            self.biases_N += self.bias_update_rate * torch.sign(c_avg - sizes_N.to(b.device))
         return y_BSD

@@ -7,11 +7,12 @@ pass and its backward are one HIP kernel each.
 import torch
 import torch.nn as nn
 
-from . import _hip
+from . import _layer
 
 
-class TopKRouterFunction(torch.autograd.Function):
-    """(x_BSD, Wg_DN, biases_N, N, K, Ks) -> (x_BSD, mask_NM int32 [N,M], s_NM fp32 [N,M]).
+class TopKRouterFunction:
+    """(x_BSD, Wg_DN, biases_N, N, K, Ks) -> (x_BSD, mask_NM int32 [N,M], s_NM fp32 [N,M]): the
+    autograd function of the router, native (csrc/layer_binding.cpp).
 
     s_NM is the transposed view of an [M,N] matrix, as in the reference
     (momoe/topk_router.py:120); x_BSD is passed through so its gradient picks up
@@ -19,45 +20,8 @@ class TopKRouterFunction(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, x_BSD, Wg_DN, biases_N, N, K, Ks):
-        B, S, D = x_BSD.shape
-        M = B * S
-        assert Wg_DN.dtype == torch.bfloat16, "Wg_DN must be of type torch.bfloat16"
-        dev = Wg_DN.device
-        if dev.type != "cuda":
-            raise RuntimeError("TopKRouter weights must live on the GPU: there is no CPU compute path")
-        with torch.cuda.device(dev):
-            x_MD = x_BSD.reshape(M, D).to(device=dev, dtype=torch.bfloat16)
-            logits = x_MD @ Wg_DN
-            bias = biases_N.to(device=dev, dtype=torch.float32).contiguous()
-            mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M = _hip.router_fwd(logits.contiguous(), bias, K, Ks)
-        ctx.save_for_backward(x_MD, Wg_DN, mask_NM, p_sel_MN, s_MN, Ng_M, Ks_M)
-        ctx.Ks = Ks
-        ctx.mark_non_differentiable(mask_NM)
-        return x_BSD, mask_NM, s_MN.T
-
-    @staticmethod
-    def backward(ctx, G_x_BSD, _, G_s_NM):
-        x_MD, Wg_DN, mask_NM, p_sel_MN, s_MN, Ng_M, Ks_M = ctx.saved_tensors
-        M, D = x_MD.shape
-        dev = Wg_DN.device
-        with torch.cuda.device(dev):
-            G_x_MD = None
-            if G_x_BSD is not None:
-                G_x_MD = G_x_BSD.reshape(M, D).to(device=dev, dtype=torch.bfloat16)
-            if G_s_NM is None:
-                G_Wg = torch.zeros_like(Wg_DN)
-                G_x = G_x_MD if G_x_MD is not None else torch.zeros_like(x_MD)
-            else:
-                G_s = G_s_NM.to(device=dev, dtype=torch.float32)
-                G_logit = _hip.router_bwd(G_s, p_sel_MN, s_MN, Ng_M, Ks_M, mask_NM, ctx.Ks)
-                if G_x_MD is None:
-                    G_x = G_logit @ Wg_DN.T
-                else:
-                    G_x = torch.addmm(G_x_MD, G_logit, Wg_DN.T)
-                G_Wg = x_MD.T @ G_logit
-        shape = G_x_BSD.shape if G_x_BSD is not None else (1, M, D)
-        return G_x.view(shape), G_Wg, None, None, None, None
+    def apply(x_BSD, Wg_DN, biases_N, N, K, Ks):
+        return _layer.router(x_BSD, Wg_DN, biases_N, N, K, Ks)
 
 
 class TopKRouter(nn.Module):
