@@ -11,6 +11,8 @@
 //   pass 3 (scatter): per panel, each set bit learns its sorted row
 //                     (expert base + panel base + wave base + rank in ballot) and
 //                     its slot (set bits of the token in earlier experts).
+// Up to kPlaceCounts panel counts and kPlaceMaxExperts experts, passes 2 and 3 are one launch
+// (index_place_kernel): every panel's workgroup sums the counts it needs by itself.
 #include <mutex>
 
 #include "common.hpp"
@@ -41,8 +43,9 @@ __device__ __forceinline__ uint32_t load_panel_bits(const int32_t* __restrict__ 
 }
 
 __global__ __launch_bounds__(kPanelTokens) void index_count_kernel(
-    const int32_t* __restrict__ mask, int64_t sn, int64_t sm, int M, int N, int NC,
-    int32_t* __restrict__ part /*[N][NC]*/, int32_t* __restrict__ tokcnt /*[NG][M]*/) {
+    const int32_t* __restrict__ mask, int64_t sn, int64_t sm, int M, int N,
+    int32_t* __restrict__ part /*(expert i, panel c) at i * pn + c * pc*/, int pn, int pc,
+    int32_t* __restrict__ tokcnt /*[NG][M]*/) {
   __shared__ int32_t wcnt[kPanelExperts][4];
   const int c = blockIdx.x, g = blockIdx.y;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -57,7 +60,7 @@ __global__ __launch_bounds__(kPanelTokens) void index_count_kernel(
   __syncthreads();
   if (t < kPanelExperts) {
     const int i = g * kPanelExperts + t;
-    if (i < N) part[(int64_t)i * NC + c] = wcnt[t][0] + wcnt[t][1] + wcnt[t][2] + wcnt[t][3];
+    if (i < N) part[(int64_t)i * pn + (int64_t)c * pc] = wcnt[t][0] + wcnt[t][1] + wcnt[t][2] + wcnt[t][3];
   }
 }
 
@@ -246,30 +249,26 @@ __global__ __launch_bounds__(kPanelTokens) void index_scatter_kernel(
   }
 }
 
-// The whole index build in one launch of one workgroup, for at most 256 tokens (one token
-// panel) and 256 experts: decode-sized calls, where three dependent launches cost more than
-// the work.  Thread t is token t and reads its whole mask column up front (all loads in flight
-// at once: one memory latency), as 16 bits per group of 16 experts; one ballot per expert gives
-// the lane masks of its tokens, a scan over the experts gives cumsums and the tile table, and
-// every token then places its own K pairs from its bits and those masks.
-// the single-launch kernels: one expert's entries, and the header, in the table and (if asked
-// for) in its copy for the recomputing GEMM
+// one tile's entry, all of an expert's entries, and the header, in a table and (if asked for) in
+// its copy for the recomputing GEMM
+__device__ __forceinline__ void write_tile_entry(int32_t* table, int32_t* table_rc, int tile, int first,
+                                                 int expert, int row0, int rows) {
+  int32_t* e = table + kTileHeader + 4 * tile;
+  e[0] = expert;
+  e[1] = first;
+  e[2] = row0;
+  e[3] = rows;
+  if (table_rc != nullptr) {
+    int32_t* c = table_rc + kTileHeader + 4 * tile;
+    c[0] = expert;
+    c[1] = first;
+    c[2] = row0;
+    c[3] = rows;
+  }
+}
 __device__ __forceinline__ void write_tile_entries(int32_t* table, int32_t* table_rc, int first,
                                                    int nt, int expert, int row0, int rows) {
-  for (int k = 0; k < nt; ++k) {
-    int32_t* e = table + kTileHeader + 4 * (first + k);
-    e[0] = expert;
-    e[1] = first;
-    e[2] = row0;
-    e[3] = rows;
-    if (table_rc != nullptr) {
-      int32_t* c = table_rc + kTileHeader + 4 * (first + k);
-      c[0] = expert;
-      c[1] = first;
-      c[2] = row0;
-      c[3] = rows;
-    }
-  }
+  for (int k = 0; k < nt; ++k) write_tile_entry(table, table_rc, first + k, first, expert, row0, rows);
 }
 __device__ __forceinline__ void write_tile_header(int32_t* table, int32_t* table_rc, int ntiles,
                                                   int tile_rows) {
@@ -285,114 +284,12 @@ __device__ __forceinline__ void write_tile_header(int32_t* table, int32_t* table
   }
 }
 
-constexpr int kSmallMaxGroups = 16;
-constexpr int kSmallMaxExperts = kSmallMaxGroups * kPanelExperts;
-
-template <int NGROUPS>
-__global__ __launch_bounds__(kPanelTokens) void index_small_kernel(
-    const int32_t* __restrict__ mask, int64_t sn, int64_t sm, int M, int N, int K,
-    int64_t* __restrict__ sizes, int32_t* __restrict__ cumsums, int32_t* __restrict__ idx,
-    int32_t* __restrict__ which, int32_t* __restrict__ inv, int32_t* __restrict__ table,
-    int tile_rows_arg, int32_t* __restrict__ table_rc, int32_t* __restrict__ violations) {
-  // asked to choose the tile height: with at most 256 tokens no expert holds more than 256 rows,
-  // and taller tiles save nothing.  table_rc (only with that choice) receives the same table.
-  const int tile_rows = tile_rows_arg > 0 ? tile_rows_arg : MOMOE_RECOMPUTE_TILE_ROWS;
-  static_assert(kPanelTokens <= MOMOE_RECOMPUTE_TILE_ROWS, "one tile per expert in the one-launch kernel");
-  __shared__ uint64_t ball[NGROUPS * kPanelExperts][4];  // tokens of expert i in wave w, as a lane mask
-  __shared__ int32_t s_base[NGROUPS * kPanelExperts][4];  // sorted row of expert i's first token in wave w
-  __shared__ int32_t s_wave[4][2];
-  static_assert(NGROUPS % 4 == 0, "the experts of a token are walked as 64-bit words");
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int64_t msum = (int64_t)M * K;
-  uint32_t bits[NGROUPS];
-#pragma unroll
-  for (int g = 0; g < NGROUPS; ++g) bits[g] = load_panel_bits(mask, sn, sm, M, N, g, t);
-#pragma unroll
-  for (int g = 0; g < NGROUPS; ++g)
-#pragma unroll
-    for (int e = 0; e < kPanelExperts; ++e) {
-      const uint64_t b = __ballot((bits[g] >> e) & 1u);
-      if (lane == 0) ball[g * kPanelExperts + e][wave] = b;
-    }
-  __syncthreads();
-  // exclusive scan over the experts of (rows, row tiles): one expert per thread
-  const int v = t < N ? __popcll(ball[t][0]) + __popcll(ball[t][1]) + __popcll(ball[t][2]) + __popcll(ball[t][3]) : 0;
-  const int nt = (v + tile_rows - 1) / tile_rows;
-  const int irows = wave_inclusive_scan(v, lane), itiles = wave_inclusive_scan(nt, lane);
-  if (lane == 63) {
-    s_wave[wave][0] = irows;
-    s_wave[wave][1] = itiles;
-  }
-  __syncthreads();
-  int brow = irows - v, btile = itiles - nt;
-  for (int w = 0; w < wave; ++w) {
-    brow += s_wave[w][0];
-    btile += s_wave[w][1];
-  }
-  const int total = s_wave[0][0] + s_wave[1][0] + s_wave[2][0] + s_wave[3][0];
-  const int total_tiles = s_wave[0][1] + s_wave[1][1] + s_wave[2][1] + s_wave[3][1];
-  const bool overflow = (int64_t)total > msum;
-  if (t < N) {
-    int run = brow;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      s_base[t][w] = run;
-      run += __popcll(ball[t][w]);
-    }
-    cumsums[t] = brow;
-    sizes[t] = (int64_t)v;
-    if (!overflow) write_tile_entries(table, table_rc, btile, nt, t, brow, v);
-  }
-  if (t == 0) {
-    cumsums[N] = total;
-    if (overflow) atomicAdd(violations, 1);
-    write_tile_header(table, table_rc, overflow ? 0 : total_tiles, tile_rows);
-  }
-  // sorted rows past the last pair (a routing with fewer than M*K pairs): token 0, slot 0
-  for (int64_t r = (int64_t)total + t; r < msum; r += kPanelTokens) {
-    idx[r] = 0;
-    which[r] = 0;
-  }
-  __syncthreads();
-  // every token walks its own pairs (K of them, not N candidates), lowest expert first: one loop
-  // over all of its experts, so that a wavefront makes as many rounds as its busiest token has
-  // pairs (a loop per group of 16 experts made the sum over the groups of that maximum)
-  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  constexpr int NWORDS = NGROUPS / 4;
-  uint64_t word[NWORDS];
-#pragma unroll
-  for (int j = 0; j < NWORDS; ++j)
-    word[j] = (uint64_t)bits[4 * j] | ((uint64_t)bits[4 * j + 1] << 16) |
-              ((uint64_t)bits[4 * j + 2] << 32) | ((uint64_t)bits[4 * j + 3] << 48);
-  int k = 0;
-  for (;;) {
-    int i = -1;
-#pragma unroll
-    for (int j = NWORDS - 1; j >= 0; --j)
-      if (word[j] != 0) i = 64 * j + __ffsll((unsigned long long)word[j]) - 1;
-    if (i < 0) break;
-#pragma unroll
-    for (int j = 0; j < NWORDS; ++j)
-      if ((i >> 6) == j) word[j] &= word[j] - 1;
-    const int64_t row = (int64_t)s_base[i][wave] + __popcll(ball[i][wave] & below);
-    if (row < msum) {
-      idx[row] = t;
-      which[row] = k;
-    }
-    if (k < K) inv[(int64_t)t * K + k] = row < msum && !overflow ? (int32_t)row : -1;
-    ++k;
-  }
-  if (t < M && k != K) {
-    atomicAdd(violations, 1);
-    for (int kk = k; kk < K; ++kk) inv[(int64_t)t * K + kk] = -1;
-  }
-}
-
-// The same for at most 64 tokens, the other way round: thread e is EXPERT e and holds its row of
-// the mask as a 64-bit set of tokens.  Transposing the mask costs one ballot per token here (at
-// most 64) instead of one per expert (128 to 256 in the kernel above), a thread loads M mask
-// entries instead of N, and an expert has its few rows placed in as many rounds: a 16-token call
-// has its index in a third of the time (5.7 us against 16.5 at 128 experts).
+// The whole index build in one launch of one workgroup, for at most 64 tokens and 256 experts:
+// thread e is EXPERT e and holds its row of the mask as a 64-bit set of tokens.  Transposing the
+// mask costs one ballot per token (at most 64), a thread loads M mask entries, and an expert has
+// its few rows placed in as many rounds: 4.8 us at 16 tokens x 128 experts.  (With a thread per
+// token one workgroup can build up to 256 tokens' index, but it loads N entries per thread and
+// needs N ballots: 15 us at 131 tokens, where counting and placing in two launches take 11.)
 // MCH = ceil(M / 16): all of a thread's mask loads are in flight at once.
 constexpr int kTinyTokens = 64;
 template <int MCH>
@@ -502,6 +399,181 @@ __global__ __launch_bounds__(kPanelTokens) void index_tiny_kernel(
   }
 }
 
+// Passes 2 and 3 in one launch, for N <= kPlaceMaxExperts and N * NC <= kPlaceCounts.  Every
+// workgroup needs the rows of all experts before its panel, i.e. sums over all the counts (at most
+// 64 KiB, from L2): doing that in each of them takes less time than a one-workgroup launch in
+// front.  The panel's mask, its tokens' earlier pairs and the first counts are loaded together,
+// so that a workgroup waits for memory once or twice; bases come from LDS (read from memory
+// under the branch on a mask bit, they were waited for expert by expert).  Workgroup 0 writes what
+// does not belong to a panel: sizes, cumsums and the tile tables, tile by tile (a thread per
+// expert wrote all tiles of a large expert alone).
+// Measured at 128 experts: 1000 tokens 9.1 + 11.6 (scan, scatter) -> 7.5 us, 8192 tokens 9.7 + 13.9
+// -> 8.3; 65536 tokens x 64 experts 15.6 + 14.8 -> 18.9, and a launch fewer.
+// The line at 16384 counts: a workgroup's sums grow with the counts and there are as many
+// workgroups as panels, so the traffic goes with their square: 64 MB at 65536 tokens x 64 experts.
+constexpr int kPlaceMaxExperts = 256;
+constexpr int kPlaceCounts = 16384;
+
+__device__ __forceinline__ int last_not_above(const int32_t* a, int n, int v) {
+  int lo = 0, hi = n;  // a[lo] <= v < a[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (a[mid] <= v) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+__global__ __launch_bounds__(kPanelTokens) void index_place_kernel(
+    const int32_t* __restrict__ mask, int64_t sn, int64_t sm, int M, int N, int K, int NC, int NG,
+    const int32_t* __restrict__ part /*[NC][N]*/, const int32_t* __restrict__ tokcnt,
+    int64_t* __restrict__ sizes, int32_t* __restrict__ cumsums, int32_t* __restrict__ idx,
+    int32_t* __restrict__ which, int32_t* __restrict__ inv, int32_t* __restrict__ table,
+    int tile_rows_arg, int32_t* __restrict__ table_rc, int32_t* __restrict__ violations) {
+  __shared__ int32_t s_tot[kPlaceMaxExperts], s_pre[kPlaceMaxExperts];  // [slice][expert]
+  __shared__ int32_t s_cum[kPlaceMaxExperts], s_first[kPlaceMaxExperts];
+  __shared__ int32_t s_wave[4], s_off[kPanelExperts][4], s_height;
+  static_assert(kPlaceMaxExperts == kPanelTokens, "a thread per expert");
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t msum = (int64_t)M * K;
+  const bool writer = blockIdx.x == 0;
+  const int panel = max((int)blockIdx.x - 1, 0);
+  const int g = panel / NC, c = panel - g * NC;
+  const int m = c * kPanelTokens + t;
+  constexpr int kMaxGroups = kPlaceMaxExperts / kPanelExperts;
+  // pairs of this token in the groups of experts before g
+  int32_t cnt[kMaxGroups];
+  uint32_t bits = 0;
+  if (!writer) {
+    const int32_t* tc = tokcnt + min(m, M - 1);
+#pragma unroll
+    for (int q = 0; q < kMaxGroups; ++q) cnt[q] = tc[(int64_t)min(q, g) * M];
+    bits = load_panel_bits(mask, sn, sm, M, N, g, m);
+  }
+  // rows of every expert, and those in the panels before c: the panels are dealt to
+  // 256 / (experts rounded up to a power of two) slices of threads
+  int ep = 1;
+  while (ep < N) ep <<= 1;
+  const int e = t & (ep - 1), slice = t / ep, slices = kPanelTokens / ep;
+  int tot = 0, pre = 0;
+  for (int c0 = slice; c0 < NC; c0 += 16 * slices) {
+    int32_t v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = part[(int64_t)min(c0 + q * slices, NC - 1) * N + min(e, N - 1)];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int cc = c0 + q * slices;
+      tot += cc < NC ? v[q] : 0;
+      pre += cc < min(c, NC) ? v[q] : 0;
+    }
+  }
+  s_tot[t] = tot;
+  s_pre[t] = pre;
+  uint64_t ballots[kPanelExperts];
+#pragma unroll
+  for (int q = 0; q < kPanelExperts; ++q) ballots[q] = __ballot((bits >> q) & 1u);
+  if (lane == 0)
+#pragma unroll
+    for (int q = 0; q < kPanelExperts; ++q) s_off[q][wave] = __popcll(ballots[q]);
+  __syncthreads();
+  int v = 0, before = 0;
+  if (t < N)
+    for (int q = 0; q < slices; ++q) {
+      v += s_tot[q * ep + t];
+      before += s_pre[q * ep + t];
+    }
+  const int inc = wave_inclusive_scan(v, lane);
+  if (lane == 63) s_wave[wave] = inc;
+  __syncthreads();
+  int cum = inc - v;
+  for (int w = 0; w < wave; ++w) cum += s_wave[w];
+  const int total = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+  const bool overflow = (int64_t)total > msum;
+
+  if (writer) {
+    s_tot[t] = v;  // each thread has read its own column of the slices; others' are re-read below
+    if (t < N) {
+      cumsums[t] = cum;
+      sizes[t] = (int64_t)v;
+    }
+    s_cum[t] = cum;
+    if (t == 0) {
+      cumsums[N] = total;
+      if (overflow) atomicAdd(violations, 1);
+    }
+    // sorted rows past the last pair (a routing with fewer than M*K pairs): token 0, slot 0
+    for (int64_t r = (int64_t)total + t; r < msum; r += kPanelTokens) {
+      idx[r] = 0;
+      which[r] = 0;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int h = tile_rows_arg > 0 ? tile_rows_arg : choose_tile_rows(s_tot, N, lane);
+      if (lane == 0) s_height = h;
+    }
+    __syncthreads();
+    const int height = s_height;
+    auto write_table = [&](int32_t* dst, int32_t* copy, int rows) {
+      const int nt = (v + rows - 1) / rows;
+      const int inct = wave_inclusive_scan(nt, lane);
+      if (lane == 63) s_wave[wave] = inct;
+      __syncthreads();
+      int first = inct - nt;
+      for (int w = 0; w < wave; ++w) first += s_wave[w];
+      s_first[t] = first;
+      const int ntiles = overflow ? 0 : s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+      __syncthreads();
+      if (t == 0) write_tile_header(dst, copy, ntiles, rows);
+      for (int j = t; j < ntiles; j += kPanelTokens) {
+        // the last expert whose first tile is not after j is the one that has tiles
+        const int i = last_not_above(s_first, N, j);
+        write_tile_entry(dst, copy, j, s_first[i], i, s_cum[i], s_tot[i]);
+      }
+      __syncthreads();
+    };
+    const bool same = height == MOMOE_RECOMPUTE_TILE_ROWS;
+    write_table(table, same ? table_rc : nullptr, height);
+    if (table_rc != nullptr && !same) write_table(table_rc, nullptr, MOMOE_RECOMPUTE_TILE_ROWS);
+    return;
+  }
+
+  // sorted row of the first token of each of the panel's experts, per wavefront
+  s_cum[t] = cum + before;
+  __syncthreads();
+  if (t < kPanelExperts && g * kPanelExperts + t < N) {
+    int run = s_cum[g * kPanelExperts + t];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int n = s_off[t][w];
+      s_off[t][w] = run;
+      run += n;
+    }
+  }
+  __syncthreads();
+  int k = 0;
+#pragma unroll
+  for (int q = 0; q < kMaxGroups; ++q) k += q < g ? cnt[q] : 0;
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int q = 0; q < kPanelExperts; ++q) {
+    if ((bits >> q) & 1u) {
+      const int row = s_off[q][wave] + __popcll(ballots[q] & below);
+      if (row < msum) {
+        idx[row] = m;
+        which[row] = k;
+      }
+      // more pairs than rows: the GEMMs get an empty tile table and write nothing, so no token
+      // may point at a row (the combine then gives zeros instead of unwritten memory)
+      if (k < K) inv[(int64_t)m * K + k] = row < msum && !overflow ? row : -1;
+      ++k;
+    }
+  }
+  if (m < M && g == NG - 1 && k != K) {
+    atomicAdd(violations, 1);
+    // slots the token does not fill: -1 = "no row" (momoe_combine skips them)
+    for (int kk = k; kk < K; ++kk) inv[(int64_t)m * K + kk] = -1;
+  }
+}
+
 // A tile table for another tile height from the prefix sums of a finished index build.
 __global__ __launch_bounds__(1024) void tile_table_kernel(const int32_t* __restrict__ cumsums, int N,
                                                           int64_t msum_cap, int tile_rows,
@@ -607,16 +679,16 @@ extern "C" int momoe_index_build(const int32_t* mask_NM, int64_t stride_n, int64
                                        tile_rows, recompute_table, violations, rows_of_int4);
     return launch_status();
   }
-  if (NC == 1 && N <= kSmallMaxExperts) {
-    auto kernel = N <= 128 ? index_small_kernel<8> : index_small_kernel<kSmallMaxGroups>;
-    kernel<<<1, kPanelTokens, 0, st>>>(mask_NM, stride_n, stride_m, (int)M, (int)N, (int)K, sizes_N,
-                                       cumsums_N1, idx_Msum, which_Msum, inv_MK, tile_table,
-                                       tile_rows, recompute_table, violations);
+  dim3 grid(NC, NG);
+  const bool place = N <= kPlaceMaxExperts && N * NC <= kPlaceCounts;
+  index_count_kernel<<<grid, kPanelTokens, 0, st>>>(mask_NM, stride_n, stride_m, (int)M, (int)N, part,
+                                                    place ? 1 : NC, place ? (int)N : 1, tokcnt);
+  if (place) {
+    index_place_kernel<<<(unsigned)(NC * NG + 1), kPanelTokens, 0, st>>>(
+        mask_NM, stride_n, stride_m, (int)M, (int)N, (int)K, NC, NG, part, tokcnt, sizes_N, cumsums_N1,
+        idx_Msum, which_Msum, inv_MK, tile_table, tile_rows, recompute_table, violations);
     return launch_status();
   }
-  dim3 grid(NC, NG);
-  index_count_kernel<<<grid, kPanelTokens, 0, st>>>(mask_NM, stride_n, stride_m, (int)M, (int)N,
-                                                    NC, part, tokcnt);
   index_scan_kernel<<<1, 1024, 0, st>>>(part, (int)N, NC, M * K, sizes_N, cumsums_N1, tile_table,
                                         tile_rows, recompute_table, violations, idx_Msum,
                                         which_Msum);

@@ -81,6 +81,12 @@ def _compare(mask, K, out):
     (257, 1, 1, 0, None),       # a single expert: one 320-row tile, two of 256 rows for the recomputing GEMM
     (1024, 64, 8, 4, 1.8),      # experts of up to 1024 rows: tall tiles chosen on the device
     (700, 128, 8, 0, 1.8),
+    # the two-launch build: as many panel counts and experts as it takes, and one more of either
+    (16384, 256, 8, 0, 1.8),
+    (16385, 256, 4, 0, None),
+    (511, 257, 4, 0, None),
+    (32768, 128, 8, 2, 1.8),
+    (5000, 33, 5, 0, None),     # 64 thread slots for 33 experts, four slices of panels, 20 panels
 ])
 def test_index_bit_exact(M, N, K, Ks, skew):
     mask, _ = make_routing(M, N, K, Ks, seed=11, skew=skew)
