@@ -37,6 +37,8 @@ class MoE(nn.Module):
     def forward(self, x_BSD):
         x_BSD, mask_NM, s_NM = self.router(x_BSD, self.biases_N)
         y_BSD, sizes_N = self.momoe(x_BSD, mask_NM, s_NM)
+        if self.bias_update_rate == 0.0:  # serving: the bias stays what it was trained to
+            return y_BSD
         # under-loaded experts become easier to select, over-loaded ones harder
         B, S, _ = x_BSD.shape
         c_avg = B * S * (self.K - self.Ks) / (self.N - self.Ks)

@@ -16,6 +16,10 @@ def _logits(M, N, seed):
     (513, 200, 6, 1, True), (2048, 128, 8, 0, False),
     (77, 300, 8, 3, True),      # more than 256 experts: 8 columns per lane
     (33, 64, 3, 0, True),       # one column per lane, a partial block of tokens
+    (4096, 96, 6, 2, True),     # the most tokens with one per wavefront
+    (4097, 130, 6, 2, True),    # one more: two per wavefront, a last block of one token
+    (17, 512, 8, 1, True),      # the most experts, a last block of one token
+    (64, 8, 8, 0, True),        # every expert is chosen
 ])
 def test_router_forward(M, N, K, Ks, f32):
     from momoe_amd import _hip
@@ -44,6 +48,24 @@ def test_router_forward(M, N, K, Ks, f32):
     torch.testing.assert_close(Ng_M.cpu(), ref["Ng_M"], rtol=1e-5, atol=1e-7)
     if Ks:
         torch.testing.assert_close(Ks_M.cpu(), ref["Ks_M"], rtol=1e-5, atol=1e-7)
+
+
+def test_router_forward_takes_equal_scores_in_column_order():
+    """Whole numbers as logits (few distinct scores, the two lowest -inf through the bias) and every
+    column: of equal scores the lowest columns are taken, as a stable sort gives them."""
+    from momoe_amd import _hip
+    M, N, K = 300, 130, 8
+    lg = torch.randint(0, 3, (M, N), generator=torch.Generator().manual_seed(5)).float()
+    lg[0] = 1.0
+    bias = torch.zeros(N)
+    bias[3:] = torch.where(torch.arange(3, N) % 5 == 0, torch.tensor(0.0), torch.tensor(float("-inf")))
+    bias[40:] = float("-inf")
+    mask = _hip.router_fwd(lg.to("cuda:0"), bias.to("cuda:0"), K, 0)[0].cpu()
+    # every column's exponential is one of three values, so equal logits have equal probabilities
+    key = torch.where(torch.isinf(bias), torch.tensor(-1.0), lg)
+    want = torch.zeros(M, N, dtype=torch.int32)
+    want.scatter_(1, torch.sort(key, dim=1, descending=True, stable=True).indices[:, :K], 1)
+    assert torch.equal(mask.T, want)
 
 
 @pytest.mark.parametrize("M,N,K,Ks", [(256, 16, 4, 0), (1000, 64, 8, 4), (300, 130, 5, 2),
