@@ -43,7 +43,7 @@ struct TileCoord {
   int prow0;   // padded position of that row
   int rows;    // valid rows in this tile (1..rows per tile)
   int tn;      // column block
-  int mbase;   // first tile row owned by this wave (waves 0-3 / 4-7 split the tile's rows)
+  int mbase;   // first tile row owned by this wave (the wave rows split the tile's rows)
   int na;      // 32-row fragment rows owned by this wave (0..5)
   bool valid;
 };
@@ -56,7 +56,10 @@ struct TileCoord {
 // token rows.
 // A tile is looked up in two steps so that the table read can travel while other work runs:
 // fetch() issues the scalar loads of the workgroup's next tile, resolve() does the arithmetic.
-struct TileSched {
+// WROWS: wave rows the fragment rows of a tile are dealt to.  LIMIT: most rows the kernel takes in
+// a tile if it is less than the table may hold, else 0: tiles of a taller table are halved.
+template <int WROWS = 2, int LIMIT = 0>
+struct TileSchedT {
   static constexpr int kBandTiles = 4;
   // tile height the table was built for
   static __device__ __forceinline__ int tile_rows_of(const int* table) {
@@ -68,16 +71,18 @@ struct TileSched {
   };
   const int* table;
   int nb, bm, begin, total, chunk, xcd, pos, stride;
+  int sub;  // tiles made of one table entry
 
   // tiles before row tile `first_row_tile` (all its column blocks) are left out; a table whose
   // tiles are taller than the kernel's `max_tile_rows` yields no tiles at all
-  __device__ __forceinline__ TileSched(const int* table_, int nb_, int max_tile_rows,
-                                       int first_row_tile = 0)
+  __device__ __forceinline__ TileSchedT(const int* table_, int nb_, int max_tile_rows,
+                                        int first_row_tile = 0)
       : table(table_), nb(nb_) {
     bm = *(const int __attribute__((address_space(4)))*)(table + 1);
     const int ntiles = bm <= max_tile_rows ? *(const int __attribute__((address_space(4)))*)table : 0;
-    begin = min(first_row_tile, ntiles) * nb;
-    total = ntiles * nb;
+    sub = LIMIT > 0 && bm > LIMIT ? 2 : 1;
+    begin = min(first_row_tile, ntiles) * sub * nb;
+    total = ntiles * sub * nb;
     chunk = (total - begin + 7) >> 3;
     xcd = blockIdx.x & 7;
     pos = blockIdx.x >> 3;
@@ -91,7 +96,7 @@ struct TileSched {
     pos += stride;
     if (q >= total) return r;
     const int __attribute__((address_space(4)))* e =
-        (const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * (q / nb));
+        (const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * (q / (nb * sub)));
     r.q = q;
     r.expert = e[0];
     r.first = e[1];
@@ -108,28 +113,31 @@ struct TileSched {
     // go (the first few tiles hold one more), not full tiles plus a remainder: tiles that share
     // a weight block then take nearly equally long and stay in step, no tile streams a whole
     // weight block for a handful of rows, and only the expert's last fragment row is ragged.
-    const int nt = (r.mi + bm - 1) / bm;
-    const int nfe = (r.mi + 31) >> 5, fbase = nfe / nt, fextra = nfe - fbase * nt;
+    const int nt = (r.mi + bm - 1) / bm * sub;
+    const int nfe = (r.mi + 31) >> 5;
+    // halved tiles may outnumber the fragment rows: those left over do the last one again
+    const int ntf = LIMIT > 0 ? min(nt, nfe) : nt;
+    const int fbase = nfe / ntf, fextra = nfe - fbase * ntf;
     // Order inside an expert: bands of kBandTiles row tiles, each band crossing every column
     // block before the next band starts (row tile fastest inside a band).  The workgroups of
     // an XCD hold consecutive positions at any moment, so they share a few row tiles and a few
     // weight blocks in L2 however many rows the expert has.
-    const int qq = r.q - r.first * nb;
+    const int qq = r.q - r.first * sub * nb;
     const int band = qq / (kBandTiles * nb);
     const int in_band = qq - band * (kBandTiles * nb);
     const int band_rows = min(kBandTiles, nt - band * kBandTiles);
-    const int tl = band * kBandTiles + in_band % band_rows;
+    const int tl = min(band * kBandTiles + in_band % band_rows, ntf - 1);
     tc.tn = in_band / band_rows;
     tc.expert = r.expert;
     const int f0 = tl * fbase + min(tl, fextra);  // first fragment row of this tile
     tc.row0 = r.rstart + 32 * f0;
     tc.prow0 = padded_start(r.rstart, r.expert) + 32 * f0;
     tc.rows = min(32 * (fbase + (tl < fextra ? 1 : 0)), r.mi - 32 * f0);
-    // the tile's fragment rows are dealt to the two wave rows as evenly as possible
-    const int nf = (tc.rows + 31) >> 5, half = (nf + 1) >> 1;
-    const bool upper = wave_id() >= kWaves / 2;
-    tc.mbase = upper ? 32 * half : 0;
-    tc.na = upper ? nf - half : half;
+    // the tile's fragment rows are dealt to the wave rows as evenly as possible
+    const int nf = (tc.rows + 31) >> 5, wr = wave_id() / (kWaves / WROWS);
+    const int wbase = nf / WROWS, wextra = nf - wbase * WROWS;
+    tc.mbase = 32 * (wr * wbase + min(wr, wextra));
+    tc.na = wbase + (wr < wextra ? 1 : 0);
     return tc;
   }
   __device__ __forceinline__ TileCoord next() { return resolve(fetch()); }
@@ -148,6 +156,7 @@ struct TileSched {
     return *(const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * lo + 1);
   }
 };
+using TileSched = TileSchedT<>;
 
 __device__ __forceinline__ float bf2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }

@@ -9,10 +9,9 @@
 namespace momoe {
 namespace {
 
-// Both data-gradient GEMMs hold both row-tile geometries and follow the tile table they are given.
-constexpr int BN = 256;
-constexpr int FN = 2;    // 2x4 waves, each (32 * FM) rows x 64 columns
-using RowsB = RDma<BN>;  // weight rows, k-contiguous (the "NT" GEMMs of the data gradients)
+// Both data-gradient GEMMs hold both tall and standard row tiles and follow the tile table they are
+// given; launches with few tiles take narrow ones (takes_narrow_tiles).
+constexpr int FN = 2;  // 2x4 (4x2) waves, each (32 * FM) rows x 64 columns
 
 struct DhArgs {
   const bf16* gy;
@@ -27,8 +26,9 @@ struct DhArgs {
 // u = G_y[idx] . Wl2^T is an "NT" GEMM: both operands are k-contiguous (k = D).
 template <class G>
 struct DhProg {
-  static constexpr int FM = G::FM;
+  static constexpr int FM = G::FM, BN = G::COLS;
   using RowsA = RDma<G::AROWS>;  // gathered token rows, k-contiguous
+  using RowsB = RDma<BN>;        // weight rows, k-contiguous (an "NT" GEMM)
   using Ring = StageRing<RowsA, RowsB, G::STAGES>;  // its idle buffer is the store staging
   struct Prep {
     int32_t tok[RowsA::NCH];  // tokens of the rows this lane fetches
@@ -70,12 +70,12 @@ struct DhProg {
   }
 };
 
-template <class G>
+template <class G, class Sched = TileSched>
 __device__ __forceinline__ void dgrad_h_tiles(const DhArgs& p) {
   using Prog = DhProg<G>;
   typename Prog::Ring ring(dyn_lds());
-  TileSched sched(p.table, (p.H + BN - 1) / BN, G::MAX_ROWS);
-  const int wn = wave_id() & 3;
+  Sched sched(p.table, (p.H + G::COLS - 1) / G::COLS, MOMOE_TILE_ROWS);
+  const int wn = wave_id() % G::WCOLS;
   const int n_org[FN] = {wn * 64, wn * 64 + 32};
   Prog prog{p, p.D / kBK, wn};
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
@@ -87,6 +87,12 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
   else dgrad_h_tiles<StdTiles>(p);
   trace.finish();
 }
+__global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
+  const ClockTrace trace(p.clk);
+  dgrad_h_tiles<NarrowTiles, NarrowSched>(p);
+  trace.finish();
+}
+constexpr size_t kDhNarrowLds = DhProg<NarrowTiles>::Ring::BYTES;
 constexpr size_t kDhLds = std::max(DhProg<TallTiles>::Ring::BYTES, DhProg<StdTiles>::Ring::BYTES);
 
 // SwiGLU backward for the sorted rows whose a|b were saved by the forward.  One workgroup per
@@ -206,8 +212,9 @@ struct DxArgs {
 // gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
 template <class G>
 struct DxProg {
-  static constexpr int FM = G::FM;
+  static constexpr int FM = G::FM, BN = G::COLS;
   using BlockedA = RBlockedDma<G::AROWS>;  // sorted rows of the k-blocked gz
+  using RowsB = RDma<BN>;                  // weight rows, k-contiguous
   using Ring = StageRing<BlockedA, RowsB, G::STAGES>;
   struct Prep {};
   const DxArgs& p;
@@ -244,12 +251,12 @@ struct DxProg {
   }
 };
 
-template <class G>
+template <class G, class Sched = TileSched>
 __device__ __forceinline__ void dgrad_x_tiles(const DxArgs& p) {
   using Prog = DxProg<G>;
   typename Prog::Ring ring(dyn_lds());
-  TileSched sched(p.table, (p.D + BN - 1) / BN, G::MAX_ROWS);
-  const int wn = wave_id() & 3;
+  Sched sched(p.table, (p.D + G::COLS - 1) / G::COLS, MOMOE_TILE_ROWS);
+  const int wn = wave_id() % G::WCOLS;
   const int n_org[FN] = {wn * 64, wn * 64 + 32};
   Prog prog{p, (2 * p.H) / kBK, wn};
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
@@ -261,6 +268,12 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
   else dgrad_x_tiles<StdTiles>(p);
   trace.finish();
 }
+__global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
+  const ClockTrace trace(p.clk);
+  dgrad_x_tiles<NarrowTiles, NarrowSched>(p);
+  trace.finish();
+}
+constexpr size_t kDxNarrowLds = DxProg<NarrowTiles>::Ring::BYTES;
 constexpr size_t kDxLds = std::max(DxProg<TallTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
 
 // dL/ds [N][M] from the partial row sums in sorted order.  One workgroup per (expert, kGsTokens
@@ -325,6 +338,12 @@ extern "C" int momoe_dgrad_h(const void* Gy_MD, const void* Wl2_NHD, const int32
   if (st != MOMOE_OK) return st;
   DhArgs a{(const bf16*)Gy_MD, (const bf16*)Wl2_NHD, idx_Msum, tile_table, (bf16*)u_MsumH, (int)D,
            (int)H, clock_trace_buffer()};
+  if (takes_narrow_tiles(Msum, N, H)) {
+    static LdsLimit narrow;
+    if (!allow_lds(dgrad_h_narrow_kernel, kDhNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    dgrad_h_narrow_kernel<<<persistent_grid(), kThreads, kDhNarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   static LdsLimit lds;
   if (!allow_lds(dgrad_h_kernel, kDhLds, lds)) return MOMOE_ERR_LAUNCH;
   dgrad_h_kernel<<<persistent_grid(), kThreads, kDhLds, (hipStream_t)stream>>>(a);
@@ -380,6 +399,12 @@ extern "C" int momoe_dgrad_x(const void* gz_blocked, const void* Wl1_ND2H,
   if (st != MOMOE_OK) return st;
   DxArgs a{(const bf16*)gz_blocked, (const bf16*)Wl1_ND2H, tile_table, (bf16*)gxs_MsumD, (int)D,
            (int)H, Msum, clock_trace_buffer()};
+  if (takes_narrow_tiles(Msum, N, D)) {
+    static LdsLimit narrow;
+    if (!allow_lds(dgrad_x_narrow_kernel, kDxNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    dgrad_x_narrow_kernel<<<persistent_grid(), kThreads, kDxNarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   static LdsLimit lds;
   if (!allow_lds(dgrad_x_kernel, kDxLds, lds)) return MOMOE_ERR_LAUNCH;
   dgrad_x_kernel<<<persistent_grid(), kThreads, kDxLds, (hipStream_t)stream>>>(a);

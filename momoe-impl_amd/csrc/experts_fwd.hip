@@ -8,9 +8,7 @@
 namespace momoe {
 namespace {
 
-constexpr int BN = 256;  // GEMM columns per tile
-constexpr int FN = 2;    // 2x4 waves, each (32 * FM) rows x 64 columns
-using WeightOp = TDma;   // expert weights [k][col], k-strided
+constexpr int FN = 2;  // 2x4 (4x2) waves, each (32 * FM) rows x 64 columns
 
 struct Lin1Args {
   const bf16* x;
@@ -33,7 +31,7 @@ struct Lin1Args {
   unsigned long long* clk;
 };
 
-// Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns); a wave owns 32 `a`
+// Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave owns 32 `a`
 // columns and their 32 `b` columns, so the SwiGLU product pairs registers of the same lane.
 // BWD = false: forward / recomputation, writes h and/or a|b.  BWD = true: the a|b of the tile
 // stay in registers and go straight into the SwiGLU backward.
@@ -42,12 +40,13 @@ struct Lin1Args {
 template <bool BWD, class G>
 struct Lin1Prog {
   static_assert(!BWD || std::is_same_v<G, StdTiles>, "the SwiGLU backward epilogue fits 256-row tiles only");
-  static constexpr int FM = G::FM, BM = G::MAX_ROWS;
+  static constexpr int FM = G::FM, BM = G::MAX_ROWS, BN = G::COLS;
   using RowsOp = RDma<G::AROWS>;  // token rows, k-contiguous
+  using WeightOp = TDmaT<BN>;     // expert weights [k][col], k-strided
   using Ring = StageRing<RowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   static constexpr int BNH = BN / 2;
-  static_assert(BNH == MOMOE_GS_BLOCK, "gs_part blocks follow the hidden-column tile");
+  static_assert(!BWD || BNH == MOMOE_GS_BLOCK, "gs_part blocks follow the hidden-column tile");
   static_assert(4 * BM * sizeof(float) <= kEpilogueLds, "the dL/ds row sums reuse the staging area");
   struct Prep {
     int32_t tok[RowsOp::NCH];  // tokens of the rows this lane fetches
@@ -248,7 +247,7 @@ struct Lin1Prog {
   }
 };
 
-template <bool BWD, class G>
+template <bool BWD, class G, class Sched = TileSched>
 __device__ __forceinline__ void lin1_swiglu_tiles(const Lin1Args& p) {
   using Prog = Lin1Prog<BWD, G>;
   using Ring = typename Prog::Ring;
@@ -256,9 +255,9 @@ __device__ __forceinline__ void lin1_swiglu_tiles(const Lin1Args& p) {
   Ring ring(dyn_lds());
   // without an h output only rows >= ab_lo are wanted: experts entirely below are skipped
   const int first_tile =
-      p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
-  TileSched sched(p.table, (p.H + Prog::BNH - 1) / Prog::BNH, Prog::BM, first_tile);
-  const int wn = wave_id() & 3;
+      p.h == nullptr && p.ab_lo > 0 ? Sched::expert_tile_of_row(p.table, p.ab_lo) : 0;
+  Sched sched(p.table, (p.H + Prog::BNH - 1) / Prog::BNH, BWD ? Prog::BM : MOMOE_TILE_ROWS, first_tile);
+  const int wn = wave_id() % G::WCOLS;
   const int n_org[FN] = {wn * 32, Prog::BNH + wn * 32};
   Prog prog{p, p.D / kBK, wn};
   run_row_tiles<FM, FN>(prog, sched, ring, n_org);
@@ -276,6 +275,12 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_kernel(Lin1Args p) {
   }
   trace.finish();
 }
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  lin1_swiglu_tiles<false, NarrowTiles, NarrowSched>(p);
+  trace.finish();
+}
+constexpr size_t kLin1NarrowLds = Lin1Prog<false, NarrowTiles>::kLds;
 constexpr size_t kLin1FwdLds = std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, StdTiles>::kLds);
 constexpr size_t kLin1BwdLds = Lin1Prog<true, StdTiles>::kLds;
 
@@ -294,8 +299,9 @@ struct Lin2Args {
 
 template <class G>
 struct Lin2Prog {
-  static constexpr int FM = G::FM;
+  static constexpr int FM = G::FM, BN = G::COLS;
   using HRowsOp = RBlockedDma<G::AROWS>;  // rows of h, k-blocked
+  using WeightOp = TDmaT<BN>;             // expert weights [k][col], k-strided
   using Ring = StageRing<HRowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   struct Prep {
@@ -343,12 +349,12 @@ struct Lin2Prog {
   }
 };
 
-template <class G>
+template <class G, class Sched = TileSched>
 __device__ __forceinline__ void lin2_scale_tiles(const Lin2Args& p) {
   using Prog = Lin2Prog<G>;
   typename Prog::Ring ring(dyn_lds());
-  TileSched sched(p.table, (p.D + BN - 1) / BN, G::MAX_ROWS);
-  const int wn = wave_id() & 3;
+  Sched sched(p.table, (p.D + G::COLS - 1) / G::COLS, MOMOE_TILE_ROWS);
+  const int wn = wave_id() % G::WCOLS;
   const int n_org[FN] = {wn * 64, wn * 64 + 32};
   Prog prog{p, p.H / kBK, wn};
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
@@ -360,6 +366,12 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
   else lin2_scale_tiles<StdTiles>(p);
   trace.finish();
 }
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
+  const ClockTrace trace(p.clk);
+  lin2_scale_tiles<NarrowTiles, NarrowSched>(p);
+  trace.finish();
+}
+constexpr size_t kLin2NarrowLds = Lin2Prog<NarrowTiles>::kLds;
 constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<StdTiles>::kLds);
 
 // out[m] = sum_k rows[inv[m,k]]: one workgroup per token, 16-byte loads, fp32 accumulate.
@@ -427,6 +439,12 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
   Lin1Args a{(const bf16*)x_MD, (const bf16*)Wl1_ND2H, idx_Msum, tile_table, (bf16*)h_blocked,
              (bf16*)ab_rows, ab_row_lo, ab_row_hi, (int)D, (int)H,
              nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, Msum, clock_trace_buffer()};
+  if (takes_narrow_tiles(Msum, N, 2 * H)) {
+    static LdsLimit narrow;
+    if (!allow_lds(lin1_swiglu_narrow_kernel, kLin1NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    lin1_swiglu_narrow_kernel<<<persistent_grid(), kThreads, kLin1NarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   static LdsLimit lds;
   if (!allow_lds(lin1_swiglu_kernel<false>, kLin1FwdLds, lds)) return MOMOE_ERR_LAUNCH;
   lin1_swiglu_kernel<false><<<persistent_grid(), kThreads, kLin1FwdLds, (hipStream_t)stream>>>(a);
@@ -472,6 +490,12 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
   if (st != MOMOE_OK) return st;
   Lin2Args a{(const bf16*)h_blocked, (const bf16*)Wl2_NHD, s_NM, s_stride_n, s_stride_m,
              idx_Msum, tile_table, (bf16*)ys_MsumD, (int)D, (int)H, Msum, clock_trace_buffer()};
+  if (takes_narrow_tiles(Msum, N, D)) {
+    static LdsLimit narrow;
+    if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    lin2_scale_narrow_kernel<<<persistent_grid(), kThreads, kLin2NarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   static LdsLimit lds;
   if (!allow_lds(lin2_scale_kernel, kLin2Lds, lds)) return MOMOE_ERR_LAUNCH;
   lin2_scale_kernel<<<persistent_grid(), kThreads, kLin2Lds, (hipStream_t)stream>>>(a);

@@ -62,6 +62,7 @@
 // column 8*(r/4) + 4*(lane/32) + r%4.  Row-wise epilogues (per-row scale,
 // SwiGLU pairing, row reductions) are then lane-local and stores are 8-byte.
 #pragma once
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -191,24 +192,32 @@ struct RBlockedDma {
   static __device__ __forceinline__ bf16x8 frag(const bf16* stage, int r0, int kk) { return R::frag(stage, r0, kk); }
 };
 
-// ---- k-strided operand, 256 columns -----------------------------------------------------
+// ---- k-strided operand, 256 (128) columns -----------------------------------------------------
 // LDS stage: k-row k at elements [256k, 256k+256); 16-byte piece p of the row is stored
 // at position p ^ swz(k), swz(k) = 4*(k&3) + 16*((k>>3)&1): the 8 k-rows x 64 bytes that one
 // transpose read of a wave touches then fall into 8 different 64-byte bank groups (measured
 // 124 B/clk against 113 for a swizzle that only separates the 4 k-rows of a 16-lane group;
 // the instruction tops out at 128).  A deposit covers two k-rows (lanes 0-31 / 32-63); wave w
 // deposits k-rows [4w, 4w+4).
-struct TLayout {
-  static constexpr int COLS = 256;
-  static constexpr int NCH = kBK / (2 * kWaves);  // deposits per wave per stage
+// With 128 columns (256-byte k-rows) a deposit covers four k-rows, two consecutive k-rows fill
+// what one fills above, and swz(k) = 4*((k>>1)&1) + 8*((k>>3)&1) separates the eight.
+template <int COLS_>
+struct TLayoutT {
+  static constexpr int COLS = COLS_;
+  static_assert(COLS == 256 || COLS == 128, "swizzles written for these");
+  static constexpr int PIECES = COLS / 8;                    // 16-byte pieces of a k-row
+  static constexpr int RPD = 64 / PIECES;                    // k-rows of a deposit
+  static constexpr int NCH = kBK / (RPD * kWaves);           // deposits per wave per stage
   static constexpr int LDS_ELEMS = kBK * COLS;
-  static __device__ __forceinline__ int swz(int krow) { return 4 * (krow & 3) + 16 * ((krow >> 3) & 1); }
+  static __device__ __forceinline__ int swz(int krow) {
+    return COLS == 256 ? 4 * (krow & 3) + 16 * ((krow >> 3) & 1) : 4 * ((krow >> 1) & 1) + 8 * ((krow >> 3) & 1);
+  }
 
   // k-row and logical column (multiple of 8) fetched by this lane in deposit j
   static __device__ __forceinline__ void lane_piece(int j, int& krow, int& col) {
     const int l = threadIdx.x & 63, w = wave_id();
-    krow = w * (2 * NCH) + j * 2 + (l >> 5);
-    col = ((l & 31) ^ swz(krow)) * 8;
+    krow = w * (RPD * NCH) + j * RPD + l / PIECES;
+    col = ((l & (PIECES - 1)) ^ swz(krow)) * 8;
   }
   static __device__ __forceinline__ uint32_t deposit(uint32_t stage, int j) {
     return stage + (wave_id() * NCH + j) * (kChunkElems * 2);
@@ -226,9 +235,12 @@ struct TLayout {
   }
 };
 
+using TLayout = TLayoutT<256>;
+
 // k-strided operand with a fixed pitch between k-rows (the expert weights)
-struct TDma {
-  using L = TLayout;
+template <int COLS>
+struct TDmaT {
+  using L = TLayoutT<COLS>;
   static constexpr int NCH = L::NCH;
   static constexpr int LDS_ELEMS = L::LDS_ELEMS;
   const bf16* base;   // wave-uniform
@@ -260,6 +272,8 @@ struct TDma {
     return L::frag(stage, c0, kk);
   }
 };
+
+using TDma = TDmaT<256>;
 
 // k-strided operand whose k-rows are the sorted rows [row_begin,row_end) of one expert,
 // optionally gathered through an index.  k-rows past row_end are pointed at the expert's last
@@ -366,6 +380,10 @@ struct TGatherDmaT {
     return L::frag(stage, c0, kk);
   }
 };
+// LDS the epilogues stage their stores in (RowStager below): 4 KiB per wave
+constexpr int kStageBytesPerWave = 32 * 64 * 2;                  // NF = 2
+constexpr size_t kEpilogueLds = (size_t)kWaves * kStageBytesPerWave;
+
 // ---- the k-loop -----------------------------------------------------------------------------
 // Ring of NS LDS stage buffers; `head` is the buffer of stage 0 of the current tile and is
 // carried from tile to tile by a persistent workgroup.  FIRST = NS - 1 stages of a tile are
@@ -379,7 +397,9 @@ struct StageRing {
   using B = BOp;
   static constexpr int STAGES = NS, FIRST = NS - 1;
   static constexpr int STAGE = AOp::LDS_ELEMS + BOp::LDS_ELEMS;
-  static constexpr size_t BYTES = (size_t)NS * STAGE * sizeof(bf16);
+  // the epilogues' store staging: the idle stage buffer, or LDS of its own where that is too small
+  static constexpr bool kStagingInRing = STAGE * sizeof(bf16) >= kEpilogueLds;
+  static constexpr size_t BYTES = (size_t)NS * STAGE * sizeof(bf16) + (kStagingInRing ? 0 : kEpilogueLds);
   bf16* lds;
   uint32_t addr;  // LDS byte address of `lds`
   int head;
@@ -545,13 +565,15 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
   ring.advance(ktiles);
 }
 
-// Row-tile geometry of a kernel: two wave rows of FM 32-row fragment rows each (tiles of up to
-// 64 * FM rows, 64 columns per wave), the rows of the row operand's stage buffer (whole deposits
+// Row-tile geometry of a kernel: WROWS wave rows of FM 32-row fragment rows each (tiles of up to
+// 32 * WROWS * FM rows, 64 columns per wave), the rows of the row operand's stage buffer (whole deposits
 // of 16 rows per wave, so a multiple of 128 that holds the tallest tile) and the ring depth.
-template <int FM_, int NS_>
+template <int FM_, int NS_, int WROWS_ = 2>
 struct RowTileGeometry {
   static constexpr int FM = FM_, FN = 2;
-  static constexpr int MAX_ROWS = 64 * FM;
+  static constexpr int WROWS = WROWS_, WCOLS = kWaves / WROWS;  // the waves' arrangement
+  static constexpr int COLS = 64 * WCOLS;
+  static constexpr int MAX_ROWS = 32 * FM * WROWS;
   static constexpr int AROWS = (MAX_ROWS + 127) / 128 * 128;
   static constexpr int STAGES = NS_;
 };
@@ -564,6 +586,16 @@ using StdTiles = RowTileGeometry<4, 4>;
 // repeat the tile's last row; four such stages are all of the CU's LDS (the epilogues stage
 // their stores in the ring's idle buffer)
 using TallTiles = RowTileGeometry<5, 4>;
+// 256 rows x 128 columns, waves 4 x 2, for launches whose 256-column tiles would leave at least half
+// of the CUs without one: such a launch takes as long as one CU needs to pull one tile's operands
+// out of L2, and half the columns are twice the CUs.  Sums run over k in the same order: results are
+// bit-identical to the other geometries'.
+// Measured, 256 -> 128 columns, us: 1024 tokens over 32 experts with D = 1024, H = 512: x.Wl1 23.5 ->
+// 18.9, h.Wl2 15.5 -> 13.0, dL/dh 20.6 -> 15.3, dL/dx 22.5 -> 17.8; one token, 8 experts of D = 2048,
+// H = 768: x.Wl1 20.0 -> 16.6, h.Wl2 10.8 -> 9.1.  A fifth stage, or half the row deposits for calls of
+// few tokens, changed nothing.
+using NarrowTiles = RowTileGeometry<2, 4, 4>;
+using NarrowSched = TileSchedT<NarrowTiles::WROWS, NarrowTiles::MAX_ROWS>;
 static_assert(TallTiles::MAX_ROWS == MOMOE_TILE_ROWS && StdTiles::MAX_ROWS == MOMOE_RECOMPUTE_TILE_ROWS,
               "tile heights promised by the header");
 
@@ -572,7 +604,7 @@ template <class AOp, class BOp, int NS, int FM, int FN, class Hook>
 __device__ __forceinline__ void gemm_rows(AOp& A, BOp& B, f32x16 (&acc)[FN][FM], int ktiles,
                                           StageRing<AOp, BOp, NS>& ring, const int (&m_org)[FM],
                                           const int (&n_org)[FN], int na_, Hook hook) {
-  static_assert(FM == 4 || FM == 5, "dispatch written for 4 or 5 fragment rows per wave");
+  static_assert(FM == 2 || FM == 4 || FM == 5, "dispatch written for 2, 4 or 5 fragment rows per wave");
   const int na = __builtin_amdgcn_readfirstlane(na_);
   if constexpr (FM == 5) {
     if (na == 5) {
@@ -580,9 +612,17 @@ __device__ __forceinline__ void gemm_rows(AOp& A, BOp& B, f32x16 (&acc)[FN][FM],
       return;
     }
   }
-  if (na == 4) gemm_mainloop<AOp, BOp, NS, FM, FN, 4>(A, B, acc, ktiles, ring, m_org, n_org, hook);
-  else if (na == 3) gemm_mainloop<AOp, BOp, NS, FM, FN, 3>(A, B, acc, ktiles, ring, m_org, n_org, hook);
-  else if (na == 2) gemm_mainloop<AOp, BOp, NS, FM, FN, 2>(A, B, acc, ktiles, ring, m_org, n_org, hook);
+  if constexpr (FM >= 4) {
+    if (na == 4) {
+      gemm_mainloop<AOp, BOp, NS, FM, FN, 4>(A, B, acc, ktiles, ring, m_org, n_org, hook);
+      return;
+    }
+    if (na == 3) {
+      gemm_mainloop<AOp, BOp, NS, FM, FN, 3>(A, B, acc, ktiles, ring, m_org, n_org, hook);
+      return;
+    }
+  }
+  if (na == 2) gemm_mainloop<AOp, BOp, NS, FM, FN, 2>(A, B, acc, ktiles, ring, m_org, n_org, hook);
   else if (na == 1) gemm_mainloop<AOp, BOp, NS, FM, FN, 1>(A, B, acc, ktiles, ring, m_org, n_org, hook);
   else gemm_mainloop<AOp, BOp, NS, FM, FN, 0>(A, B, acc, ktiles, ring, m_org, n_org, hook);
 }
@@ -626,6 +666,14 @@ inline int persistent_grid() {
   return (cus + 7) / 8 * 8;
 }
 
+// Whether a launch over `cols` output columns takes NarrowTiles: with them there is still no more
+// than one tile per CU.  The routing is not known here; its row tiles are taken as if every expert
+// held a quarter more than its share (an estimate off the mark costs speed only).
+inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
+  const int64_t row_tiles = std::min(n, msum) * std::max<int64_t>(1, cdiv64(5 * msum, 4 * n * StdTiles::MAX_ROWS));
+  return 2 * row_tiles * cdiv64(cols, StdTiles::COLS) <= persistent_grid();
+}
+
 template <int FM, int FN>
 __device__ __forceinline__ void zero_acc(f32x16 (&acc)[FN][FM]) {
 #pragma unroll
@@ -648,10 +696,6 @@ __device__ __forceinline__ void store_bf16x4(bf16* p, float a, float b, float c,
   *(bf16x4*)p = pack_bf16x4(a, b, c, d);
 }
 
-// LDS the epilogues stage their stores in (RowStager below): 4 KiB per wave
-constexpr int kStageBytesPerWave = 32 * 64 * 2;                  // NF = 2
-constexpr size_t kEpilogueLds = (size_t)kWaves * kStageBytesPerWave;
-
 // ---- persistent tile loop ------------------------------------------------------------------------
 // Drives a workgroup through its (row tile, column block) pairs with everything a tile needs
 // from memory requested one tile ahead.  The tile program P supplies
@@ -666,10 +710,10 @@ constexpr size_t kEpilogueLds = (size_t)kWaves * kStageBytesPerWave;
 // While tile t is multiplied: the table entry of tile t+2 and the gathered values of tile t+1
 // are in flight; after its main loop the first stages of tile t+1 are requested, then the
 // epilogue of tile t runs.
-template <int FM, int FN, class P, class AOp, class BOp, int NS>
-__device__ __forceinline__ void run_row_tiles(P& prog, TileSched& sched, StageRing<AOp, BOp, NS>& ring,
+template <int FM, int FN, class P, class Sched, class AOp, class BOp, int NS>
+__device__ __forceinline__ void run_row_tiles(P& prog, Sched& sched, StageRing<AOp, BOp, NS>& ring,
                                               const int (&n_org)[FN]) {
-  static_assert(StageRing<AOp, BOp, NS>::STAGE * sizeof(bf16) >= kEpilogueLds, "a stage buffer holds the store staging");
+  using Ring = StageRing<AOp, BOp, NS>;
   TileCoord c0 = sched.next();
   if (!c0.valid) return;
   TileCoord c1 = sched.next();
@@ -683,7 +727,7 @@ __device__ __forceinline__ void run_row_tiles(P& prog, TileSched& sched, StageRi
   while (true) {
     f32x16 acc[FN][FM];
     zero_acc<FM, FN>(acc);
-    TileSched::Raw rn;
+    typename Sched::Raw rn;
     int m_org[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) m_org[i] = c0.mbase + 32 * i;
@@ -700,7 +744,7 @@ __device__ __forceinline__ void run_row_tiles(P& prog, TileSched& sched, StageRi
     // last stage out of it
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();
-    prog.epilogue(c0, acc, p0, ring.free_buf());
+    prog.epilogue(c0, acc, p0, Ring::kStagingInRing ? ring.free_buf() : ring.lds + NS * Ring::STAGE);
     if (!c1.valid) break;
     c0 = c1;
     p0 = p1;

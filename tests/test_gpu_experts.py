@@ -81,6 +81,29 @@ def test_random_small_shapes(seed):
         assert torch.equal(tall[k], dev[k]), k
 
 
+@pytest.mark.parametrize("M,D,H,N,K,sp", [
+    (2000, 352, 288, 72, 3, 0),     # too many tiles for narrow ones: every GEMM takes the wide ones
+    (1100, 800, 416, 16, 4, 40),    # 275 rows per expert: narrow tiles of halved 320-row ones
+    (1, 2048, 768, 128, 8, 0),      # one token
+    (640, 1056, 544, 20, 2, 0),     # narrow, column counts one fragment past a tile, 64 rows
+    (1300, 160, 1056, 24, 4, 100),  # x.Wl1 wide, the products over D columns narrow
+])
+def test_wide_and_narrow_tiles(M, D, H, N, K, sp):
+    from momoe_amd import _hip, experts
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=3)
+    dev = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+    _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
+    # any tile height gives the same sums: halved 320-row tiles, tiles of one fragment row
+    for rows in (_hip.TILE_ROWS, 32):
+        try:
+            experts.TILE_ROWS = rows
+            other = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+        finally:
+            experts.TILE_ROWS = _hip.AUTO_TILE_ROWS
+        for k in dev:
+            assert torch.equal(other[k], dev[k]), (rows, k)
+
+
 @pytest.mark.parametrize("gather_a", [True, False])
 def test_weight_gradient_of_cut_experts(gather_a):
     # experts of 20000 / 3 / 0 / 5000 rows: the first is contracted in pieces that meet in the
