@@ -280,6 +280,35 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Arg
   lin1_swiglu_tiles<false, NarrowTiles, NarrowSched>(p);
   trace.finish();
 }
+
+// The few-row tiles (FewRows): its own operands and loop, the epilogue of the narrow ones.
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p) {
+  using Prog = Lin1Prog<false, FewRows::G>;
+  const ClockTrace trace(p.clk);
+  bf16* lds = dyn_lds();
+  const int first_tile = p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
+  TileSched sched(p.table, (p.H + Prog::BNH - 1) / Prog::BNH, MOMOE_TILE_ROWS, first_tile);
+  const int n_org[FN] = {0, Prog::BNH};
+  const Prog prog{p, 0, 0};
+  const int D = p.D, H = p.H;
+  FewRows op;
+  for (TileCoord t = sched.next(); t.valid; t = sched.next()) {
+    t.mbase = 0;
+    t.na = 1;
+    op.rows(p.x, FewRows::BK, D, [&](int row, int piece) {
+      return (uint32_t)p.idx[t.row0 + min(row, t.rows - 1)] * (uint32_t)(2 * D) + piece * 16;
+    });
+    const int j0 = t.tn * Prog::BNH;
+    op.weights(p.w1 + (int64_t)t.expert * D * 2 * H, D,
+               [&](int c) { return (c / Prog::BNH) * H + min(j0 + (c % Prog::BNH), H - 8); }, 2 * H);
+    f32x16 acc[FN][1];
+    __builtin_amdgcn_s_barrier();  // the previous tile's partial sums have been read
+    op.multiply(acc, lds, D, n_org);
+    if (wave_id() == 0) prog.epilogue_fwd(t, acc, FewRows::staging(lds));
+    wait_lgkm0();
+  }
+  trace.finish();
+}
 constexpr size_t kLin1NarrowLds = Lin1Prog<false, NarrowTiles>::kLds;
 constexpr size_t kLin1FwdLds = std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, StdTiles>::kLds);
 constexpr size_t kLin1BwdLds = Lin1Prog<true, StdTiles>::kLds;
@@ -371,6 +400,37 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args
   lin2_scale_tiles<NarrowTiles, NarrowSched>(p);
   trace.finish();
 }
+
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
+  using Prog = Lin2Prog<FewRows::G>;
+  const ClockTrace trace(p.clk);
+  bf16* lds = dyn_lds();
+  TileSched sched(p.table, (p.D + FewRows::G::COLS - 1) / FewRows::G::COLS, MOMOE_TILE_ROWS);
+  const int n_org[FN] = {0, 32};
+  const Prog prog{p, 0, 0};
+  const int D = p.D, H = p.H;
+  FewRows op;
+  for (TileCoord t = sched.next(); t.valid; t = sched.next()) {
+    t.mbase = 0;
+    t.na = 1;
+    Prog::Prep prep;
+    prog.gather(t, prep);
+    // h is k-blocked: a stage is four blocks of 32 k-values
+    const uint32_t block = (uint32_t)p.msum * (kBK * 2);
+    op.rows(p.h + (int64_t)t.row0 * kBK, 4 * p.msum * kBK, H, [&](int row, int piece) {
+      return (uint32_t)min(row, t.rows - 1) * (kBK * 2) + (piece >> 2) * block + (piece & 3) * 16;
+    });
+    const int d0 = t.tn * FewRows::G::COLS;
+    op.weights(p.w2 + (int64_t)t.expert * H * D, H, [&](int c) { return min(d0 + c, D - 8); }, D);
+    prog.late(t, prep);
+    f32x16 acc[FN][1];
+    __builtin_amdgcn_s_barrier();  // the previous tile's partial sums have been read
+    op.multiply(acc, lds, H, n_org);
+    if (wave_id() == 0) prog.epilogue(t, acc, prep, FewRows::staging(lds));
+    wait_lgkm0();
+  }
+  trace.finish();
+}
 constexpr size_t kLin2NarrowLds = Lin2Prog<NarrowTiles>::kLds;
 constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<StdTiles>::kLds);
 
@@ -439,6 +499,12 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
   Lin1Args a{(const bf16*)x_MD, (const bf16*)Wl1_ND2H, idx_Msum, tile_table, (bf16*)h_blocked,
              (bf16*)ab_rows, ab_row_lo, ab_row_hi, (int)D, (int)H,
              nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, Msum, clock_trace_buffer()};
+  if (takes_few_rows_tiles(M, Msum, N, 2 * H)) {
+    static LdsLimit few;
+    if (!allow_lds(lin1_swiglu_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
+    lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   if (takes_narrow_tiles(Msum, N, 2 * H)) {
     static LdsLimit narrow;
     if (!allow_lds(lin1_swiglu_narrow_kernel, kLin1NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
@@ -490,6 +556,12 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
   if (st != MOMOE_OK) return st;
   Lin2Args a{(const bf16*)h_blocked, (const bf16*)Wl2_NHD, s_NM, s_stride_n, s_stride_m,
              idx_Msum, tile_table, (bf16*)ys_MsumD, (int)D, (int)H, Msum, clock_trace_buffer()};
+  if (takes_few_rows_tiles(M, Msum, N, D)) {
+    static LdsLimit few;
+    if (!allow_lds(lin2_scale_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
+    lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
   if (takes_narrow_tiles(Msum, N, D)) {
     static LdsLimit narrow;
     if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;

@@ -204,13 +204,14 @@ struct RBlockedDma {
 template <int COLS_>
 struct TLayoutT {
   static constexpr int COLS = COLS_;
-  static_assert(COLS == 256 || COLS == 128, "swizzles written for these");
+  static_assert(COLS == 256 || COLS == 128 || COLS == 64, "swizzles written for these");
   static constexpr int PIECES = COLS / 8;                    // 16-byte pieces of a k-row
   static constexpr int RPD = 64 / PIECES;                    // k-rows of a deposit
   static constexpr int NCH = kBK / (RPD * kWaves);           // deposits per wave per stage
   static constexpr int LDS_ELEMS = kBK * COLS;
   static __device__ __forceinline__ int swz(int krow) {
-    return COLS == 256 ? 4 * (krow & 3) + 16 * ((krow >> 3) & 1) : 4 * ((krow >> 1) & 1) + 8 * ((krow >> 3) & 1);
+    if (COLS == 256) return 4 * (krow & 3) + 16 * ((krow >> 3) & 1);
+    return COLS == 128 ? 4 * ((krow >> 1) & 1) + 8 * ((krow >> 3) & 1) : 4 * ((krow >> 3) & 1);
   }
 
   // k-row and logical column (multiple of 8) fetched by this lane in deposit j
@@ -810,5 +811,127 @@ struct RowStager {
     }
   }
 };
+
+// ---- few rows: the waves share the contraction --------------------------------------------------
+// Tiles of at most 32 rows x 64 columns for the forward of calls with at most 32 tokens (no expert
+// holds more) that still have no more than one such tile per CU.  One CU pulls weights from HBM at 46
+// GB/s at most, so a call of a few experts takes as long as the CUs it uses are few, and 64
+// columns give it twice those of NarrowTiles.  To keep as many bytes on the way, a stage holds 128
+// k-values; wave w multiplies the 16 of slice w with all columns, nothing but the fragment reads
+// lies between two barriers, and the eight slices' sums meet in LDS at the end of the tile.
+// Measured against NarrowTiles, weights not in any cache: one token, 8 experts of D = 2048, H = 768: the
+// forward 35.0 -> 30.8 us; with the weights cached x.Wl1 16.6 -> 13.5 us, h.Wl2 9.1 -> 9.9 (launch and
+// the chain table -> row ids -> rows are most of both).  64 x 128 tiles with half the k-values a
+// stage took 14.8 and 9.8.  With more than one tile per CU the gap between two tiles, in which
+// nothing is on the way, would cost what the CUs gain.
+struct FewRows {
+  static constexpr int ROWS = 32, BK = 128, STAGES = 5;
+  using G = RowTileGeometry<1, 4, 8>;  // 64 columns and the accumulators of one wave, for the epilogues
+  using W = TLayoutT<G::COLS>;         // its swizzle and fragment reads hold for 128 k-rows as for 32
+  static constexpr int FN = G::FN;
+  static constexpr int A_ELEMS = ROWS * BK, W_ELEMS = BK * G::COLS, STAGE = A_ELEMS + W_ELEMS;
+  static constexpr int WCH = W_ELEMS / (kChunkElems * kWaves), LOADS = 1 + WCH;  // deposits per wave
+  static_assert(G::FM == 1 && G::COLS == 64 && BK == 16 * kWaves && A_ELEMS == kChunkElems * kWaves && WCH == 2,
+                "a wave's share of a stage");
+  static constexpr size_t BYTES = (size_t)STAGES * STAGE * sizeof(bf16) + kStageBytesPerWave;
+  static_assert((kWaves - 1) * FN * 1024 * sizeof(float) <= (size_t)STAGES * STAGE * sizeof(bf16),
+                "the partial sums fit where the stages were");
+
+  const bf16 *abase, *wbase;   // wave-uniform
+  uint32_t aoff, atail;        // byte offset of this lane's piece; in a last stage that is not whole
+  uint32_t woff[WCH], wtail[WCH];
+  int64_t astride, wstride;    // elements between stages
+
+  // A row is 256 bytes = 16 pieces, piece p stored at p ^ (row & 15): the 16 rows x 16 bytes of 16
+  // lanes of a fragment read lie in 16 different 16-byte bank groups.  aoffset(row, piece) = byte
+  // offset from base of 8 k-values of a row (every row < 32 readable).  A last stage of 32, 64 or
+  // 96 k-values repeats its first 32 in the rest, which nobody multiplies.
+  template <class AOff>
+  __device__ __forceinline__ void rows(const bf16* base, int64_t stage_stride, int K, AOff aoffset) {
+    const int l = threadIdx.x & 63, row = 4 * wave_id() + (l >> 4), piece = (l & 15) ^ (row & 15);
+    abase = base;
+    astride = stage_stride;
+    aoff = aoffset(row, piece);
+    atail = aoffset(row, 8 * piece < K % BK ? piece : piece & 3);
+  }
+  template <class ColOff>
+  __device__ __forceinline__ void weights(const bf16* base, int K, ColOff coloff, int64_t ld) {
+    const int l = threadIdx.x & 63;
+    wbase = base;
+    wstride = (int64_t)BK * ld;
+#pragma unroll
+    for (int j = 0; j < WCH; ++j) {
+      const int krow = wave_id() * (8 * WCH) + 8 * j + (l >> 3);
+      const int64_t col = coloff(((l & 7) ^ W::swz(krow)) * 8);
+      woff[j] = (uint32_t)((col + (int64_t)krow * ld) * 2);
+      wtail[j] = (uint32_t)((col + (int64_t)(krow < K % BK ? krow : krow & 31) * ld) * 2);
+    }
+  }
+  __device__ __forceinline__ void issue(int kt, int K, uint32_t stage) const {
+    const int w = wave_id();
+    const bool tail = kt * BK + BK > K;  // uniform
+    dma16(abase + kt * astride, tail ? atail : aoff, stage + w * (kChunkElems * 2));
+#pragma unroll
+    for (int j = 0; j < WCH; ++j)
+      dma16(wbase + kt * wstride, tail ? wtail[j] : woff[j],
+            stage + A_ELEMS * 2 + (w * WCH + j) * (kChunkElems * 2));
+  }
+  // acc of wave 0 = the tile's sums over K (a multiple of 32) k-values; the other waves' acc is left
+  // undefined.  Every wave must be done with `lds` on entry; on return wave 0 may still be reading
+  // it.  n_org: {0, 32}.
+  __device__ __forceinline__ void multiply(f32x16 (&acc)[FN][1], bf16* lds, int K, const int (&n_org)[FN]) const {
+    const int slice = wave_id(), l = threadIdx.x & 63;
+    const int ktiles = (K + BK - 1) / BK;
+    const uint32_t addr = lds_address(lds);
+    zero_acc<1, FN>(acc);
+    for (int s = 0; s < min(STAGES - 1, ktiles); ++s) issue(s, K, addr + s * (STAGE * 2));
+    int cur = 0, next = STAGES - 1;  // buffers of stage kt and of the stage to request
+    for (int kt = 0; kt < ktiles; ++kt) {
+      wait_stage<LOADS, STAGES>(kt, ktiles);
+      wait_lgkm0();  // this wave's reads of stage kt-1, whose buffer is requested into next
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + STAGES - 1 < ktiles) issue(kt + STAGES - 1, K, addr + next * (STAGE * 2));
+      const bf16* sa = lds + cur * STAGE;
+      if (kt * BK + 16 * slice < K) {
+        const int row = l & 31, piece = (2 * slice + (l >> 5)) ^ (row & 15);
+        const bf16x8 af = *(const bf16x8*)(sa + row * BK + piece * 8);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[j][0] = mfma32(W::frag(sa + A_ELEMS, n_org[j], slice), af, acc[j][0]);
+      }
+      cur = cur + 1 == STAGES ? 0 : cur + 1;
+      next = next + 1 == STAGES ? 0 : next + 1;
+    }
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();  // the last stage has been read: partial sums take its place
+    auto at = [&](int sl, int j, int q) { return (f32x4*)lds + ((sl - 1) * FN + j) * 256 + q * 64 + l; };
+    if (slice > 0) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *at(slice, j, q) = f32x4{acc[j][0][4 * q], acc[j][0][4 * q + 1], acc[j][0][4 * q + 2], acc[j][0][4 * q + 3]};
+    }
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    if (slice > 0) return;
+#pragma unroll
+    for (int sl = 1; sl < kWaves; ++sl)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = *at(sl, j, q);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[j][0][4 * q + r] += v[r];
+        }
+  }
+  static __device__ __forceinline__ bf16* staging(bf16* lds) { return lds + STAGES * STAGE; }
+};
+
+// Whether a forward GEMM over `cols` output columns takes FewRows tiles.
+inline bool takes_few_rows_tiles(int64_t m, int64_t msum, int64_t n, int64_t cols) {
+  return m <= FewRows::ROWS && std::min(n, msum) * cdiv64(cols, FewRows::G::COLS) <= persistent_grid();
+}
 
 }  // namespace momoe

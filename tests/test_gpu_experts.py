@@ -104,6 +104,19 @@ def test_wide_and_narrow_tiles(M, D, H, N, K, sp):
             assert torch.equal(other[k], dev[k]), (rows, k)
 
 
+@pytest.mark.parametrize("M,D,H,N,K,Ks,sp", [
+    (1, 2048, 768, 128, 8, 0, 0),    # one token
+    (32, 96, 160, 8, 3, 1, 100),     # the most rows a tile takes, last stages of 96 and 32 k-values
+    (31, 64, 32, 5, 5, 0, 50),       # last stages of 64 and 32
+    (17, 640, 544, 4, 2, 0, 0),      # five stages: one more than are in flight, columns past a tile
+    (33, 448, 320, 4, 2, 0, 0),      # one token too many for it
+])
+def test_tiles_of_few_rows(M, D, H, N, K, Ks, sp):
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, Ks=Ks, seed=4)
+    dev = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+    _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
+
+
 @pytest.mark.parametrize("gather_a", [True, False])
 def test_weight_gradient_of_cut_experts(gather_a):
     # experts of 20000 / 3 / 0 / 5000 rows: the first is contracted in pieces that meet in the
