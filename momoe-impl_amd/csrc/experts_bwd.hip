@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
   const ClockTrace trace(p.clk);
-  dgrad_h_tiles<NarrowTiles, NarrowSched>(p);
+  dgrad_h_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   trace.finish();
 }
 constexpr size_t kDhNarrowLds = DhProg<NarrowTiles>::Ring::BYTES;
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
   const ClockTrace trace(p.clk);
-  dgrad_x_tiles<NarrowTiles, NarrowSched>(p);
+  dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   trace.finish();
 }
 constexpr size_t kDxNarrowLds = DxProg<NarrowTiles>::Ring::BYTES;

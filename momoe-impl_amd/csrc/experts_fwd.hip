@@ -42,7 +42,7 @@ struct Lin1Prog {
   static_assert(!BWD || std::is_same_v<G, StdTiles>, "the SwiGLU backward epilogue fits 256-row tiles only");
   static constexpr int FM = G::FM, BM = G::MAX_ROWS, BN = G::COLS;
   using RowsOp = RDma<G::AROWS>;  // token rows, k-contiguous
-  using WeightOp = TDmaT<BN>;     // expert weights [k][col], k-strided
+  using WeightOp = TDmaT<BN, G::ONCE>;     // expert weights [k][col], k-strided
   using Ring = StageRing<RowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   static constexpr int BNH = BN / 2;
@@ -275,10 +275,20 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_kernel(Lin1Args p) {
   }
   trace.finish();
 }
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Args p) {
+// One geometry only (NarrowTiles, OnceTiles).
+template <class G>
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_geometry_kernel(Lin1Args p) {
   const ClockTrace trace(p.clk);
-  lin1_swiglu_tiles<false, NarrowTiles, NarrowSched>(p);
+  lin1_swiglu_tiles<false, G, OneGeometrySched<G>>(p);
   trace.finish();
+}
+template <class G>
+int launch_lin1_geometry(const Lin1Args& a, hipStream_t st) {
+  static LdsLimit lds;
+  constexpr size_t bytes = Lin1Prog<false, G>::kLds;
+  if (!allow_lds(lin1_swiglu_geometry_kernel<G>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin1_swiglu_geometry_kernel<G><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  return launch_status();
 }
 
 // The few-row tiles (FewRows): its own operands and loop, the epilogue of the narrow ones.
@@ -309,7 +319,6 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1A
   }
   trace.finish();
 }
-constexpr size_t kLin1NarrowLds = Lin1Prog<false, NarrowTiles>::kLds;
 constexpr size_t kLin1FwdLds = std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, StdTiles>::kLds);
 constexpr size_t kLin1BwdLds = Lin1Prog<true, StdTiles>::kLds;
 
@@ -330,7 +339,7 @@ template <class G>
 struct Lin2Prog {
   static constexpr int FM = G::FM, BN = G::COLS;
   using HRowsOp = RBlockedDma<G::AROWS>;  // rows of h, k-blocked
-  using WeightOp = TDmaT<BN>;             // expert weights [k][col], k-strided
+  using WeightOp = TDmaT<BN, G::ONCE>;             // expert weights [k][col], k-strided
   using Ring = StageRing<HRowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   struct Prep {
@@ -395,10 +404,19 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
   else lin2_scale_tiles<StdTiles>(p);
   trace.finish();
 }
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
+template <class G>
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_geometry_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
-  lin2_scale_tiles<NarrowTiles, NarrowSched>(p);
+  lin2_scale_tiles<G, OneGeometrySched<G>>(p);
   trace.finish();
+}
+template <class G>
+int launch_lin2_geometry(const Lin2Args& a, hipStream_t st) {
+  static LdsLimit lds;
+  constexpr size_t bytes = Lin2Prog<G>::kLds;
+  if (!allow_lds(lin2_scale_geometry_kernel<G>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin2_scale_geometry_kernel<G><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  return launch_status();
 }
 
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
@@ -431,7 +449,6 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Ar
   }
   trace.finish();
 }
-constexpr size_t kLin2NarrowLds = Lin2Prog<NarrowTiles>::kLds;
 constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<StdTiles>::kLds);
 
 // out[m] = sum_k rows[inv[m,k]]: one workgroup per token, 16-byte loads, fp32 accumulate.
@@ -505,12 +522,8 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
     lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, 2 * H)) {
-    static LdsLimit narrow;
-    if (!allow_lds(lin1_swiglu_narrow_kernel, kLin1NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    lin1_swiglu_narrow_kernel<<<persistent_grid(), kThreads, kLin1NarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
-  }
+  if (takes_narrow_tiles(Msum, N, 2 * H)) return launch_lin1_geometry<NarrowTiles>(a, (hipStream_t)stream);
+  if (weights_read_once(Msum, N, 4 * N * D * H)) return launch_lin1_geometry<OnceTiles>(a, (hipStream_t)stream);
   static LdsLimit lds;
   if (!allow_lds(lin1_swiglu_kernel<false>, kLin1FwdLds, lds)) return MOMOE_ERR_LAUNCH;
   lin1_swiglu_kernel<false><<<persistent_grid(), kThreads, kLin1FwdLds, (hipStream_t)stream>>>(a);
@@ -562,12 +575,8 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
     lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, D)) {
-    static LdsLimit narrow;
-    if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    lin2_scale_narrow_kernel<<<persistent_grid(), kThreads, kLin2NarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
-  }
+  if (takes_narrow_tiles(Msum, N, D)) return launch_lin2_geometry<NarrowTiles>(a, (hipStream_t)stream);
+  if (weights_read_once(Msum, N, 2 * N * D * H)) return launch_lin2_geometry<OnceTiles>(a, (hipStream_t)stream);
   static LdsLimit lds;
   if (!allow_lds(lin2_scale_kernel, kLin2Lds, lds)) return MOMOE_ERR_LAUNCH;
   lin2_scale_kernel<<<persistent_grid(), kThreads, kLin2Lds, (hipStream_t)stream>>>(a);

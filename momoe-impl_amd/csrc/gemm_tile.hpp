@@ -89,12 +89,19 @@ __device__ __forceinline__ void dma16(const bf16* g, uint32_t lds_wave_base) {
                "s"(__builtin_amdgcn_readfirstlane(lds_wave_base))
                : "memory");
 }
-// same, the source given as a wave-uniform base plus a per-lane byte offset
+// same, the source given as a wave-uniform base plus a per-lane byte offset; ONCE: the data is read
+// once (non-temporal)
+template <bool ONCE = false>
 __device__ __forceinline__ void dma16(const bf16* uniform_base, uint32_t byte_offset,
                                       uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_offset),
-               "s"(uniform_base), "s"(__builtin_amdgcn_readfirstlane(lds_wave_base))
-               : "memory");
+  if (ONCE)
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(byte_offset),
+                 "s"(uniform_base), "s"(__builtin_amdgcn_readfirstlane(lds_wave_base))
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_offset),
+                 "s"(uniform_base), "s"(__builtin_amdgcn_readfirstlane(lds_wave_base))
+                 : "memory");
 }
 
 // wait until at most N vector-memory operations of this wave are outstanding
@@ -239,7 +246,7 @@ struct TLayoutT {
 using TLayout = TLayoutT<256>;
 
 // k-strided operand with a fixed pitch between k-rows (the expert weights)
-template <int COLS>
+template <int COLS, bool ONCE = false>
 struct TDmaT {
   using L = TLayoutT<COLS>;
   static constexpr int NCH = L::NCH;
@@ -265,7 +272,7 @@ struct TDmaT {
   __device__ __forceinline__ void issue(int kt, uint32_t stage) {
     const bf16* b = base + kt * kstride;
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) dma16(b, off[j], L::deposit(stage, j));
+    for (int j = 0; j < NCH; ++j) dma16<ONCE>(b, off[j], L::deposit(stage, j));
   }
   template <int S>
   __device__ __forceinline__ void issue_head(uint32_t stage) { issue(S, stage); }
@@ -569,8 +576,9 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
 // Row-tile geometry of a kernel: WROWS wave rows of FM 32-row fragment rows each (tiles of up to
 // 32 * WROWS * FM rows, 64 columns per wave), the rows of the row operand's stage buffer (whole deposits
 // of 16 rows per wave, so a multiple of 128 that holds the tallest tile) and the ring depth.
-template <int FM_, int NS_, int WROWS_ = 2>
+template <int FM_, int NS_, int WROWS_ = 2, bool ONCE_ = false>
 struct RowTileGeometry {
+  static constexpr bool ONCE = ONCE_;  // an expert's weights are read by one row tile
   static constexpr int FM = FM_, FN = 2;
   static constexpr int WROWS = WROWS_, WCOLS = kWaves / WROWS;  // the waves' arrangement
   static constexpr int COLS = 64 * WCOLS;
@@ -596,7 +604,14 @@ using TallTiles = RowTileGeometry<5, 4>;
 // H = 768: x.Wl1 20.0 -> 16.6, h.Wl2 10.8 -> 9.1.  A fifth stage, or half the row deposits for calls of
 // few tokens, changed nothing.
 using NarrowTiles = RowTileGeometry<2, 4, 4>;
-using NarrowSched = TileSchedT<NarrowTiles::WROWS, NarrowTiles::MAX_ROWS>;
+// tile order of a kernel that holds one geometry of 256-row tiles whatever the table's height
+template <class G>
+using OneGeometrySched = TileSchedT<G::WROWS, G::MAX_ROWS>;
+// StdTiles whose k-strided weights are read with the non-temporal hint, for experts that are a
+// single row tile: their weights then pass through the L2 once and leave the token rows in it,
+// and HBM delivers a stream of such reads faster.  (k-contiguous weights come as half lines, a
+// stage apart: with the hint the second half is fetched again, dL/dh 112 -> 152 us.)
+using OnceTiles = RowTileGeometry<4, 4, 2, true>;
 static_assert(TallTiles::MAX_ROWS == MOMOE_TILE_ROWS && StdTiles::MAX_ROWS == MOMOE_RECOMPUTE_TILE_ROWS,
               "tile heights promised by the header");
 
@@ -669,10 +684,23 @@ inline int persistent_grid() {
 
 // Whether a launch over `cols` output columns takes NarrowTiles: with them there is still no more
 // than one tile per CU.  The routing is not known here; its row tiles are taken as if every expert
-// held a quarter more than its share (an estimate off the mark costs speed only).
+// held a quarter more than its share (an estimate off the mark costs speed only).  Beyond one
+// tile per CU the weights' way from HBM sets the pace: dL/dh of 1000 tokens over 128 experts with
+// 768 columns takes 112 us in two rounds of wide tiles, 113 in three of narrow ones.
 inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
   const int64_t row_tiles = std::min(n, msum) * std::max<int64_t>(1, cdiv64(5 * msum, 4 * n * StdTiles::MAX_ROWS));
   return 2 * row_tiles * cdiv64(cols, StdTiles::COLS) <= persistent_grid();
+}
+
+// Whether a launch over weight matrices of `weight_bytes` takes OnceTiles.  Measured at D = 2048, H =
+// 768, N = 128, K = 8 with cold weights, a forward without -> with the hint: 16 tokens 143 -> 130
+// us, 131 tokens 223 -> 202, 1000 (62 rows per expert) 261 -> 247, 1300 (81) 273 -> 261; at 162
+// rows it is slower (h.Wl2 117 -> 119), at 512 x.Wl1 by 4 %: the line lies at a third of a tile.
+// Matrices that fit the 256 MiB last-level cache keep their place in it without the hint: a step
+// whose backward reads them again took 175 -> 191 us (1000 tokens, 128 MB).  The recomputing GEMM
+// does not gain (171 us either way at 62 rows).
+inline bool weights_read_once(int64_t msum, int64_t n, int64_t weight_bytes) {
+  return 3 * msum <= n * OnceTiles::MAX_ROWS && weight_bytes >= (256ll << 20);
 }
 
 template <int FM, int FN>

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 import oracle
-from gpu_util import (assert_close, rel_err, run_device_layer, run_oracle_layer,
+from gpu_util import (assert_close, device_layer_inputs, oracle_forward_for_tokens, rel_err,
+                      run_device_layer, run_oracle_layer,
                       sampled_parity_on_device_inputs as _sampled_parity_on_device_inputs)
 from helpers import make_layer_inputs
 
@@ -102,6 +103,30 @@ def test_wide_and_narrow_tiles(M, D, H, N, K, sp):
             experts.TILE_ROWS = _hip.AUTO_TILE_ROWS
         for k in dev:
             assert torch.equal(other[k], dev[k]), (rows, k)
+
+
+@pytest.mark.parametrize("M,D,H,N,K,skew", [
+    (300, 2080, 544, 120, 2, None),   # both matrices above 256 MiB, no dimension a multiple of the tile
+    (1300, 2080, 544, 120, 2, 1.8),   # experts of several row tiles, 320-row ones halved
+])
+def test_weights_read_once(M, D, H, N, K, skew):
+    """The forward only: no kernel of the backward reads weights this way."""
+    import momoe_amd
+    from momoe_amd import _hip, experts
+    x, _, W1, W2, mask, s = device_layer_inputs(M, D, H, N, K, skew=skew)
+    layer = momoe_amd.MoMoE(D, H, N, K, Wl1_ND2H=W1, Wl2_NHD=W2)
+    args = x.reshape(1, M, D), mask.to("cuda:0"), s.T.contiguous().to("cuda:0").T
+    with torch.no_grad():
+        y, sizes = layer(*args)
+        try:
+            experts.TILE_ROWS = _hip.TILE_ROWS
+            tall, _ = layer(*args)
+        finally:
+            experts.TILE_ROWS = _hip.AUTO_TILE_ROWS
+    assert torch.equal(sizes.cpu(), (mask != 0).sum(1)) and torch.equal(tall, y)
+    tok = torch.arange(0, M, M // 16)[:16]
+    want, _ = oracle_forward_for_tokens(x, W1, W2, mask, s, tok)
+    assert_close(y.reshape(M, D)[tok.to("cuda:0")], want, "y (sampled tokens)")
 
 
 @pytest.mark.parametrize("M,D,H,N,K,Ks,sp", [
