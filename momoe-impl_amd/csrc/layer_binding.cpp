@@ -95,6 +95,15 @@ Tensor empty_f32(at::IntArrayRef size, const at::Device& dev) {
   throw py::error_already_set();
 }
 
+// Whether a call has to go through its autograd function.  A forward-mode tangent counts: the
+// function refuses it, where the plain forward would drop it without a word.
+bool wants_autograd(std::initializer_list<const Tensor*> inputs) {
+  bool any = false;
+  for (const Tensor* t : inputs)
+    any = any || (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined();
+  return any;
+}
+
 // ---- experts -----------------------------------------------------------------------------------
 // What the index build leaves for the rest of the forward and for the backward, in one allocation:
 // [cumsums N+1 | idx Msum | inv Msum | tile table | tile table of the recomputing GEMM], every part
@@ -297,9 +306,7 @@ std::pair<Tensor, Tensor> experts(const Tensor& x, const Tensor& W1, const Tenso
       W2.size(1) != W1.size(2) / 2 || W2.size(2) != x.size(2))
     throw_python(PyExc_AssertionError, "x_BSD [B,S,D], Wl1_ND2H [N,D,2H] and Wl2_NHD [N,H,D] do not fit together");
   const int64_t msum = x.size(0) * x.size(1) * K;
-  const bool grad = at::GradMode::is_enabled() &&
-                    (x.requires_grad() || W1.requires_grad() || W2.requires_grad() || s.requires_grad());
-  if (!grad) {  // nothing is kept for a backward that cannot happen
+  if (!wants_autograd({&x, &W1, &W2, &s})) {  // nothing is kept for a backward that cannot happen
     Forward f = experts_forward(x, W1, W2, mask, s, K, 0, false, tile_rows, check);
     return {f.y, f.sizes};
   }
@@ -381,7 +388,7 @@ std::tuple<Tensor, Tensor, Tensor> router(const Tensor& x, const Tensor& Wg, con
   if (Wg.scalar_type() != at::kBFloat16) throw_python(PyExc_AssertionError, "Wg_DN must be of type torch.bfloat16");
   TORCH_CHECK(Wg.is_cuda(), "TopKRouter weights must live on the GPU: there is no CPU compute path");
   TORCH_CHECK(x.dim() == 3, "x_BSD must be [B, S, D]");
-  if (!at::GradMode::is_enabled() || !(x.requires_grad() || Wg.requires_grad())) {
+  if (!wants_autograd({&x, &Wg})) {
     Routed r = router_forward(x, Wg, biases, N, K, Ks);
     return {x, r.mask, r.s_MN.t()};
   }

@@ -354,6 +354,25 @@ def test_input_formats_and_partial_gradients():
     assert not yn.requires_grad and torch.equal(yn, yc.detach())
 
 
+@pytest.mark.parametrize("grad", [True, False])
+def test_forward_mode_is_refused(grad):
+    """Neither function has a forward-mode rule: a tangent on an input is an error, also where no
+    input wants a gradient, never a result without it."""
+    import momoe_amd
+    import torch.autograd.forward_ad as fwAD
+    x, W1, W2, mask, s, _ = make_layer_inputs(32, 64, 32, 4, 2, seed=1)
+    layer = momoe_amd.MoMoE(64, 32, 4, 2, Wl1_ND2H=W1.to("cuda:0"), Wl2_NHD=W2.to("cuda:0"))
+    moe = momoe_amd.MoE(64, 32, 4, 2, 0, Wg_DN=torch.randn(64, 4).to("cuda:0"), Wl1_ND2H=W1.to("cuda:0"),
+                        Wl2_NHD=W2.to("cuda:0"))
+    xd = x.to("cuda:0", torch.bfloat16).reshape(1, 32, 64)
+    with fwAD.dual_level(), torch.set_grad_enabled(grad):
+        dual = fwAD.make_dual(xd, torch.ones_like(xd))
+        with pytest.raises(RuntimeError):
+            layer(dual, mask.to("cuda:0"), s.to("cuda:0"))
+        with pytest.raises(RuntimeError):
+            moe(dual)
+
+
 def test_recomputing_gemm_ignores_a_table_of_taller_tiles():
     """momoe_lin1_swiglu_bwd takes row tiles of at most 256 rows: given the 320-row table of the other
     GEMMs it must leave its outputs alone instead of computing on tiles it cannot hold."""
