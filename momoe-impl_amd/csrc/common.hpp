@@ -192,6 +192,16 @@ struct ClockTrace {
   }
 };
 
+// Data of at least this size is not read back from the 256 MiB last-level cache by a kernel that
+// passes over it once: such reads go with the non-temporal hint.  (Smaller data just written is
+// still there, and the hint gives that up: 4 to 7 % of a forward or step at a few MiB.)
+constexpr int64_t kBeyondCache = 256ll << 20;
+template <bool ONCE, class T>
+__device__ __forceinline__ T load_maybe_once(const T* p) {
+  if (ONCE) return __builtin_nontemporal_load(p);
+  return *p;
+}
+
 inline int launch_status() {
   return hipGetLastError() == hipSuccess ? MOMOE_OK : MOMOE_ERR_LAUNCH;
 }

@@ -697,10 +697,11 @@ inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
 // us, 131 tokens 223 -> 202, 1000 (62 rows per expert) 261 -> 247, 1300 (81) 273 -> 261; at 162
 // rows it is slower (h.Wl2 117 -> 119), at 512 x.Wl1 by 4 %: the line lies at a third of a tile.
 // Matrices that fit the 256 MiB last-level cache keep their place in it without the hint: a step
-// whose backward reads them again took 175 -> 191 us (1000 tokens, 128 MB).  The recomputing GEMM
-// does not gain (171 us either way at 62 rows).
+// whose backward reads them again took 175 -> 191 us (1000 tokens, 128 MB).  For the same reason
+// the recomputing GEMM goes without it: dL/dx reads Wl1 again, and with the hint a step took
+// 982 -> 949 us (1000 tokens) but 313 -> 327 (64 tokens, D = 2048, H = 1024, N = 32, K = 4).
 inline bool weights_read_once(int64_t msum, int64_t n, int64_t weight_bytes) {
-  return 3 * msum <= n * OnceTiles::MAX_ROWS && weight_bytes >= (256ll << 20);
+  return 3 * msum <= n * OnceTiles::MAX_ROWS && weight_bytes >= kBeyondCache;
 }
 
 template <int FM, int FN>
