@@ -47,7 +47,8 @@ extern "C" {
  * weights (e.g. experts of 513..640 rows: two row tiles instead of three), else the shorter. */
 #define MOMOE_TILE_ROWS 320
 #define MOMOE_RECOMPUTE_TILE_ROWS 256
-/* column-block width of the partial row sums written by momoe_lin1_swiglu_bwd */
+/* column-block width of the partial row sums written by momoe_lin1_swiglu_bwd (half of it where
+ * momoe_gs_parts says so: momoe_lin1_swiglu_bwd_parts) */
 #define MOMOE_GS_BLOCK 128
 
 int momoe_abi_version(void);
@@ -210,7 +211,7 @@ int momoe_combine(const void* rows_MsumD, const int32_t* inv_MK, void* out_MD,
  *
  * momoe_swiglu_bwd_saved: the same from the saved a|b (bf16) of the rows below Msave; the row
  * sum is spread over the first ceil(H/256) parts, the other parts get zeros
- * (nparts = ceil(H / MOMOE_GS_BLOCK)).
+ * (nparts = ceil(H / MOMOE_GS_BLOCK), or as many as momoe_lin1_swiglu_bwd_parts is given).
  *
  * Which of the two produces a row (the reference's own choice is per tile of its autotuned
  * height, momoe/momoe.py:486): rows are taken in groups of 32 counted from their expert's first
@@ -229,6 +230,19 @@ int momoe_lin1_swiglu_bwd(const void* x_MD, const void* Wl1_ND2H, const int32_t*
                           int64_t row_lo, void* gz_blocked, void* hsT_GH32, int64_t ld_hsT,
                           float* gs_part,
                           int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum, void* stream);
+
+/* momoe_lin1_swiglu_bwd with `nparts` partial row sums per row, gs_part fp32 [nparts][Msum]:
+ * ceil(H/MOMOE_GS_BLOCK), as above, or momoe_gs_parts(H, N, Msum) (anything else:
+ * MOMOE_ERR_BAD_ARG).  The latter is twice as many where the launch has few output tiles: it then
+ * works on tiles half as wide, each with a partial sum of its own, on twice the CUs.
+ */
+int64_t momoe_gs_parts(int64_t H, int64_t N, int64_t Msum);
+int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2H, const int32_t* idx_Msum,
+                                const int32_t* tile_table, const void* u_MsumH,
+                                const float* s_NM, int64_t s_stride_n, int64_t s_stride_m,
+                                int64_t row_lo, void* gz_blocked, void* hsT_GH32, int64_t ld_hsT,
+                                float* gs_part, int64_t nparts,
+                                int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum, void* stream);
 
 int momoe_swiglu_bwd_saved(const void* ab_save, const void* u_MsumH,
                            const float* s_NM, int64_t s_stride_n, int64_t s_stride_m,

@@ -234,7 +234,7 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     // s*h in groups of 32 padded sorted rows, feature-major inside a group: the layout the Wl2
     // gradient reads fastest
     Tensor hst = empty_bf16({momoe_padded_rows(msum, N) / 32, H, 32}, dev);
-    const int64_t nparts = (H + MOMOE_GS_BLOCK - 1) / MOMOE_GS_BLOCK;
+    const int64_t nparts = momoe_gs_parts(H, N, msum);
     Tensor gs_part = empty_f32({nparts, msum}, dev);
     if (msave > 0)
       MOMOE_CALL(momoe_swiglu_bwd_saved, st, ab_save.data_ptr(), u.data_ptr(), s.data_ptr<float>(), s.stride(0),
@@ -251,9 +251,9 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                    own.data_ptr<int32_t>());
         table_rc = own.data_ptr<int32_t>();
       }
-      MOMOE_CALL(momoe_lin1_swiglu_bwd, st, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc, u.data_ptr(),
-                 s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz.data_ptr(), hst.data_ptr(), H,
-                 gs_part.data_ptr<float>(), M, D, H, N, msum);
+      call("momoe_lin1_swiglu_bwd", st, momoe_lin1_swiglu_bwd_parts, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc,
+           u.data_ptr(), s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz.data_ptr(), hst.data_ptr(), H,
+           gs_part.data_ptr<float>(), nparts, M, D, H, N, msum);
     }
     u.reset();
     if (need_s) {

@@ -54,6 +54,9 @@ _SIGNATURES = {
     "momoe_dgrad_h": (_int, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "momoe_lin1_swiglu_bwd": (_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64, _p,
                                      _i64, _i64, _i64, _i64, _i64, _p]),
+    "momoe_gs_parts": (_i64, [_i64, _i64, _i64]),
+    "momoe_lin1_swiglu_bwd_parts": (_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64, _p,
+                                           _i64, _i64, _i64, _i64, _i64, _i64, _p]),
     "momoe_swiglu_bwd_saved": (_int, [_p, _p, _p, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _p, _i64,
                                       _i64, _i64, _i64, _i64, _p]),
     "momoe_gs_scatter": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _p]),

@@ -58,6 +58,26 @@ def test_size_queries_and_argument_validation(lib):
     assert lib.momoe_wgrad_workspace_bytes(i64(2), i64(64), i64(64), i64(100)) == 0
 
 
+@pytest.mark.parametrize("H,N,msum,parts", [
+    (512, 32, 4096, 8),       # 128 tiles of 256 columns: 64-column parts
+    (544, 32, 4096, 5),       # 160 tiles: 128-column parts
+    (1024, 128, 65536, 8),
+    (64, 8, 256, 1), (96, 8, 256, 2), (2048, 8, 16, 32), (0, 8, 256, -1),
+])
+def test_parts_of_the_gate_gradient(lib, H, N, msum, parts):
+    i64, p = ctypes.c_int64, ctypes.c_void_p
+    lib.momoe_gs_parts.restype = i64
+    got = lib.momoe_gs_parts(i64(H), i64(N), i64(msum))
+    assert got == parts
+    if H:  # another number of parts than the two documented ones is refused before any launch
+        a = p(4096)
+        for n in (0, got + 1, 2 * got + 2):
+            if n == -(-H // 128):
+                continue
+            assert lib.momoe_lin1_swiglu_bwd_parts(a, a, a, a, a, a, i64(1), i64(1), i64(0), a, a, i64(H), a, i64(n),
+                                                   i64(256), i64(64), i64(H), i64(N), i64(msum), p(0)) == 1
+
+
 def test_host_modules_refuse_cpu_tensors():
     import torch
     import momoe_amd
