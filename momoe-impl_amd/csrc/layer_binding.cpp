@@ -330,7 +330,11 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
   const c10::DeviceGuard guard(dev);
   Routed r;
   r.x_MD = x_BSD.reshape({M, D}).to(dev, at::kBFloat16);
+  // autocast may give the product another type than its operands'; the kernel reads two of them
   const Tensor logits = at::mm(r.x_MD, Wg).contiguous();
+  if (logits.scalar_type() != at::kBFloat16 && logits.scalar_type() != at::kFloat)
+    throw_python(PyExc_AssertionError, std::string("the gate logits must be bfloat16 or float32, got ") +
+                                           c10::toString(logits.scalar_type()));
   TORCH_CHECK(logits.size(1) == N, "Wg_DN must have N = ", N, " columns");
   const Tensor bias = biases.to(dev, at::kFloat).contiguous();
   TORCH_CHECK(bias.numel() == N, "biases_N must have N = ", N, " elements");
@@ -339,7 +343,7 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
   r.p_sel = empty_f32({M, N}, dev);
   r.norms = empty_f32({2, M}, dev);  // per token: sum over the selected, over the shared experts
   float* norms = r.norms.data_ptr<float>();
-  MOMOE_CALL(momoe_router_fwd, stream_of(dev), logits.data_ptr(), 0, bias.data_ptr<float>(), M, N, K, Ks,
+  MOMOE_CALL(momoe_router_fwd, stream_of(dev), logits.data_ptr(), logits.scalar_type() == at::kFloat, bias.data_ptr<float>(), M, N, K, Ks,
              r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M);
   return r;
 }

@@ -148,6 +148,28 @@ def test_moe_wrapper_against_oracle_and_state_dict():
     assert moe.biases_N[-1].item() == float("-inf")
 
 
+@pytest.mark.parametrize("grad", [True, False])
+def test_router_under_autocast(grad):
+    """autocast decides the type of the gate product: bfloat16 changes nothing, float16 (its default)
+    is refused, since the kernel reads bfloat16 and float32 logits only."""
+    import momoe_amd
+    torch.manual_seed(3)
+    D, H, N, K, Ks = 64, 32, 8, 3, 1
+    moe = momoe_amd.MoE(D, H, N, K, Ks, bias_update_rate=0.0)
+    x = torch.randn(2, 24, D, device="cuda", dtype=torch.bfloat16)
+    with torch.set_grad_enabled(grad):
+        want = [*moe.router(x, moe.biases_N), moe(x)]
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            got = [*moe.router(x, moe.biases_N), moe(x)]
+        with torch.autocast("cuda", dtype=torch.float16):
+            with pytest.raises(AssertionError, match="logits"):
+                moe.router(x, moe.biases_N)
+            with pytest.raises(AssertionError, match="logits"):
+                moe(x)
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and torch.equal(g, w)
+
+
 def test_training_smoke_loss_decreases():
     # scaled-down version of the reference's only test (momoe/test.py): AdamW on
     # mean((y - x)^2); the loss starts near 1 and must go down.
