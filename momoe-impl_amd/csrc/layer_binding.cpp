@@ -10,10 +10,13 @@
 // memory.
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
+#include <torch/library.h>
 
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -102,6 +105,16 @@ bool wants_autograd(std::initializer_list<const Tensor*> inputs) {
   for (const Tensor* t : inputs)
     any = any || (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined();
   return any;
+}
+
+// A call under torch.jit.trace, made again through the operator momoe::`name` (TORCH_LIBRARY
+// below), whose kernel is the calling function itself: the tracer records operators that pass
+// the dispatcher.  Of a plain call it would see the allocations only and record a graph that
+// returns unwritten memory.
+template <class Result, class... Args>
+Result call_recorded(const char* name, Args... args) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Result(Args...)>().call(
+      std::forward<Args>(args)...);
 }
 
 // ---- experts -----------------------------------------------------------------------------------
@@ -296,8 +309,12 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
   }
 };
 
-std::pair<Tensor, Tensor> experts(const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& mask,
-                                  const Tensor& s, int64_t K, double save_percent, int64_t tile_rows, bool check) {
+std::tuple<Tensor, Tensor> experts(const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& mask,
+                                   const Tensor& s, int64_t K, double save_percent, int64_t tile_rows, bool check) {
+  if (torch::jit::tracer::isTracing())
+    return call_recorded<std::tuple<Tensor, Tensor>, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                         const Tensor&, int64_t, double, int64_t, bool>("momoe::experts", x, W1, W2, mask, s, K,
+                                                                        save_percent, tile_rows, check);
   if (W1.device() != W2.device())
     throw_python(PyExc_AssertionError, "All weights must be on the same device, but got: Wl1_ND2H.device = " +
                                     W1.device().str() + ", Wl2_NHD.device = " + W2.device().str());
@@ -389,6 +406,9 @@ struct RouterFn : torch::autograd::Function<RouterFn> {
 
 std::tuple<Tensor, Tensor, Tensor> router(const Tensor& x, const Tensor& Wg, const Tensor& biases, int64_t N, int64_t K,
                                           int64_t Ks) {
+  if (torch::jit::tracer::isTracing())
+    return call_recorded<std::tuple<Tensor, Tensor, Tensor>, const Tensor&, const Tensor&, const Tensor&, int64_t,
+                         int64_t, int64_t>("momoe::router", x, Wg, biases, N, K, Ks);
   if (Wg.scalar_type() != at::kBFloat16) throw_python(PyExc_AssertionError, "Wg_DN must be of type torch.bfloat16");
   TORCH_CHECK(Wg.is_cuda(), "TopKRouter weights must live on the GPU: there is no CPU compute path");
   TORCH_CHECK(x.dim() == 3, "x_BSD must be [B, S, D]");
@@ -409,6 +429,16 @@ void bias_update(Tensor biases, const Tensor& sizes, double c_avg, double rate) 
 }
 
 }  // namespace
+
+// The operators of a traced call.  A graph keeps the integers and flags it was traced with, the sizes
+// are those of the tensors it is run on.
+TORCH_LIBRARY(momoe, m) {
+  m.def("experts(Tensor x_BSD, Tensor Wl1_ND2H, Tensor Wl2_NHD, Tensor mask_NM, Tensor s_NM, int K, "
+        "float save_percent, int tile_rows, bool check) -> (Tensor, Tensor)",
+        torch::dispatch(c10::DispatchKey::CompositeImplicitAutograd, TORCH_FN(experts)));
+  m.def("router(Tensor(a) x_BSD, Tensor Wg_DN, Tensor biases_N, int N, int K, int Ks) -> (Tensor(a), Tensor, Tensor)",
+        torch::dispatch(c10::DispatchKey::CompositeImplicitAutograd, TORCH_FN(router)));
+}
 
 PYBIND11_MODULE(_layer, m) {
   m.def("experts", &experts, py::call_guard<py::gil_scoped_release>());

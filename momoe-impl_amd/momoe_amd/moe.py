@@ -43,7 +43,9 @@ class MoE(nn.Module):
         B, S, _ = x_BSD.shape
         c_avg = B * S * (self.K - self.Ks) / (self.N - self.Ks)
         b = self.biases_N
-        if b.dtype == torch.float32 and b.is_contiguous() and b.device == sizes_N.device and not b.requires_grad:
+        # (a trace has to see the update, and sees operators of torch only)
+        if (b.dtype == torch.float32 and b.is_contiguous() and b.device == sizes_N.device and not b.requires_grad
+                and not torch.jit.is_tracing()):
             _layer.bias_update(b, sizes_N, c_avg, self.bias_update_rate)
         else:
             self.biases_N += self.bias_update_rate * torch.sign(c_avg - sizes_N.to(b.device))

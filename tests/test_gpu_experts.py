@@ -355,6 +355,49 @@ def test_input_formats_and_partial_gradients():
 
 
 @pytest.mark.parametrize("grad", [True, False])
+def test_traced_modules_run_the_layer(grad):
+    """A graph of torch.jit.trace does on other inputs, of other sizes too, what the module does:
+    results, gradients and the selection bias's update."""
+    import momoe_amd
+    dev = "cuda:0"
+    D, H, N, K, Ks = 64, 32, 8, 3, 1
+    torch.manual_seed(4)
+    eager = momoe_amd.MoE(D, H, N, K, Ks, save_percent=50, bias_update_rate=0.5)
+    module = momoe_amd.MoE(D, H, N, K, Ks, save_percent=50, bias_update_rate=0.5)
+    module.load_state_dict(eager.state_dict())
+
+    def inputs(M, seed):
+        x, _, _, mask, s, dy = make_layer_inputs(M, D, H, N, K, Ks, seed=seed)
+        return (x.to(dev, torch.bfloat16).reshape(1, M, D), mask.to(dev), s.to(dev),
+                dy.to(dev, torch.bfloat16).reshape(1, M, D))
+
+    x, mask, s, _ = inputs(40, 1)
+    with torch.set_grad_enabled(grad):
+        traced_experts = torch.jit.trace(module.momoe, (x, mask, s))
+        traced_router = torch.jit.trace(module.router, (x, module.biases_N))
+        traced = torch.jit.trace(module, x, check_trace=False)  # a call moves the bias
+    module.load_state_dict(eager.state_dict())
+    for M, seed in ((40, 2), (40, 3), (40, 4), (75, 5)):
+        x, mask, s, dy = inputs(M, seed)
+        results = []
+        for moe, router, experts_of in ((eager, eager.router, eager.momoe), (traced, traced_router, traced_experts)):
+            params = eager if moe is eager else module
+            params.zero_grad(set_to_none=True)
+            xd, sd = x.clone().requires_grad_(grad), s.clone().requires_grad_(grad)
+            with torch.set_grad_enabled(grad):
+                y, sizes = experts_of(xd, mask, sd)
+                xr, chosen, gates = router(xd, params.biases_N)
+                out = [y, sizes, xr, chosen, gates, moe(xd)]
+            if grad:
+                torch.autograd.backward([y, gates, out[5]], [dy, torch.ones_like(gates), dy])
+                out += [xd.grad, sd.grad, params.router.Wg_DN.grad, params.momoe.Wl1_ND2H.grad,
+                        params.momoe.Wl2_NHD.grad]
+            results.append([t.detach() for t in out] + [params.biases_N.detach().clone()])
+        for i, (a, b) in enumerate(zip(*results)):
+            assert a.dtype == b.dtype and torch.equal(a, b), (M, i)
+
+
+@pytest.mark.parametrize("grad", [True, False])
 def test_forward_mode_is_refused(grad):
     """Neither function has a forward-mode rule: a tangent on an input is an error, also where no
     input wants a gradient, never a result without it."""
