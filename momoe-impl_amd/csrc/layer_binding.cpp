@@ -117,6 +117,18 @@ Result call_recorded(const char* name, Args... args) {
       std::forward<Args>(args)...);
 }
 
+// A tensor that a backward hands to kernels by pointer, as the forward saved it.  A saved-tensor hook
+// may have put any other in its place: one on the host, of another type or shorter would be read
+// past its end on the device.  `packed`: contiguous and on a 16-byte boundary.
+const Tensor& as_saved(const Tensor& t, const char* name, const at::Device& dev, at::ScalarType type,
+                       at::IntArrayRef sizes, bool packed = true) {
+  TORCH_CHECK(t.defined() && t.device() == dev && t.scalar_type() == type && t.sizes() == sizes &&
+                  (!packed || (t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0)),
+              "backward: the saved tensor ", name, " came back from its hook as something else than ", type, " ", sizes,
+              " on ", dev, packed ? ", contiguous" : "");
+  return t;
+}
+
 // ---- experts -----------------------------------------------------------------------------------
 // What the index build leaves for the rest of the forward and for the backward, in one allocation:
 // [cumsums N+1 | idx Msum | inv Msum | tile table | tile table of the recomputing GEMM], every part
@@ -213,6 +225,10 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     ctx->saved_data["msave"] = msave;
     ctx->saved_data["tile_rows"] = tile_rows;
     ctx->saved_data["want_rc"] = want_rc;
+    ctx->saved_data["device"] = f.W1.device();
+    ctx->saved_data["D"] = f.W1.size(1);
+    ctx->saved_data["N"] = f.W2.size(0);
+    ctx->saved_data["H"] = f.W2.size(1);
     ctx->save_for_backward({f.x, f.s, f.W1, f.W2, f.index, f.ab_save});
     ctx->mark_non_differentiable({f.sizes});
     ctx->set_materialize_grads(false);
@@ -220,21 +236,26 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const variable_list saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &s = saved[1], &W1 = saved[2], &W2 = saved[3], &ab_save = saved[5];
     const int64_t K = ctx->saved_data["K"].toInt(), msave = ctx->saved_data["msave"].toInt();
     const int64_t tile_rows = ctx->saved_data["tile_rows"].toInt();
     const bool need_x = ctx->needs_input_grad(0), need_w1 = ctx->needs_input_grad(1),
                need_w2 = ctx->needs_input_grad(2), need_s = ctx->needs_input_grad(4);
     variable_list out(9);
     if (!grads[0].defined()) return out;
-    const at::Device dev = W1.device(), gdev = grads[0].device();
-    const int64_t B = grads[0].size(0), S = grads[0].size(1), D = grads[0].size(2), M = B * S;
-    const int64_t N = W2.size(0), H = W2.size(1), msum = M * K;
+    const at::Device dev = ctx->saved_data["device"].toDevice(), gdev = grads[0].device();
+    const int64_t D = ctx->saved_data["D"].toInt(), N = ctx->saved_data["N"].toInt(), H = ctx->saved_data["H"].toInt();
+    const int64_t B = grads[0].size(0), S = grads[0].size(1), M = B * S, msum = M * K;
+    Index ib(M, N, K, tile_rows, ctx->saved_data["want_rc"].toBool());
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor& x = as_saved(saved[0], "x", dev, at::kBFloat16, {M, D});
+    const Tensor& s = as_saved(saved[1], "s", dev, at::kFloat, {N, M}, /*packed=*/false);
+    const Tensor& W1 = as_saved(saved[2], "Wl1", dev, at::kBFloat16, {N, D, 2 * H});
+    const Tensor& W2 = as_saved(saved[3], "Wl2", dev, at::kBFloat16, {N, H, D});
+    ib.base = as_saved(saved[4], "index", dev, at::kInt, {ib.ints}).data_ptr<int32_t>();
+    const Tensor& ab_save = saved[5];
+    if (msave > 0) as_saved(ab_save, "a|b", dev, at::kBFloat16, {msave, 2 * H});
     const c10::DeviceGuard guard(dev);
     const hipStream_t st = stream_of(dev);
-    Index ib(M, N, K, tile_rows, ctx->saved_data["want_rc"].toBool());
-    ib.base = saved[4].data_ptr<int32_t>();
     const Tensor Gy = grads[0].reshape({M, D}).to(dev, at::kBFloat16).contiguous();
 
     // dL/dh before the gate weight, in sorted order
@@ -371,16 +392,24 @@ struct RouterFn : torch::autograd::Function<RouterFn> {
     Routed r = router_forward(x, Wg, biases, N, K, Ks);
     ctx->save_for_backward({r.x_MD, Wg, r.mask, r.p_sel, r.s_MN, r.norms});
     ctx->saved_data["Ks"] = Ks;
+    ctx->saved_data["N"] = N;
     ctx->saved_data["shape"] = x.sizes().vec();
+    ctx->saved_data["device"] = Wg.device();
     ctx->mark_non_differentiable({r.mask});
     ctx->set_materialize_grads(false);
     return {x, r.mask, r.s_MN.t()};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &Wg = saved[1], &mask = saved[2], &p_sel = saved[3], &s_MN = saved[4], &norms = saved[5];
-    const at::Device dev = Wg.device();
-    const int64_t M = x.size(0), D = x.size(1), N = Wg.size(1);
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    const at::Device dev = ctx->saved_data["device"].toDevice();
+    const int64_t M = shape[0] * shape[1], D = shape[2], N = ctx->saved_data["N"].toInt();
+    const Tensor& x = as_saved(saved[0], "x", dev, at::kBFloat16, {M, D}, /*packed=*/false);
+    const Tensor& Wg = as_saved(saved[1], "Wg", dev, at::kBFloat16, {D, N}, /*packed=*/false);
+    const Tensor& mask = as_saved(saved[2], "mask", dev, at::kInt, {N, M});
+    const Tensor& p_sel = as_saved(saved[3], "p", dev, at::kFloat, {M, N});
+    const Tensor& s_MN = as_saved(saved[4], "s", dev, at::kFloat, {M, N});
+    const Tensor& norms = as_saved(saved[5], "norms", dev, at::kFloat, {2, M});
     const bool need_x = ctx->needs_input_grad(0), need_wg = ctx->needs_input_grad(1);
     const c10::DeviceGuard guard(dev);
     variable_list out(6);
@@ -399,7 +428,7 @@ struct RouterFn : torch::autograd::Function<RouterFn> {
     } else if (need_wg) {
       out[1] = at::zeros_like(Wg);
     }
-    if (need_x && G_x.defined()) out[0] = G_x.reshape(ctx->saved_data["shape"].toIntVector());
+    if (need_x && G_x.defined()) out[0] = G_x.reshape(shape);
     return out;
   }
 };

@@ -397,6 +397,53 @@ def test_traced_modules_run_the_layer(grad):
             assert a.dtype == b.dtype and torch.equal(a, b), (M, i)
 
 
+def test_saved_tensor_hooks():
+    """A hook may hand every saved tensor back as a copy; one that hands back something else than was
+    saved (host memory, another type, fewer elements) is refused before any kernel reads it."""
+    import momoe_amd
+    dev = "cuda:0"
+    D, H, N, K, M = 64, 32, 4, 2, 48
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=6)
+    moe = momoe_amd.MoE(D, H, N, K, 0, save_percent=50, bias_update_rate=0.0, Wg_DN=torch.randn(D, N).to(dev),
+                        Wl1_ND2H=W1.to(dev), Wl2_NHD=W2.to(dev))
+    xd = x.to(dev, torch.bfloat16).reshape(1, M, D).requires_grad_()
+    sd, dyd, maskd = s.to(dev).requires_grad_(), dy.to(dev, torch.bfloat16).reshape(1, M, D), mask.to(dev)
+
+    def experts():
+        y, _ = moe.momoe(xd, maskd, sd)
+        return [y], [dyd]
+
+    def router():
+        _, _, gates = moe.router(xd, moe.biases_N)
+        return [gates], [torch.ones_like(gates) * 0.5 + gates.detach()]
+
+    def gradients(call, unpack):
+        saved = []
+
+        def pack(t):
+            saved.append(t.clone())
+            return len(saved) - 1
+
+        for t in (xd, sd, *moe.parameters()):
+            t.grad = None
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda i: unpack(i, saved[i])):
+            out, grads = call()
+        torch.autograd.backward(out, grads)
+        return [t.grad for t in (xd, sd, *moe.parameters()) if t.grad is not None], len(saved)
+
+    def at(i, change):  # the i-th saved tensor changed, the others as they were
+        return lambda j, t: change(t) if i == j else t
+
+    for call, count in ((experts, 6), (router, 6)):
+        want, n = gradients(call, lambda i, t: t)
+        got, _ = gradients(call, lambda i, t: t.cpu().to(dev))
+        assert n == count and len(want) >= 2 and all(torch.equal(a, b) for a, b in zip(got, want))
+        for i in range(count):
+            for change in (torch.Tensor.cpu, lambda t: t.to(torch.float16), lambda t: t[..., :-1].contiguous()):
+                with pytest.raises(RuntimeError, match="saved tensor"):
+                    gradients(call, at(i, change))
+
+
 @pytest.mark.parametrize("grad", [True, False])
 def test_forward_mode_is_refused(grad):
     """Neither function has a forward-mode rule: a tangent on an input is an error, also where no
