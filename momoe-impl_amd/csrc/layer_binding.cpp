@@ -14,6 +14,7 @@
 #include <torch/extension.h>
 #include <torch/library.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <tuple>
@@ -34,7 +35,7 @@ struct TimedCall {
   hipEvent_t begin, end;
 };
 std::mutex g_timing_mutex;
-bool g_timing = false;  // written with no launch in flight; a stale read only skips a record
+std::atomic<bool> g_timing{false};  // read by every thread that launches; a stale read only skips a record
 std::vector<TimedCall> g_calls;
 
 void timing_start() {
@@ -63,7 +64,7 @@ std::vector<std::pair<std::string, double>> timing_take() {
 template <class Fn, class... Args>
 void call(const char* name, hipStream_t st, Fn fn, Args... args) {
   int code;
-  if (!g_timing) {
+  if (!g_timing.load(std::memory_order_relaxed)) {
     code = fn(args..., (void*)st);
   } else {
     TimedCall t{name, nullptr, nullptr};
