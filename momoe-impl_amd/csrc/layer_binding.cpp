@@ -31,21 +31,15 @@ using torch::autograd::variable_list;
 
 // ---- launch timing (kernel_timer in _hip.py): an event pair around every library call ---------
 struct TimedCall {
-  const char* name;
+  std::string name;
   hipEvent_t begin, end;
 };
 std::mutex g_timing_mutex;
 std::atomic<bool> g_timing{false};  // read by every thread that launches; a stale read only skips a record
 std::vector<TimedCall> g_calls;
 
-void timing_start() {
-  std::lock_guard<std::mutex> lock(g_timing_mutex);
-  g_timing = true;
-}
-void timing_stop() {
-  std::lock_guard<std::mutex> lock(g_timing_mutex);
-  g_timing = false;
-}
+void timing_start() { g_timing.store(true, std::memory_order_relaxed); }
+void timing_stop() { g_timing.store(false, std::memory_order_relaxed); }
 // durations in ms of the calls recorded so far; the device must be idle
 std::vector<std::pair<std::string, double>> timing_take() {
   std::lock_guard<std::mutex> lock(g_timing_mutex);
@@ -61,21 +55,27 @@ std::vector<std::pair<std::string, double>> timing_take() {
   return out;
 }
 
+// fn(), with an event pair around it on `st` while launches are timed
+template <class Fn>
+auto timed(const char* name, hipStream_t st, Fn fn) {
+  if (!g_timing.load(std::memory_order_relaxed)) return fn();
+  TimedCall t{name, nullptr, nullptr};
+  const bool begun = hipEventCreate(&t.begin) == hipSuccess && hipEventCreate(&t.end) == hipSuccess &&
+                     hipEventRecord(t.begin, st) == hipSuccess;
+  auto result = fn();
+  if (begun && hipEventRecord(t.end, st) == hipSuccess) {
+    std::lock_guard<std::mutex> lock(g_timing_mutex);
+    g_calls.push_back(std::move(t));
+  } else {
+    if (t.begin) (void)hipEventDestroy(t.begin);
+    if (t.end) (void)hipEventDestroy(t.end);
+  }
+  return result;
+}
+
 template <class Fn, class... Args>
 void call(const char* name, hipStream_t st, Fn fn, Args... args) {
-  int code;
-  if (!g_timing.load(std::memory_order_relaxed)) {
-    code = fn(args..., (void*)st);
-  } else {
-    TimedCall t{name, nullptr, nullptr};
-    const bool ok = hipEventCreate(&t.begin) == hipSuccess && hipEventCreate(&t.end) == hipSuccess &&
-                    hipEventRecord(t.begin, st) == hipSuccess;
-    code = fn(args..., (void*)st);
-    if (ok && hipEventRecord(t.end, st) == hipSuccess) {
-      std::lock_guard<std::mutex> lock(g_timing_mutex);
-      g_calls.push_back(t);
-    }
-  }
+  const int code = timed(name, st, [&] { return fn(args..., (void*)st); });
   TORCH_CHECK(code == MOMOE_OK, name, " failed: status ", code, " (", momoe_status_string(code), ")");
 }
 #define MOMOE_CALL(fn, st, ...) call(#fn, st, fn, __VA_ARGS__)
@@ -477,4 +477,8 @@ PYBIND11_MODULE(_layer, m) {
   m.def("timing_start", &timing_start);
   m.def("timing_stop", &timing_stop);
   m.def("timing_take", &timing_take);
+  // a library call made from Python, recorded like those made here
+  m.def("timed", [](const std::string& name, uintptr_t stream, const py::function& fn) {
+    return timed(name.c_str(), (hipStream_t)stream, [&] { return py::object(fn()); });
+  });
 }

@@ -83,22 +83,36 @@ def status_string(code):
 
 
 class kernel_timer:
-    """Context manager: record a HIP event pair around every library call the modules make inside
-    it (on torch's current stream).  `durations_ms()` returns
-    [(entry point, milliseconds), ...] in call order."""
+    """Context manager: record a HIP event pair around every library call made inside it, by the
+    modules or through the wrappers below (on the stream of the call).  `durations_ms()`
+    synchronises and returns [(entry point, milliseconds), ...] of the calls so far, in call
+    order; it may be called inside the block as well as after it."""
+
+    _active = None  # the timer that the calls being recorded belong to
 
     def __enter__(self):
+        if kernel_timer._active is not None:
+            kernel_timer._active._collect()
+        self.records = []
+        kernel_timer._active = self
         _layer.timing_start()
         return self
 
     def __exit__(self, *exc):
         _layer.timing_stop()
-        torch.cuda.synchronize()
-        self.records = _layer.timing_take()
+        if kernel_timer._active is self:
+            self._collect()
+        kernel_timer._active = None
         return False
 
+    def _collect(self):
+        torch.cuda.synchronize()
+        self.records += _layer.timing_take()
+
     def durations_ms(self):
-        return self.records
+        if kernel_timer._active is self:
+            self._collect()
+        return list(self.records)
 
 
 class clock_trace:
@@ -169,7 +183,8 @@ def hbm_stream_probe(weights_NKC, launches=5):
 
 
 def _call(name, *args):
-    code = getattr(_lib, name)(*args)
+    # (the stream is every entry point's last argument)
+    code = _layer.timed(name, args[-1], lambda: getattr(_lib, name)(*args))
     if code != 0:
         raise RuntimeError(f"{name} failed: status {code} ({status_string(code)})")
 

@@ -298,6 +298,31 @@ def test_measurement_aids_of_the_benchmark():
     assert tf > 250 and 500 < clk < 3000, (tf, clk)
 
 
+def test_kernel_timer_inside_its_block_and_through_the_wrappers():
+    import momoe_amd
+    from momoe_amd import _hip
+    x, W1, W2, mask, s, _ = make_layer_inputs(40, 64, 32, 4, 2, seed=8)
+    dev = "cuda:0"
+    layer = momoe_amd.MoMoE(64, 32, 4, 2, Wl1_ND2H=W1.to(dev), Wl2_NHD=W2.to(dev))
+    xd, maskd, sd = x.to(dev, torch.bfloat16).reshape(1, 40, 64), mask.to(dev), s.to(dev)
+    forward = ["momoe_index_build", "momoe_lin1_swiglu_fwd", "momoe_lin2_scale_fwd", "momoe_combine"]
+    names = lambda timer: [n for n, ms in timer.durations_ms() if ms >= 0]
+    with _hip.kernel_timer() as kt, torch.no_grad():
+        assert kt.durations_ms() == []
+        layer(xd, maskd, sd)
+        assert names(kt) == forward
+        ib = _hip.index_build(maskd, 2)
+        with pytest.raises(RuntimeError, match="unsupported"):  # refused calls are calls too
+            _hip.tile_table_build(ib["cumsums_N"], 40, 2, 31)
+        layer(xd, maskd, sd)
+    want = forward + ["momoe_index_build", "momoe_tile_table_build"] + forward
+    assert names(kt) == want and names(kt) == want
+    layer(xd, maskd, sd)  # not timed
+    with _hip.kernel_timer() as kt2:
+        _hip.index_build(maskd, 2)
+    assert names(kt2) == ["momoe_index_build"] and names(kt) == want
+
+
 def test_backward_row_limit_is_reported_in_the_forward():
     # the Wl1 gradient takes fewer than 8 388 608 (token, expert) pairs per call (32-bit offsets
     # into the k-blocked gz): a larger training batch is refused before anything is launched,
