@@ -313,9 +313,8 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1A
   const Prog prog{p, 0, 0};
   const int D = p.D, H = p.H;
   FewRows op;
-  for (TileCoord t = sched.next(); t.valid; t = sched.next()) {
-    t.mbase = 0;
-    t.na = 1;
+  for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
+    const TileCoord t = FewRows::piece(left);
     op.rows(p.x, FewRows::BK, D, [&](int row, int piece) {
       return (uint32_t)p.idx[t.row0 + min(row, t.rows - 1)] * (uint32_t)(2 * D) + piece * 16;
     });
@@ -439,9 +438,8 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Ar
   const Prog prog{p, 0, 0};
   const int D = p.D, H = p.H;
   FewRows op;
-  for (TileCoord t = sched.next(); t.valid; t = sched.next()) {
-    t.mbase = 0;
-    t.na = 1;
+  for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
+    const TileCoord t = FewRows::piece(left);
     Prog::Prep prep;
     prog.gather(t, prep);
     // h is k-blocked: a stage is four blocks of 32 k-values

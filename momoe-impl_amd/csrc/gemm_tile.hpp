@@ -842,12 +842,13 @@ struct RowStager {
 };
 
 // ---- few rows: the waves share the contraction --------------------------------------------------
-// Tiles of at most 32 rows x 64 columns for the forward of calls with at most 32 tokens (no expert
-// holds more) that still have no more than one such tile per CU.  One CU pulls weights from HBM at 46
-// GB/s at most, so a call of a few experts takes as long as the CUs it uses are few, and 64
-// columns give it twice those of NarrowTiles.  To keep as many bytes on the way, a stage holds 128
-// k-values; wave w multiplies the 16 of slice w with all columns, nothing but the fragment reads
-// lies between two barriers, and the eight slices' sums meet in LDS at the end of the tile.
+// Tiles of at most 32 rows x 64 columns for the forward of calls with at most 32 tokens (an expert
+// holds no more, unless its list repeats some: piece()) that still have no more than one such tile
+// per CU.  One CU pulls weights from HBM at 46 GB/s at most, so a call of a few experts takes as long
+// as the CUs it uses are few, and 64 columns give it twice those of NarrowTiles.  To keep as many
+// bytes on the way, a stage holds 128 k-values; wave w multiplies the 16 of slice w with all
+// columns, nothing but the fragment reads lies between two barriers, and the eight slices' sums meet
+// in LDS at the end of the tile.
 // Measured against NarrowTiles, weights not in any cache: one token, 8 experts of D = 2048, H = 768: the
 // forward 35.0 -> 30.8 us; with the weights cached x.Wl1 16.6 -> 13.5 us, h.Wl2 9.1 -> 9.9 (launch and
 // the chain table -> row ids -> rows are most of both).  64 x 128 tiles with half the k-values a
@@ -956,11 +957,29 @@ struct FewRows {
         }
   }
   static __device__ __forceinline__ bf16* staging(bf16* lds) { return lds + STAGES * STAGE; }
+
+  // A tile of the table is worked on in pieces of ROWS rows: one for a mask of at most ROWS tokens,
+  // more if the caller's index lists a token several times for an expert.  t holds the rows left.
+  static __device__ __forceinline__ TileCoord piece(TileCoord t) {
+    t.rows = min(t.rows, ROWS);
+    t.mbase = 0;
+    t.na = 1;
+    return t;
+  }
+  static __device__ __forceinline__ TileCoord following(TileSched& sched, TileCoord t) {
+    if (t.rows <= ROWS) return sched.next();
+    t.row0 += ROWS;
+    t.rows -= ROWS;
+    return t;
+  }
 };
 
-// Whether a forward GEMM over `cols` output columns takes FewRows tiles.
+// Whether a forward GEMM over `cols` output columns takes FewRows tiles.  More rows than tokens x
+// experts mean repeated tokens and tiles of several pieces throughout, and their number would have
+// no bound (the offsets into h are 32-bit).
 inline bool takes_few_rows_tiles(int64_t m, int64_t msum, int64_t n, int64_t cols) {
-  return m <= FewRows::ROWS && std::min(n, msum) * cdiv64(cols, FewRows::G::COLS) <= persistent_grid();
+  return m <= FewRows::ROWS && msum <= m * n &&
+         std::min(n, msum) * cdiv64(cols, FewRows::G::COLS) <= persistent_grid();
 }
 
 }  // namespace momoe

@@ -142,6 +142,36 @@ def test_tiles_of_few_rows(M, D, H, N, K, Ks, sp):
     _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
 
 
+@pytest.mark.parametrize("rows", [32, 256, 320])
+@pytest.mark.parametrize("sizes", [[33, 0, 1, 64, 2, 0, 0, 0], [0, 0, 250, 0, 0, 0, 0, 0], [0, 700, 5, 0, 0, 31, 0, 0]])
+def test_index_that_repeats_tokens(sizes, rows):
+    """The entry points take any list of tokens per expert, also of few tokens an expert holds many times."""
+    from momoe_amd import _hip
+    M, D, H, N, dev = 32, 160, 96, len(sizes), "cuda:0"
+    x, W1, W2, _, s, _ = make_layer_inputs(M, D, H, N, 2, seed=13)
+    msum = sum(sizes)
+    cumsums = torch.zeros(N + 1, dtype=torch.int32)
+    cumsums[1:] = torch.cumsum(torch.tensor(sizes), 0)
+    idx = torch.randint(0, M, (msum,), generator=torch.Generator().manual_seed(2), dtype=torch.int32)
+    s = torch.rand(N, M, generator=torch.Generator().manual_seed(3))
+    b = lambda t: t.to(dev, torch.bfloat16)
+    table = _hip.tile_table_build(cumsums.to(dev), 1, msum, rows)
+    h = torch.full((H // 32, msum, 32), 7.0, device=dev, dtype=torch.bfloat16)
+    ys = torch.full((msum, D), 7.0, device=dev, dtype=torch.bfloat16)
+    _hip.lin1_swiglu_fwd(b(x), b(W1), idx.to(dev), table, h, None, 0, 0)
+    _hip.lin2_scale_fwd(h, b(W2), s.to(dev), idx.to(dev), table, ys, M)
+    f = lambda t: t.to(torch.bfloat16).float()
+    got_h = h.permute(1, 0, 2).reshape(msum, H).float().cpu()
+    for i in range(N):
+        r = slice(int(cumsums[i]), int(cumsums[i + 1]))
+        if sizes[i] == 0:
+            continue
+        tok = idx[r].long()
+        ab = f(x)[tok] @ f(W1)[i]
+        assert_close(got_h[r], ab[:, :H] * torch.nn.functional.silu(ab[:, H:]), f"h of expert {i}")
+        assert_close(ys[r], (got_h[r] @ f(W2)[i]) * s[i, tok][:, None], f"rows of expert {i}")
+
+
 @pytest.mark.parametrize("gather_a", [True, False])
 def test_weight_gradient_of_cut_experts(gather_a):
     # experts of 20000 / 3 / 0 / 5000 rows: the first is contracted in pieces that meet in the
