@@ -45,6 +45,7 @@ struct TileCoord {
   int tn;      // column block
   int mbase;   // first tile row owned by this wave (the wave rows split the tile's rows)
   int na;      // 32-row fragment rows owned by this wave (0..5)
+  bool alone;  // the only row tile of its expert
   bool valid;
 };
 
@@ -115,6 +116,7 @@ struct TileSchedT {
     // weight block for a handful of rows, and only the expert's last fragment row is ragged.
     const int nt = (r.mi + bm - 1) / bm * sub;
     const int nfe = (r.mi + 31) >> 5;
+    tc.alone = nt == 1;
     // halved tiles may outnumber the fragment rows: those left over do the last one again
     const int ntf = LIMIT > 0 ? min(nt, nfe) : nt;
     const int fbase = nfe / ntf, fextra = nfe - fbase * ntf;

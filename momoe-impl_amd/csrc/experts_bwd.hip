@@ -27,6 +27,7 @@ struct DhArgs {
 template <class G>
 struct DhProg {
   static constexpr int FM = G::FM, BN = G::COLS;
+  static constexpr bool MAY_ONCE = false;
   using RowsA = RDma<G::AROWS>;  // gathered token rows, k-contiguous
   using RowsB = RDma<BN>;        // weight rows, k-contiguous (an "NT" GEMM)
   using Ring = StageRing<RowsA, RowsB, G::STAGES>;  // its idle buffer is the store staging
@@ -216,6 +217,7 @@ struct DxArgs {
 template <class G>
 struct DxProg {
   static constexpr int FM = G::FM, BN = G::COLS;
+  static constexpr bool MAY_ONCE = false;
   using BlockedA = RBlockedDma<G::AROWS>;  // sorted rows of the k-blocked gz
   using RowsB = RDma<BN>;                  // weight rows, k-contiguous
   using Ring = StageRing<BlockedA, RowsB, G::STAGES>;

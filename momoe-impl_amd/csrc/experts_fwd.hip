@@ -41,8 +41,9 @@ template <bool BWD, class G>
 struct Lin1Prog {
   static_assert(!BWD || G::MAX_ROWS == StdTiles::MAX_ROWS, "the SwiGLU backward epilogue fits 256-row tiles only");
   static constexpr int FM = G::FM, BM = G::MAX_ROWS, BN = G::COLS;
+  static constexpr bool MAY_ONCE = G::MAY_ONCE;
   using RowsOp = RDma<G::AROWS>;  // token rows, k-contiguous
-  using WeightOp = TDmaT<BN, G::ONCE>;     // expert weights [k][col], k-strided
+  using WeightOp = TDmaT<BN, MAY_ONCE>;  // expert weights [k][col], k-strided
   using Ring = StageRing<RowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   static constexpr int BNH = BN / 2;
@@ -76,6 +77,7 @@ struct Lin1Prog {
     const int j0 = t.tn * BNH;
     A.init(p.x, [&](int, int j) { return (uint32_t)g.tok[j] * (uint32_t)(2 * D); });
     B.init(w, [&](int c) { return (c / BNH) * H + min(j0 + (c % BNH), H - 8); }, 2 * H);
+    if (MAY_ONCE) B.once = t.alone;
   }
   // epi: store staging; in the backward also the row-sum exchange
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x16 (&acc)[FN][FM], const Prep& g, bf16* epi) const {
@@ -265,33 +267,34 @@ __device__ __forceinline__ void lin1_swiglu_tiles(const Lin1Args& p) {
   run_row_tiles<FM, FN>(prog, sched, ring, n_org);
 }
 
-// The forward holds both geometries and follows the tile table it is given.
-template <bool BWD>
+// The forward holds two geometries, Short for tables of at most 256 rows, and follows the tile table
+// it is given.
+template <bool BWD, class Short>
 __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_kernel(Lin1Args p) {
   const ClockTrace trace(p.clk);
   if constexpr (BWD) {
-    lin1_swiglu_tiles<true, StdTiles>(p);
+    lin1_swiglu_tiles<true, Short>(p);
   } else {
-    if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) lin1_swiglu_tiles<false, TallTiles>(p);
-    else lin1_swiglu_tiles<false, StdTiles>(p);
+    if (TileSched::tile_rows_of(p.table) > Short::MAX_ROWS) lin1_swiglu_tiles<false, TallTiles>(p);
+    else lin1_swiglu_tiles<false, Short>(p);
   }
   trace.finish();
 }
-// One geometry only (NarrowTiles, OnceTiles).
-template <class G>
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_geometry_kernel(Lin1Args p) {
-  const ClockTrace trace(p.clk);
-  lin1_swiglu_tiles<false, G, OneGeometrySched<G>>(p);
-  trace.finish();
-}
-template <class G>
-int launch_lin1_geometry(const Lin1Args& a, hipStream_t st) {
+template <bool BWD, class Short>
+int launch_lin1(const Lin1Args& a, hipStream_t st) {
   static LdsLimit lds;
-  constexpr size_t bytes = Lin1Prog<false, G>::kLds;
-  if (!allow_lds(lin1_swiglu_geometry_kernel<G>, bytes, lds)) return MOMOE_ERR_LAUNCH;
-  lin1_swiglu_geometry_kernel<G><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  constexpr size_t bytes =
+      BWD ? Lin1Prog<BWD, Short>::kLds : std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, Short>::kLds);
+  if (!allow_lds(lin1_swiglu_kernel<BWD, Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin1_swiglu_kernel<BWD, Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
 }
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  lin1_swiglu_tiles<false, NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  trace.finish();
+}
+constexpr size_t kLin1FwdNarrowLds = Lin1Prog<false, NarrowTiles>::kLds;
 
 // The SwiGLU backward on NarrowTiles: twice as many partial row sums, each over 64 hidden columns.
 // 1024 tokens over 32 experts, D = 1024, H = 512: 27.5 -> 21.6 us.
@@ -329,8 +332,6 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1A
   }
   trace.finish();
 }
-constexpr size_t kLin1FwdLds = std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, StdTiles>::kLds);
-constexpr size_t kLin1BwdLds = Lin1Prog<true, StdTiles>::kLds;
 
 struct Lin2Args {
   const bf16* h;
@@ -348,8 +349,9 @@ struct Lin2Args {
 template <class G>
 struct Lin2Prog {
   static constexpr int FM = G::FM, BN = G::COLS;
+  static constexpr bool MAY_ONCE = G::MAY_ONCE;
   using HRowsOp = RBlockedDma<G::AROWS>;  // rows of h, k-blocked
-  using WeightOp = TDmaT<BN, G::ONCE>;             // expert weights [k][col], k-strided
+  using WeightOp = TDmaT<BN, MAY_ONCE>;  // expert weights [k][col], k-strided
   using Ring = StageRing<HRowsOp, WeightOp, G::STAGES>;
   static constexpr size_t kLds = Ring::BYTES;
   struct Prep {
@@ -373,6 +375,7 @@ struct Lin2Prog {
     const int d0 = t.tn * BN;
     A.init(p.h, p.msum, t.row0, t.rows);
     B.init(w, [&](int c) { return min(d0 + c, D - 8); }, D);
+    if (MAY_ONCE) B.once = t.alone;
   }
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x16 (&acc)[FN][FM], const Prep& g, bf16* epi) const {
     const int D = p.D;
@@ -408,26 +411,27 @@ __device__ __forceinline__ void lin2_scale_tiles(const Lin2Args& p) {
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
 }
 
+template <class Short>
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
-  if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) lin2_scale_tiles<TallTiles>(p);
-  else lin2_scale_tiles<StdTiles>(p);
+  if (TileSched::tile_rows_of(p.table) > Short::MAX_ROWS) lin2_scale_tiles<TallTiles>(p);
+  else lin2_scale_tiles<Short>(p);
   trace.finish();
 }
-template <class G>
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_geometry_kernel(Lin2Args p) {
-  const ClockTrace trace(p.clk);
-  lin2_scale_tiles<G, OneGeometrySched<G>>(p);
-  trace.finish();
-}
-template <class G>
-int launch_lin2_geometry(const Lin2Args& a, hipStream_t st) {
+template <class Short>
+int launch_lin2(const Lin2Args& a, hipStream_t st) {
   static LdsLimit lds;
-  constexpr size_t bytes = Lin2Prog<G>::kLds;
-  if (!allow_lds(lin2_scale_geometry_kernel<G>, bytes, lds)) return MOMOE_ERR_LAUNCH;
-  lin2_scale_geometry_kernel<G><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  constexpr size_t bytes = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<Short>::kLds);
+  if (!allow_lds(lin2_scale_kernel<Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin2_scale_kernel<Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
 }
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
+  const ClockTrace trace(p.clk);
+  lin2_scale_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  trace.finish();
+}
+constexpr size_t kLin2NarrowLds = Lin2Prog<NarrowTiles>::kLds;
 
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
   using Prog = Lin2Prog<FewRows::G>;
@@ -458,7 +462,6 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Ar
   }
   trace.finish();
 }
-constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<StdTiles>::kLds);
 
 // out[m] = sum_k rows[inv[m,k]]: one workgroup per token, 16-byte loads, fp32 accumulate.
 // The row numbers and then the rows are fetched 8 at a time with unconditional loads (a missing
@@ -533,12 +536,14 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
     lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, 2 * H)) return launch_lin1_geometry<NarrowTiles>(a, (hipStream_t)stream);
-  if (weights_read_once(Msum, N, 4 * N * D * H)) return launch_lin1_geometry<OnceTiles>(a, (hipStream_t)stream);
-  static LdsLimit lds;
-  if (!allow_lds(lin1_swiglu_kernel<false>, kLin1FwdLds, lds)) return MOMOE_ERR_LAUNCH;
-  lin1_swiglu_kernel<false><<<persistent_grid(), kThreads, kLin1FwdLds, (hipStream_t)stream>>>(a);
-  return launch_status();
+  if (takes_narrow_tiles(Msum, N, 2 * H)) {
+    static LdsLimit narrow;
+    if (!allow_lds(lin1_swiglu_narrow_kernel, kLin1FwdNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    lin1_swiglu_narrow_kernel<<<persistent_grid(), kThreads, kLin1FwdNarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
+  if (weights_read_once(Msum, N, 4 * N * D * H)) return launch_lin1<false, OnceTiles>(a, (hipStream_t)stream);
+  return launch_lin1<false, StdTiles>(a, (hipStream_t)stream);
 }
 
 extern "C" int64_t momoe_gs_parts(int64_t H, int64_t N, int64_t Msum) {
@@ -587,10 +592,7 @@ extern "C" int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2
     lin1_swiglu_bwd_narrow_kernel<<<persistent_grid(), kThreads, kLin1BwdNarrowLds, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  static LdsLimit lds;
-  if (!allow_lds(lin1_swiglu_kernel<true>, kLin1BwdLds, lds)) return MOMOE_ERR_LAUNCH;
-  lin1_swiglu_kernel<true><<<persistent_grid(), kThreads, kLin1BwdLds, (hipStream_t)stream>>>(a);
-  return launch_status();
+  return launch_lin1<true, StdTiles>(a, (hipStream_t)stream);
 }
 
 extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, const float* s_NM,
@@ -612,12 +614,14 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
     lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, D)) return launch_lin2_geometry<NarrowTiles>(a, (hipStream_t)stream);
-  if (weights_read_once(Msum, N, 2 * N * D * H)) return launch_lin2_geometry<OnceTiles>(a, (hipStream_t)stream);
-  static LdsLimit lds;
-  if (!allow_lds(lin2_scale_kernel, kLin2Lds, lds)) return MOMOE_ERR_LAUNCH;
-  lin2_scale_kernel<<<persistent_grid(), kThreads, kLin2Lds, (hipStream_t)stream>>>(a);
-  return launch_status();
+  if (takes_narrow_tiles(Msum, N, D)) {
+    static LdsLimit narrow;
+    if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+    lin2_scale_narrow_kernel<<<persistent_grid(), kThreads, kLin2NarrowLds, (hipStream_t)stream>>>(a);
+    return launch_status();
+  }
+  if (weights_read_once(Msum, N, 2 * N * D * H)) return launch_lin2<OnceTiles>(a, (hipStream_t)stream);
+  return launch_lin2<StdTiles>(a, (hipStream_t)stream);
 }
 
 extern "C" int momoe_combine(const void* rows_MsumD, const int32_t* inv_MK, void* out_MD,

@@ -245,15 +245,18 @@ struct TLayoutT {
 
 using TLayout = TLayoutT<256>;
 
-// k-strided operand with a fixed pitch between k-rows (the expert weights)
-template <int COLS, bool ONCE = false>
+// k-strided operand with a fixed pitch between k-rows (the expert weights).  MAY_ONCE: the tiles for
+// which `once` is set read it with the non-temporal hint.
+template <int COLS, bool MAY_ONCE_ = false>
 struct TDmaT {
+  static constexpr bool MAY_ONCE = MAY_ONCE_;
   using L = TLayoutT<COLS>;
   static constexpr int NCH = L::NCH;
   static constexpr int LDS_ELEMS = L::LDS_ELEMS;
   const bf16* base;   // wave-uniform
   uint32_t off[NCH];  // byte offset of this lane's piece of deposit j from `base`, at k=0
   int64_t kstride;
+  int once = 0;  // wave-uniform
 
   // coloff(c) -> element offset from base_ of (k=0, tile column c), c a multiple of 8;
   // columns outside the matrix must be clamped by the caller to something readable.
@@ -269,10 +272,15 @@ struct TDmaT {
     }
     kstride = (int64_t)kBK * ld;
   }
-  __device__ __forceinline__ void issue(int kt, uint32_t stage) {
+  template <bool ONCE>
+  __device__ __forceinline__ void issue_as(int kt, uint32_t stage) {
     const bf16* b = base + kt * kstride;
 #pragma unroll
     for (int j = 0; j < NCH; ++j) dma16<ONCE>(b, off[j], L::deposit(stage, j));
+  }
+  __device__ __forceinline__ void issue(int kt, uint32_t stage) {
+    if (MAY_ONCE && __builtin_amdgcn_readfirstlane(once)) issue_as<true>(kt, stage);
+    else issue_as<false>(kt, stage);
   }
   template <int S>
   __device__ __forceinline__ void issue_head(uint32_t stage) { issue(S, stage); }
@@ -282,6 +290,15 @@ struct TDmaT {
 };
 
 using TDma = TDmaT<256>;
+
+// Such an operand within a tile whose choice is known: no branch in the main loop.
+template <class Op, bool ONCE>
+struct KnownOnce {
+  static constexpr int NCH = Op::NCH, LDS_ELEMS = Op::LDS_ELEMS;
+  Op& op;
+  __device__ __forceinline__ void issue(int kt, uint32_t stage) { op.template issue_as<ONCE>(kt, stage); }
+  static __device__ __forceinline__ bf16x8 frag(const bf16* stage, int c0, int kk) { return Op::frag(stage, c0, kk); }
+};
 
 // k-strided operand whose k-rows are the sorted rows [row_begin,row_end) of one expert,
 // optionally gathered through an index.  k-rows past row_end are pointed at the expert's last
@@ -426,8 +443,8 @@ struct StageRing {
   __device__ __forceinline__ bf16* free_buf() const { return lds + slot(head + FIRST) * STAGE; }
 };
 
-template <class AOp, class BOp, int NS>
-__device__ __forceinline__ void gemm_issue(AOp& A, BOp& B, StageRing<AOp, BOp, NS>& ring, int kt) {
+template <class AOp, class BOp, class Ring>
+__device__ __forceinline__ void gemm_issue(AOp& A, BOp& B, Ring& ring, int kt) {
   const uint32_t st = ring.buf_addr(kt);
   A.issue(kt, st);
   B.issue(kt, st + AOp::LDS_ELEMS * 2);
@@ -490,9 +507,9 @@ __device__ __forceinline__ void wait_stage(int kt, int ktiles) {
 // under the whole main loop (they enter the vmcnt queue between two stages, which can only
 // make the stage waits err on the long side).  On return the ring has advanced to the next
 // tile; all buffers but the last stage's are free, other waves may still be reading that one.
-template <class AOp, class BOp, int NS, int FM, int FN, int NA, class Hook>
+template <class AOp, class BOp, int NS, int FM, int FN, int NA, class Ring, class Hook>
 __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][FM], int ktiles,
-                                              StageRing<AOp, BOp, NS>& ring, const int (&m_org)[FM],
+                                              Ring& ring, const int (&m_org)[FM],
                                               const int (&n_org)[FN], Hook hook, int ktail = kBK) {
   constexpr int kStages = NS, kFirst = NS - 1;
   static_assert(kKSteps == 2, "written for 2 k-steps per stage");
@@ -576,9 +593,9 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
 // Row-tile geometry of a kernel: WROWS wave rows of FM 32-row fragment rows each (tiles of up to
 // 32 * WROWS * FM rows, 64 columns per wave), the rows of the row operand's stage buffer (whole deposits
 // of 16 rows per wave, so a multiple of 128 that holds the tallest tile) and the ring depth.
-template <int FM_, int NS_, int WROWS_ = 2, bool ONCE_ = false>
+template <int FM_, int NS_, int WROWS_ = 2, bool MAY_ONCE_ = false>
 struct RowTileGeometry {
-  static constexpr bool ONCE = ONCE_;  // an expert's weights are read by one row tile
+  static constexpr bool MAY_ONCE = MAY_ONCE_;  // weights that one row tile reads take the non-temporal hint
   static constexpr int FM = FM_, FN = 2;
   static constexpr int WROWS = WROWS_, WCOLS = kWaves / WROWS;  // the waves' arrangement
   static constexpr int COLS = 64 * WCOLS;
@@ -607,19 +624,19 @@ using NarrowTiles = RowTileGeometry<2, 4, 4>;
 // tile order of a kernel that holds one geometry of 256-row tiles whatever the table's height
 template <class G>
 using OneGeometrySched = TileSchedT<G::WROWS, G::MAX_ROWS>;
-// StdTiles whose k-strided weights are read with the non-temporal hint, for experts that are a
-// single row tile: their weights then pass through the L2 once and leave the token rows in it,
-// and HBM delivers a stream of such reads faster.  (k-contiguous weights come as half lines, a
-// stage apart: with the hint the second half is fetched again, dL/dh 112 -> 152 us.)
+// StdTiles that read the k-strided weights of an expert that is a single row tile with the
+// non-temporal hint: they then pass through the L2 once and leave the token rows in it, and HBM
+// delivers a stream of such reads faster.  An expert of several row tiles reads its weights several
+// times, all but the first out of the caches, so its tiles go without.  (k-contiguous weights come as
+// half lines, a stage apart: with the hint the second half is fetched again, dL/dh 112 -> 152 us.)
 using OnceTiles = RowTileGeometry<4, 4, 2, true>;
 static_assert(TallTiles::MAX_ROWS == MOMOE_TILE_ROWS && StdTiles::MAX_ROWS == MOMOE_RECOMPUTE_TILE_ROWS,
               "tile heights promised by the header");
 
 // main loop for a wave that owns `na` fragment rows starting at tile row m_org[0]
-template <class AOp, class BOp, int NS, int FM, int FN, class Hook>
-__device__ __forceinline__ void gemm_rows(AOp& A, BOp& B, f32x16 (&acc)[FN][FM], int ktiles,
-                                          StageRing<AOp, BOp, NS>& ring, const int (&m_org)[FM],
-                                          const int (&n_org)[FN], int na_, Hook hook) {
+template <class AOp, class BOp, int NS, int FM, int FN, class Ring, class Hook>
+__device__ __forceinline__ void gemm_rows(AOp& A, BOp& B, f32x16 (&acc)[FN][FM], int ktiles, Ring& ring,
+                                          const int (&m_org)[FM], const int (&n_org)[FN], int na_, Hook hook) {
   static_assert(FM == 2 || FM == 4 || FM == 5, "dispatch written for 2, 4 or 5 fragment rows per wave");
   const int na = __builtin_amdgcn_readfirstlane(na_);
   if constexpr (FM == 5) {
@@ -696,6 +713,12 @@ inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
 // 768, N = 128, K = 8 with cold weights, a forward without -> with the hint: 16 tokens 143 -> 130
 // us, 131 tokens 223 -> 202, 1000 (62 rows per expert) 261 -> 247, 1300 (81) 273 -> 261; at 162
 // rows it is slower (h.Wl2 117 -> 119), at 512 x.Wl1 by 4 %: the line lies at a third of a tile.
+// The mean is all the host knows; of a skewed routing the tiles themselves decide (TileCoord::alone).
+// A forward without the hint -> with it on every tile -> on the tiles that are their expert's only
+// one: 1000 tokens, two shared experts, 321 -> 319 -> 294 us; load falling as rank^-1.8, 1300 tokens,
+// 226 -> 260 -> 227; 600 tokens, D = 4096, H = 2048, N = 48, K = 6, 463 -> 525 -> 463; a table of
+// 320-row tiles (D = 4096, H = 1024, N = 64, K = 4, two shared), which takes TallTiles without
+// it, 219 -> 266 (halved tiles) -> 216.
 // Matrices that fit the 256 MiB last-level cache keep their place in it without the hint: a step
 // whose backward reads them again took 175 -> 191 us (1000 tokens, 128 MB).  For the same reason
 // the recomputing GEMM goes without it: dL/dx reads Wl1 again, and with the hint a step took
@@ -737,6 +760,7 @@ __device__ __forceinline__ void store_bf16x4(bf16* p, float a, float b, float c,
 //   epilogue(tile, acc, prep, staging)        may use late()'s results; staging = kEpilogueLds
 //                                             bytes of LDS for the workgroup
 //   ktiles                                    stages per tile
+//   MAY_ONCE                                  B is a TDmaT whose setup sets `once` for the tiles that are alone
 // While tile t is multiplied: the table entry of tile t+2 and the gathered values of tile t+1
 // are in flight; after its main loop the first stages of tile t+1 are requested, then the
 // epilogue of tile t runs.
@@ -761,11 +785,21 @@ __device__ __forceinline__ void run_row_tiles(P& prog, Sched& sched, StageRing<A
     int m_org[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) m_org[i] = c0.mbase + 32 * i;
-    gemm_rows<AOp, BOp, NS, FM, FN>(A, B, acc, prog.ktiles, ring, m_org, n_org, c0.na, [&] {
+    auto hook = [&] {
       prog.late(c0, p0);
       if (c1.valid) prog.gather(c1, p1);
       rn = sched.fetch();
-    });
+    };
+    if constexpr (P::MAY_ONCE) {
+      KnownOnce<BOp, true> once{B};
+      KnownOnce<BOp, false> again{B};
+      if (__builtin_amdgcn_readfirstlane(c0.alone))
+        gemm_rows<AOp, decltype(once), NS, FM, FN>(A, once, acc, prog.ktiles, ring, m_org, n_org, c0.na, hook);
+      else
+        gemm_rows<AOp, decltype(again), NS, FM, FN>(A, again, acc, prog.ktiles, ring, m_org, n_org, c0.na, hook);
+    } else {
+      gemm_rows<AOp, BOp, NS, FM, FN>(A, B, acc, prog.ktiles, ring, m_org, n_org, c0.na, hook);
+    }
     if (c1.valid) {
       prog.setup(c1, p1, A, B);
       gemm_issue_first(A, B, ring, prog.ktiles);  // travels during this tile's epilogue
