@@ -90,11 +90,14 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
   const ClockTrace trace(p.clk);
-  dgrad_h_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  if (narrow_tiles_fit(p.table, (p.H + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+    dgrad_h_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  else
+    dgrad_h_tiles<StdTiles>(p);
   trace.finish();
 }
-constexpr size_t kDhNarrowLds = DhProg<NarrowTiles>::Ring::BYTES;
 constexpr size_t kDhLds = std::max(DhProg<TallTiles>::Ring::BYTES, DhProg<StdTiles>::Ring::BYTES);
+constexpr size_t kDhNarrowLds = std::max(DhProg<NarrowTiles>::Ring::BYTES, DhProg<StdTiles>::Ring::BYTES);
 
 // SwiGLU backward for the sorted rows whose a|b were saved by the forward.  One workgroup per
 // group of 32 padded sorted rows (an expert's rows start at a multiple of 32 in padded
@@ -275,11 +278,14 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
   const ClockTrace trace(p.clk);
-  dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  if (narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+    dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  else
+    dgrad_x_tiles<StdTiles>(p);
   trace.finish();
 }
-constexpr size_t kDxNarrowLds = DxProg<NarrowTiles>::Ring::BYTES;
 constexpr size_t kDxLds = std::max(DxProg<TallTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
+constexpr size_t kDxNarrowLds = std::max(DxProg<NarrowTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
 
 // dL/ds [N][M] from the partial row sums in sorted order.  One workgroup per (expert, kGsTokens
 // tokens) writes its piece whole, zeros included, through LDS: every line of the matrix is stored

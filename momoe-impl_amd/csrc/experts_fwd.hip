@@ -244,7 +244,10 @@ struct Lin1Prog {
       float sum = red[threadIdx.x];
 #pragma unroll
       for (int w = 1; w < G::WCOLS; ++w) sum += red[w * BM + threadIdx.x];
-      p.gs_part[(int64_t)tc.tn * p.msum + tc.row0 + threadIdx.x] = sum;
+      float* part = p.gs_part + (int64_t)tc.tn * (G::HALF_PARTS ? 2 : 1) * p.msum + tc.row0 + threadIdx.x;
+      *part = sum;
+      // (the columns' second half has its share in the first part)
+      if (G::HALF_PARTS && j0 - wn * 32 + BNH / 2 < H) part[p.msum] = 0.0f;
     }
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();  // `red` is rewritten by the next tile
@@ -289,21 +292,27 @@ int launch_lin1(const Lin1Args& a, hipStream_t st) {
   lin1_swiglu_kernel<BWD, Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
 }
+// Few tiles: NarrowTiles if the table holds as few as the launch was chosen for.  The SwiGLU backward
+// writes twice as many partial row sums, each over 64 hidden columns: 1024 tokens over 32 experts,
+// D = 1024, H = 512: 27.5 -> 21.6 us.
+template <bool BWD>
 __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Args p) {
+  // the backward's table has no taller tiles
+  using Sched = std::conditional_t<BWD, TileSchedT<NarrowTiles::WROWS>, OneGeometrySched<NarrowTiles>>;
+  constexpr int BNH = NarrowTiles::COLS / 2;
   const ClockTrace trace(p.clk);
-  lin1_swiglu_tiles<false, NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  if (narrow_tiles_fit(p.table, (p.H + BNH - 1) / BNH)) lin1_swiglu_tiles<BWD, NarrowTiles, Sched>(p);
+  else lin1_swiglu_tiles<BWD, StdTilesHalfParts>(p);
   trace.finish();
 }
-constexpr size_t kLin1FwdNarrowLds = Lin1Prog<false, NarrowTiles>::kLds;
-
-// The SwiGLU backward on NarrowTiles: twice as many partial row sums, each over 64 hidden columns.
-// 1024 tokens over 32 experts, D = 1024, H = 512: 27.5 -> 21.6 us.
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_bwd_narrow_kernel(Lin1Args p) {
-  const ClockTrace trace(p.clk);
-  lin1_swiglu_tiles<true, NarrowTiles, TileSchedT<NarrowTiles::WROWS>>(p);
-  trace.finish();
+template <bool BWD>
+int launch_lin1_narrow(const Lin1Args& a, hipStream_t st) {
+  static LdsLimit lds;
+  constexpr size_t bytes = std::max(Lin1Prog<BWD, NarrowTiles>::kLds, Lin1Prog<BWD, StdTilesHalfParts>::kLds);
+  if (!allow_lds(lin1_swiglu_narrow_kernel<BWD>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin1_swiglu_narrow_kernel<BWD><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  return launch_status();
 }
-constexpr size_t kLin1BwdNarrowLds = Lin1Prog<true, NarrowTiles>::kLds;
 
 // The few-row tiles (FewRows): its own operands and loop, the epilogue of the narrow ones.
 __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p) {
@@ -428,10 +437,13 @@ int launch_lin2(const Lin2Args& a, hipStream_t st) {
 }
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
-  lin2_scale_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  if (narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+    lin2_scale_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
+  else
+    lin2_scale_tiles<StdTiles>(p);
   trace.finish();
 }
-constexpr size_t kLin2NarrowLds = Lin2Prog<NarrowTiles>::kLds;
+constexpr size_t kLin2NarrowLds = std::max(Lin2Prog<NarrowTiles>::kLds, Lin2Prog<StdTiles>::kLds);
 
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
   using Prog = Lin2Prog<FewRows::G>;
@@ -536,12 +548,7 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
     lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, 2 * H)) {
-    static LdsLimit narrow;
-    if (!allow_lds(lin1_swiglu_narrow_kernel, kLin1FwdNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    lin1_swiglu_narrow_kernel<<<persistent_grid(), kThreads, kLin1FwdNarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
-  }
+  if (takes_narrow_tiles(Msum, N, 2 * H)) return launch_lin1_narrow<false>(a, (hipStream_t)stream);
   if (weights_read_once(Msum, N, 4 * N * D * H)) return launch_lin1<false, OnceTiles>(a, (hipStream_t)stream);
   return launch_lin1<false, StdTiles>(a, (hipStream_t)stream);
 }
@@ -586,12 +593,7 @@ extern "C" int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2
   Lin1Args a{(const bf16*)x_MD, (const bf16*)Wl1_ND2H, idx_Msum, tile_table, nullptr, nullptr,
              row_lo, Msum, (int)D, (int)H, (const bf16*)u_MsumH, s_NM, s_stride_n, s_stride_m,
              (bf16*)gz_blocked, (bf16*)hsT_GH32, ld_hsT, gs_part, Msum, clock_trace_buffer()};
-  if (narrow) {
-    static LdsLimit lds_narrow;
-    if (!allow_lds(lin1_swiglu_bwd_narrow_kernel, kLin1BwdNarrowLds, lds_narrow)) return MOMOE_ERR_LAUNCH;
-    lin1_swiglu_bwd_narrow_kernel<<<persistent_grid(), kThreads, kLin1BwdNarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
-  }
+  if (narrow) return launch_lin1_narrow<true>(a, (hipStream_t)stream);
   return launch_lin1<true, StdTiles>(a, (hipStream_t)stream);
 }
 

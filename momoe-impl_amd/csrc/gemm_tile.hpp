@@ -596,6 +596,7 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
 template <int FM_, int NS_, int WROWS_ = 2, bool MAY_ONCE_ = false>
 struct RowTileGeometry {
   static constexpr bool MAY_ONCE = MAY_ONCE_;  // weights that one row tile reads take the non-temporal hint
+  static constexpr bool HALF_PARTS = false;
   static constexpr int FM = FM_, FN = 2;
   static constexpr int WROWS = WROWS_, WCOLS = kWaves / WROWS;  // the waves' arrangement
   static constexpr int COLS = 64 * WCOLS;
@@ -621,6 +622,10 @@ using TallTiles = RowTileGeometry<5, 4>;
 // H = 768: x.Wl1 20.0 -> 16.6, h.Wl2 10.8 -> 9.1.  A fifth stage, or half the row deposits for calls of
 // few tokens, changed nothing.
 using NarrowTiles = RowTileGeometry<2, 4, 4>;
+// StdTiles of a SwiGLU backward that has a partial dL/ds per 64 hidden columns, as NarrowTiles write it
+struct StdTilesHalfParts : StdTiles {
+  static constexpr bool HALF_PARTS = true;
+};
 // tile order of a kernel that holds one geometry of 256-row tiles whatever the table's height
 template <class G>
 using OneGeometrySched = TileSchedT<G::WROWS, G::MAX_ROWS>;
@@ -699,14 +704,27 @@ inline int persistent_grid() {
   return (cus + 7) / 8 * 8;
 }
 
-// Whether a launch over `cols` output columns takes NarrowTiles: with them there is still no more
-// than one tile per CU.  The routing is not known here; its row tiles are taken as if every expert
-// held a quarter more than its share (an estimate off the mark costs speed only).  Beyond one
-// tile per CU the weights' way from HBM sets the pace: dL/dh of 1000 tokens over 128 experts with
-// 768 columns takes 112 us in two rounds of wide tiles, 113 in three of narrow ones.
+// Whether a launch over `cols` output columns takes the kernel that holds NarrowTiles: if with them
+// there is still no more than one tile per CU.  The routing is not known here; its row tiles are taken as
+// if every expert held a quarter more than its share, and the kernel goes by the table
+// (narrow_tiles_fit).  Beyond one tile per CU the weights' way from HBM sets the pace: dL/dh of 1000
+// tokens over 128 experts with 768 columns takes 112 us in two rounds of wide tiles, 113 in three of
+// narrow ones.
 inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
   const int64_t row_tiles = std::min(n, msum) * std::max<int64_t>(1, cdiv64(5 * msum, 4 * n * StdTiles::MAX_ROWS));
   return 2 * row_tiles * cdiv64(cols, StdTiles::COLS) <= persistent_grid();
+}
+
+// In that kernel: whether the table's tiles in `nb` column blocks of NarrowTiles are at most one per
+// workgroup; if not it takes StdTiles.  Forward and step with D = 1024, H = 512, N = 32, K = 4, wide
+// tiles -> narrow ones regardless -> by this rule, us: 1024 tokens, one expert shared (37 tiles x 8) 66
+// -> 79 -> 67 and 249 -> 265 -> 247; 320 tokens, one shared (33 x 8) 55 -> 59 -> 54 and 168 -> 175 ->
+// 163; 700 tokens, load falling as rank^-1.8 (25 x 8) 57 -> 43 -> 43 and 205 -> 166 -> 168.
+// Tables of 320-row tiles stay narrow, halved.  Past 2 x 256 halves that may lose (33 x 8: 70 -> 67 or
+// 71 -> 76 us, 39 x 8: 71 -> 82), but TallTiles in this kernel too cost every launch 0.5 us.
+__device__ __forceinline__ bool narrow_tiles_fit(const int32_t* table, int nb) {
+  const int tiles = load_uniform(table), rows = load_uniform(table + 1);  // both at once
+  return __builtin_expect((rows > StdTiles::MAX_ROWS) | (tiles * nb <= (int)gridDim.x), 1);
 }
 
 // Whether a launch over weight matrices of `weight_bytes` takes OnceTiles.  Measured at D = 2048, H =
