@@ -44,7 +44,8 @@ def _compile_layer():
     import sysconfig
     from torch.utils import cpp_extension
     obj = os.path.join(OBJ, "layer_binding.o")
-    inc = [f"-I{p}" for p in [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_path("include")]]
+    # "cuda" adds the include directory of the ROCm that torch finds, as library_paths does below
+    inc = [f"-I{p}" for p in [*cpp_extension.include_paths("cuda"), sysconfig.get_path("include")]]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-Wno-deprecated-declarations",
            *inc, "-c", os.path.join(CSRC, "layer_binding.cpp"), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
