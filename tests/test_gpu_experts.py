@@ -516,6 +516,50 @@ def test_forward_mode_is_refused(grad):
             moe(dual)
 
 
+@pytest.mark.parametrize("M,D,H,N,K,sp", [
+    (300, 128, 96, 8, 3, 40),      # few tiles: the module has a partial dL/ds per 64 hidden columns
+    (2000, 352, 288, 72, 3, 100),
+    (2000, 352, 288, 72, 3, 0),
+])
+def test_entry_points_one_by_one(M, D, H, N, K, sp):
+    """The launch sequence of a forward and backward through the C entry points, in buffers of the
+    caller's own, gives what the module gives."""
+    from momoe_amd import _hip
+    dev = "cuda:0"
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=9)
+    want = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+    b = lambda t: t.to(dev, torch.bfloat16)
+    new = lambda *size, dtype=torch.bfloat16: torch.full(size, 7, device=dev, dtype=dtype)
+    x, W1, W2, Gy, sd = b(x), b(W1), b(W2), b(dy), s.T.contiguous().to(dev).T
+    msum, msave = M * K, M * K * sp // 100
+    ib = _hip.index_build(mask.to(dev), K, recompute_table=True)
+    idx, cumsums, inv, table = (ib[k] for k in ("idx_Msum", "cumsums_N", "inv_MK", "tile_table"))
+
+    h, ab, ys, y = new(H // 32, msum, 32), new(msave, 2 * H) if msave else None, new(msum, D), new(M, D)
+    _hip.lin1_swiglu_fwd(x, W1, idx, table, h, ab, 0, msave)
+    _hip.lin2_scale_fwd(h, W2, sd, idx, table, ys, M)
+    _hip.combine(ys, inv, y)
+
+    u, gz, hsT = new(msum, H), new(2 * H // 32, msum, 32), new(_hip.padded_rows(msum, N) // 32, H, 32)
+    gs_part, Gs = new(-(-H // _hip.GS_BLOCK), msum, dtype=torch.float32), new(N, M, dtype=torch.float32)
+    GW1, GW2, gxs, Gx = new(N, D, 2 * H), new(N, H, D), new(msum, D), new(M, D)
+    ws = lambda X, Y: min(msum * H * 2, _hip.wgrad_workspace_bytes(N, X, Y, msum))
+    _hip.dgrad_h(Gy, W2, idx, table, u)
+    if msave:
+        _hip.swiglu_bwd_saved(ab, u, sd, idx, cumsums, msave, gz, hsT, gs_part)
+    _hip.lin1_swiglu_bwd(x, W1, idx, ib["recompute_table"], u, sd, msave, gz, hsT, gs_part)
+    _hip.gs_scatter(gs_part, idx, cumsums, Gs)
+    _hip.wgrad(hsT, None, Gy, idx, cumsums, GW2, M, msum, workspace_bytes=ws(H, D), a_transposed=True)
+    _hip.wgrad(x, idx, gz, None, cumsums, GW1, M, msum, workspace_bytes=ws(D, 2 * H), b_kblocked=True)
+    _hip.dgrad_x(gz, W1, table, gxs, M)
+    _hip.combine(gxs, inv, Gx)
+    torch.cuda.synchronize()
+    for k, got in (("sizes", ib["sizes_N"]), ("y", y), ("G_x", Gx), ("G_W1", GW1), ("G_W2", GW2)):
+        assert torch.equal(got.cpu(), want[k]), k
+    # fp32 sums of at most ceil(H/64) partial sums in another grouping
+    torch.testing.assert_close(Gs.cpu(), want["G_s"], rtol=1e-5, atol=1e-5 * want["G_s"].abs().max().item())
+
+
 def test_recomputing_gemm_ignores_a_table_of_taller_tiles():
     """momoe_lin1_swiglu_bwd takes row tiles of at most 256 rows: given the 320-row table of the other
     GEMMs it must leave its outputs alone instead of computing on tiles it cannot hold."""
