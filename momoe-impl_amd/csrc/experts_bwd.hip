@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
   const ClockTrace trace(p.clk);
-  if (narrow_tiles_fit(p.table, (p.H + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+  if (__builtin_expect(narrow_tiles_fit(p.table, (p.H + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     dgrad_h_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
     dgrad_h_tiles<StdTiles>(p);
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
   const ClockTrace trace(p.clk);
-  if (narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+  if (__builtin_expect(narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
     dgrad_x_tiles<StdTiles>(p);

@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Arg
   using Sched = std::conditional_t<BWD, TileSchedT<NarrowTiles::WROWS>, OneGeometrySched<NarrowTiles>>;
   constexpr int BNH = NarrowTiles::COLS / 2;
   const ClockTrace trace(p.clk);
-  if (narrow_tiles_fit(p.table, (p.H + BNH - 1) / BNH)) lin1_swiglu_tiles<BWD, NarrowTiles, Sched>(p);
+  if (__builtin_expect(narrow_tiles_fit(p.table, (p.H + BNH - 1) / BNH), 1)) lin1_swiglu_tiles<BWD, NarrowTiles, Sched>(p);
   else lin1_swiglu_tiles<BWD, StdTilesHalfParts>(p);
   trace.finish();
 }
@@ -437,7 +437,7 @@ int launch_lin2(const Lin2Args& a, hipStream_t st) {
 }
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
-  if (narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS))
+  if (__builtin_expect(narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     lin2_scale_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
     lin2_scale_tiles<StdTiles>(p);

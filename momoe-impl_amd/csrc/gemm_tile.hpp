@@ -626,7 +626,7 @@ using NarrowTiles = RowTileGeometry<2, 4, 4>;
 struct StdTilesHalfParts : StdTiles {
   static constexpr bool HALF_PARTS = true;
 };
-// tile order of a kernel that holds one geometry of 256-row tiles whatever the table's height
+// tile order of NarrowTiles: the table may be of either height
 template <class G>
 using OneGeometrySched = TileSchedT<G::WROWS, G::MAX_ROWS>;
 // StdTiles that read the k-strided weights of an expert that is a single row tile with the
@@ -724,7 +724,7 @@ inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
 // 71 -> 76 us, 39 x 8: 71 -> 82), but TallTiles in this kernel too cost every launch 0.5 us.
 __device__ __forceinline__ bool narrow_tiles_fit(const int32_t* table, int nb) {
   const int tiles = load_uniform(table), rows = load_uniform(table + 1);  // both at once
-  return __builtin_expect((rows > StdTiles::MAX_ROWS) | (tiles * nb <= (int)gridDim.x), 1);
+  return (rows > StdTiles::MAX_ROWS) | (tiles * nb <= (int)gridDim.x);
 }
 
 // Whether a launch over weight matrices of `weight_bytes` takes OnceTiles.  Measured at D = 2048, H =
