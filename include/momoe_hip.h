@@ -37,9 +37,9 @@ extern "C" {
 
 /* Rows per row tile of the grouped GEMMs.  A tile table is built for one tile height
  * (momoe_index_build, momoe_tile_table_build).  momoe_lin1_swiglu_fwd, momoe_lin2_scale_fwd,
- * momoe_dgrad_h and momoe_dgrad_x take tables of any height up to MOMOE_TILE_ROWS: they hold
- * one code path for heights up to MOMOE_RECOMPUTE_TILE_ROWS and one for taller tiles, and follow
- * the table.  momoe_lin1_swiglu_bwd takes heights up to MOMOE_RECOMPUTE_TILE_ROWS (its epilogue
+ * momoe_dgrad_h and momoe_dgrad_x take tables of any height up to MOMOE_TILE_ROWS and any list of
+ * tokens per expert; which of their tile shapes a launch takes follows from its sizes and, on the device,
+ * from the table (its height, its number of tiles, whether a tile is its expert's only one).  momoe_lin1_swiglu_bwd takes heights up to MOMOE_RECOMPUTE_TILE_ROWS (its epilogue
  * leaves no registers for a taller tile).  A kernel given a table of a greater height than it
  * takes returns without writing anything.
  * tile_rows = 0 in momoe_index_build lets the library choose between the two heights from the
@@ -234,7 +234,8 @@ int momoe_lin1_swiglu_bwd(const void* x_MD, const void* Wl1_ND2H, const int32_t*
 /* momoe_lin1_swiglu_bwd with `nparts` partial row sums per row, gs_part fp32 [nparts][Msum]:
  * ceil(H/MOMOE_GS_BLOCK), as above, or momoe_gs_parts(H, N, Msum) (anything else:
  * MOMOE_ERR_BAD_ARG).  The latter is twice as many where the launch has few output tiles: it then
- * works on tiles half as wide, each with a partial sum of its own, on twice the CUs.
+ * works on tiles half as wide, each with a partial sum of its own, on twice the CUs; or, if the table
+ * holds more tiles than CUs, on whole ones, and the second partial sum of each is zero.
  */
 int64_t momoe_gs_parts(int64_t H, int64_t N, int64_t Msum);
 int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2H, const int32_t* idx_Msum,
