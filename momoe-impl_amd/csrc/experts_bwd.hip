@@ -82,10 +82,13 @@ __device__ __forceinline__ void dgrad_h_tiles(const DhArgs& p) {
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
 }
 
-__global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
-  const ClockTrace trace(p.clk);
+__device__ __forceinline__ void dgrad_h_by_table(const DhArgs& p) {
   if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) dgrad_h_tiles<TallTiles>(p);
   else dgrad_h_tiles<StdTiles>(p);
+}
+__global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
+  const ClockTrace trace(p.clk);
+  dgrad_h_by_table(p);
   trace.finish();
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
@@ -93,11 +96,11 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
   if (__builtin_expect(narrow_tiles_fit(p.table, (p.H + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     dgrad_h_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
-    dgrad_h_tiles<StdTiles>(p);
+    dgrad_h_by_table(p);
   trace.finish();
 }
 constexpr size_t kDhLds = std::max(DhProg<TallTiles>::Ring::BYTES, DhProg<StdTiles>::Ring::BYTES);
-constexpr size_t kDhNarrowLds = std::max(DhProg<NarrowTiles>::Ring::BYTES, DhProg<StdTiles>::Ring::BYTES);
+constexpr size_t kDhNarrowLds = std::max(DhProg<NarrowTiles>::Ring::BYTES, kDhLds);
 
 // SwiGLU backward for the sorted rows whose a|b were saved by the forward.  One workgroup per
 // group of 32 padded sorted rows (an expert's rows start at a multiple of 32 in padded
@@ -270,10 +273,13 @@ __device__ __forceinline__ void dgrad_x_tiles(const DxArgs& p) {
   run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
 }
 
-__global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
-  const ClockTrace trace(p.clk);
+__device__ __forceinline__ void dgrad_x_by_table(const DxArgs& p) {
   if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) dgrad_x_tiles<TallTiles>(p);
   else dgrad_x_tiles<StdTiles>(p);
+}
+__global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
+  const ClockTrace trace(p.clk);
+  dgrad_x_by_table(p);
   trace.finish();
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
@@ -281,11 +287,11 @@ __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
   if (__builtin_expect(narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
-    dgrad_x_tiles<StdTiles>(p);
+    dgrad_x_by_table(p);
   trace.finish();
 }
 constexpr size_t kDxLds = std::max(DxProg<TallTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
-constexpr size_t kDxNarrowLds = std::max(DxProg<NarrowTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
+constexpr size_t kDxNarrowLds = std::max(DxProg<NarrowTiles>::Ring::BYTES, kDxLds);
 
 // dL/ds [N][M] from the partial row sums in sorted order.  One workgroup per (expert, kGsTokens
 // tokens) writes its piece whole, zeros included, through LDS: every line of the matrix is stored

@@ -270,24 +270,29 @@ __device__ __forceinline__ void lin1_swiglu_tiles(const Lin1Args& p) {
   run_row_tiles<FM, FN>(prog, sched, ring, n_org);
 }
 
-// The forward holds two geometries, Short for tables of at most 256 rows, and follows the tile table
-// it is given.
+// The wide tiles: Short for tables of at most 256 rows, the forward also the tall ones.
 template <bool BWD, class Short>
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_kernel(Lin1Args p) {
-  const ClockTrace trace(p.clk);
+__device__ __forceinline__ void lin1_swiglu_by_table(const Lin1Args& p) {
   if constexpr (BWD) {
     lin1_swiglu_tiles<true, Short>(p);
   } else {
     if (TileSched::tile_rows_of(p.table) > Short::MAX_ROWS) lin1_swiglu_tiles<false, TallTiles>(p);
     else lin1_swiglu_tiles<false, Short>(p);
   }
+}
+template <bool BWD, class Short>
+constexpr size_t kLin1Lds = BWD ? Lin1Prog<BWD, Short>::kLds
+                                : std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, Short>::kLds);
+template <bool BWD, class Short>
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  lin1_swiglu_by_table<BWD, Short>(p);
   trace.finish();
 }
 template <bool BWD, class Short>
 int launch_lin1(const Lin1Args& a, hipStream_t st) {
   static LdsLimit lds;
-  constexpr size_t bytes =
-      BWD ? Lin1Prog<BWD, Short>::kLds : std::max(Lin1Prog<false, TallTiles>::kLds, Lin1Prog<false, Short>::kLds);
+  constexpr size_t bytes = kLin1Lds<BWD, Short>;
   if (!allow_lds(lin1_swiglu_kernel<BWD, Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
   lin1_swiglu_kernel<BWD, Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
@@ -301,14 +306,16 @@ __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_narrow_kernel(Lin1Arg
   using Sched = std::conditional_t<BWD, TileSchedT<NarrowTiles::WROWS>, OneGeometrySched<NarrowTiles>>;
   constexpr int BNH = NarrowTiles::COLS / 2;
   const ClockTrace trace(p.clk);
-  if (__builtin_expect(narrow_tiles_fit(p.table, (p.H + BNH - 1) / BNH), 1)) lin1_swiglu_tiles<BWD, NarrowTiles, Sched>(p);
-  else lin1_swiglu_tiles<BWD, StdTilesHalfParts>(p);
+  if (__builtin_expect(narrow_tiles_fit(p.table, (p.H + BNH - 1) / BNH), 1))
+    lin1_swiglu_tiles<BWD, NarrowTiles, Sched>(p);
+  else
+    lin1_swiglu_by_table<BWD, StdTilesHalfParts>(p);
   trace.finish();
 }
 template <bool BWD>
 int launch_lin1_narrow(const Lin1Args& a, hipStream_t st) {
   static LdsLimit lds;
-  constexpr size_t bytes = std::max(Lin1Prog<BWD, NarrowTiles>::kLds, Lin1Prog<BWD, StdTilesHalfParts>::kLds);
+  constexpr size_t bytes = std::max(Lin1Prog<BWD, NarrowTiles>::kLds, kLin1Lds<BWD, StdTilesHalfParts>);
   if (!allow_lds(lin1_swiglu_narrow_kernel<BWD>, bytes, lds)) return MOMOE_ERR_LAUNCH;
   lin1_swiglu_narrow_kernel<BWD><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
@@ -421,16 +428,22 @@ __device__ __forceinline__ void lin2_scale_tiles(const Lin2Args& p) {
 }
 
 template <class Short>
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
-  const ClockTrace trace(p.clk);
+__device__ __forceinline__ void lin2_scale_by_table(const Lin2Args& p) {
   if (TileSched::tile_rows_of(p.table) > Short::MAX_ROWS) lin2_scale_tiles<TallTiles>(p);
   else lin2_scale_tiles<Short>(p);
+}
+template <class Short>
+constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<Short>::kLds);
+template <class Short>
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
+  const ClockTrace trace(p.clk);
+  lin2_scale_by_table<Short>(p);
   trace.finish();
 }
 template <class Short>
 int launch_lin2(const Lin2Args& a, hipStream_t st) {
   static LdsLimit lds;
-  constexpr size_t bytes = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<Short>::kLds);
+  constexpr size_t bytes = kLin2Lds<Short>;
   if (!allow_lds(lin2_scale_kernel<Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
   lin2_scale_kernel<Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
@@ -440,10 +453,10 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args
   if (__builtin_expect(narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
     lin2_scale_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
   else
-    lin2_scale_tiles<StdTiles>(p);
+    lin2_scale_by_table<StdTiles>(p);
   trace.finish();
 }
-constexpr size_t kLin2NarrowLds = std::max(Lin2Prog<NarrowTiles>::kLds, Lin2Prog<StdTiles>::kLds);
+constexpr size_t kLin2NarrowLds = std::max(Lin2Prog<NarrowTiles>::kLds, kLin2Lds<StdTiles>);
 
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
   using Prog = Lin2Prog<FewRows::G>;

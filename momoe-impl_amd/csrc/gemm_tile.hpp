@@ -716,15 +716,15 @@ inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
 }
 
 // In that kernel: whether the table's tiles in `nb` column blocks of NarrowTiles are at most one per
-// workgroup; if not it takes StdTiles.  Forward and step with D = 1024, H = 512, N = 32, K = 4, wide
-// tiles -> narrow ones regardless -> by this rule, us: 1024 tokens, one expert shared (37 tiles x 8) 66
-// -> 79 -> 67 and 249 -> 265 -> 247; 320 tokens, one shared (33 x 8) 55 -> 59 -> 54 and 168 -> 175 ->
-// 163; 700 tokens, load falling as rank^-1.8 (25 x 8) 57 -> 43 -> 43 and 205 -> 166 -> 168.
-// Tables of 320-row tiles stay narrow, halved.  Past 2 x 256 halves that may lose (33 x 8: 70 -> 67 or
-// 71 -> 76 us, 39 x 8: 71 -> 82), but TallTiles in this kernel too cost every launch 0.5 us.
+// workgroup (two halves of a 320-row one); if not it takes the wide tiles of the table's height.
+// Callers mark the narrow path as the expected one: behind the test it cost a launch 0.1 to 0.5 us less
+// than past the wide path's code.
+// Forward and step with D = 1024, H = 512, N = 32, K = 4, wide tiles -> narrow ones regardless -> by
+// this rule, us: 1024 tokens, one expert shared (37 tiles x 8) 66 -> 79 -> 67 and 249 -> 265 -> 247;
+// 1300 tokens, load falling as rank^-1.8 (39 x 8 of 320 rows) 70 -> 80 -> 71 and 268 -> 284 -> 270; 700
+// tokens of that kind (25 x 8) 57 -> 43 -> 43 and 205 -> 166 -> 168.
 __device__ __forceinline__ bool narrow_tiles_fit(const int32_t* table, int nb) {
-  const int tiles = load_uniform(table), rows = load_uniform(table + 1);  // both at once
-  return (rows > StdTiles::MAX_ROWS) | (tiles * nb <= (int)gridDim.x);
+  return load_uniform(table) * nb <= (int)gridDim.x;
 }
 
 // Whether a launch over weight matrices of `weight_bytes` takes OnceTiles.  Measured at D = 2048, H =
