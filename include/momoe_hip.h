@@ -105,7 +105,8 @@ int64_t momoe_hbm_stream_probe(const void* matrix, int64_t blocks, int64_t krows
  * MOMOE_TILE_ROWS (anything else: MOMOE_ERR_UNSUPPORTED; the GEMMs deal whole 32-row fragment
  * rows to an expert's tiles), or 0: the library
  * picks MOMOE_RECOMPUTE_TILE_ROWS or MOMOE_TILE_ROWS on the device (table[1] holds the choice);
- * momoe_tile_table_ints(M, N, K, 0) sizes the table for either.
+ * momoe_tile_table_ints(M, N, K, 0) sizes the table for either.  momoe_gemm_tile_rows says which
+ * suits a launch.
  * recompute_table (may be NULL; only with tile_rows = 0, MOMOE_ERR_BAD_ARG otherwise)
  * int32[momoe_tile_table_ints(M, N, K, MOMOE_RECOMPUTE_TILE_ROWS)]: receives the table for tiles of
  * MOMOE_RECOMPUTE_TILE_ROWS rows, which momoe_lin1_swiglu_bwd needs whatever height was chosen
@@ -116,6 +117,11 @@ int64_t momoe_hbm_stream_probe(const void* matrix, int64_t blocks, int64_t krows
  */
 int64_t momoe_tile_table_ints(int64_t M, int64_t N, int64_t K, int tile_rows);
 int64_t momoe_index_workspace_bytes(int64_t M, int64_t N);
+/* Which tables suit momoe_lin1_swiglu_fwd (cols = 2H output columns, a contraction over D), momoe_lin2_scale_fwd
+ * (D, H), momoe_dgrad_h (H, D) and momoe_dgrad_x (D, 2H) of these sizes: MOMOE_RECOMPUTE_TILE_ROWS where the launch takes
+ * shapes of at most so many rows (a taller table's tiles are halved for it), 0 where the
+ * table of the library's own choice is the better one. */
+int momoe_gemm_tile_rows(int64_t Msum, int64_t N, int64_t cols, int64_t contraction);
 int momoe_index_build(const int32_t* mask_NM, int64_t stride_n, int64_t stride_m,
                       int64_t M, int64_t N, int64_t K,
                       int64_t* sizes_N, int32_t* cumsums_N1, int32_t* idx_Msum,

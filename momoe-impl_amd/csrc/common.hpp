@@ -58,8 +58,9 @@ struct TileCoord {
 // A tile is looked up in two steps so that the table read can travel while other work runs:
 // fetch() issues the scalar loads of the workgroup's next tile, resolve() does the arithmetic.
 // WROWS: wave rows the fragment rows of a tile are dealt to.  LIMIT: most rows the kernel takes in
-// a tile if it is less than the table may hold, else 0: tiles of a taller table are halved.
-template <int WROWS = 2, int LIMIT = 0>
+// a tile if it is less than the table may hold, else 0: tiles of a taller table are halved.  WAVES: of a
+// workgroup.
+template <int WROWS = 2, int LIMIT = 0, int WAVES = kWaves>
 struct TileSchedT {
   static constexpr int kBandTiles = 4;
   // tile height the table was built for
@@ -72,6 +73,7 @@ struct TileSchedT {
   };
   const int* table;
   int nb, bm, begin, total, chunk, xcd, pos, stride;
+  int limit;  // tiles of this XCD
   int sub;  // tiles made of one table entry
 
   // tiles before row tile `first_row_tile` (all its column blocks) are left out; a table whose
@@ -88,14 +90,19 @@ struct TileSchedT {
     xcd = blockIdx.x & 7;
     pos = blockIdx.x >> 3;
     stride = gridDim.x >> 3;
+    limit = max(0, min(chunk, total - begin - xcd * chunk));
   }
   __device__ __forceinline__ Raw fetch() {
-    Raw r;
-    r.any = false;
-    if (pos >= chunk) return r;
-    const int q = begin + xcd * chunk + pos;
+    const int at = pos;
     pos += stride;
-    if (q >= total) return r;
+    return entry(at, at < limit);
+  }
+  // tile `at` of this XCD's
+  __device__ __forceinline__ Raw entry(int at, bool any) const {
+    Raw r;
+    r.any = any;
+    if (!any) return r;
+    const int q = begin + xcd * chunk + at;
     const int __attribute__((address_space(4)))* e =
         (const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * (q / (nb * sub)));
     r.q = q;
@@ -103,7 +110,6 @@ struct TileSchedT {
     r.first = e[1];
     r.rstart = e[2];
     r.mi = e[3];
-    r.any = true;
     return r;
   }
   __device__ __forceinline__ TileCoord resolve(const Raw& r) const {
@@ -135,12 +141,15 @@ struct TileSchedT {
     tc.row0 = r.rstart + 32 * f0;
     tc.prow0 = padded_start(r.rstart, r.expert) + 32 * f0;
     tc.rows = min(32 * (fbase + (tl < fextra ? 1 : 0)), r.mi - 32 * f0);
-    // the tile's fragment rows are dealt to the wave rows as evenly as possible
-    const int nf = (tc.rows + 31) >> 5, wr = wave_id() / (kWaves / WROWS);
+    deal(tc);
+    return tc;
+  }
+  // the tile's fragment rows are dealt to the wave rows as evenly as possible
+  static __device__ __forceinline__ void deal(TileCoord& tc) {
+    const int nf = (tc.rows + 31) >> 5, wr = wave_id() / (WAVES / WROWS);
     const int wbase = nf / WROWS, wextra = nf - wbase * WROWS;
     tc.mbase = 32 * (wr * wbase + min(wr, wextra));
     tc.na = wbase + (wr < wextra ? 1 : 0);
-    return tc;
   }
   __device__ __forceinline__ TileCoord next() { return resolve(fetch()); }
   // first row tile of the expert that holds sorted row `row` (number of row tiles if the row

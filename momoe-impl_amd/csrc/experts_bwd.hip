@@ -4,14 +4,14 @@
 // gradient into [N, M].
 #include <algorithm>
 
-#include "gemm_tile.hpp"
+#include "gemm_span.hpp"
 
 namespace momoe {
 namespace {
 
-// Both data-gradient GEMMs hold both tall and standard row tiles and follow the tile table they are
-// given; launches with few tiles take narrow ones (takes_narrow_tiles).
-constexpr int FN = 2;  // 2x4 (4x2) waves, each (32 * FM) rows x 64 columns
+// Both data-gradient GEMMs take WideSpan tiles; launches with few tiles the narrow ones of
+// gemm_tile.hpp (takes_narrow_tiles).
+constexpr int FN = 2;  // of those: 2x4 (4x2) waves, each (32 * FM) rows x 64 columns
 
 struct DhArgs {
   const bf16* gy;
@@ -22,6 +22,40 @@ struct DhArgs {
   int D, H;
   unsigned long long* clk;
 };
+
+// u = G_y[idx] . Wl2^T: both operands are k-contiguous (k = D).
+template <class G_>
+struct DhSpan {
+  using G = G_;
+  using Rows = SpanGatheredRows<256>;
+  using Weights = SpanPitchedRows<G::COLS>;
+  using Ids = FetchIds;
+  struct Late {};
+  const DhArgs& p;
+  const int K, n_org;
+
+  __device__ __forceinline__ explicit DhSpan(const DhArgs& p_)
+      : p(p_), K(p_.D), n_org(wave_id() % G::WCOLS * (16 * G::FN)) {}
+  __device__ __forceinline__ void gather(const TileCoord& t, Ids& g) const { g.gather(t, p.idx); }
+  __device__ __forceinline__ void late(const TileCoord&, const Ids&, Late&) const {}
+  __device__ __forceinline__ void settle(Ids& g) const { momoe::settle(g.tok); }
+  __device__ __forceinline__ void settle(Late&) const {}
+  __device__ __forceinline__ void setup(const TileCoord& t, const Ids& g, Rows& A, Weights& W) const {
+    A.init(p.gy, [&](int j, int l) { return (uint32_t)g.of(j, l) * (uint32_t)(2 * p.D); });
+    W.init(p.w2 + (int64_t)t.expert * p.H * p.D, p.D, t.tn * G::COLS, p.H);
+  }
+  template <int NA>
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late&,
+                                           bf16* staging) const {
+    store_rows(tc, acc, staging, p.u, p.H, tc.tn * G::COLS + n_org, fresh_lane(), [](int) { return 1.0f; });
+  }
+};
+
+__global__ __launch_bounds__(kSpanThreads, 1) void dgrad_h_kernel(DhArgs p) {
+  const ClockTrace trace(p.clk);
+  run_span_tiles<DhSpan<WideSpan>>(p, (p.H + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  trace.finish();
+}
 
 // u = G_y[idx] . Wl2^T is an "NT" GEMM: both operands are k-contiguous (k = D).
 template <class G>
@@ -85,11 +119,6 @@ __device__ __forceinline__ void dgrad_h_tiles(const DhArgs& p) {
 __device__ __forceinline__ void dgrad_h_by_table(const DhArgs& p) {
   if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) dgrad_h_tiles<TallTiles>(p);
   else dgrad_h_tiles<StdTiles>(p);
-}
-__global__ __launch_bounds__(kThreads, 2) void dgrad_h_kernel(DhArgs p) {
-  const ClockTrace trace(p.clk);
-  dgrad_h_by_table(p);
-  trace.finish();
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_h_narrow_kernel(DhArgs p) {
   const ClockTrace trace(p.clk);
@@ -220,6 +249,40 @@ struct DxArgs {
 };
 
 // gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
+template <class G_>
+struct DxSpan {
+  using G = G_;
+  using Rows = SpanBlockedRows<256>;
+  using Weights = SpanPitchedRows<G::COLS>;
+  struct Ids {};
+  struct Late {};
+  const DxArgs& p;
+  const int K, n_org;
+
+  __device__ __forceinline__ explicit DxSpan(const DxArgs& p_)
+      : p(p_), K(2 * p_.H), n_org(wave_id() % G::WCOLS * (16 * G::FN)) {}
+  __device__ __forceinline__ void gather(const TileCoord&, Ids&) const {}
+  __device__ __forceinline__ void late(const TileCoord&, const Ids&, Late&) const {}
+  __device__ __forceinline__ void settle(Ids&) const {}
+  __device__ __forceinline__ void settle(Late&) const {}
+  __device__ __forceinline__ void setup(const TileCoord& t, const Ids&, Rows& A, Weights& W) const {
+    A.init(p.gz, p.msum, t.row0, t.rows);
+    W.init(p.w1 + (int64_t)t.expert * p.D * K, K, t.tn * G::COLS, p.D);
+  }
+  template <int NA>
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late&,
+                                           bf16* staging) const {
+    store_rows(tc, acc, staging, p.gxs, p.D, tc.tn * G::COLS + n_org, fresh_lane(), [](int) { return 1.0f; });
+  }
+};
+
+__global__ __launch_bounds__(kSpanThreads, 1) void dgrad_x_kernel(DxArgs p) {
+  const ClockTrace trace(p.clk);
+  run_span_tiles<DxSpan<WideSpan>>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  trace.finish();
+}
+
+// gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
 template <class G>
 struct DxProg {
   static constexpr int FM = G::FM, BN = G::COLS;
@@ -276,11 +339,6 @@ __device__ __forceinline__ void dgrad_x_tiles(const DxArgs& p) {
 __device__ __forceinline__ void dgrad_x_by_table(const DxArgs& p) {
   if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) dgrad_x_tiles<TallTiles>(p);
   else dgrad_x_tiles<StdTiles>(p);
-}
-__global__ __launch_bounds__(kThreads, 2) void dgrad_x_kernel(DxArgs p) {
-  const ClockTrace trace(p.clk);
-  dgrad_x_by_table(p);
-  trace.finish();
 }
 __global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
   const ClockTrace trace(p.clk);
@@ -355,15 +413,13 @@ extern "C" int momoe_dgrad_h(const void* Gy_MD, const void* Wl2_NHD, const int32
   if (st != MOMOE_OK) return st;
   DhArgs a{(const bf16*)Gy_MD, (const bf16*)Wl2_NHD, idx_Msum, tile_table, (bf16*)u_MsumH, (int)D,
            (int)H, clock_trace_buffer()};
-  if (takes_narrow_tiles(Msum, N, H)) {
-    static LdsLimit narrow;
-    if (!allow_lds(dgrad_h_narrow_kernel, kDhNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    dgrad_h_narrow_kernel<<<persistent_grid(), kThreads, kDhNarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
+  if (takes_span_tiles(Msum, N, H, D)) {
+    static LdsLimit span;
+    return launch_span(dgrad_h_kernel, a, span, (hipStream_t)stream);
   }
-  static LdsLimit lds;
-  if (!allow_lds(dgrad_h_kernel, kDhLds, lds)) return MOMOE_ERR_LAUNCH;
-  dgrad_h_kernel<<<persistent_grid(), kThreads, kDhLds, (hipStream_t)stream>>>(a);
+  static LdsLimit narrow;
+  if (!allow_lds(dgrad_h_narrow_kernel, kDhNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+  dgrad_h_narrow_kernel<<<persistent_grid(), kThreads, kDhNarrowLds, (hipStream_t)stream>>>(a);
   return launch_status();
 }
 
@@ -417,14 +473,12 @@ extern "C" int momoe_dgrad_x(const void* gz_blocked, const void* Wl1_ND2H,
   if (st != MOMOE_OK) return st;
   DxArgs a{(const bf16*)gz_blocked, (const bf16*)Wl1_ND2H, tile_table, (bf16*)gxs_MsumD, (int)D,
            (int)H, Msum, clock_trace_buffer()};
-  if (takes_narrow_tiles(Msum, N, D)) {
-    static LdsLimit narrow;
-    if (!allow_lds(dgrad_x_narrow_kernel, kDxNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    dgrad_x_narrow_kernel<<<persistent_grid(), kThreads, kDxNarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
+  if (takes_span_tiles(Msum, N, D, 2 * H)) {
+    static LdsLimit span;
+    return launch_span(dgrad_x_kernel, a, span, (hipStream_t)stream);
   }
-  static LdsLimit lds;
-  if (!allow_lds(dgrad_x_kernel, kDxLds, lds)) return MOMOE_ERR_LAUNCH;
-  dgrad_x_kernel<<<persistent_grid(), kThreads, kDxLds, (hipStream_t)stream>>>(a);
+  static LdsLimit narrow;
+  if (!allow_lds(dgrad_x_narrow_kernel, kDxNarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+  dgrad_x_narrow_kernel<<<persistent_grid(), kThreads, kDxNarrowLds, (hipStream_t)stream>>>(a);
   return launch_status();
 }

@@ -3,7 +3,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_tile.hpp"
+#include "gemm_span.hpp"
 
 namespace momoe {
 namespace {
@@ -30,6 +30,99 @@ struct Lin1Args {
   int64_t msum;
   unsigned long long* clk;
 };
+
+// The forward.  Tile = up to 256 rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave's
+// first half of fragments are `a` columns, the second their `b` columns, so the SwiGLU product pairs
+// registers of the same lane.
+template <class G_>
+struct Lin1Span {
+  using G = G_;
+  static constexpr int BNH = G::COLS / 2, WIDTH = 8 * G::FN;  // hidden columns of a tile, of a wave
+  using Rows = SpanGatheredRows<256>;
+  using Weights = SpanCols<G::COLS, true>;
+  using Ids = FetchIds;
+  struct Late {};
+  const Lin1Args& p;
+  const int K, n_org;
+
+  __device__ __forceinline__ explicit Lin1Span(const Lin1Args& p_)
+      : p(p_), K(p_.D), n_org(wave_id() % G::WCOLS * WIDTH) {}
+  __device__ __forceinline__ void gather(const TileCoord& t, Ids& g) const { g.gather(t, p.idx); }
+  __device__ __forceinline__ void late(const TileCoord&, const Ids&, Late&) const {}
+  __device__ __forceinline__ void settle(Ids& g) const { momoe::settle(g.tok); }
+  __device__ __forceinline__ void settle(Late&) const {}
+  __device__ __forceinline__ void setup(const TileCoord& t, const Ids& g, Rows& A, Weights& W) const {
+    const int D = p.D, H = p.H, j0 = t.tn * BNH;
+    A.init(p.x, [&](int j, int l) { return (uint32_t)g.of(j, l) * (uint32_t)(2 * D); });
+    W.init(p.w1 + (int64_t)t.expert * D * 2 * H, 2 * H,
+           [&](int c) { return (c / BNH) * H + min(j0 + (c % BNH), H - 8); });
+  }
+  template <int NA>
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late&,
+                                           bf16* staging) const {
+    constexpr int HF = G::FN / 2;
+    using Stager = SpanStager<WIDTH>;
+    const int H = p.H, j0 = tc.tn * BNH + n_org;  // first hidden column of this wave
+    const Stager stager(staging, fresh_lane());
+    const int rows = tc.rows - tc.mbase;
+    const int64_t r0 = (int64_t)tc.row0 + tc.mbase;
+    if (p.h) {
+      // h is k-blocked for the next GEMM: 32 hidden columns of consecutive rows are one piece of memory
+      bf16* const first = p.h + ((int64_t)(j0 >> 5) * p.msum + r0) * 32;  // uniform
+      const uint32_t off = (stager.block_row() * 32 + stager.block_col()) * 2;
+      bf16x8 v[2][Stager::PASSES];
+      auto store = [&](int i) {
+#pragma unroll
+        for (int q = 0; q < Stager::PASSES; ++q)
+          store16(first + ((int64_t)q * p.msum + 16 * i) * 32, off, 16 * i + stager.block_row() < rows && j0 + 32 * q < H,
+                  v[i & 1][q]);
+      };
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+#pragma unroll
+        for (int f = 0; f < HF; ++f) {
+          float hv[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float a = acc[f][i][e], b = acc[HF + f][i][e];
+            hv[e] = a * b * sigmoidf_fast(b);
+          }
+          stager.put(i & 1, f, pack_bf16x4(hv[0], hv[1], hv[2], hv[3]));
+        }
+        if (i > 0) store(i - 1);
+#pragma unroll
+        for (int q = 0; q < Stager::PASSES; ++q) v[i & 1][q] = stager.get_block(i & 1, q);
+      }
+      store(NA - 1);
+    }
+    if (p.ab) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+#pragma unroll
+          for (int f = 0; f < HF; ++f) stager.put(half, f, pack_bf16x4(acc[half * HF + f][i], 1.0f));
+#pragma unroll
+          for (int q = 0; q < Stager::PASSES; ++q) {
+            const int row = 16 * i + stager.row(q), col = j0 + stager.col(q);
+            const bf16x8 v = stager.get(half, q);
+            store16(p.ab + (r0 + 16 * i) * 2 * H + half * H + j0,
+                    ((uint32_t)stager.row(q) * 2 * H + stager.col(q)) * 2,
+                    row < rows && col < H && r0 + row >= p.ab_lo && r0 + row < p.ab_hi, v);
+          }
+        }
+    }
+  }
+};
+
+__global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_fwd_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  // without an h output only rows >= ab_lo are wanted: experts entirely below are skipped
+  const int first = p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
+  using Prog = Lin1Span<WideSpan>;
+  run_span_tiles<Prog>(p, (p.H + Prog::BNH - 1) / Prog::BNH, MOMOE_TILE_ROWS, first);
+  trace.finish();
+}
 
 // Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave owns 32 `a`
 // columns and their 32 `b` columns, so the SwiGLU product pairs registers of the same lane.
@@ -362,6 +455,43 @@ struct Lin2Args {
   unsigned long long* clk;
 };
 
+template <class G_>
+struct Lin2Span {
+  using G = G_;
+  using Rows = SpanBlockedRows<256>;   // rows of h, k-blocked
+  using Weights = SpanCols<G::COLS>;
+  using Ids = RowIds;     // tokens of the rows this wave holds in the accumulators
+  using Late = RowScales; // their gate weights
+  const Lin2Args& p;
+  const int K, n_org;
+
+  __device__ __forceinline__ explicit Lin2Span(const Lin2Args& p_)
+      : p(p_), K(p_.H), n_org(wave_id() % G::WCOLS * (16 * G::FN)) {}
+  __device__ __forceinline__ void gather(const TileCoord& t, Ids& g) const { g.gather(t, p.idx); }
+  __device__ __forceinline__ void late(const TileCoord& t, const Ids& g, Late& s) const {
+    s.load(t, g, p.s, p.ssn, p.ssm);
+  }
+  __device__ __forceinline__ void settle(Ids& g) const { g.settle(); }
+  __device__ __forceinline__ void settle(Late& s) const { s.settle(); }
+  __device__ __forceinline__ void setup(const TileCoord& t, const Ids&, Rows& A, Weights& W) const {
+    const int D = p.D, d0 = t.tn * G::COLS;
+    A.init(p.h, p.msum, t.row0, t.rows);
+    W.init(p.w2 + (int64_t)t.expert * p.H * D, D, [&](int c) { return min(d0 + c, D - 8); });
+  }
+  template <int NA>
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late& s,
+                                           bf16* staging) const {
+    const int lane = fresh_lane();
+    store_rows(tc, acc, staging, p.ys, p.D, tc.tn * G::COLS + n_org, lane, [&](int i) { return s.of(i, lane); });
+  }
+};
+
+__global__ __launch_bounds__(kSpanThreads, 1) void lin2_scale_kernel(Lin2Args p) {
+  const ClockTrace trace(p.clk);
+  run_span_tiles<Lin2Span<WideSpan>>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  trace.finish();
+}
+
 template <class G>
 struct Lin2Prog {
   static constexpr int FM = G::FM, BN = G::COLS;
@@ -435,7 +565,7 @@ __device__ __forceinline__ void lin2_scale_by_table(const Lin2Args& p) {
 template <class Short>
 constexpr size_t kLin2Lds = std::max(Lin2Prog<TallTiles>::kLds, Lin2Prog<Short>::kLds);
 template <class Short>
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_kernel(Lin2Args p) {
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_once_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
   lin2_scale_by_table<Short>(p);
   trace.finish();
@@ -444,8 +574,8 @@ template <class Short>
 int launch_lin2(const Lin2Args& a, hipStream_t st) {
   static LdsLimit lds;
   constexpr size_t bytes = kLin2Lds<Short>;
-  if (!allow_lds(lin2_scale_kernel<Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
-  lin2_scale_kernel<Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
+  if (!allow_lds(lin2_scale_once_kernel<Short>, bytes, lds)) return MOMOE_ERR_LAUNCH;
+  lin2_scale_once_kernel<Short><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
 }
 __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args p) {
@@ -561,9 +691,18 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
     lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, 2 * H)) return launch_lin1_narrow<false>(a, (hipStream_t)stream);
-  if (weights_read_once(Msum, N, 4 * N * D * H)) return launch_lin1<false, OnceTiles>(a, (hipStream_t)stream);
-  return launch_lin1<false, StdTiles>(a, (hipStream_t)stream);
+  if (takes_span_tiles(Msum, N, 2 * H, D)) {
+    static LdsLimit span;
+    return launch_span(lin1_swiglu_fwd_kernel, a, span, (hipStream_t)stream);
+  }
+  if (!takes_narrow_tiles(Msum, N, 2 * H) && weights_read_once(Msum, N, 4 * N * D * H))
+    return launch_lin1<false, OnceTiles>(a, (hipStream_t)stream);
+  return launch_lin1_narrow<false>(a, (hipStream_t)stream);
+}
+
+extern "C" int momoe_gemm_tile_rows(int64_t Msum, int64_t N, int64_t cols, int64_t contraction) {
+  if (Msum <= 0 || N <= 0 || cols <= 0 || contraction <= 0) return 0;
+  return takes_span_tiles(Msum, N, cols, contraction) ? MOMOE_RECOMPUTE_TILE_ROWS : 0;
 }
 
 extern "C" int64_t momoe_gs_parts(int64_t H, int64_t N, int64_t Msum) {
@@ -629,14 +768,16 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
     lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
-  if (takes_narrow_tiles(Msum, N, D)) {
-    static LdsLimit narrow;
-    if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
-    lin2_scale_narrow_kernel<<<persistent_grid(), kThreads, kLin2NarrowLds, (hipStream_t)stream>>>(a);
-    return launch_status();
+  if (takes_span_tiles(Msum, N, D, H)) {
+    static LdsLimit span;
+    return launch_span(lin2_scale_kernel, a, span, (hipStream_t)stream);
   }
-  if (weights_read_once(Msum, N, 2 * N * D * H)) return launch_lin2<OnceTiles>(a, (hipStream_t)stream);
-  return launch_lin2<StdTiles>(a, (hipStream_t)stream);
+  if (!takes_narrow_tiles(Msum, N, D) && weights_read_once(Msum, N, 2 * N * D * H))
+    return launch_lin2<OnceTiles>(a, (hipStream_t)stream);
+  static LdsLimit narrow;
+  if (!allow_lds(lin2_scale_narrow_kernel, kLin2NarrowLds, narrow)) return MOMOE_ERR_LAUNCH;
+  lin2_scale_narrow_kernel<<<persistent_grid(), kThreads, kLin2NarrowLds, (hipStream_t)stream>>>(a);
+  return launch_status();
 }
 
 extern "C" int momoe_combine(const void* rows_MsumD, const int32_t* inv_MK, void* out_MD,

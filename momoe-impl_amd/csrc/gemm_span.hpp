@@ -1,0 +1,669 @@
+// Workgroup-level bf16 GEMM for gfx950 (CDNA4): 256 x 256 (256 x 128) fp32 tiles, 64 k-values a stage.
+//
+// A workgroup of 4 wavefronts, one per SIMD with the SIMD's whole register file, computes a tile
+// with v_mfma_f32_16x16x32_bf16; each wave owns 128 x 128 (128 x 64) of it in 8 x 8 (8 x 4)
+// accumulators of 4 registers.  One workgroup per CU, persistent.
+//
+// What bounds such a loop on MI355X is energy: under sustained MFMA load the chip is power-limited and
+// the shader clock falls until the power fits, so time follows what is spent on multiplications,
+// LDS reads and transfers, and idle issue slots come on top.  Hence:
+//   * 128 x 128 per wave: a wave reads 256 rows and columns of LDS for 16384 products per k, where
+//     two waves per SIMD with 128 x 64 each read 384.
+//   * the 16 x 16 x 32 MFMA: the same products at 2.0 PFLOP/s where 32 x 32 x 16 sustains 1.75 on
+//     random operands.
+//   * 64 k-values a stage: a row of a k-contiguous operand is a whole 128-byte line, asked for once
+//     (with 32 k-values every line was asked for twice).
+//   * a lone wave per SIMD hides nothing behind another wave, so everything is placed by hand: between
+//     the MFMAs of one half of a stage (32 k-values) lie the fragment reads of the next half
+//     and one operand's transfers, a few MFMAs apart; two register sets of fragments.
+//   * the request stream runs on across tiles: the last two stages of a tile request the
+//     first two of the next one, and nothing drains before the epilogue or refills after it.
+// Uniform product of 131072 rows in 16 experts, K = N = 4096, N(0,1) x N(0,0.02) operands, harness of
+// the loop alone, TFLOP/s: 8 waves with 32 x 32 x 16 and 32 k-values a stage 1022 -> 8 waves, 64
+// k-values 1273 -> 4 waves 1229 -> 8 waves with 16 x 16 x 32 1293 -> 4 waves with 16 x 16 x 32 1393.
+//
+// LDS: a ring of stages for each operand, one deeper for the weights, which come from HBM where rows
+// mostly come out of L2: 3 x 32 KiB and 2 x 32 KiB with 256 columns, 4 x 16 and 3 x 32 with 128.
+//
+// Global memory goes straight to LDS with global_load_lds_dwordx4; every lane chooses its own 16
+// bytes, so the LDS image is swizzled by permuting which piece a lane fetches, and the same freedom
+// does all predication: what does not exist is pointed at something that does, masked at the store.
+//
+// The MFMA's first input is the weight-side fragment (16 columns), its second the row-side one
+// (16 rows): a lane holds, for one tile row (lane%16), columns 4*(lane/16) .. +3.
+#pragma once
+#include <cmath>
+
+#include "gemm_tile.hpp"
+
+namespace momoe {
+
+constexpr int kSpan = 64;                   // k-extent of a stage
+constexpr int kHalf = 32;                   // k-extent of one MFMA and of the smallest contraction
+constexpr int kSpanThreads = 256;
+constexpr int kSpanWaves = kSpanThreads / 64;
+constexpr size_t kSpanLds = 160 << 10;      // all of a CU's
+
+template <int V>
+struct IntC {
+  static constexpr int value = V;
+};
+template <int I, int N, class F>
+__device__ __forceinline__ void unrolled(F f) {
+  if constexpr (I < N) {
+    f(IntC<I>{});
+    unrolled<I + 1, N>(f);
+  }
+}
+__device__ __forceinline__ void order_fence() { __builtin_amdgcn_sched_barrier(0); }
+__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+// The lane, as a value of its own each time: what is derived from it is computed where it is used.  Taken
+// from lane_id() in a tile's set-up or epilogue it would be hoisted out of the tile loop, and a main
+// loop that owns every register has it spilled; each reload then waits for the stores before it
+// (h.Wl2 with 1024 k-values: 449 us where 300 are due).
+__device__ __forceinline__ int fresh_lane() {
+  int l = lane_id();
+  asm volatile("" : "+v"(l));
+  return l;
+}
+__device__ __forceinline__ f32x4 mfma16(bf16x8 first, bf16x8 second, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(first, second, c, 0, 0, 0);
+}
+
+// 16 bytes per lane, global -> LDS, as dma16; the LDS address is the sum of a scalar and a constant
+template <int IMM>
+__device__ __forceinline__ void dma16_at(const void* uniform_base, uint32_t byte_offset, uint32_t lds_wave_base) {
+  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_offset), "s"(uniform_base),
+               "s"(lds_wave_base), "n"(IMM)
+               : "memory", "scc");
+}
+
+// Stores 16 bytes per lane at a uniform base plus a byte offset below 2 GiB; lanes that are not `valid` store
+// nothing.  Without a branch: under a divergent one the compiler took what follows it for divergent, too.
+__device__ __forceinline__ void store16(void* uniform_base, uint32_t byte_offset, bool valid, bf16x8 v) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_base, 0, 0x7FFFFFFF, 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, 0);
+}
+
+// ---- operands -------------------------------------------------------------------------------------
+// Common to all: DEP deposits (wave-wide transfers of 1 KiB) per wave and stage; source(k) is where the
+// stage that starts at k-value k (a multiple of 32) lies, deposit<j>(source, slot) requests the j-th into
+// the slot at LDS byte address slot - 1024 * wave; Lane(org) prepares the fragment reads of this lane for rows (columns) org.., frag(slot, lane, i, h) is the
+// fragment of the 16 rows from org + 16 i, half h of the stage.
+
+// Rows of 64 k-values, k-contiguous.  LDS [ROWS][64]: the 16-byte piece p of row r at position
+// p ^ ((r / 2) % 8), so that the 16 rows x 16 bytes of 16 lanes of a fragment read cover all banks.
+template <int ROWS>
+struct SpanRowsLayout {
+  static constexpr int DEP = ROWS / 32;
+  // row that lane l fetches in the first deposit; the others lie 32 rows apart
+  static __device__ __forceinline__ int first_row(int l) { return wave_id() * 8 + (l >> 3); }
+  // piece of a row that it fetches (the same in every deposit), as a byte offset
+  static __device__ __forceinline__ uint32_t piece_bytes(int l) { return ((l & 7) ^ ((first_row(l) >> 1) & 7)) * 16; }
+  static constexpr int at(int j) { return j * kSpanWaves * 1024; }
+  static constexpr int ELEMS = ROWS * kSpan;
+  struct Lane {
+    int o[2];
+    __device__ __forceinline__ explicit Lane(int org) {
+      const int r = lane_id() & 15, g = lane_id() >> 4;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) o[h] = (org + r) * kSpan + ((4 * h + g) ^ (r >> 1)) * 8;
+    }
+  };
+  static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
+    return *(const bf16x8*)(slot + ln.o[h] + i * (16 * kSpan));
+  }
+};
+
+// gathered rows: one byte offset per deposit
+template <int ROWS>
+struct SpanGatheredRows : SpanRowsLayout<ROWS> {
+  using L = SpanRowsLayout<ROWS>;
+  const bf16* base;
+  uint32_t off[L::DEP];
+  // rowbytes(j, l) = byte offset from base_ of the row that lane l fetches in deposit j
+  template <class RowBytes>
+  __device__ __forceinline__ void init(const bf16* base_, RowBytes rowbytes) {
+    base = base_;
+    const int l = fresh_lane();
+    const uint32_t piece = L::piece_bytes(l);
+#pragma unroll
+    for (int j = 0; j < L::DEP; ++j) off[j] = rowbytes(j, l) + piece;
+  }
+  // nothing more will be needed: one line per deposit from here on
+  __device__ __forceinline__ void idle() {
+#pragma unroll
+    for (int j = 0; j < L::DEP; ++j) off[j] = 0;
+  }
+  __device__ __forceinline__ const bf16* source(int k) const { return base + k; }
+  template <int j>
+  __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
+    dma16_at<L::at(j)>(src, off[j], slot);
+  }
+};
+
+// Rows at a fixed pitch (k-contiguous weights).  The matrix holds a multiple of 32 rows, and a deposit
+// of the four waves covers 32: where the tile sticks out the last 32 are repeated.
+template <int ROWS>
+struct SpanPitchedRows : SpanRowsLayout<ROWS> {
+  using L = SpanRowsLayout<ROWS>;
+  const bf16* base;
+  uint32_t off, pitch;  // bytes
+  int last;             // first row, relative to the tile, of the matrix' last 32
+  __device__ __forceinline__ void init(const bf16* mat, int K, int row0, int nrows) {
+    pitch = (uint32_t)K * 2;
+    base = mat + (int64_t)row0 * K;
+    const int l = fresh_lane();
+    off = (uint32_t)L::first_row(l) * pitch + L::piece_bytes(l);
+    last = nrows - 32 - row0;
+  }
+  __device__ __forceinline__ void idle() { off = 0, last = 0; }
+  __device__ __forceinline__ const bf16* source(int k) const { return base + k; }
+  template <int j>
+  __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
+    dma16_at<L::at(j)>((const char*)src + (uint32_t)min(32 * j, last) * pitch, off, slot);
+  }
+};
+
+// Sorted rows of a k-blocked matrix: element (row, k) at mat[((k / 32) * nrows + row) * 32 + k % 32].
+// LDS [2][ROWS][32], each half as the matrix has it, piece p of row r at p ^ swz(r).
+template <int ROWS>
+struct SpanBlockedRows {
+  // 0, 2, 3, 1 for consecutive groups of 4 rows: a 16-byte LDS read serves lanes 0-3, 12-15, 20-23 and
+  // 24-27 in one clock, 4-11, 16-19 and 28-31 in the next; with r / 4 itself lanes 0-3 and 20-23 met
+  // in the same banks (a third of the LDS' busy cycles)
+  static __device__ __forceinline__ int swz(int r) { return ((r >> 2) & 1) * 2 ^ ((r >> 3) & 1) * 3; }
+  static constexpr int DEP = ROWS / 32, PER_HALF = DEP / 2;
+  static constexpr int ELEMS = ROWS * kSpan;
+  const bf16* base;
+  int64_t kstride;  // elements between k-blocks
+  uint32_t off[PER_HALF];
+  __device__ __forceinline__ void init(const bf16* mat, int64_t nrows, int64_t row0, int nvalid) {
+    kstride = nrows * kHalf;
+    base = mat + row0 * kHalf;
+    const int l = fresh_lane();
+#pragma unroll
+    for (int j = 0; j < PER_HALF; ++j) {
+      const int row = (j * kSpanWaves + wave_id()) * 16 + (l >> 2);
+      off[j] = (uint32_t)min(row, nvalid - 1) * (kHalf * 2) + (((l & 3) ^ swz(row)) * 16);
+    }
+  }
+  __device__ __forceinline__ void idle() {
+#pragma unroll
+    for (int j = 0; j < PER_HALF; ++j) off[j] = 0;
+  }
+  __device__ __forceinline__ const bf16* source(int k) const { return base + (int64_t)(k / kHalf) * kstride; }
+  template <int j>
+  __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
+    constexpr int h = j / PER_HALF, q = j % PER_HALF;
+    dma16_at<h * (ROWS * kHalf * 2) + q * kSpanWaves * 1024>(h ? src + kstride : src, off[q], slot);
+  }
+  struct Lane {
+    int o;
+    __device__ __forceinline__ explicit Lane(int org) {
+      const int r = lane_id() & 15, g = lane_id() >> 4;
+      o = (org + r) * kHalf + (g ^ swz(r)) * 8;
+    }
+  };
+  static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
+    return *(const bf16x8*)(slot + ln.o + h * (ROWS * kHalf) + i * (16 * kHalf));
+  }
+};
+
+// k-strided columns at a fixed pitch ([k][n] weights).  LDS [64][COLS]; the 16-byte piece p of k-row k at
+// p ^ swz(k).  A fragment is two ds_read_b64_tr_b16, the LDS transpose read: within each group of 16
+// lanes, lane i supplies the address of columns 4 * (i % 4) .. +3 of k-row i / 4 and receives column
+// i of those 4 k-rows.  The 8 k-rows x 32 bytes of 32 lanes then lie in different banks.
+// PAIRED: the wave's second half of fragments are the columns COLS / 2 further on.
+template <int COLS, bool PAIRED = false>
+struct SpanCols {
+  static constexpr int DEP = COLS / 32, FN = COLS / 32;
+  static constexpr int ELEMS = COLS * kSpan;
+  static constexpr int PIECES = COLS / 8, RPD = 64 / PIECES;  // pieces of a k-row, k-rows of a deposit
+  static constexpr int STEP = RPD * kSpanWaves;                // k-rows of a deposit of all waves
+  static constexpr int PATTERNS = STEP < 16 ? 2 : 1;           // swizzles met by this lane's deposits
+  static_assert(COLS == 256 || COLS == 128, "deposits of 8 or 16 k-rows");
+  static __device__ __forceinline__ int swz(int k) { return 2 * (k & 3) + 8 * ((k >> 3) & 1); }
+  const bf16* base;
+  uint32_t off[PATTERNS], pitch;  // bytes
+  // coloff(c) = element offset from base_ of tile column c (a multiple of 8) of k-row 0, readable
+  template <class ColOff>
+  __device__ __forceinline__ void init(const bf16* base_, int ld, ColOff coloff) {
+    base = base_;
+    pitch = (uint32_t)ld * 2;
+    const int l = fresh_lane(), krow = wave_id() * RPD + l / PIECES;
+#pragma unroll
+    for (int q = 0; q < PATTERNS; ++q)
+      off[q] = (uint32_t)krow * pitch + (uint32_t)coloff(((l % PIECES) ^ swz(krow + STEP * q)) * 8) * 2;
+  }
+  __device__ __forceinline__ void idle() {
+    pitch = 0;
+#pragma unroll
+    for (int q = 0; q < PATTERNS; ++q) off[q] = 0;
+  }
+  __device__ __forceinline__ const bf16* source(int k) const { return (const bf16*)((const char*)base + (int64_t)k * pitch); }
+  template <int j>
+  __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
+    dma16_at<j * kSpanWaves * 1024>((const char*)src + (uint32_t)(STEP * j) * pitch, off[j % PATTERNS], slot);
+  }
+  struct Lane {
+    int o;  // first fragment
+    __device__ __forceinline__ explicit Lane(int org) {
+      const int l = lane_id(), krow = 8 * (l >> 4) + ((l & 15) >> 2), col = org + 4 * (l & 3);
+      o = krow * COLS + (((col >> 3) ^ swz(krow)) << 3) + (col & 7);
+    }
+  };
+  static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
+    // (pieces 1 to 3 bits up are permuted, so what is added to a column there is an exclusive or)
+    const int far = PAIRED && i >= FN / 2 ? COLS / 2 : 0, n = PAIRED ? i % (FN / 2) : i;
+    const int flip = 16 * n + (far < 128 ? far : 0);
+    const bf16* p = slot + (ln.o ^ flip) + (far - (flip - 16 * n)) + h * (kHalf * COLS);
+    const bf16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + 4 * COLS);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+// ---- tile geometries --------------------------------------------------------------------------------
+// Waves 2 x 2, each 128 rows and COLS / 2 columns.
+struct WideSpan {
+  static constexpr int COLS = 256, MAX_ROWS = 256;
+  static constexpr int AHEAD = 2;               // stages of rows in LDS; of weights one more
+  static constexpr int FM = 8, FN = COLS / 32;  // 16-row and 16-column fragments of a wave
+  static constexpr int WROWS = 2, WCOLS = 2;
+};
+
+// Tile order: that of TileSchedT (tables of taller tiles are halved) as long as an XCD has a tile for every
+// workgroup.  What is left after its last full round, if that is at most half a round, is cut by its
+// 32-row fragment rows into as many pieces, up to 8, as there are workgroups for, and every workgroup
+// does one: without the cut a launch with 324 tiles for 256 CUs takes as long as one with 512.
+template <class G>
+struct SpanSched {
+  using Tiles = TileSchedT<G::WROWS, G::MAX_ROWS, kSpanWaves>;
+  struct Raw {
+    typename Tiles::Raw tile;
+    bool piece;
+  };
+  Tiles tiles;
+  int rest, cut;  // tiles that are cut, into how many pieces (0: nothing left to do)
+  __device__ __forceinline__ SpanSched(const int* table, int nb, int max_tile_rows, int first)
+      : tiles(table, nb, max_tile_rows, first) {
+    rest = tiles.limit % tiles.stride;
+    cut = 8 * rest <= tiles.stride ? 8 : 4 * rest <= tiles.stride ? 4 : 2;
+    if (2 * rest > tiles.stride || rest == 0) cut = 0;
+    else tiles.limit -= rest;
+  }
+  __device__ __forceinline__ int order() const { return blockIdx.x >> 3; }  // of this workgroup in its XCD
+  __device__ __forceinline__ Raw fetch() {
+    const bool whole = tiles.pos < tiles.limit;
+    Raw r;
+    r.piece = !whole && cut > 0 && order() < rest * cut;
+    r.tile = tiles.entry(whole ? tiles.pos : tiles.limit + order() / max(cut, 1), whole || r.piece);
+    if (!whole) rest = 0;
+    tiles.pos += tiles.stride;
+    return r;
+  }
+  __device__ __forceinline__ TileCoord resolve(const Raw& r) const {
+    TileCoord tc = tiles.resolve(r.tile);
+    if (!r.piece || !tc.valid) return tc;
+    const int nf = (tc.rows + 31) >> 5, part = order() % cut;
+    const int base = nf / cut, extra = nf - base * cut, f0 = part * base + min(part, extra);
+    tc.row0 += 32 * f0;
+    tc.prow0 += 32 * f0;
+    tc.rows = min(32 * (base + (part < extra ? 1 : 0)), tc.rows - 32 * f0);
+    tc.valid = tc.rows > 0;
+    Tiles::deal(tc);
+    return tc;
+  }
+  __device__ __forceinline__ TileCoord next() { return resolve(fetch()); }
+};
+
+// ---- the k-loop -----------------------------------------------------------------------------------
+// Stages of a contraction over K k-values, a multiple of 32 and at least 64 AHEAD.  The last one starts at
+// K - 64 and is multiplied by its second half only where K is an odd multiple of 32.
+struct SpanStages {
+  int full, count, kmax;
+  bool tail;
+  __device__ __forceinline__ explicit SpanStages(int K)
+      : full(K / kSpan), count((K + kSpan - 1) / kSpan), kmax(K - kSpan), tail(K % kSpan != 0) {}
+  __device__ __forceinline__ int after(int k) const { return min(k + kSpan, kmax); }  // k-origin of the next stage
+};
+
+constexpr int kStagingElems = 4096;  // a wave's share of the epilogue's staging
+
+// Keeps `v` in its register from here on: the compiler waits for the load behind it now and not at
+// its next use.
+template <class T>
+__device__ __forceinline__ void settle(T& v) {
+  static_assert(sizeof(T) == 4, "one register");
+  asm volatile("" : "+v"(v));
+}
+
+// Drives a workgroup through its (row tile, column block) pairs.  The tile program P supplies
+//   P::G, P::Rows, P::Weights                  geometry and operands
+//   P::Ids, P::Late                            per-tile values that come from loads; Late's depend on Ids'
+//   gather(tile, ids) / late(tile, ids, late)  issue those loads
+//   settle(ids) / settle(late)                 settle() each register of them
+//   setup(tile, ids, A, W)                     operand set-up
+//   epilogue(tile, acc, ids, late, staging)    acc [FN][fragment rows]; staging: kStagingElems of LDS per wave
+//   K, n_org[FN]                               contraction length, first columns of the fragments
+// While tile t is multiplied, the ids of tile t+2, the late values of tile t+1 and the table entry of
+// tile t+3 are on their way.  All of them settle at the end of tile t's epilogue: the compiler does
+// not see the transfers, so its wait for any load is a wait for every transfer older than the
+// youngest few, which cost a memory latency per tile in the middle of a stage; there the transfers
+// have had the epilogue to arrive.
+// The launch has `nb` column blocks; `first`: row tiles left out.
+template <class P, class Args>
+__device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max_tile_rows, int first = 0) {
+  using G = typename P::G;
+  using Sched = SpanSched<G>;
+  Sched sched(args.table, nb, max_tile_rows, first);
+  P prog(args);
+  using Rows = typename P::Rows;
+  using Weights = typename P::Weights;
+  constexpr int FM = G::FM, FN = G::FN, AHEAD = G::AHEAD;
+  constexpr int ROWS_AT = (AHEAD + 1) * Weights::ELEMS;  // the rows' ring lies behind the weights'
+  static_assert((ROWS_AT + AHEAD * Rows::ELEMS) * sizeof(bf16) <= kSpanLds, "the rings fit the LDS");
+  static_assert(Weights::ELEMS >= kSpanWaves * kStagingElems, "a stage of weights holds the epilogue's staging");
+  bf16* const lds = dyn_lds();
+  const uint32_t addr = lds_address(lds) + wave_id() * 1024;
+  auto wslot = [&](int s) { return addr + (uint32_t)s * (Weights::ELEMS * 2); };
+  auto aslot = [&](int s) { return addr + (uint32_t)(ROWS_AT + s * Rows::ELEMS) * 2; };
+  auto wptr = [&](int s) { return (const bf16*)lds + s * Weights::ELEMS; };
+  auto aptr = [&](int s) { return (const bf16*)lds + ROWS_AT + s * Rows::ELEMS; };
+  auto wnext = [](int s) { return s == AHEAD ? 0 : s + 1; };
+  auto anext = [](int s) { return s == AHEAD - 1 ? 0 : s + 1; };
+
+  TileCoord c0 = sched.next();
+  if (!c0.valid) return;
+  typename P::Ids g0, g1, g2;
+  typename P::Late l0, l1;
+  Rows A;
+  Weights W;
+  prog.gather(c0, g0);
+  const SpanStages st(prog.K);
+  prog.setup(c0, g0, A, W);
+  int k = 0;  // k-origin of the stage to be requested
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) {
+    const bf16 *wsrc = W.source(k), *asrc = A.source(k);
+    unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wslot(s)); });
+    unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, aslot(s)); });
+    k = st.after(k);
+  }
+  TileCoord c1 = sched.next();
+  g1 = g0;
+  if (c1.valid) prog.gather(c1, g1);
+  TileCoord c2 = sched.next();
+  const typename Weights::Lane wlane(prog.n_org);
+  prog.settle(g0);
+  prog.settle(g1);
+  prog.late(c0, g0, l0);
+  wait_vmcnt<(AHEAD - 1) * (Weights::DEP + Rows::DEP)>();
+  __builtin_amdgcn_s_barrier();
+  order_fence();
+  g2 = g1;
+  l1 = l0;
+  int sw = 0, sa = 0;  // slots of the stage at hand
+  while (true) {
+    if (c2.valid) prog.gather(c2, g2);
+    if (c1.valid) prog.late(c1, g1, l1);
+    const typename Sched::Raw rn = sched.fetch();
+
+    // this tile for a wave with NA fragment rows
+    auto tile = [&](auto NAC) {
+      constexpr int NA = decltype(NAC)::value, NM = NA * FN;
+      f32x4 acc[FN][NA > 0 ? NA : 1];
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      const typename Rows::Lane alane(c0.mbase);
+      bf16x8 af[2][NA > 0 ? NA : 1], wf[2][FN];
+      // fragment r (weights first) of half h of the stage in slots s, s+1 into register set b
+      auto read = [&](int b, int r, const bf16* w, const bf16* a, int h) {
+        if constexpr (NA > 0) {
+          if (r < FN) wf[b][r] = Weights::frag(w, wlane, r, h);
+          else af[b][r - FN] = Rows::frag(a, alane, r - FN, h);
+        }
+      };
+      // MFMAs of register set B; between them the reads of half H of (w, a) into the other set, and `dep`'s
+      // DEP deposits
+      auto multiply = [&](auto B, auto READ, const bf16* w, const bf16* a, auto H, auto DEPC, auto dep) {
+        constexpr int b = decltype(B)::value, h = decltype(H)::value, DEP = decltype(DEPC)::value;
+        constexpr int NR = decltype(READ)::value ? FN + NA : 0;
+        constexpr int PER = NM > 0 ? (2 * NR + NM - 1) / (NM > 0 ? NM : 1) : 0;  // reads behind an MFMA of the first half
+        if constexpr (NM == 0) {
+          unrolled<0, DEP>([&](auto D) { dep(D); });
+        } else {
+          unrolled<0, NM>([&](auto MC) {
+            constexpr int m = decltype(MC)::value, j = m / NA, i = (j & 1) ? NA - 1 - m % NA : m % NA;
+            acc[j][i] = mfma16(wf[b][j], af[b][i], acc[j][i]);
+            unrolled<0, PER>([&](auto R) {
+              constexpr int r = m * PER + decltype(R)::value;
+              if constexpr (r < NR) read(b ^ 1, r, w, a, h);
+            });
+            unrolled<0, DEP>([&](auto D) {
+              constexpr int d = decltype(D)::value;
+              if constexpr (((2 * d + 1) * NM) / (2 * DEP) == m) dep(D);
+            });
+            order_fence();
+          });
+        }
+      };
+      // the next stage has landed, all but what was requested after it; every wave is done reading this one
+      auto turn = [&] {
+        wait_vmcnt<(AHEAD - 1) * Weights::DEP + (AHEAD - 2) * Rows::DEP>();
+        wait_lgkm0();
+        __builtin_amdgcn_s_barrier();
+        order_fence();
+      };
+      const bf16 *w = wptr(sw), *a = aptr(sa);
+#pragma unroll
+      for (int r = 0; r < FN + NA; ++r) read(0, r, w, a, 0);
+      order_fence();
+      int t = 0, end = st.count - AHEAD;
+      while (true) {
+        const int stop = min(end, st.full);
+#pragma unroll 1
+        for (; t < stop; ++t) {
+          const bf16 *wsrc = W.source(k), *asrc = A.source(k);
+          const uint32_t wto = wslot(sw == 0 ? AHEAD : sw - 1), ato = aslot(sa);
+          sw = wnext(sw);
+          sa = anext(sa);
+          const bf16 *nw = wptr(sw), *na = aptr(sa);
+          multiply(IntC<0>{}, IntC<1>{}, w, a, IntC<1>{}, IntC<Weights::DEP>{},
+                   [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
+          turn();
+          multiply(IntC<1>{}, IntC<1>{}, nw, na, IntC<0>{}, IntC<Rows::DEP>{},
+                   [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
+          k = st.after(k);
+          w = nw;
+          a = na;
+        }
+        if (end == st.count) break;
+        k = 0;  // from here on the next tile's stages are requested
+        end = st.count;
+        if (c1.valid) {
+          prog.setup(c1, g1, A, W);
+        } else {
+          A.idle();
+          W.idle();
+        }
+      }
+      if (st.tail) {
+        const bf16 *wsrc = W.source(k), *asrc = A.source(k);
+        const int before = sw == 0 ? AHEAD : sw - 1;
+        unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wslot(before)); });
+#pragma unroll
+        for (int r = 0; r < FN + NA; ++r) read(0, r, w, a, 1);
+        multiply(IntC<0>{}, IntC<0>{}, w, a, IntC<1>{}, IntC<0>{}, [](auto) {});
+        turn();
+        unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, aslot(sa)); });
+        k = st.after(k);
+        sw = wnext(sw);
+        sa = anext(sa);
+      }
+      // staging: where the finished tile's last weights were; every wave has read them, and the next ones are
+      // requested behind the barrier below
+      if constexpr (NA > 0) prog.epilogue(c0, acc, g0, l0, lds + (sw == 0 ? AHEAD : sw - 1) * Weights::ELEMS);
+    };
+    const int na = __builtin_amdgcn_readfirstlane(c0.na);
+    if (na == 4) tile(IntC<8>{});
+    else if (na == 3) tile(IntC<6>{});
+    else if (na == 2) tile(IntC<4>{});
+    else if (na == 1) tile(IntC<2>{});
+    else tile(IntC<0>{});
+    prog.settle(g2);
+    prog.settle(l1);
+    if (!c1.valid) break;
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    c0 = c1;
+    c1 = c2;
+    c2 = sched.resolve(rn);
+    g0 = g1;
+    g1 = g2;
+    l0 = l1;
+  }
+  wait_vmcnt<0>();  // no transfer may outlive the workgroup's LDS
+}
+
+// Whether a launch over `cols` output columns takes these tiles rather than those of gemm_tile.hpp.  Not
+// where most CUs would go without one (takes_narrow_tiles), nor with few rows per expert: a tile of few
+// rows is a stream of weights, and then what is on the way counts, two to three stages of 32 k-values at
+// any time in that ring, one of 64 here.  Otherwise by the rounds of tiles the CUs take, a tile costing 0.4
+// for its weights and 0.6 for 256 rows, and of it all 0.8 here plus an epilogue that nothing hides,
+// 0.07 of a contraction over 1024: an expert of 260 rows is two tiles here and one of 320 rows there.
+// The routing is not known; the rows per expert are taken as those of one with the same chance for
+// every expert.
+// (The k-loop needs two stages.)
+// Measured, there -> here in us (x.Wl1, h.Wl2, dL/dh, dL/dx): 8192 tokens, D = 2048, H = 1024, N = 128, K = 8
+// 538 -> 498, 302 -> 286, 293 -> 252, 562 -> 493; 7680, D = 2176, H = 1152, N = 64, K = 6 438 -> 388, 257 -> 234,
+// 260 -> 209, 459 -> 388; 4000, D = 1024, H = 512, N = 64, K = 4 (64 tiles of 320 rows, 81 of 256) 39 -> 47,
+// 27 -> 31, 36 -> 27, 39 -> 43: here only dL/dh.
+inline bool takes_span_tiles(int64_t msum, int64_t n, int64_t cols, int64_t contraction) {
+  if (contraction < WideSpan::AHEAD * kSpan || takes_narrow_tiles(msum, n, cols) || few_rows_per_expert(msum, n)) return false;
+  const double mean = (double)msum / n, spread = std::sqrt(mean), blocks = (double)cdiv64(cols, WideSpan::COLS);
+  // row tiles per expert of at most `height` rows (normal spread, its tail by the logistic curve)
+  auto row_tiles = [&](double height) {
+    double t = 1.0;
+    for (int k = 1; k * height < mean + 6 * spread; ++k) t += 1.0 / (1.0 + std::exp(1.7 * (k * height - mean) / spread));
+    return t;
+  };
+  auto tile_cost = [&](double tiles) { return 0.4 + 0.6 * mean / (tiles * StdTiles::MAX_ROWS); };
+  const double tall = std::min(row_tiles(TallTiles::MAX_ROWS), row_tiles(StdTiles::MAX_ROWS)), ours = row_tiles(WideSpan::MAX_ROWS);
+  const double rounds = n * ours * blocks / persistent_grid(), rest = rounds - std::floor(rounds);
+  const double pieces = rest > 0.5 ? 1.0 : rest > 0.25 ? 0.65 : rest > 0.125 ? 0.45 : 0.3;  // SpanSched
+  return (0.8 + 73.0 / contraction) * tile_cost(ours) * (std::floor(rounds) + pieces) <=
+         tile_cost(tall) * std::ceil(n * tall * blocks / persistent_grid() - 0.05);
+}
+
+template <class Kernel, class Args>
+inline int launch_span(Kernel kernel, const Args& a, LdsLimit& lim, hipStream_t st) {
+  if (!allow_lds(kernel, kSpanLds, lim)) return MOMOE_ERR_LAUNCH;
+  kernel<<<persistent_grid(), kSpanThreads, kSpanLds, st>>>(a);
+  return launch_status();
+}
+
+// ---- ids ------------------------------------------------------------------------------------------
+// Tokens of a tile's rows for SpanGatheredRows: lane l keeps that of row 32 * (l / 8) + 8 * wave + l % 8
+struct FetchIds {
+  int32_t tok;
+  __device__ __forceinline__ void gather(const TileCoord& t, const int32_t* idx) {
+    const int l = fresh_lane();
+    tok = idx[t.row0 + min(32 * (l >> 3) + 8 * wave_id() + (l & 7), t.rows - 1)];
+  }
+  // of the row that lane l, this one, fetches in deposit j
+  __device__ __forceinline__ int32_t of(int j, int l) const { return __shfl(tok, 8 * j + (l >> 3)); }
+};
+
+// Tokens of the 128 rows a wave holds in its accumulators: lane l keeps those of rows l and 64 + l
+struct RowIds {
+  int32_t tok[2];
+  __device__ __forceinline__ void gather(const TileCoord& t, const int32_t* idx) {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) tok[q] = idx[t.row0 + min(t.mbase + 64 * q + l, t.rows - 1)];
+  }
+  __device__ __forceinline__ void settle() { momoe::settle(tok[0]), momoe::settle(tok[1]); }
+};
+// their gate weights
+struct RowScales {
+  float s[2];
+  __device__ __forceinline__ void load(const TileCoord& t, const RowIds& g, const float* s_NM, int64_t ssn, int64_t ssm) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) s[q] = s_NM[(int64_t)t.expert * ssn + (int64_t)g.tok[q] * ssm];
+  }
+  __device__ __forceinline__ void settle() { momoe::settle(s[0]), momoe::settle(s[1]); }
+  // of the row that lane l, this one, holds in fragment row i
+  __device__ __forceinline__ float of(int i, int l) const { return __shfl(s[i / 4], 16 * (i % 4) + (l & 15)); }
+};
+
+// ---- coalesced epilogue stores ----------------------------------------------------------------------
+// One 16-row fragment row of a wave at a time passes through a staging area (16 rows x WIDTH columns) and
+// leaves as 16 bytes per lane, lanes along the rows: whole lines.  Wave-private: no barrier is
+// involved.  With two areas in turn a row's reads travel while the one before it is stored.
+template <int WIDTH>
+struct SpanStager {
+  static constexpr int CHUNKS = WIDTH / 8, PASSES = 16 * CHUNKS / 64;
+  static constexpr int ELEMS = 16 * WIDTH;
+  static_assert(2 * ELEMS <= kStagingElems, "two areas");
+  static constexpr int ROWS_PER_BANK_ROW = 256 / (2 * WIDTH);
+  static __device__ __forceinline__ int swz(int row) { return (row / ROWS_PER_BANK_ROW) & (CHUNKS - 1); }
+  bf16* st;
+  int l;  // fresh_lane() of the epilogue
+  __device__ __forceinline__ SpanStager(bf16* staging, int lane) : st(staging + wave_id() * kStagingElems), l(lane) {}
+  // this lane's four columns of fragment f
+  __device__ __forceinline__ void put(int area, int f, bf16x4 v) const {
+    const int row = l & 15;
+    *(bf16x4*)(st + area * ELEMS + row * WIDTH + ((2 * f + (l >> 5)) ^ swz(row)) * 8 + ((l >> 4) & 1) * 4) = v;
+  }
+  // pass p: 8 columns from col(p) of row(p)
+  __device__ __forceinline__ int row(int p) const { return p * (64 / CHUNKS) + l / CHUNKS; }
+  __device__ __forceinline__ int col(int p) const { return ((l % CHUNKS) ^ swz(row(p))) * 8; }
+  __device__ __forceinline__ bf16x8 get(int area, int p) const {
+    return *(const bf16x8*)(st + area * ELEMS + row(p) * WIDTH + (l % CHUNKS) * 8);
+  }
+  // the same with a pass of 32 columns of 16 rows: 8 columns from 32 p + block_col() of block_row()
+  __device__ __forceinline__ int block_row() const { return l >> 2; }
+  __device__ __forceinline__ int block_col() const { return (l & 3) * 8; }
+  __device__ __forceinline__ bf16x8 get_block(int area, int p) const {
+    return *(const bf16x8*)(st + area * ELEMS + (l >> 2) * WIDTH + ((4 * p + (l & 3)) ^ swz(l >> 2)) * 8);
+  }
+};
+__device__ __forceinline__ bf16x4 pack_bf16x4(f32x4 v, float s) {
+  return bf16x4{(bf16)(v[0] * s), (bf16)(v[1] * s), (bf16)(v[2] * s), (bf16)(v[3] * s)};
+}
+
+// A wave's accumulators as rows of a row-major matrix of `cols` columns, from column col0; scale(i) is that of
+// the lane's row in fragment row i; lane = fresh_lane()
+template <int FN, int NA, class Scale>
+__device__ __forceinline__ void store_rows(const TileCoord& tc, f32x4 (&acc)[FN][NA], bf16* staging, bf16* out, int cols,
+                                           int col0, int lane, Scale scale) {
+  using Stager = SpanStager<16 * FN>;
+  const Stager stager(staging, lane);
+  bf16* const first = out + ((int64_t)tc.row0 + tc.mbase) * cols + col0;  // uniform
+  const int rows = tc.rows - tc.mbase;
+  uint32_t off[Stager::PASSES];
+#pragma unroll
+  for (int p = 0; p < Stager::PASSES; ++p) off[p] = ((uint32_t)stager.row(p) * (uint32_t)cols + stager.col(p)) * 2;
+  bf16x8 v[2][Stager::PASSES];
+  auto store = [&](int i) {
+#pragma unroll
+    for (int p = 0; p < Stager::PASSES; ++p)
+      store16(first + (int64_t)(16 * i) * cols, off[p], 16 * i + stager.row(p) < rows && col0 + stager.col(p) < cols,
+              v[i & 1][p]);
+  };
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const float s = scale(i);
+#pragma unroll
+    for (int f = 0; f < FN; ++f) stager.put(i & 1, f, pack_bf16x4(acc[f][i], s));
+    if (i > 0) store(i - 1);
+#pragma unroll
+    for (int p = 0; p < Stager::PASSES; ++p) v[i & 1][p] = stager.get(i & 1, p);
+  }
+  store(NA - 1);
+}
+
+}  // namespace momoe

@@ -741,8 +741,9 @@ __device__ __forceinline__ bool narrow_tiles_fit(const int32_t* table, int nb) {
 // whose backward reads them again took 175 -> 191 us (1000 tokens, 128 MB).  For the same reason
 // the recomputing GEMM goes without it: dL/dx reads Wl1 again, and with the hint a step took
 // 982 -> 949 us (1000 tokens) but 313 -> 327 (64 tokens, D = 2048, H = 1024, N = 32, K = 4).
+inline bool few_rows_per_expert(int64_t msum, int64_t n) { return 3 * msum <= n * OnceTiles::MAX_ROWS; }
 inline bool weights_read_once(int64_t msum, int64_t n, int64_t weight_bytes) {
-  return 3 * msum <= n * OnceTiles::MAX_ROWS && weight_bytes >= kBeyondCache;
+  return few_rows_per_expert(msum, n) && weight_bytes >= kBeyondCache;
 }
 
 template <int FM, int FN>

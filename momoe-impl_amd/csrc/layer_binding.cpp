@@ -132,11 +132,11 @@ const Tensor& as_saved(const Tensor& t, const char* name, const at::Device& dev,
 
 // ---- experts -----------------------------------------------------------------------------------
 // What the index build leaves for the rest of the forward and for the backward, in one allocation:
-// [cumsums N+1 | idx Msum | inv Msum | tile table | tile table of the recomputing GEMM], every part
+// [cumsums N+1 | idx Msum | inv Msum | tile table | table of tiles of at most 256 rows], every part
 // on a 16-byte boundary.  The parts are found again from the sizes alone.
 struct Index {
   int64_t M, N, K, tile_rows;
-  bool with_rc;
+  bool with_rc;  // with the second table; the first one is then of the library's choice
   int64_t off_idx, off_inv, off_table, off_rc, ints;
   Index(int64_t M_, int64_t N_, int64_t K_, int64_t tile_rows_, bool with_rc_)
       : M(M_), N(N_), K(K_), tile_rows(tile_rows_), with_rc(with_rc_) {
@@ -153,6 +153,10 @@ struct Index {
   int32_t* inv() const { return base + off_inv; }
   int32_t* table() const { return base + off_table; }
   int32_t* table_rc() const { return with_rc ? base + off_rc : nullptr; }
+  // the one that suits a GEMM of `cols` output columns
+  int32_t* table_for(int64_t cols, int64_t contraction) const {
+    return with_rc && momoe_gemm_tile_rows(M * K, N, cols, contraction) != 0 ? table_rc() : table();
+  }
 };
 
 struct Forward {
@@ -197,11 +201,11 @@ Forward experts_forward(const Tensor& x_BSD, const Tensor& Wl1, const Tensor& Wl
   {
     // h in blocks of 32 hidden columns, [H/32][Msum][32]: the layout the down projection reads
     const Tensor h = empty_bf16({H / 32, msum, 32}, dev);
-    MOMOE_CALL(momoe_lin1_swiglu_fwd, st, f.x.data_ptr(), f.W1.data_ptr(), ib.idx(), ib.table(), h.data_ptr(),
+    MOMOE_CALL(momoe_lin1_swiglu_fwd, st, f.x.data_ptr(), f.W1.data_ptr(), ib.idx(), ib.table_for(2 * H, D), h.data_ptr(),
                msave > 0 ? f.ab_save.data_ptr() : nullptr, (int64_t)0, msave, M, D, H, N, msum);
     ys = empty_bf16({msum, D}, dev);
     MOMOE_CALL(momoe_lin2_scale_fwd, st, h.data_ptr(), f.W2.data_ptr(), f.s.data_ptr<float>(), f.s.stride(0),
-               f.s.stride(1), ib.idx(), ib.table(), ys.data_ptr(), M, D, H, N, msum);
+               f.s.stride(1), ib.idx(), ib.table_for(D, H), ys.data_ptr(), M, D, H, N, msum);
   }
   f.y = empty_bf16({B, S, D}, dev);
   MOMOE_CALL(momoe_combine, st, ys.data_ptr(), ib.inv(), f.y.data_ptr(), M, D, K, msum);
@@ -214,13 +218,33 @@ Forward experts_forward(const Tensor& x_BSD, const Tensor& Wl1, const Tensor& Wl
   return f;
 }
 
+// Tile height left to the library (tile_rows = 0): one table of 256 rows if that suits all these GEMMs (output
+// columns, contraction), else the library's choice, and that one next to it if any wants it.
+void choose_tables(std::initializer_list<std::pair<int64_t, int64_t>> gemms, int64_t msum, int64_t N, int64_t& tile_rows,
+                   bool& with_rc) {
+  if (tile_rows != 0) {
+    with_rc = false;
+    return;
+  }
+  bool all = true;
+  for (const auto& g : gemms) {
+    const bool short_tiles = momoe_gemm_tile_rows(msum, N, g.first, g.second) != 0;
+    all = all && short_tiles;
+    with_rc = with_rc || short_tiles;
+  }
+  if (!all) return;
+  tile_rows = MOMOE_RECOMPUTE_TILE_ROWS;
+  with_rc = false;
+}
+
 struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& W1, const Tensor& W2,
                                const Tensor& mask, const Tensor& s, int64_t K, int64_t msave, int64_t tile_rows,
                                bool check) {
-    // the backward's recomputing GEMM walks row tiles of its own height: with the height left to
-    // the library, the index build writes that table too
-    const bool want_rc = msave < x.size(0) * x.size(1) * K && tile_rows == 0;
+    // the recomputing GEMM's tiles have at most 256 rows
+    bool want_rc = msave < x.size(0) * x.size(1) * K;
+    const int64_t D = W1.size(1), H = W2.size(1);
+    choose_tables({{2 * H, D}, {D, H}, {H, D}, {D, 2 * H}}, x.size(0) * x.size(1) * K, W1.size(0), tile_rows, want_rc);
     Forward f = experts_forward(x, W1, W2, mask, s, K, msave, want_rc, tile_rows, check);
     ctx->saved_data["K"] = K;
     ctx->saved_data["msave"] = msave;
@@ -261,7 +285,8 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
 
     // dL/dh before the gate weight, in sorted order
     Tensor u = empty_bf16({msum, H}, dev);
-    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table(), u.data_ptr(), M, D, H, N, msum);
+    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u.data_ptr(), M, D, H, N,
+               msum);
     // SwiGLU backward: rows with saved a|b read them; the others recompute a|b = x.Wl1 and consume
     // them straight from the GEMM's accumulators.
     // G_a|G_b in blocks of 32 columns, [2H/32][Msum][32]: the layout dL/dx contracts over
@@ -276,11 +301,10 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                  s.stride(1), ib.idx(), ib.cumsums(), msave, gz.data_ptr(), hst.data_ptr(), H,
                  gs_part.data_ptr<float>(), nparts, M, H, N, msum);
     if (msave < msum) {
-      // the recomputing GEMM takes shorter row tiles than the others: its own table, from the
-      // index build, or made here when the tile height was given
+      // the recomputing GEMM takes no taller tiles: a table of its own where another height was given
       Tensor own;
-      const int32_t* table_rc = ib.table_rc();
-      if (table_rc == nullptr) {
+      const int32_t* table_rc = ib.with_rc ? ib.table_rc() : ib.table();
+      if (tile_rows != 0 && tile_rows != MOMOE_RECOMPUTE_TILE_ROWS) {
         own = empty_i32(momoe_tile_table_ints(M, N, K, MOMOE_RECOMPUTE_TILE_ROWS), dev);
         MOMOE_CALL(momoe_tile_table_build, st, ib.cumsums(), N, msum, MOMOE_RECOMPUTE_TILE_ROWS,
                    own.data_ptr<int32_t>());
@@ -322,7 +346,7 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     }
     if (need_x) {
       const Tensor gxs = empty_bf16({msum, D}, dev);
-      MOMOE_CALL(momoe_dgrad_x, st, gz.data_ptr(), W1.data_ptr(), ib.table(), gxs.data_ptr(), M, D, H, N, msum);
+      MOMOE_CALL(momoe_dgrad_x, st, gz.data_ptr(), W1.data_ptr(), ib.table_for(D, 2 * H), gxs.data_ptr(), M, D, H, N, msum);
       Tensor Gx = empty_bf16({B, S, D}, dev);
       MOMOE_CALL(momoe_combine, st, gxs.data_ptr(), ib.inv(), Gx.data_ptr(), M, D, K, msum);
       out[0] = gdev == dev ? Gx : Gx.to(gdev);
@@ -346,7 +370,9 @@ std::tuple<Tensor, Tensor> experts(const Tensor& x, const Tensor& W1, const Tens
     throw_python(PyExc_AssertionError, "x_BSD [B,S,D], Wl1_ND2H [N,D,2H] and Wl2_NHD [N,H,D] do not fit together");
   const int64_t msum = x.size(0) * x.size(1) * K;
   if (!wants_autograd({&x, &W1, &W2, &s})) {  // nothing is kept for a backward that cannot happen
-    Forward f = experts_forward(x, W1, W2, mask, s, K, 0, false, tile_rows, check);
+    bool with_rc = false;
+    choose_tables({{2 * W2.size(1), W1.size(1)}, {W1.size(1), W2.size(1)}}, msum, W1.size(0), tile_rows, with_rc);
+    Forward f = experts_forward(x, W1, W2, mask, s, K, 0, with_rc, tile_rows, check);
     return {f.y, f.sizes};
   }
   // the Wl1 gradient addresses the eight 32-column blocks of a gz tile with 32-bit byte offsets

@@ -23,9 +23,10 @@ from . import _hip, _layer
 # every forward (one device synchronisation per call) and raise on a violation.
 CHECK_ROUTING = False
 
-# Row-tile height of the grouped GEMMs: _hip.AUTO_TILE_ROWS leaves the choice between 256 and 320
-# rows to the index build, which makes it on the device from the routing.  A fixed height (a
-# multiple of 32 from 32 to _hip.TILE_ROWS) is for experiments and for tests that must cover both code paths.
+# Row-tile height of the grouped GEMMs: _hip.AUTO_TILE_ROWS leaves it to the library, 256 rows for the
+# launches that take no taller tiles whole and for the others 256 or 320, chosen by the index build on the
+# device from the routing.  A fixed height (a multiple of 32 from 32 to _hip.TILE_ROWS) is for
+# experiments and for tests that must cover every code path.
 TILE_ROWS = _hip.AUTO_TILE_ROWS
 
 

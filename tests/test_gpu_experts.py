@@ -105,6 +105,31 @@ def test_wide_and_narrow_tiles(M, D, H, N, K, sp):
             assert torch.equal(other[k], dev[k]), (rows, k)
 
 
+@pytest.mark.parametrize("M,D,H,N,K,Ks,skew,sp", [
+    (8000, 352, 544, 8, 2, 0, None, 0),      # a full round of x.Wl1 and 6 to 9 tiles per XCD in 2 or 4 pieces each;
+                                             # contractions of 5.5, 8.5 and 17 stages, columns past a tile
+    (3000, 480, 608, 30, 4, 0, None, 60),    # 2 to 6 tiles per XCD in 4 or 8 pieces
+    (4100, 544, 352, 10, 4, 1, 1.0, 100),    # skew: tiles of 1 to 8 fragment rows
+    (2900, 352, 544, 20, 6, 2, 0.3, 30),
+])
+def test_tiles_of_64_k_values(M, D, H, N, K, Ks, skew, sp):
+    from momoe_amd import _hip, experts
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, Ks=Ks, seed=6, skew=skew)
+    gemms = ((2 * H, D), (D, H), (H, D), (D, 2 * H))
+    assert any(_hip._lib.momoe_gemm_tile_rows(M * K, N, *g) == _hip.RECOMPUTE_TILE_ROWS for g in gemms)
+    dev = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+    _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
+    # halved tiles of 320 rows, tiles of three fragment rows: the same sums
+    for rows in (_hip.TILE_ROWS, 96):
+        try:
+            experts.TILE_ROWS = rows
+            other = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
+        finally:
+            experts.TILE_ROWS = _hip.AUTO_TILE_ROWS
+        for k in ("y", "G_x"):
+            assert torch.equal(other[k], dev[k]), (rows, k)
+
+
 @pytest.mark.parametrize("M,D,H,N,K,Ks,skew,rows", [
     (1024, 992, 480, 32, 4, 1, 0.5, 256),    # a partial dL/ds per 64 of 480 hidden columns: 8
     (1000, 1024, 416, 32, 4, 2, 0.3, 256),   # 7: the last 128-column tile has no second one
