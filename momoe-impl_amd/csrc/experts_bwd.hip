@@ -47,7 +47,8 @@ struct DhSpan {
   template <int NA>
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late&,
                                            bf16* staging) const {
-    store_rows(tc, acc, staging, p.u, p.H, tc.tn * G::COLS + n_org, fresh_lane(), [](int) { return 1.0f; });
+    store_rows(acc, staging, p.u, (int64_t)tc.row0 + tc.mbase, tc.rows - tc.mbase, p.H, tc.tn * G::COLS + n_org,
+               fresh_lane(), [](int) { return 1.0f; });
   }
 };
 
@@ -272,7 +273,8 @@ struct DxSpan {
   template <int NA>
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late&,
                                            bf16* staging) const {
-    store_rows(tc, acc, staging, p.gxs, p.D, tc.tn * G::COLS + n_org, fresh_lane(), [](int) { return 1.0f; });
+    store_rows(acc, staging, p.gxs, (int64_t)tc.row0 + tc.mbase, tc.rows - tc.mbase, p.D, tc.tn * G::COLS + n_org,
+               fresh_lane(), [](int) { return 1.0f; });
   }
 };
 

@@ -67,6 +67,7 @@ struct Lin1Span {
     const int rows = tc.rows - tc.mbase;
     const int64_t r0 = (int64_t)tc.row0 + tc.mbase;
     if (p.h) {
+      keep_in_place(acc);
       // h is k-blocked for the next GEMM: 32 hidden columns of consecutive rows are one piece of memory
       bf16* const first = p.h + ((int64_t)(j0 >> 5) * p.msum + r0) * 32;  // uniform
       const uint32_t off = (stager.block_row() * 32 + stager.block_col()) * 2;
@@ -96,6 +97,7 @@ struct Lin1Span {
       store(NA - 1);
     }
     if (p.ab) {
+      keep_in_place(acc);
 #pragma unroll
       for (int i = 0; i < NA; ++i)
 #pragma unroll
@@ -482,7 +484,8 @@ struct Lin2Span {
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late& s,
                                            bf16* staging) const {
     const int lane = fresh_lane();
-    store_rows(tc, acc, staging, p.ys, p.D, tc.tn * G::COLS + n_org, lane, [&](int i) { return s.of(i, lane); });
+    store_rows(acc, staging, p.ys, (int64_t)tc.row0 + tc.mbase, tc.rows - tc.mbase, p.D, tc.tn * G::COLS + n_org, lane,
+               [&](int i) { return s.of(i, lane); });
   }
 };
 

@@ -80,9 +80,11 @@ __device__ __forceinline__ void dma16_at(const void* uniform_base, uint32_t byte
 
 // Stores 16 bytes per lane at a uniform base plus a byte offset below 2 GiB; lanes that are not `valid` store
 // nothing.  Without a branch: under a divergent one the compiler took what follows it for divergent, too.
+// STREAM: non-temporal.
+template <bool STREAM = false>
 __device__ __forceinline__ void store16(void* uniform_base, uint32_t byte_offset, bool valid, bf16x8 v) {
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_base, 0, 0x7FFFFFFF, 0x00027000);
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, STREAM ? 2 : 0);
 }
 
 // ---- operands -------------------------------------------------------------------------------------
@@ -105,7 +107,7 @@ struct SpanRowsLayout {
   struct Lane {
     int o[2];
     __device__ __forceinline__ explicit Lane(int org) {
-      const int r = lane_id() & 15, g = lane_id() >> 4;
+      const int l = fresh_lane(), r = l & 15, g = l >> 4;
 #pragma unroll
       for (int h = 0; h < 2; ++h) o[h] = (org + r) * kSpan + ((4 * h + g) ^ (r >> 1)) * 8;
     }
@@ -201,7 +203,7 @@ struct SpanBlockedRows {
   struct Lane {
     int o;
     __device__ __forceinline__ explicit Lane(int org) {
-      const int r = lane_id() & 15, g = lane_id() >> 4;
+      const int l = fresh_lane(), r = l & 15, g = l >> 4;
       o = (org + r) * kHalf + (g ^ swz(r)) * 8;
     }
   };
@@ -249,7 +251,7 @@ struct SpanCols {
   struct Lane {
     int o;  // first fragment
     __device__ __forceinline__ explicit Lane(int org) {
-      const int l = lane_id(), krow = 8 * (l >> 4) + ((l & 15) >> 2), col = org + 4 * (l & 3);
+      const int l = fresh_lane(), krow = 8 * (l >> 4) + ((l & 15) >> 2), col = org + 4 * (l & 3);
       o = krow * COLS + (((col >> 3) ^ swz(krow)) << 3) + (col & 7);
     }
   };
@@ -328,6 +330,60 @@ struct SpanStages {
   __device__ __forceinline__ int after(int k) const { return min(k + kSpan, kmax); }  // k-origin of the next stage
 };
 
+// Copies of the accumulators to vector registers are made after this point, where they are used: made ahead,
+// beside a main loop's fragments, they were spilled, and every reload waits for the stores before it.
+template <int FN, int NA>
+__device__ __forceinline__ void keep_in_place(f32x4 (&acc)[FN][NA]) {
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+#pragma unroll
+    for (int i = 0; i < NA; ++i) asm volatile("" : "+a"(acc[j][i]));
+}
+
+// A wave's fragments of a stage, NA of rows and FN of weights, in two register sets
+template <class Rows, class Weights, int FN, int NA>
+struct SpanFrags {
+  static constexpr int NM = NA * FN;
+  typename Rows::Lane alane;
+  typename Weights::Lane wlane;
+  bf16x8 af[2][NA > 0 ? NA : 1], wf[2][FN];
+  __device__ __forceinline__ SpanFrags(int m_org, int n_org) : alane(m_org), wlane(n_org) {}
+  // fragment R (weights first) of half H of the stage at (w, a) into register set B
+  template <int B, int R, int H>
+  __device__ __forceinline__ void read(const bf16* w, const bf16* a) {
+    if constexpr (NA == 0) return;
+    else if constexpr (R < FN) wf[B][R] = Weights::frag(w, wlane, R, H);
+    else af[B][R - FN] = Rows::frag(a, alane, R - FN, H);
+  }
+  template <int B, int H>
+  __device__ __forceinline__ void read_all(const bf16* w, const bf16* a) {
+    unrolled<0, FN + NA>([&](auto R) { read<B, decltype(R)::value, H>(w, a); });
+  }
+  // The products of register set B; between them the reads of half H (-1: none) of (w, a) into the other set,
+  // and DEP calls of `dep`
+  template <int B, int H, int DEP, class Dep>
+  __device__ __forceinline__ void multiply(f32x4 (&acc)[FN][NA > 0 ? NA : 1], const bf16* w, const bf16* a, Dep dep) {
+    if constexpr (NM == 0) {
+      unrolled<0, DEP>([&](auto D) { dep(D); });
+    } else {
+      constexpr int NR = H >= 0 ? FN + NA : 0, PER = (2 * NR + NM - 1) / NM;  // reads behind an MFMA: in the first half
+      unrolled<0, NM>([&](auto MC) {
+        constexpr int m = decltype(MC)::value, j = m / NA, i = (j & 1) ? NA - 1 - m % NA : m % NA;
+        acc[j][i] = mfma16(wf[B][j], af[B][i], acc[j][i]);
+        unrolled<0, PER>([&](auto R) {
+          constexpr int r = m * PER + decltype(R)::value;
+          if constexpr (r < NR) read<B ^ 1, r, (H > 0 ? 1 : 0)>(w, a);
+        });
+        unrolled<0, DEP>([&](auto D) {
+          constexpr int d = decltype(D)::value;
+          if constexpr (((2 * d + 1) * NM) / (2 * DEP) == m) dep(D);
+        });
+        order_fence();
+      });
+    }
+  }
+};
+
 constexpr int kStagingElems = 4096;  // a wave's share of the epilogue's staging
 
 // Keeps `v` in its register from here on: the compiler waits for the load behind it now and not at
@@ -394,7 +450,6 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
   g1 = g0;
   if (c1.valid) prog.gather(c1, g1);
   TileCoord c2 = sched.next();
-  const typename Weights::Lane wlane(prog.n_org);
   prog.settle(g0);
   prog.settle(g1);
   prog.late(c0, g0, l0);
@@ -411,45 +466,13 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
 
     // this tile for a wave with NA fragment rows
     auto tile = [&](auto NAC) {
-      constexpr int NA = decltype(NAC)::value, NM = NA * FN;
+      constexpr int NA = decltype(NAC)::value;
       f32x4 acc[FN][NA > 0 ? NA : 1];
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int i = 0; i < NA; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      const typename Rows::Lane alane(c0.mbase);
-      bf16x8 af[2][NA > 0 ? NA : 1], wf[2][FN];
-      // fragment r (weights first) of half h of the stage in slots s, s+1 into register set b
-      auto read = [&](int b, int r, const bf16* w, const bf16* a, int h) {
-        if constexpr (NA > 0) {
-          if (r < FN) wf[b][r] = Weights::frag(w, wlane, r, h);
-          else af[b][r - FN] = Rows::frag(a, alane, r - FN, h);
-        }
-      };
-      // MFMAs of register set B; between them the reads of half H of (w, a) into the other set, and `dep`'s
-      // DEP deposits
-      auto multiply = [&](auto B, auto READ, const bf16* w, const bf16* a, auto H, auto DEPC, auto dep) {
-        constexpr int b = decltype(B)::value, h = decltype(H)::value, DEP = decltype(DEPC)::value;
-        constexpr int NR = decltype(READ)::value ? FN + NA : 0;
-        constexpr int PER = NM > 0 ? (2 * NR + NM - 1) / (NM > 0 ? NM : 1) : 0;  // reads behind an MFMA of the first half
-        if constexpr (NM == 0) {
-          unrolled<0, DEP>([&](auto D) { dep(D); });
-        } else {
-          unrolled<0, NM>([&](auto MC) {
-            constexpr int m = decltype(MC)::value, j = m / NA, i = (j & 1) ? NA - 1 - m % NA : m % NA;
-            acc[j][i] = mfma16(wf[b][j], af[b][i], acc[j][i]);
-            unrolled<0, PER>([&](auto R) {
-              constexpr int r = m * PER + decltype(R)::value;
-              if constexpr (r < NR) read(b ^ 1, r, w, a, h);
-            });
-            unrolled<0, DEP>([&](auto D) {
-              constexpr int d = decltype(D)::value;
-              if constexpr (((2 * d + 1) * NM) / (2 * DEP) == m) dep(D);
-            });
-            order_fence();
-          });
-        }
-      };
+      SpanFrags<Rows, Weights, FN, NA> fr(c0.mbase, prog.n_org);
       // the next stage has landed, all but what was requested after it; every wave is done reading this one
       auto turn = [&] {
         wait_vmcnt<(AHEAD - 1) * Weights::DEP + (AHEAD - 2) * Rows::DEP>();
@@ -458,8 +481,7 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
         order_fence();
       };
       const bf16 *w = wptr(sw), *a = aptr(sa);
-#pragma unroll
-      for (int r = 0; r < FN + NA; ++r) read(0, r, w, a, 0);
+      fr.template read_all<0, 0>(w, a);
       order_fence();
       int t = 0, end = st.count - AHEAD;
       while (true) {
@@ -471,11 +493,11 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
           sw = wnext(sw);
           sa = anext(sa);
           const bf16 *nw = wptr(sw), *na = aptr(sa);
-          multiply(IntC<0>{}, IntC<1>{}, w, a, IntC<1>{}, IntC<Weights::DEP>{},
-                   [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
+          fr.template multiply<0, 1, Weights::DEP>(
+              acc, w, a, [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
           turn();
-          multiply(IntC<1>{}, IntC<1>{}, nw, na, IntC<0>{}, IntC<Rows::DEP>{},
-                   [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
+          fr.template multiply<1, 0, Rows::DEP>(
+              acc, nw, na, [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
           k = st.after(k);
           w = nw;
           a = na;
@@ -494,9 +516,8 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
         const bf16 *wsrc = W.source(k), *asrc = A.source(k);
         const int before = sw == 0 ? AHEAD : sw - 1;
         unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wslot(before)); });
-#pragma unroll
-        for (int r = 0; r < FN + NA; ++r) read(0, r, w, a, 1);
-        multiply(IntC<0>{}, IntC<0>{}, w, a, IntC<1>{}, IntC<0>{}, [](auto) {});
+        fr.template read_all<0, 1>(w, a);
+        fr.template multiply<0, -1, 0>(acc, w, a, [](auto) {});
         turn();
         unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, aslot(sa)); });
         k = st.after(k);
@@ -505,6 +526,7 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
       }
       // staging: where the finished tile's last weights were; every wave has read them, and the next ones are
       // requested behind the barrier below
+      keep_in_place(acc);
       if constexpr (NA > 0) prog.epilogue(c0, acc, g0, l0, lds + (sw == 0 ? AHEAD : sw - 1) * Weights::ELEMS);
     };
     const int na = __builtin_amdgcn_readfirstlane(c0.na);
@@ -635,15 +657,14 @@ __device__ __forceinline__ bf16x4 pack_bf16x4(f32x4 v, float s) {
   return bf16x4{(bf16)(v[0] * s), (bf16)(v[1] * s), (bf16)(v[2] * s), (bf16)(v[3] * s)};
 }
 
-// A wave's accumulators as rows of a row-major matrix of `cols` columns, from column col0; scale(i) is that of
+// A wave's accumulators as `rows` rows, from row0, of a row-major matrix of `cols` columns, from column col0; scale(i) is that of
 // the lane's row in fragment row i; lane = fresh_lane()
-template <int FN, int NA, class Scale>
-__device__ __forceinline__ void store_rows(const TileCoord& tc, f32x4 (&acc)[FN][NA], bf16* staging, bf16* out, int cols,
+template <bool STREAM = false, int FN, int NA, class Scale>
+__device__ __forceinline__ void store_rows(f32x4 (&acc)[FN][NA], bf16* staging, bf16* out, int64_t row0, int rows, int cols,
                                            int col0, int lane, Scale scale) {
   using Stager = SpanStager<16 * FN>;
   const Stager stager(staging, lane);
-  bf16* const first = out + ((int64_t)tc.row0 + tc.mbase) * cols + col0;  // uniform
-  const int rows = tc.rows - tc.mbase;
+  bf16* const first = out + row0 * cols + col0;  // uniform
   uint32_t off[Stager::PASSES];
 #pragma unroll
   for (int p = 0; p < Stager::PASSES; ++p) off[p] = ((uint32_t)stager.row(p) * (uint32_t)cols + stager.col(p)) * 2;
@@ -651,7 +672,7 @@ __device__ __forceinline__ void store_rows(const TileCoord& tc, f32x4 (&acc)[FN]
   auto store = [&](int i) {
 #pragma unroll
     for (int p = 0; p < Stager::PASSES; ++p)
-      store16(first + (int64_t)(16 * i) * cols, off[p], 16 * i + stager.row(p) < rows && col0 + stager.col(p) < cols,
+      store16<STREAM>(first + (int64_t)(16 * i) * cols, off[p], 16 * i + stager.row(p) < rows && col0 + stager.col(p) < cols,
               v[i & 1][p]);
   };
 #pragma unroll
