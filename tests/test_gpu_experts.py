@@ -298,6 +298,59 @@ def test_weight_gradient_from_a_transposed_operand(sizes, M):
         _hip.wgrad(grouped(A), None, grouped(B), None, cumsums, GW, M, msum, a_transposed=True, b_transposed=True)
 
 
+@pytest.mark.parametrize("sizes,X,Y", [
+    ([0, 1, 33, 64, 65, 130, 1100, 257], 264, 328),     # 206 rows per expert on average, edges in X and Y
+    ([2000, 0, 31, 1500], 512, 256),                     # whole tiles; two experts that are cut by rows
+    ([129, 1, 0, 300, 128, 127, 95, 5], 520, 72),        # 98 rows per expert: the short loop
+])
+@pytest.mark.parametrize("form", ["gather_a", "gather_b", "a_transposed", "b_transposed", "b_kblocked"])
+def test_weight_gradient_loops_at_the_edges(sizes, X, Y, form):
+    # Bound: products of bf16 pairs are exact in fp32, so n of them sum to within n 2^-24 of their
+    # absolute sum, and the result is rounded to bf16 once (2^-8 relative).
+    from momoe_amd import _hip
+    dev = "cuda:0"
+    if form == "b_kblocked":
+        Y = Y // 32 * 32
+    N, msum, M = len(sizes), sum(sizes), 1500
+    M = max(M, max(sizes))
+    c = [0] + list(torch.tensor(sizes).cumsum(0).tolist())
+    cumsums = torch.tensor(c, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(21)
+    A = torch.randn(M if form == "gather_a" else msum, X, generator=g, device=dev).to(torch.bfloat16)
+    B = torch.randn(M if form == "gather_b" else msum, Y, generator=g, device=dev).to(torch.bfloat16)
+    ids = torch.randint(0, M, (msum,), generator=g, device=dev, dtype=torch.int32)
+
+    def grouped(rows):
+        mpad = _hip.padded_rows(msum, N)
+        T = torch.full((mpad, rows.shape[1]), float("nan"), device=dev, dtype=rows.dtype)
+        for e in range(N):
+            p0, n = (c[e] + 31) // 32 * 32 + 32 * e, sizes[e]
+            T[p0:p0 + (n + 31) // 32 * 32] = 0
+            T[p0:p0 + n] = rows[c[e]:c[e + 1]]
+        return T.reshape(mpad // 32, 32, -1).permute(0, 2, 1).contiguous()
+
+    a, b, kw, ga, gb = A, B, {}, None, None
+    rows_a, rows_b = A, B
+    if form == "gather_a":
+        ga, rows_a = ids, A[ids.long()]
+    elif form == "gather_b":
+        gb, rows_b = ids, B[ids.long()]
+    elif form == "a_transposed":
+        a, kw = grouped(A), dict(a_transposed=True)
+    elif form == "b_transposed":
+        b, kw = grouped(B), dict(b_transposed=True)
+    else:
+        b, kw = B.reshape(msum, Y // 32, 32).permute(1, 0, 2).contiguous(), dict(b_kblocked=True)
+    for ws in (None, 0):
+        GW = torch.full((N, X, Y), float("nan"), device=dev, dtype=torch.bfloat16)
+        _hip.wgrad(a, ga, b, gb, cumsums, GW, M, msum, workspace_bytes=ws, **kw)
+        for e in range(N):
+            pa, pb = (t[c[e]:c[e + 1]].double().cpu() for t in (rows_a, rows_b))
+            want, size = pa.T @ pb, pa.abs().T @ pb.abs()
+            bound = want.abs() * 2.0**-8 + size * (sizes[e] * 2.0**-24 * (1 + 2.0**-8))
+            assert torch.all((GW[e].double().cpu() - want).abs() <= bound), f"expert {e} ws={ws}"
+
+
 def test_experts_without_tokens_get_zero_weight_grads():
     M, D, H, N, K = 256, 128, 64, 8, 2
     x, W1, W2, _, _, dy = make_layer_inputs(M, D, H, N, K, seed=9)
