@@ -237,8 +237,11 @@ struct WorkItems {
       return items_before(lo) + (int)((c - pl.cost[lo] + each - 1) / each);
     };
     const int64_t total_cost = pl.cost[p.N];
-    int2 run = {0, 0};
-    if (THREADS != kSpanThreads || !whole_rounds(pl, items_before, run))
+    const int total = items_before(p.N), all = gridDim.x;
+    int2 run;
+    if (total <= all)  // one each
+      run = {total * xcd / 8, total * (xcd + 1) / 8};
+    else if (THREADS != kSpanThreads || !whole_rounds(pl, items_before, run))
       run = {item_at(total_cost * xcd / 8), item_at(total_cost * (xcd + 1) / 8)};
     g_end = uniform(run.y);
     pos = uniform(run.x) + (int)(blockIdx.x >> 3);
