@@ -27,6 +27,7 @@ struct DhArgs {
 template <class G_>
 struct DhSpan {
   using G = G_;
+  static constexpr bool EXCHANGE = false;
   using Rows = SpanGatheredRows<256>;
   using Weights = SpanPitchedRows<G::COLS>;
   using Ids = FetchIds;
@@ -253,6 +254,7 @@ struct DxArgs {
 template <class G_>
 struct DxSpan {
   using G = G_;
+  static constexpr bool EXCHANGE = false;
   using Rows = SpanBlockedRows<256>;
   using Weights = SpanPitchedRows<G::COLS>;
   struct Ids {};

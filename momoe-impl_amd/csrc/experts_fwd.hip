@@ -37,6 +37,7 @@ struct Lin1Args {
 template <class G_>
 struct Lin1Span {
   using G = G_;
+  static constexpr bool EXCHANGE = false;
   static constexpr int BNH = G::COLS / 2, WIDTH = 8 * G::FN;  // hidden columns of a tile, of a wave
   using Rows = SpanGatheredRows<256>;
   using Weights = SpanCols<G::COLS, true>;
@@ -124,6 +125,176 @@ __global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_fwd_kernel(Lin1Ar
   using Prog = Lin1Span<WideSpan>;
   run_span_tiles<Prog>(p, (p.H + Prog::BNH - 1) / Prog::BNH, MOMOE_TILE_ROWS, first);
   trace.finish();
+}
+
+// The recomputing backward (momoe/momoe.py:421-535), on the tiles of the forward: the a|b of the tile stay in registers and go
+// straight into the SwiGLU backward.  With u = dL/dh before the gate weight s,  G_a = s u b sig(b),
+// G_b = s u a sig(b) (1 + b (1 - sig(b))),  hs = s a b sig(b),  and the row sums of u a b sig(b) over the
+// tile's 128 hidden columns.
+struct Lin1BwdSpan {
+  using G = WideSpan;
+  static constexpr bool EXCHANGE = true;
+  static constexpr int BNH = G::COLS / 2, WIDTH = 8 * G::FN, HF = G::FN / 2;
+  static_assert(BNH == MOMOE_GS_BLOCK && G::WCOLS == 2, "a tile's row sums are one part, from two waves");
+  using Rows = SpanGatheredRows<256>;
+  using Weights = SpanCols<G::COLS, true>;
+  using Stager = SpanStager<WIDTH>;
+  struct Ids {
+    FetchIds fetch;
+    RowIds rows;  // of the accumulators
+  };
+  using Late = RowScales;
+  const Lin1Args& p;
+  const int K, n_org;
+
+  __device__ __forceinline__ explicit Lin1BwdSpan(const Lin1Args& p_)
+      : p(p_), K(p_.D), n_org(wave_id() % G::WCOLS * WIDTH) {}
+  __device__ __forceinline__ void gather(const TileCoord& t, Ids& g) const { g.fetch.gather(t, p.idx), g.rows.gather(t, p.idx); }
+  __device__ __forceinline__ void late(const TileCoord& t, const Ids& g, Late& l) const { l.load(t, g.rows, p.s, p.ssn, p.ssm); }
+  __device__ __forceinline__ void settle(Ids& g) const { momoe::settle(g.fetch.tok), g.rows.settle(); }
+  __device__ __forceinline__ void settle(Late& l) const { l.settle(); }
+  __device__ __forceinline__ void setup(const TileCoord& t, const Ids& g, Rows& A, Weights& W) const {
+    const int D = p.D, H = p.H, j0 = t.tn * BNH;
+    A.init(p.x, [&](int j, int l) { return (uint32_t)g.fetch.of(j, l) * (uint32_t)(2 * D); });
+    W.init(p.w1 + (int64_t)t.expert * D * 2 * H, 2 * H,
+           [&](int c) { return (c / BNH) * H + min(j0 + (c % BNH), H - 8); });
+  }
+  // Rows below the save boundary are not this kernel's: the boundary is moved down to a multiple of 32
+  // rows from the expert's first row (tiles start at such multiples), so that a whole group of 32 rows is
+  // either produced here or by momoe_swiglu_bwd_saved.
+  __device__ __forceinline__ int first_row(const TileCoord& tc) const {
+    return p.ab_lo > tc.row0 ? (int)((p.ab_lo - tc.row0) & ~(int64_t)31) : 0;
+  }
+  // Staging areas: 0 G_a, 1 G_b, 2 and 3 hs of 32 rows.
+  template <int NA>
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x4 (&acc)[G::FN][NA], const Ids&, const Late& scales,
+                                           bf16* staging) const {
+    static_assert(4 * Stager::ELEMS <= kStagingElems && NA % 2 == 0, "four areas; groups of 32 rows");
+    const int H = p.H, j0 = tc.tn * BNH + n_org;  // first hidden column of this wave
+    const int l = fresh_lane();
+    const Stager stager(staging, l);
+    const int rows = tc.rows - tc.mbase, lo = first_row(tc) - tc.mbase;
+    const int64_t r0 = (int64_t)tc.row0 + tc.mbase;
+    const bf16* const u0 = p.u + r0 * H;  // uniform
+    bf16x4 uq[2][HF];
+    auto load_u = [&](int i) {
+      const uint32_t at = ((uint32_t)min(16 * i + (l & 15), rows - 1) * (uint32_t)H + 4 * (l >> 4)) * 2;
+#pragma unroll
+      for (int f = 0; f < HF; ++f) uq[i & 1][f] = *(const bf16x4*)((const char*)(u0 + (j0 + 16 * f < H ? j0 + 16 * f : 0)) + at);
+    };
+    // gz is k-blocked ([2H/32][Msum][32], the layout dL/dx contracts over): 32 columns of consecutive rows are one
+    // piece of memory
+    bf16* const gza = p.gz + ((int64_t)(j0 >> 5) * p.msum + r0) * 32;  // uniform
+    const int64_t to_b = (int64_t)(H >> 5) * p.msum * 32;
+    const uint32_t off = (stager.block_row() * 32 + stager.block_col()) * 2;
+    bf16x8 v[2][2][Stager::PASSES];
+    auto store_gz = [&](int i) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int q = 0; q < Stager::PASSES; ++q)
+          store16(gza + half * to_b + ((int64_t)q * p.msum + 16 * i) * 32, off,
+                  16 * i + stager.block_row() < rows && 16 * i >= lo && j0 + 32 * q < H, v[i & 1][half][q]);
+    };
+    // hs^T leaves as 8 consecutive rows of a column per lane.  Rows past the expert's last one are zeros: the
+    // padding that the weight-gradient GEMM reads.
+    bf16* const hst = p.hst + ((int64_t)((tc.prow0 + tc.mbase) >> 5) * p.ldt + j0) * 32;  // uniform
+    const uint32_t hoff = (l & 15) * 64 + (l >> 4) * 16;
+    bf16x8 hv[HF];
+    auto store_hs = [&](int i) {
+#pragma unroll
+      for (int q = 0; q < HF; ++q)
+        store16(hst + ((int64_t)(i / 2) * p.ldt + 16 * q) * 32, hoff, 16 * i >= lo && j0 + 16 * q < H, hv[q]);
+    };
+    load_u(0);
+    float gsums[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      if (i + 1 < NA) load_u(i + 1);
+      const float sv = scales.of(i, l);
+      const bool some = 16 * i + (l & 15) < rows;
+      float gsum = 0.0f;
+#pragma unroll
+      for (int f = 0; f < HF; ++f) {
+        float va[4], vb[4], hs[4], part = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = acc[f][i][e], b = acc[HF + f][i][e];
+          const float u = (float)uq[i & 1][f][e];
+          const float sg = sigmoidf_fast(b);
+          const float t = b * sg;  // silu(b)
+          const float hval = a * t;
+          part += u * hval;
+          const float gh = sv * u;
+          va[e] = gh * t;
+          // d silu / d b = sg (1 + b (1 - sg)) = sg + t - t sg
+          vb[e] = (gh * a) * __builtin_fmaf(-t, sg, sg + t);
+          hs[e] = some ? sv * hval : 0.0f;
+        }
+        if (j0 + 16 * f < H) gsum += part;
+        momoe::settle(gsum);  // (summed up later, u and its factors were kept until then)
+        stager.put(0, f, pack_bf16x4(va[0], va[1], va[2], va[3]));
+        stager.put(1, f, pack_bf16x4(vb[0], vb[1], vb[2], vb[3]));
+        stager.put(2 + (i & 1), f, pack_bf16x4(hs[0], hs[1], hs[2], hs[3]));
+      }
+      gsums[i] = gsum;
+      if (i > 0) store_gz(i - 1);
+      if (i > 0 && i % 2 == 0) store_hs(i - 1);
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int q = 0; q < Stager::PASSES; ++q) v[i & 1][half][q] = stager.get_block(half, q);
+      if (i % 2 == 1) {
+#pragma unroll
+        for (int q = 0; q < HF; ++q) hv[q] = stager.get_rows(2, q);
+      }
+      order_fence();  // (loads of several rounds ahead were spilled)
+    }
+    store_gz(NA - 1);
+    store_hs(NA - 1);
+    // this wave's row sums, for finish()
+    float* const red = (float*)(staging + wave_id() * kStagingElems);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      float g = gsums[i] + __shfl_xor(gsums[i], 16);
+      g += __shfl_xor(g, 32);
+      red[16 * i + (l & 15)] = g;  // (the same from four lanes)
+    }
+  }
+  __device__ __forceinline__ void finish(const TileCoord& tc, bf16* staging) const {
+    if (n_org != 0) return;  // wave-uniform: the other column half's wave is the next one
+    const int l = fresh_lane(), lo = first_row(tc) - tc.mbase, rows = min(tc.rows - tc.mbase, 32 * tc.na);
+    const float* const red = (const float*)(staging + wave_id() * kStagingElems);
+    float* const part = p.gs_part + (int64_t)tc.tn * p.msum + tc.row0 + tc.mbase;  // uniform
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int row = 64 * q + l;
+      store4(part, row * 4, row < rows && row >= lo, red[row] + red[row + kStagingElems / 2]);
+    }
+  }
+};
+
+// Bound by the loop of gemm_span.hpp; the epilogue is some 6 us of a tile, of which the stores of gz (128 KB) and
+// hs^T (64 KB) need 5 at the HBM's rate.
+__global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_bwd_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  const int first = p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
+  run_span_tiles<Lin1BwdSpan>(p, (p.H + Lin1BwdSpan::BNH - 1) / Lin1BwdSpan::BNH, WideSpan::MAX_ROWS, first);
+  trace.finish();
+}
+
+// Whether a launch takes it rather than the 8 waves of Lin1Prog<true, StdTiles>: with as much work per workgroup
+// as pays for the longer start and the last epilogue, about 3 us.  A tile costs 0.4 for its weights and 0.6 for
+// 256 rows.
+// Measured, there -> here in us: 65536 tokens, D = 4096, H = 2048, N = 64, K = 8 17297 -> 14150; 8192, 2048, 1024, 128, 8
+// 664 -> 561; 7680, 2176, 1152, 64, 6 509 -> 437; 4000, 1024, 512, 64, 4 69 -> 57; 2048, 2048, 1024, 128, 8 (128
+// rows per expert) 275 -> 267; in one round of tiles 3000, 3072, 1024, 32, 2 112 -> 102; 16000, 1024, 256, 128, 1
+// (125 rows per expert, one round) 34 -> 38; 12000, 256, 128, 32, 4 21.6 -> 23.7.
+inline bool takes_span_recompute(int64_t msum, int64_t n, int64_t h, int64_t d) {
+  if (d < WideSpan::AHEAD * kSpan || few_rows_per_expert(msum, n)) return false;
+  const double mean = (double)msum / n, tiles = std::ceil(mean / WideSpan::MAX_ROWS);
+  const double rounds = std::max(1.0, n * tiles * (double)cdiv64(h, Lin1BwdSpan::BNH) / persistent_grid());
+  return rounds * d * (0.4 + 0.6 * mean / (tiles * WideSpan::MAX_ROWS)) >= 780;
 }
 
 // Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave owns 32 `a`
@@ -460,6 +631,7 @@ struct Lin2Args {
 template <class G_>
 struct Lin2Span {
   using G = G_;
+  static constexpr bool EXCHANGE = false;
   using Rows = SpanBlockedRows<256>;   // rows of h, k-blocked
   using Weights = SpanCols<G::COLS>;
   using Ids = RowIds;     // tokens of the rows this wave holds in the accumulators
@@ -749,6 +921,10 @@ extern "C" int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2
              row_lo, Msum, (int)D, (int)H, (const bf16*)u_MsumH, s_NM, s_stride_n, s_stride_m,
              (bf16*)gz_blocked, (bf16*)hsT_GH32, ld_hsT, gs_part, Msum, clock_trace_buffer()};
   if (narrow) return launch_lin1_narrow<true>(a, (hipStream_t)stream);
+  if (takes_span_recompute(Msum, N, H, D)) {
+    static LdsLimit span;
+    return launch_span(lin1_swiglu_bwd_kernel, a, span, (hipStream_t)stream);
+  }
   return launch_lin1<true, StdTiles>(a, (hipStream_t)stream);
 }
 

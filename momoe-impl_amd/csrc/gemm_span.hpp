@@ -87,6 +87,12 @@ __device__ __forceinline__ void store16(void* uniform_base, uint32_t byte_offset
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, STREAM ? 2 : 0);
 }
 
+// the same for 4 bytes
+__device__ __forceinline__ void store4(float* uniform_base, uint32_t byte_offset, bool valid, float v) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_base, 0, 0x7FFFFFFF, 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, 0);
+}
+
 // ---- operands -------------------------------------------------------------------------------------
 // Common to all: DEP deposits (wave-wide transfers of 1 KiB) per wave and stage; source(k) is where the
 // stage that starts at k-value k (a multiple of 32) lies, deposit<j>(source, slot) requests the j-th into
@@ -401,6 +407,7 @@ __device__ __forceinline__ void settle(T& v) {
 //   settle(ids) / settle(late)                 settle() each register of them
 //   setup(tile, ids, A, W)                     operand set-up
 //   epilogue(tile, acc, ids, late, staging)    acc [FN][fragment rows]; staging: kStagingElems of LDS per wave
+//   EXCHANGE, finish(tile, staging)            if the waves leave values for each other there: behind a barrier
 //   K, n_org[FN]                               contraction length, first columns of the fragments
 // While tile t is multiplied, the ids of tile t+2, the late values of tile t+1 and the table entry of
 // tile t+3 are on their way.  All of them settle at the end of tile t's epilogue: the compiler does
@@ -535,6 +542,11 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
     else if (na == 2) tile(IntC<4>{});
     else if (na == 1) tile(IntC<2>{});
     else tile(IntC<0>{});
+    if constexpr (P::EXCHANGE) {
+      wait_lgkm0();
+      __builtin_amdgcn_s_barrier();
+      prog.finish(c0, lds + (sw == 0 ? AHEAD : sw - 1) * Weights::ELEMS);
+    }
     prog.settle(g2);
     prog.settle(l1);
     if (!c1.valid) break;
@@ -646,7 +658,16 @@ struct SpanStager {
   __device__ __forceinline__ bf16x8 get(int area, int p) const {
     return *(const bf16x8*)(st + area * ELEMS + row(p) * WIDTH + (l % CHUNKS) * 8);
   }
-  // the same with a pass of 32 columns of 16 rows: 8 columns from 32 p + block_col() of block_row()
+  // 8 rows, from 8 * (l / 16), of column 16 p + l % 16 of the 32 rows in areas `area` and `area` + 1
+  __device__ __forceinline__ bf16x8 get_rows(int area, int p) const {
+    const int row = 8 * (l >> 4) + ((l & 15) >> 2);  // (lds_read_tr4: this lane names the address of a neighbour's)
+    auto at = [&](int r) {
+      return st + (area + (r >> 4)) * ELEMS + (r & 15) * WIDTH + ((2 * p + ((l & 3) >> 1)) ^ swz(r & 15)) * 8 + (l & 1) * 4;
+    };
+    const bf16x4 lo = lds_read_tr4(at(row)), hi = lds_read_tr4(at(row + 4));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  // as row(), col() and get() with a pass of 32 columns of 16 rows: 8 columns from 32 p + block_col() of block_row()
   __device__ __forceinline__ int block_row() const { return l >> 2; }
   __device__ __forceinline__ int block_col() const { return (l & 3) * 8; }
   __device__ __forceinline__ bf16x8 get_block(int area, int p) const {

@@ -666,6 +666,70 @@ def test_recomputing_gemm_ignores_a_table_of_taller_tiles():
     assert not bool((run(own)[0] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,D,H,N,K,Ks,skew,row_lo", [
+    (3000, 1056, 416, 12, 4, 0, None, 0),     # 16.5 stages; a column block whose second half is past H
+    (2500, 2080, 352, 14, 4, 1, 1.0, 4001),   # tiles of 1 to 8 fragment rows, a boundary inside an expert
+    (2600, 2048, 288, 24, 3, 0, 0.5, 2048),   # one 32-column block in the last tile
+])
+def test_recomputing_gemm_in_the_span_loop(M, D, H, N, K, Ks, skew, row_lo):
+    """G_z, hs^T and the partial dL/ds against 64-bit arithmetic.  Bounds: a and b are fp32 sums of D exact
+    products, D 2^-24 of their absolute sum off; that error times the derivatives (|silu'| <= 1.1, |silu''| <=
+    0.5); fp32 arithmetic and the fast exp and reciprocal, 2^-19 of the factors; bf16 results, 2^-8."""
+    from momoe_amd import _hip
+    dev = "cuda:0"
+    x, W1, _, mask, s, _ = make_layer_inputs(M, D, H, N, K, Ks=Ks, seed=8, skew=skew)
+    msum = M * K
+    ib = _hip.index_build(mask.to(dev), K, recompute_table=True)
+    idx, c = ib["idx_Msum"], [0] + mask.sum(1).cumsum(0).tolist()
+    xb, W1b, sd = x.to(dev).to(torch.bfloat16), W1.to(dev).to(torch.bfloat16), s.to(dev)
+    u = torch.randn(msum, H, generator=torch.Generator(device=dev).manual_seed(3), device=dev).to(torch.bfloat16)
+
+    def run(table):
+        full = lambda *shape, dt=torch.bfloat16: torch.full(shape, 7.0, device=dev, dtype=dt)
+        out = (full(2 * H // 32, msum, 32), full(_hip.padded_rows(msum, N) // 32, H, 32),
+               full(-(-H // _hip.GS_BLOCK), msum, dt=torch.float32))
+        _hip.lin1_swiglu_bwd(xb, W1b, idx, table, u, sd, row_lo, *out)
+        return out
+
+    tall = _hip.tile_table_build(ib["cumsums_N"], M, K, _hip.TILE_ROWS)
+    assert all(bool((t == 7.0).all()) for t in run(tall))  # tiles too tall: nothing is written
+    gz, hsT, gs = run(ib["recompute_table"])
+    gz = gz.permute(1, 0, 2).reshape(msum, 2 * H)
+    hs = hsT.permute(0, 2, 1).reshape(-1, H)
+    assert torch.isfinite(gs).all()
+    for e in range(N):
+        r0, r1 = c[e], c[e + 1]
+        lo = r0 + max(0, row_lo - r0) // 32 * 32  # groups of 32 rows from the expert's first
+        if row_lo >= r1:  # its rows are all below
+            assert bool((gz[r0:r1] == 7.0).all()) and bool((gs[:, r0:r1] == 7.0).all())
+            continue
+        assert bool((gz[r0:lo] == 7.0).all()) and bool((gs[:, r0:lo] == 7.0).all())
+        tok, x64, w64 = idx[lo:r1].long(), xb[idx[lo:r1].long()].double().cpu(), W1b[e].double().cpu()
+        ab, size = x64 @ w64, x64.abs() @ w64.abs() * (D * 2.0**-24)
+        (va, vb), (ea, eb) = ab.split(H, 1), size.split(H, 1)
+        sv, u64 = sd[e, tok].double().cpu()[:, None], u[lo:r1].double().cpu()
+        sg = torch.sigmoid(vb)
+        silu, d = vb * sg, sg * (1 + vb * (1 - sg))
+        su, near = (sv * u64).abs(), 2.0**-19 * (1 + va.abs()) * (1 + vb.abs())
+
+        def check(got, want, err, what):
+            bound = want.abs() * 2.0**-8 + 1.01 * err
+            assert bool(((got.double().cpu() - want).abs() <= bound).all()), f"{what} of expert {e}"
+
+        eh = 1.1 * va.abs() * eb + silu.abs() * ea + near  # of a silu(b)
+        check(gz[lo:r1, :H], sv * u64 * silu, su * (1.1 * eb + near), "G_a")
+        check(gz[lo:r1, H:], sv * u64 * va * d, su * (1.1 * ea + 0.5 * va.abs() * eb + near), "G_b")
+        p0 = (r0 + 31) // 32 * 32 + 32 * e + lo - r0
+        n = r1 - lo
+        check(hs[p0:p0 + n], sv * va * silu, sv.abs() * eh, "hs")
+        assert bool((hs[p0 + n:p0 + (n + 31) // 32 * 32] == 0).all())
+        for b in range(gs.shape[0]):
+            cols = slice(128 * b, min(H, 128 * b + 128))
+            t = u64[:, cols] * (va * silu)[:, cols]
+            err = (u64.abs() * eh)[:, cols].sum(1) + 128 * 2.0**-24 * t.abs().sum(1)
+            assert bool(((gs[b, lo:r1].double().cpu() - t.sum(1)).abs() <= err).all()), f"dL/ds {b} of expert {e}"
+
+
 @pytest.mark.parametrize("sp", [0, 40])
 def test_both_row_tile_geometries_give_the_same_layer(sp):
     """Experts of 1..700 rows on 256-row and on 320-row tiles (and on the library's own choice): the
