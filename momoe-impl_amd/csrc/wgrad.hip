@@ -614,9 +614,9 @@ namespace span {
 constexpr int kPlanLds = kSpanLds - kSpanWaves * kStagingElems * sizeof(bf16);
 static_assert((size_t)(kMaxWgradExperts + 1) * 20 + 512 <= kPlanLds, "prefix sums overlay the rings");
 
-// Common to the operands: set_tile() says where a tile's stages come from; request(span, t) starts the loads
-// that the deposits of a span's stage t need, a stage ahead; begin(span, t) precedes the deposits of
-// stage t, deposit<j>(slot) requests one.  Rows past the end are the
+// Common to the operands: set_tile() says where a tile's stages come from; request() starts the loads
+// that the deposits of a stage need, a stage ahead, those of the span given to restart() in turn; begin(span, t)
+// precedes the deposits of stage t, prepare<j>() uses up what was loaded for one, deposit<j>(slot) requests it.  Rows past the end are the
 // expert's last one: the M side's zeros meet finite numbers if the expert's are finite.  The stages of a
 // span without rows take row and token 0: the list may hold nothing yet.
 
@@ -634,24 +634,32 @@ struct RowsOperand {
   const int32_t* gather;
   uint32_t colb[4];  // byte offset of this lane's columns, by the swizzle of its k-row
   ids_t next;        // of the stage whose deposits come next: tokens, or rows from the span's first one
+  uint32_t off[DEP]; // byte offsets of its prepared deposits
+  int at, origin, last, some;  // row of this wave's next id, the span's first and last, all ones if it has any
   uint32_t upper;    // all ones in the lanes that fetch the second k-row of a deposit
   static __device__ __forceinline__ int wave_offset() { return wave_id() * (ROWS * 512); }
   __device__ __forceinline__ RowsOperand(const bf16* mat_, int64_t ld, const int32_t* gather_)
       : mat(mat_), ldb((uint32_t)(ld * 2)), gather(gather_), upper(lane_id() >= 32 ? 0xFFFFFFFFu : 0u) {}
-  __device__ __forceinline__ void request(const Span& sp, int t) {
-    const int first = sp.rb + t * kSpan + wave_id() * ROWS, last = max(sp.re - 1, 0);
+  // the requests that follow are for the span's stages in turn
+  __device__ __forceinline__ void restart(const Span& sp) {
+    at = sp.rb + wave_id() * ROWS;
+    origin = sp.rb;
+    last = max(sp.re - 1, 0);
+    some = sp.re > 0 ? -1 : 0;
+  }
+  __device__ __forceinline__ void request() {
     if (gather == nullptr) {  // kernel-uniform
 #pragma unroll
-      for (int i = 0; i < ROWS; ++i) next[i] = min(first + i, last) - sp.rb;
-    } else if (first + ROWS - 1 <= last) {
-      next = *(const ids_t __attribute__((address_space(4)))*)(gather + first);
+      for (int i = 0; i < ROWS; ++i) next[i] = min(at + i, last) - origin;
+    } else if (at + ROWS - 1 <= last) {
+      next = *(const ids_t __attribute__((address_space(4)))*)(gather + at);
     } else {
 #pragma unroll
-      for (int i = 0; i < ROWS; ++i) next[i] = load_uniform(gather + min(first + i, last));
-      const int some = sp.re > 0 ? -1 : 0;
+      for (int i = 0; i < ROWS; ++i) next[i] = load_uniform(gather + min(at + i, last));
 #pragma unroll
       for (int i = 0; i < ROWS; ++i) next[i] &= some;
     }
+    at += kSpan;
   }
   // columns [col0, col0 + 256) of the matrix; columns >= ncols are clamped to column 0
   __device__ __forceinline__ void set_tile(const bf16* mat_, const Span& sp, int col0, int ncols) {
@@ -666,9 +674,14 @@ struct RowsOperand {
   }
   __device__ __forceinline__ void begin(const Span&, int) {}
   template <int j>
-  __device__ __forceinline__ void deposit(uint32_t slot) const {
+  __device__ __forceinline__ void prepare() {
     const uint32_t lo = (uint32_t)next[2 * j] * ldb, hi = (uint32_t)next[2 * j + 1] * ldb;
-    dma16_at<j * 1024>(mat, lo + (upper & (hi - lo)) + colb[(j & 1) + 2 * (j >> 2)], slot);
+    off[j] = lo + (upper & (hi - lo)) + colb[(j & 1) + 2 * (j >> 2)];
+    settle(off[j]);  // (here, between products, and not where it is used)
+  }
+  template <int j>
+  __device__ __forceinline__ void deposit(uint32_t slot) const {
+    dma16_at<j * 1024>(mat, off[j], slot);
   }
   static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) { return L::frag(slot, ln, i, h); }
 };
@@ -686,7 +699,8 @@ struct BlockedRowsOperand {
   int last;  // of the rows of the stage at hand
   static __device__ __forceinline__ int wave_offset() { return wave_id() * 1024; }
   __device__ __forceinline__ BlockedRowsOperand(const bf16* mat_, int64_t ld, const int32_t*) : mat(mat_), nrows(ld) {}
-  __device__ __forceinline__ void request(const Span&, int) {}
+  __device__ __forceinline__ void restart(const Span&) {}
+  __device__ __forceinline__ void request() {}
   // features [col0, col0+256) (col0 a multiple of 256); features >= ncols are clamped to col0
   __device__ __forceinline__ void set_tile(const bf16* mat_, const Span&, int col0, int ncols) {
     mat = mat_ + (int64_t)(col0 >> 5) * nrows * 32;
@@ -698,6 +712,8 @@ struct BlockedRowsOperand {
       colb[q] = (uint32_t)(((int64_t)(cc >> 5) * nrows * 32 + (cc & 31)) * 2);
     }
   }
+  template <int j>
+  __device__ __forceinline__ void prepare() {}
   __device__ __forceinline__ void begin(const Span& sp, int t) {
     const int first = min(sp.rb + t * kSpan, max(sp.re - 1, 0));
     src = mat + (int64_t)first * 32;
@@ -723,7 +739,8 @@ struct TransposedOperand {
   uint32_t off[L::PER_HALF];
   static __device__ __forceinline__ int wave_offset() { return wave_id() * 1024; }
   __device__ __forceinline__ TransposedOperand(const bf16* mat_, int64_t ld, const int32_t*) : mat(mat_), gstride(ld * 32) {}
-  __device__ __forceinline__ void request(const Span&, int) {}
+  __device__ __forceinline__ void restart(const Span&) {}
+  __device__ __forceinline__ void request() {}
   // features [f0, f0+256) of the matrix; features >= nfeat are clamped to the last one
   __device__ __forceinline__ void set_tile(const bf16* mat_, const Span&, int f0, int nfeat) {
     mat = mat_ + (int64_t)f0 * 32;
@@ -734,6 +751,8 @@ struct TransposedOperand {
       off[q] = (uint32_t)min(row, nfeat - 1 - f0) * 64 + (((l & 3) ^ L::swz(row)) * 16);
     }
   }
+  template <int j>
+  __device__ __forceinline__ void prepare() {}
   __device__ __forceinline__ void begin(const Span& sp, int t) {
     const int groups = (sp.re - sp.rb + 31) >> 5, g = max(0, min(2 * t, groups - 1));
     src = mat + (int64_t)((sp.prow >> 5) + (groups > 0 ? g : 0)) * (groups > 0 ? gstride : 0);
@@ -817,28 +836,49 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
   BOp B(p.b, p.ldb, p.gb);
   A.set_tile(p.a, c0.rows, c0.x0, p.X);
   B.set_tile(p.b, c0.rows, c0.y0, p.Y);
+  A.restart(c0.rows);
+  B.restart(c0.rows);
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    A.request(c0.rows, s);
-    B.request(c0.rows, s);
+    A.request();
+    B.request();
     A.begin(c0.rows, s);
     B.begin(c0.rows, s);
-    unrolled<0, BOp::DEP>([&](auto D) { B.template deposit<decltype(D)::value>(bslot(s)); });
-    unrolled<0, AOp::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(aslot(s)); });
+    unrolled<0, BOp::DEP>([&](auto D) {
+      B.template prepare<decltype(D)::value>();
+      B.template deposit<decltype(D)::value>(bslot(s));
+    });
+    unrolled<0, AOp::DEP>([&](auto D) {
+      A.template prepare<decltype(D)::value>();
+      A.template deposit<decltype(D)::value>(aslot(s));
+    });
   }
   wait_vmcnt<AOp::DEP + BOp::DEP>();
   __builtin_amdgcn_s_barrier();
   order_fence();
   int sb = 0, sa = 0;  // slots of the stage at hand
-  int asked = 2;       // stages of c0 whose loads have been started
+  int togo = c0.rows.stages() - 2;  // stages of the span at hand whose loads have not been started
+  bool behind = true;               // the loads for the deposits that come next have not
   while (true) {
     WTile c1 = next_tile();
     if (!c1.valid) c1.rows = c0.rows, c1.x0 = c0.x0, c1.y0 = c0.y0;  // requests past the last item repeat its first stages
     const int rows = c0.rows.re - c0.rows.rb, real = (rows + kSpan - 1) / kSpan, count = c0.rows.stages();
-    if (asked < 3) {  // the stage requested first below: a third one, or the next item's first
-      A.request(count > 2 ? c0.rows : c1.rows, count > 2 ? 2 : 0);
-      B.request(count > 2 ? c0.rows : c1.rows, count > 2 ? 2 : 0);
-    }
+    bool in_next = false;  // the loads have gone on to the next item
+    // the loads for the stage after those started; past the next item's end the next round makes up for it
+    auto request_next = [&] {
+      behind = togo == 0 && in_next;
+      if (behind) return;
+      if (togo == 0) {
+        in_next = true;
+        togo = c1.rows.stages();
+        A.restart(c1.rows);
+        B.restart(c1.rows);
+      }
+      --togo;
+      A.request();
+      B.request();
+    };
+    if (behind) request_next();
     TileAcc acc;
 #pragma unroll
     for (int f = 0; f < FN; ++f)
@@ -856,12 +896,12 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
     };
     Span from = c0.rows;  // the span of the stages being requested,
     int ft = 2, fn = count;  // the one at hand, their number
-    // the loads for the stage after it; past the next item's end the next round makes up for it
-    auto request_next = [&](auto& op) {
-      const bool more = ft + 1 < fn;
-      const Span sp = {more ? from.rb : c1.rows.rb, more ? from.re : c1.rows.re, 0};
-      op.request(sp, more ? ft + 1 : 0);
-    };
+    // Scalar loads share the wait counter of the LDS reads, and the products wait for those at the start of
+    // each half: the loads start behind the wait in the middle of a stage, when both operands have used up the
+    // last ones, and have half a stage.  The scalar unit issues one instruction in four cycles, and between the
+    // halves no product runs: with A's loads at a stage's end and some 60 instructions in that place instead
+    // of 25, the Wl1 gradient of 65536 tokens (D = 4096, H = 2048, N = 64, K = 8) took 15.2 ms instead of 14.3.
+    static_assert(AOp::DEP == BOp::DEP, "prepared together");
     int t = 0, end = count - 2;
     while (true) {
       const int stop = min(end, real - 1);
@@ -871,13 +911,17 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
         sb = next3(sb);
         sa ^= 1;
         const bf16 *nb = bptr(sb), *na = aptr(sa);
+        auto deposit_b = [&](auto D) {
+          B.template prepare<decltype(D)::value>();
+          B.template deposit<decltype(D)::value>(bto);
+          A.template prepare<decltype(D)::value>();
+        };
         B.begin(from, ft);
-        fr.template multiply<0, 1, BOp::DEP>(acc, b, a, [&](auto D) { B.template deposit<decltype(D)::value>(bto); });
+        fr.template multiply<0, 1, BOp::DEP>(acc, b, a, deposit_b);
         turn();
-        request_next(B);  // (behind the wait for the scalar loads before it)
+        request_next();
         A.begin(from, ft);
         fr.template multiply<1, 0, AOp::DEP>(acc, nb, na, [&](auto D) { A.template deposit<decltype(D)::value>(ato); });
-        request_next(A);
         ++ft;
         b = nb;
         a = na;
@@ -910,15 +954,20 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
         }
         order_fence();
       };
+      auto deposit_b = [&](auto D) {
+        B.template prepare<decltype(D)::value>();
+        B.template deposit<decltype(D)::value>(bto);
+        A.template prepare<decltype(D)::value>();
+      };
       B.begin(from, ft);
       if (left > 0) {
         if (left < kHalf) mask(IntC<0>{}, left);
-        fr.template multiply<0, 1, BOp::DEP>(acc, b, a, [&](auto D) { B.template deposit<decltype(D)::value>(bto); });
+        fr.template multiply<0, 1, BOp::DEP>(acc, b, a, deposit_b);
       } else {
-        unrolled<0, BOp::DEP>([&](auto D) { B.template deposit<decltype(D)::value>(bto); });
+        unrolled<0, BOp::DEP>(deposit_b);
       }
       turn();
-      request_next(B);
+      request_next();
       A.begin(from, ft);
       if (left > kHalf) {
         if (left < kSpan) mask(IntC<1>{}, left - kHalf);
@@ -926,10 +975,8 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
       } else {
         unrolled<0, AOp::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(ato); });
       }
-      request_next(A);
       ++ft;
     }
-    asked = fn > 2 ? 3 : 2;
     // staging: where the item's last stage of B was (run_span_tiles)
     bf16* const staging = lds + (sb == 0 ? 2 : sb - 1) * ELEMS;
     if (!CUT || c0.slot < 0) {
