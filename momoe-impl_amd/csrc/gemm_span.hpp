@@ -111,15 +111,15 @@ struct SpanRowsLayout {
   static constexpr int at(int j) { return j * kSpanWaves * 1024; }
   static constexpr int ELEMS = ROWS * kSpan;
   struct Lane {
-    int o[2];
+    int o[2];  // bytes
     __device__ __forceinline__ explicit Lane(int org) {
       const int l = fresh_lane(), r = l & 15, g = l >> 4;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) o[h] = (org + r) * kSpan + ((4 * h + g) ^ (r >> 1)) * 8;
+      for (int h = 0; h < 2; ++h) o[h] = (org + r) * (2 * kSpan) + ((4 * h + g) ^ (r >> 1)) * 16;
     }
   };
   static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
-    return *(const bf16x8*)(slot + ln.o[h] + i * (16 * kSpan));
+    return *(const bf16x8*)((const char*)slot + ln.o[h] + i * (32 * kSpan));
   }
 };
 
@@ -143,7 +143,7 @@ struct SpanGatheredRows : SpanRowsLayout<ROWS> {
 #pragma unroll
     for (int j = 0; j < L::DEP; ++j) off[j] = 0;
   }
-  __device__ __forceinline__ const bf16* source(int k) const { return base + k; }
+  __device__ __forceinline__ const bf16* source(int k) const { return base + (uint32_t)k; }
   template <int j>
   __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
     dma16_at<L::at(j)>(src, off[j], slot);
@@ -166,7 +166,7 @@ struct SpanPitchedRows : SpanRowsLayout<ROWS> {
     last = nrows - 32 - row0;
   }
   __device__ __forceinline__ void idle() { off = 0, last = 0; }
-  __device__ __forceinline__ const bf16* source(int k) const { return base + k; }
+  __device__ __forceinline__ const bf16* source(int k) const { return base + (uint32_t)k; }
   template <int j>
   __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
     dma16_at<L::at(j)>((const char*)src + (uint32_t)min(32 * j, last) * pitch, off, slot);
@@ -210,11 +210,11 @@ struct SpanBlockedRows {
     int o;
     __device__ __forceinline__ explicit Lane(int org) {
       const int l = fresh_lane(), r = l & 15, g = l >> 4;
-      o = (org + r) * kHalf + (g ^ swz(r)) * 8;
+      o = (org + r) * (2 * kHalf) + (g ^ swz(r)) * 16;
     }
   };
   static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
-    return *(const bf16x8*)(slot + ln.o + h * (ROWS * kHalf) + i * (16 * kHalf));
+    return *(const bf16x8*)((const char*)slot + ln.o + h * (ROWS * kHalf * 2) + i * (32 * kHalf));
   }
 };
 
@@ -249,23 +249,23 @@ struct SpanCols {
 #pragma unroll
     for (int q = 0; q < PATTERNS; ++q) off[q] = 0;
   }
-  __device__ __forceinline__ const bf16* source(int k) const { return (const bf16*)((const char*)base + (int64_t)k * pitch); }
+  __device__ __forceinline__ const bf16* source(int k) const { return (const bf16*)((const char*)base + (uint32_t)k * pitch); }
   template <int j>
   __device__ __forceinline__ void deposit(const bf16* src, uint32_t slot) const {
     dma16_at<j * kSpanWaves * 1024>((const char*)src + (uint32_t)(STEP * j) * pitch, off[j % PATTERNS], slot);
   }
   struct Lane {
-    int o;  // first fragment
+    int o;  // first fragment, in bytes
     __device__ __forceinline__ explicit Lane(int org) {
       const int l = fresh_lane(), krow = 8 * (l >> 4) + ((l & 15) >> 2), col = org + 4 * (l & 3);
-      o = krow * COLS + (((col >> 3) ^ swz(krow)) << 3) + (col & 7);
+      o = (krow * COLS + (((col >> 3) ^ swz(krow)) << 3) + (col & 7)) * 2;
     }
   };
   static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
     // (pieces 1 to 3 bits up are permuted, so what is added to a column there is an exclusive or)
     const int far = PAIRED && i >= FN / 2 ? COLS / 2 : 0, n = PAIRED ? i % (FN / 2) : i;
     const int flip = 16 * n + (far < 128 ? far : 0);
-    const bf16* p = slot + (ln.o ^ flip) + (far - (flip - 16 * n)) + h * (kHalf * COLS);
+    const bf16* p = (const bf16*)((const char*)slot + (ln.o ^ (2 * flip))) + (far - (flip - 16 * n)) + h * (kHalf * COLS);
     const bf16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + 4 * COLS);
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   }
@@ -429,12 +429,18 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
   static_assert(Weights::ELEMS >= kSpanWaves * kStagingElems, "a stage of weights holds the epilogue's staging");
   bf16* const lds = dyn_lds();
   const uint32_t addr = lds_address(lds) + wave_id() * 1024;
-  auto wslot = [&](int s) { return addr + (uint32_t)s * (Weights::ELEMS * 2); };
-  auto aslot = [&](int s) { return addr + (uint32_t)(ROWS_AT + s * Rows::ELEMS) * 2; };
-  auto wptr = [&](int s) { return (const bf16*)lds + s * Weights::ELEMS; };
-  auto aptr = [&](int s) { return (const bf16*)lds + ROWS_AT + s * Rows::ELEMS; };
-  auto wnext = [](int s) { return s == AHEAD ? 0 : s + 1; };
-  auto anext = [](int s) { return s == AHEAD - 1 ? 0 : s + 1; };
+  // slots by their byte offsets: of the stage before the one at hand, of that one, of the next one
+  static_assert(AHEAD == 2, "three slots of weights, two of rows");
+  constexpr uint32_t WSLOT = Weights::ELEMS * 2, ASLOT = Rows::ELEMS * 2;
+  struct Ring {
+    uint32_t wlast = 2 * WSLOT, w = 0, wnext = WSLOT, a = ROWS_AT * 2, anext = ROWS_AT * 2 + ASLOT;
+    __device__ __forceinline__ void turn() {
+      const uint32_t old = wlast, olda = a;
+      wlast = w, w = wnext, wnext = old;
+      a = anext, anext = olda;
+    }
+  } ring;
+  auto at = [&](uint32_t offset) { return (const bf16*)((const char*)lds + offset); };
 
   TileCoord c0 = sched.next();
   if (!c0.valid) return;
@@ -449,8 +455,8 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
 #pragma unroll
   for (int s = 0; s < AHEAD; ++s) {
     const bf16 *wsrc = W.source(k), *asrc = A.source(k);
-    unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wslot(s)); });
-    unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, aslot(s)); });
+    unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, addr + s * WSLOT); });
+    unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, addr + ROWS_AT * 2 + s * ASLOT); });
     k = st.after(k);
   }
   TileCoord c1 = sched.next();
@@ -465,7 +471,6 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
   order_fence();
   g2 = g1;
   l1 = l0;
-  int sw = 0, sa = 0;  // slots of the stage at hand
   while (true) {
     if (c2.valid) prog.gather(c2, g2);
     if (c1.valid) prog.late(c1, g1, l1);
@@ -487,8 +492,7 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
         __builtin_amdgcn_s_barrier();
         order_fence();
       };
-      const bf16 *w = wptr(sw), *a = aptr(sa);
-      fr.template read_all<0, 0>(w, a);
+      fr.template read_all<0, 0>(at(ring.w), at(ring.a));
       order_fence();
       int t = 0, end = st.count - AHEAD;
       while (true) {
@@ -496,18 +500,14 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
 #pragma unroll 1
         for (; t < stop; ++t) {
           const bf16 *wsrc = W.source(k), *asrc = A.source(k);
-          const uint32_t wto = wslot(sw == 0 ? AHEAD : sw - 1), ato = aslot(sa);
-          sw = wnext(sw);
-          sa = anext(sa);
-          const bf16 *nw = wptr(sw), *na = aptr(sa);
+          const uint32_t wto = addr + ring.wlast, ato = addr + ring.a;
           fr.template multiply<0, 1, Weights::DEP>(
-              acc, w, a, [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
+              acc, at(ring.w), at(ring.a), [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
           turn();
           fr.template multiply<1, 0, Rows::DEP>(
-              acc, nw, na, [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
+              acc, at(ring.wnext), at(ring.anext), [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
           k = st.after(k);
-          w = nw;
-          a = na;
+          ring.turn();
         }
         if (end == st.count) break;
         k = 0;  // from here on the next tile's stages are requested
@@ -521,20 +521,18 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
       }
       if (st.tail) {
         const bf16 *wsrc = W.source(k), *asrc = A.source(k);
-        const int before = sw == 0 ? AHEAD : sw - 1;
-        unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wslot(before)); });
-        fr.template read_all<0, 1>(w, a);
-        fr.template multiply<0, -1, 0>(acc, w, a, [](auto) {});
+        unrolled<0, Weights::DEP>([&](auto D) { W.template deposit<decltype(D)::value>(wsrc, addr + ring.wlast); });
+        fr.template read_all<0, 1>(at(ring.w), at(ring.a));
+        fr.template multiply<0, -1, 0>(acc, at(ring.w), at(ring.a), [](auto) {});
         turn();
-        unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, aslot(sa)); });
+        unrolled<0, Rows::DEP>([&](auto D) { A.template deposit<decltype(D)::value>(asrc, addr + ring.a); });
         k = st.after(k);
-        sw = wnext(sw);
-        sa = anext(sa);
+        ring.turn();
       }
       // staging: where the finished tile's last weights were; every wave has read them, and the next ones are
       // requested behind the barrier below
       keep_in_place(acc);
-      if constexpr (NA > 0) prog.epilogue(c0, acc, g0, l0, lds + (sw == 0 ? AHEAD : sw - 1) * Weights::ELEMS);
+      if constexpr (NA > 0) prog.epilogue(c0, acc, g0, l0, (bf16*)at(ring.wlast));
     };
     const int na = __builtin_amdgcn_readfirstlane(c0.na);
     if (na == 4) tile(IntC<8>{});
@@ -545,7 +543,7 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
     if constexpr (P::EXCHANGE) {
       wait_lgkm0();
       __builtin_amdgcn_s_barrier();
-      prog.finish(c0, lds + (sw == 0 ? AHEAD : sw - 1) * Weights::ELEMS);
+      prog.finish(c0, (bf16*)at(ring.wlast));
     }
     prog.settle(g2);
     prog.settle(l1);
