@@ -1,4 +1,5 @@
-// Workgroup-level bf16 GEMM building blocks for gfx950 (CDNA4).
+// Workgroup-level bf16 GEMM building blocks for gfx950 (CDNA4): the short loop, for launches of few tiles or
+// few rows per expert.  Large ones take that of gemm_span.hpp (takes_span_tiles there).
 //
 // A workgroup of 8 wavefronts (two per SIMD: a lone wave leaves ~15% of the MFMA
 // issue slots empty) computes a 256 x 256 or, where registers and LDS allow, a 320 x 256 fp32
