@@ -315,6 +315,8 @@ int momoe_dgrad_x(const void* gz_blocked, const void* Wl1_ND2H, const int32_t* t
 #define MOMOE_LAYOUT_KBLOCKED 2
 int64_t momoe_padded_rows(int64_t Msum, int64_t N);
 int64_t momoe_wgrad_workspace_bytes(int64_t N, int64_t X, int64_t Y, int64_t Msum);
+/* Rows of a stage of the loop that such a launch runs in, 32 or 64 (0: no such launch). */
+int momoe_wgrad_stage_rows(int64_t N, int64_t X, int64_t Y, int64_t Msum, int b_layout);
 int momoe_wgrad(const void* A, int64_t lda, int a_layout, const int32_t* a_gather,
                 const void* B, int64_t ldb, int b_layout, const int32_t* b_gather,
                 const int32_t* cumsums_N1, void* GW_NXY,

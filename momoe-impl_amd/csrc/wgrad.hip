@@ -831,12 +831,11 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
   const ClockTrace trace(p.clk);
   WorkItems<CUT, kSpanThreads> items(p);
   // Tiles of experts without rows: stores that nothing waits for, behind the loop.  As two stages of it such a tile
-  // waited for the stores of the tile before it, for the stages' transfers and for its own stores; stored in front of
-  // the loop the zeros held up its first tile (182 -> 167 us where it is 159 now), and between its tiles they
-  // cost the loop registers (65536 tokens, D = 4096, H = 2048, Wl1 gradient: 14.7 -> 15.1 ms).
-  // Before -> now in us: X = Y = 1024, 56 of 64 experts empty, 2048 rows in each other 78 -> 59; X = 2048, Y = 1536,
-  // 28 of 32 empty, 4096 rows 184 -> 159; in a step of 2048 tokens, D = 2048, H = 1408, half of 64 experts empty,
-  // Wl2 and Wl1 gradient 173 -> 145 and 299 -> 266.
+  // waited for the stores of the tile before it, for the stages' transfers and for its own stores.  Before -> now in
+  // us: X = Y = 1024, 56 of 64 experts empty, 3584 rows in each other 114 -> 99; X = 2048, Y = 1536, 28 of 32 empty,
+  // 4096 rows 184 -> 158.  Stored in front of the loop the zeros held up its first tile (the second of these: 167),
+  // and between its tiles they cost the loop registers (65536 tokens, D = 4096, H = 2048, Wl1 gradient: 14.7 ->
+  // 15.1 ms).
   auto no_rows = [](const WTile& t) { return t.rows.re <= t.rows.rb && (!CUT || t.slot < 0); };
   const WorkItems<CUT, kSpanThreads> all_items = items;
   auto next_tile = [&] {
@@ -1086,13 +1085,21 @@ int launch(const WgradArgs& a, bool can_cut, hipStream_t st) {
 
 }  // namespace span
 
-// Which loop: with at least 192 rows per expert on average that of gemm_span.hpp.  Below, an expert is a
-// few stages, one of which may be empty, and the eight waves of the other start and store sooner.
-// Measured, Wl2 and Wl1 gradient in us, 32 rows a stage -> 64: 8192 rows per expert (D = 4096, H = 2048) 8365 ->
-// 6694, 17061 -> 15356; 720 (D = 2176, H = 1152) 303 -> 269, 521 -> 488; 512 (D = 2048, H = 1024) 329 -> 298,
-// 637 -> 619; 256 201 -> 196, 378 -> 371; 187 (D = 512, H = 256) 13.0 -> 13.6, 13.0 -> 14.3; 128 140 -> 141,
-// 261 -> 262; 62 (D = 1024, H = 512) 23 -> 27, 35 -> 41; 32 (D = 128, H = 64) 8.5 -> 10.5 both.
-inline bool takes_span_loop(const WgradArgs& a) { return (int64_t)a.msum >= 192 * (int64_t)a.N; }
+// Which loop: that of gemm_span.hpp from 416 rows per expert on average, and where a workgroup has ten tiles or more from 192,
+// 256 with a k-blocked operand.  Below, an expert is a few stages, the last of which may be half empty, and the
+// eight waves of the other start and store sooner; many tiles hide the start and most of the stores.
+// Measured, rows spread as by a router without preferences, Wl2 and Wl1 gradient in us, 32 rows a stage -> 64.
+// 32 and 16 tiles a workgroup (D = 2048, H = 1024, N = 128; H = 2048, N = 64): 192 rows 215 -> 205, 396 -> 375; 214 ->
+// 199, 361 -> 381; 256 249 -> 237, 454 -> 435; 241 -> 231, 426 -> 431; 512 369 -> 336, 729 -> 658; 357 -> 336, 698 -> 661.
+// 11 and 20 (2176, 1152, 64): 192 131 -> 135, 223 -> 232; 256 154 -> 153, 266 -> 268; 768 339 -> 305, 603 -> 558.
+// 4 and 8 (4096, 1024, 16): 256 68 -> 74, 113 -> 119; 304 73 -> 80, 124 -> 133; 512 105 -> 99, 182 -> 167.
+// 3 and 6 (2048, 768, 32): 256 57 -> 59, 93 -> 94; 400 71 -> 73, 123 -> 124; 448 77 -> 74, 133 -> 131.
+// 2 and 4 (1024, 512, 64): 192 39 -> 42, 60 -> 63; 400 64 -> 69, 90 -> 90; 448 69 -> 67, 100 -> 96; one or less
+// (512, 256, 64): 192 15.6 -> 17.6, 18.9 -> 20.9; 400 28 -> 29, 33 -> 33.
+inline bool takes_span_loop(int64_t msum, int64_t n, int64_t x, int64_t y, bool kblocked) {
+  const bool many_tiles = cdiv64(x, BX) * cdiv64(y, BY) * n >= 10 * (int64_t)persistent_grid();
+  return msum >= (many_tiles ? kblocked ? 256 : 192 : 416) * n;
+}
 
 }  // namespace
 }  // namespace momoe
@@ -1112,6 +1119,11 @@ extern "C" int64_t momoe_wgrad_workspace_bytes(int64_t N, int64_t X, int64_t Y, 
 extern "C" int64_t momoe_padded_rows(int64_t Msum, int64_t N) {
   if (Msum < 0 || N < 0) return -1;
   return ((Msum + 31) & ~(int64_t)31) + 32 * N;
+}
+
+extern "C" int momoe_wgrad_stage_rows(int64_t N, int64_t X, int64_t Y, int64_t Msum, int b_layout) {
+  if (N <= 0 || X <= 0 || Y <= 0 || Msum <= 0) return 0;
+  return takes_span_loop(Msum, N, X, Y, b_layout == MOMOE_LAYOUT_KBLOCKED) ? kSpan : kBK;
 }
 
 extern "C" int momoe_wgrad(const void* A, int64_t lda, int a_layout, const int32_t* a_gather,
@@ -1167,7 +1179,7 @@ extern "C" int momoe_wgrad(const void* A, int64_t lda, int a_layout, const int32
   // an expert holds at most M rows: if that is short of the cutting length, nothing is cut
   const bool can_cut = kc != 0x7fffffff && cdiv64(std::min(M, Msum), kBK) >= 2 * (int64_t)kc;
   hipStream_t st = (hipStream_t)stream;
-  if (takes_span_loop(a)) {
+  if (takes_span_loop(Msum, N, X, Y, bk)) {
     if (at) return span::launch<span::TransposedOperand, span::RowsOperand>(a, can_cut, st);
     if (bt) return span::launch<span::RowsOperand, span::TransposedOperand>(a, can_cut, st);
     if (bk) return span::launch<span::RowsOperand, span::BlockedRowsOperand>(a, can_cut, st);

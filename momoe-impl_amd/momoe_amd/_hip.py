@@ -63,6 +63,7 @@ _SIGNATURES = {
     "momoe_gs_scatter": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _p]),
     "momoe_dgrad_x": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "momoe_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
+    "momoe_wgrad_stage_rows": (_int, [_i64, _i64, _i64, _i64, _int]),
     "momoe_padded_rows": (_i64, [_i64, _i64]),
     "momoe_wgrad": (_int, [_p, _i64, _int, _p, _p, _i64, _int, _p, _p, _p, _i64, _i64, _i64, _i64,
                            _i64, _p, _i64, _p]),
