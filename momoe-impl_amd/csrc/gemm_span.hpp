@@ -576,10 +576,11 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
 inline bool takes_span_tiles(int64_t msum, int64_t n, int64_t cols, int64_t contraction) {
   if (contraction < WideSpan::AHEAD * kSpan || takes_narrow_tiles(msum, n, cols) || few_rows_per_expert(msum, n)) return false;
   const double mean = (double)msum / n, spread = std::sqrt(mean), blocks = (double)cdiv64(cols, WideSpan::COLS);
-  // row tiles per expert of at most `height` rows (normal spread, its tail by the logistic curve)
+  // row tiles per expert of at most `height` rows (normal spread, its tail by the logistic curve, which in
+  // double precision is 1 from 24 spreads below the mean on)
   auto row_tiles = [&](double height) {
-    double t = 1.0;
-    for (int k = 1; k * height < mean + 6 * spread; ++k) t += 1.0 / (1.0 + std::exp(1.7 * (k * height - mean) / spread));
+    double t = 1.0 + std::max(0.0, std::floor((mean - 24 * spread) / height));
+    for (double k = t; k * height < mean + 6 * spread; ++k) t += 1.0 / (1.0 + std::exp(1.7 * (k * height - mean) / spread));
     return t;
   };
   auto tile_cost = [&](double tiles) { return 0.4 + 0.6 * mean / (tiles * StdTiles::MAX_ROWS); };

@@ -1,4 +1,7 @@
 """CPU: which loop a launch takes, by its sizes (256 workgroups, the library's count without a GPU)."""
+import math
+import time
+
 import pytest
 
 from momoe_amd import _hip
@@ -31,3 +34,33 @@ def test_rows_of_a_weight_gradient_stage(rows_per_expert, N, X, Y, b_layout, sta
 
 def test_no_weight_gradient_launch():
     assert _hip._lib.momoe_wgrad_stage_rows(8, 64, 64, 0, ROWS) == 0
+
+
+def _row_tiles(mean, height, first=0):
+    """Row tiles per expert as the choice of loop for the row-tile GEMMs estimates them, the first terms taken as 1."""
+    spread, t, k = math.sqrt(mean), 1.0 + first, 1 + first
+    while k * height < mean + 6 * spread:
+        t += 1 / (1 + math.exp(1.7 * (k * height - mean) / spread))
+        k += 1
+    return t
+
+
+@pytest.mark.parametrize("mean", [1, 90, 300, 515, 4096, 8000, 131072])
+def test_terms_left_out_of_the_sum_of_row_tiles_are_ones(mean):
+    for height in (256, 320):
+        first, spread = math.floor((mean - 24 * math.sqrt(mean)) / height), math.sqrt(mean)
+        assert _row_tiles(mean, height) == _row_tiles(mean, height, max(0, first))
+        if first > 0:
+            assert 1 / (1 + math.exp(1.7 * (first * height - mean) / spread)) == 1
+
+
+def test_choice_for_many_rows_per_expert_is_quick():
+    """Host time of a choice does not grow with the rows per expert (120 ms for these with every term added)."""
+    lib = _hip._lib
+    lib.momoe_gemm_tile_rows(1 << 10, 1, 4096, 4096)
+    best = 1.0
+    for _ in range(5):
+        t0 = time.perf_counter()
+        lib.momoe_gemm_tile_rows(1 << 30, 1, 4096, 4096)
+        best = min(best, time.perf_counter() - t0)
+    assert best < 1e-3
