@@ -563,16 +563,24 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
 // Whether a launch over `cols` output columns takes these tiles rather than those of gemm_tile.hpp.  Not
 // where most CUs would go without one (takes_narrow_tiles), nor with few rows per expert: a tile of few
 // rows is a stream of weights, and then what is on the way counts, two to three stages of 32 k-values at
-// any time in that ring, one of 64 here.  Otherwise by the rounds of tiles the CUs take, a tile costing 0.4
+// any time in that ring, one of 64 here; nor in one round of one tile per expert with at most 512 k-values, where
+// the start and the last stores are much of the time.  Otherwise by the rounds of tiles the CUs take, a tile costing 0.4
 // for its weights and 0.6 for 256 rows, and of it all 0.8 here plus an epilogue that nothing hides,
 // 0.07 of a contraction over 1024: an expert of 260 rows is two tiles here and one of 320 rows there.
-// The routing is not known; the rows per expert are taken as those of one with the same chance for
-// every expert.
 // (The k-loop needs two stages.)
 // Measured, there -> here in us (x.Wl1, h.Wl2, dL/dh, dL/dx): 8192 tokens, D = 2048, H = 1024, N = 128, K = 8
 // 538 -> 498, 302 -> 286, 293 -> 252, 562 -> 493; 7680, D = 2176, H = 1152, N = 64, K = 6 438 -> 388, 257 -> 234,
 // 260 -> 209, 459 -> 388; 4000, D = 1024, H = 512, N = 64, K = 4 (64 tiles of 320 rows, 81 of 256) 39 -> 47,
-// 27 -> 31, 36 -> 27, 39 -> 43: here only dL/dh.
+// 27 -> 31, 36 -> 27, 39 -> 43: here only dL/dh.  D = 512, H = 256, N = 96, 130
+// rows per expert, x.Wl1 18.2 -> 20.8, dL/dx 18.2 -> 19.6: there.
+// The routing is not known; the rows per expert are taken as those of one with the same chance for
+// every expert, whose row counts spread by the root of their mean.  The choice is the wrong one for some loads without
+// any spread: of 257 to 320 rows each, one tile of 320 would do where two are taken.  A choice that allowed for
+// those would cost the others several times as much.  There -> here, 300 rows per expert, all the same | spread:
+// x.Wl1 with D = 2048, H = 1024, N = 64 163 -> 178 | 218 -> 178, N = 128 327 -> 352 | 374 -> 355; h.Wl2 with N = 64 95 ->
+// 101 | 116 -> 100; dL/dx 180 -> 186 | 221 -> 184.  A forward of such loads takes up to 9 % more than there, a step with its backward
+// 0 to 6 % less.  (Tiles of six and four fragment rows instead of five and five, a wave row being two, changed
+// nothing: 0.2 to 0.4 % more over 5760 launches.)
 inline bool takes_span_tiles(int64_t msum, int64_t n, int64_t cols, int64_t contraction) {
   if (contraction < WideSpan::AHEAD * kSpan || takes_narrow_tiles(msum, n, cols) || few_rows_per_expert(msum, n)) return false;
   const double mean = (double)msum / n, spread = std::sqrt(mean), blocks = (double)cdiv64(cols, WideSpan::COLS);
@@ -585,6 +593,7 @@ inline bool takes_span_tiles(int64_t msum, int64_t n, int64_t cols, int64_t cont
   };
   auto tile_cost = [&](double tiles) { return 0.4 + 0.6 * mean / (tiles * StdTiles::MAX_ROWS); };
   const double tall = std::min(row_tiles(TallTiles::MAX_ROWS), row_tiles(StdTiles::MAX_ROWS)), ours = row_tiles(WideSpan::MAX_ROWS);
+  if (contraction <= 512 && ours < 1.05 && n * blocks <= persistent_grid()) return false;
   const double rounds = n * ours * blocks / persistent_grid(), rest = rounds - std::floor(rounds);
   const double pieces = rest > 0.5 ? 1.0 : rest > 0.25 ? 0.65 : rest > 0.125 ? 0.45 : 0.3;  // SpanSched
   return (0.8 + 73.0 / contraction) * tile_cost(ours) * (std::floor(rounds) + pieces) <=

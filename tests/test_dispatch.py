@@ -64,3 +64,18 @@ def test_choice_for_many_rows_per_expert_is_quick():
         lib.momoe_gemm_tile_rows(1 << 30, 1, 4096, 4096)
         best = min(best, time.perf_counter() - t0)
     assert best < 1e-3
+
+
+# Times in us of the loops with 32 and 64 k-values a stage, rows spread as by a router without preferences
+@pytest.mark.parametrize("rows_per_expert,N,cols,contraction,span", [
+    (130, 96, 512, 512, False),      # x.Wl1, 18.2, 20.8: one round, a short contraction
+    (176, 96, 512, 512, False),      # dL/dx, 20.4, 21.6
+    (300, 96, 512, 512, False),      # x.Wl1, 27, 31
+    (224, 48, 3072, 512, True),      # h.Wl2, 66, 57: three rounds
+    (512, 128, 2048, 2048, True),
+    (62, 128, 2048, 2048, False),    # few rows per expert
+    (300, 64, 2048, 2048, True),     # x.Wl1, 218, 178 (163, 178 with 300 rows in every expert)
+])
+def test_loop_of_the_row_tile_gemms(rows_per_expert, N, cols, contraction, span):
+    rows = _hip._lib.momoe_gemm_tile_rows(rows_per_expert * N, N, cols, contraction)
+    assert rows == (_hip.RECOMPUTE_TILE_ROWS if span else 0)
