@@ -237,6 +237,9 @@ int momoe_lin1_swiglu_bwd(const void* x_MD, const void* Wl1_ND2H, const int32_t*
                           float* gs_part,
                           int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum, void* stream);
 
+/* k-values of a stage of the loop that such a launch runs in, 32 or 64 (0: no such launch). */
+int momoe_recompute_stage_k(int64_t Msum, int64_t N, int64_t D, int64_t H);
+
 /* momoe_lin1_swiglu_bwd with `nparts` partial row sums per row, gs_part fp32 [nparts][Msum]:
  * ceil(H/MOMOE_GS_BLOCK), as above, or momoe_gs_parts(H, N, Msum) (anything else:
  * MOMOE_ERR_BAD_ARG).  The latter is twice as many where the launch has few output tiles: it then

@@ -289,12 +289,13 @@ __global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_bwd_kernel(Lin1Ar
 // Measured, there -> here in us: 65536 tokens, D = 4096, H = 2048, N = 64, K = 8 17297 -> 14150; 8192, 2048, 1024, 128, 8
 // 664 -> 561; 7680, 2176, 1152, 64, 6 509 -> 437; 4000, 1024, 512, 64, 4 69 -> 57; 2048, 2048, 1024, 128, 8 (128
 // rows per expert) 275 -> 267; in one round of tiles 3000, 3072, 1024, 32, 2 112 -> 102; 16000, 1024, 256, 128, 1
-// (125 rows per expert, one round) 34 -> 38; 12000, 256, 128, 32, 4 21.6 -> 23.7.
+// (125 rows per expert, one round) 34 -> 38; 12000, 256, 128, 32, 4 21.6 -> 23.7.  At the line, D = 1024, H = 512: N = 64,
+// 176 and 200 rows per expert 43 -> 49 and 44 -> 48; N = 32, 320, 400 and 512 rows 35 -> 34, 39 -> 40 and 71 -> 54.
 inline bool takes_span_recompute(int64_t msum, int64_t n, int64_t h, int64_t d) {
   if (d < WideSpan::AHEAD * kSpan || few_rows_per_expert(msum, n)) return false;
   const double mean = (double)msum / n, tiles = std::ceil(mean / WideSpan::MAX_ROWS);
   const double rounds = std::max(1.0, n * tiles * (double)cdiv64(h, Lin1BwdSpan::BNH) / persistent_grid());
-  return rounds * d * (0.4 + 0.6 * mean / (tiles * WideSpan::MAX_ROWS)) >= 780;
+  return rounds * d * (0.4 + 0.6 * mean / (tiles * WideSpan::MAX_ROWS)) >= 900;
 }
 
 // Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave owns 32 `a`
@@ -878,6 +879,11 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
 extern "C" int momoe_gemm_tile_rows(int64_t Msum, int64_t N, int64_t cols, int64_t contraction) {
   if (Msum <= 0 || N <= 0 || cols <= 0 || contraction <= 0) return 0;
   return takes_span_tiles(Msum, N, cols, contraction) ? MOMOE_RECOMPUTE_TILE_ROWS : 0;
+}
+
+extern "C" int momoe_recompute_stage_k(int64_t Msum, int64_t N, int64_t D, int64_t H) {
+  if (Msum <= 0 || N <= 0 || D <= 0 || H <= 0) return 0;
+  return takes_span_recompute(Msum, N, H, D) ? kSpan : kBK;
 }
 
 extern "C" int64_t momoe_gs_parts(int64_t H, int64_t N, int64_t Msum) {

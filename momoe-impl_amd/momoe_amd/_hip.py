@@ -41,6 +41,7 @@ _SIGNATURES = {
     "momoe_hbm_stream_probe": (_i64, [_p, _i64, _i64, _i64, _p]),
     "momoe_tile_table_ints": (_i64, [_i64, _i64, _i64, _int]),
     "momoe_gemm_tile_rows": (_int, [_i64, _i64, _i64, _i64]),
+    "momoe_recompute_stage_k": (_int, [_i64, _i64, _i64, _i64]),
     "momoe_index_workspace_bytes": (_i64, [_i64, _i64]),
     "momoe_index_build": (_int, [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _int,
                                  _p, _p, _i64, _p, _p]),

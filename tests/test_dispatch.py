@@ -79,3 +79,20 @@ def test_choice_for_many_rows_per_expert_is_quick():
 def test_loop_of_the_row_tile_gemms(rows_per_expert, N, cols, contraction, span):
     rows = _hip._lib.momoe_gemm_tile_rows(rows_per_expert * N, N, cols, contraction)
     assert rows == (_hip.RECOMPUTE_TILE_ROWS if span else 0)
+
+
+@pytest.mark.parametrize("rows_per_expert,N,D,H,stage", [
+    (176, 64, 1024, 512, 32),   # 43, 49
+    (200, 64, 1024, 512, 32),   # 44, 48
+    (130, 64, 1024, 512, 32),   # 35, 40
+    (512, 32, 1024, 512, 64),   # 71, 54
+    (152, 32, 2048, 768, 64),   # 65, 58
+    (512, 128, 2048, 1024, 64),
+    (62, 128, 2048, 768, 32),
+])
+def test_loop_of_the_recomputing_gemm(rows_per_expert, N, D, H, stage):
+    assert _hip._lib.momoe_recompute_stage_k(rows_per_expert * N, N, D, H) == stage
+
+
+def test_no_recomputing_launch():
+    assert _hip._lib.momoe_recompute_stage_k(0, 8, 64, 64) == 0
