@@ -105,18 +105,19 @@ def test_wide_and_narrow_tiles(M, D, H, N, K, sp):
             assert torch.equal(other[k], dev[k]), (rows, k)
 
 
-@pytest.mark.parametrize("M,D,H,N,K,Ks,skew,sp", [
-    (8000, 352, 544, 8, 2, 0, None, 0),      # a full round of x.Wl1 and 6 to 9 tiles per XCD in 2 or 4 pieces each;
+@pytest.mark.parametrize("M,D,H,N,K,Ks,skew,sp,span", [
+    (8000, 352, 544, 8, 2, 0, None, 0, (1, 1, 1, 1)),  # a full round of x.Wl1 and 6 to 9 tiles per XCD in 2 or 4 pieces each;
                                              # contractions of 5.5, 8.5 and 17 stages, columns past a tile
-    (3000, 480, 608, 30, 4, 0, None, 60),    # 2 to 6 tiles per XCD in 4 or 8 pieces
-    (4100, 544, 352, 10, 4, 1, 1.0, 100),    # skew: tiles of 1 to 8 fragment rows
-    (2900, 352, 544, 20, 6, 2, 0.3, 30),
+    (3000, 480, 608, 30, 4, 0, None, 60, (1, 0, 1, 0)),  # 2 to 6 tiles per XCD in 4 or 8 pieces
+    (4100, 544, 352, 10, 4, 1, 1.0, 100, (1, 1, 1, 1)),  # skew: tiles of 1 to 8 fragment rows
+    (2900, 352, 544, 20, 6, 2, 0.3, 30, (1, 1, 1, 1)),
 ])
-def test_tiles_of_64_k_values(M, D, H, N, K, Ks, skew, sp):
+def test_tiles_of_64_k_values(M, D, H, N, K, Ks, skew, sp, span):
+    """span: which of x.Wl1, h.Wl2, dL/dh and dL/dx run in the loop of 64 k-values a stage."""
     from momoe_amd import _hip, experts
     x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, Ks=Ks, seed=6, skew=skew)
     gemms = ((2 * H, D), (D, H), (H, D), (D, 2 * H))
-    assert any(_hip._lib.momoe_gemm_tile_rows(M * K, N, *g) == _hip.RECOMPUTE_TILE_ROWS for g in gemms)
+    assert tuple(_hip._lib.momoe_gemm_tile_rows(M * K, N, *g) // _hip.RECOMPUTE_TILE_ROWS for g in gemms) == span
     dev = run_device_layer(x, W1, W2, mask, s, dy, K, sp)
     _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
     # halved tiles of 320 rows, tiles of three fragment rows: the same sums
@@ -298,14 +299,27 @@ def test_weight_gradient_from_a_transposed_operand(sizes, M):
         _hip.wgrad(grouped(A), None, grouped(B), None, cumsums, GW, M, msum, a_transposed=True, b_transposed=True)
 
 
-@pytest.mark.parametrize("sizes,X,Y", [
-    ([0, 1, 33, 64, 65, 130, 1100, 257], 264, 328),     # 206 rows per expert on average, edges in X and Y
-    ([0, 1, 33, 64, 65, 130, 3200, 257], 264, 328),     # the same in the loop of 64 rows a stage
-    ([2000, 0, 31, 1500], 512, 256),                     # whole tiles; two experts that are cut by rows
-    ([129, 1, 0, 300, 128, 127, 95, 5], 520, 72),        # 98 rows per expert: the short loop
+def _pieces(lib, sizes, X, Y, M):
+    """Pieces that momoe_wgrad cuts the experts' rows into, given all the workspace it can use: at least kc
+    stages of 32 rows each, so that the partial tiles fit, and none where no expert can hold two such pieces."""
+    N, msum, tiles = len(sizes), sum(sizes), -(-X // 256) * -(-Y // 256)
+    room = min(lib.momoe_wgrad_workspace_bytes(N, X, Y, msum) // 262144, 8 * 256)
+    kc = max(64, -(-tiles * (msum // 32 + N) // room)) if room else 1 << 30
+    if -(-min(M, msum) // 32) < 2 * kc:
+        return [1] * N
+    return [max(1, -(-n // 32) // kc) for n in sizes]
+
+
+@pytest.mark.parametrize("sizes,X,Y,stage,pieces", [
+    ([0, 1, 33, 64, 65, 130, 1100, 257], 264, 328, 32, 1),  # 206 rows per expert on average, edges in X and Y
+    ([0, 1, 33, 64, 65, 130, 3200, 257], 264, 328, 64, 1),  # the same in the loop of 64 rows a stage
+    ([2000, 0, 31, 1500], 512, 256, 64, 1),                  # whole tiles
+    ([129, 1, 0, 300, 128, 127, 95, 5], 520, 72, 32, 1),     # 98 rows per expert: the short loop
+    ([9031, 31, 0, 6000], 264, 328, 64, 4),                  # cut by rows, into pieces of 71 groups of 32
+    ([31, 9031, 0, 6] + [2] * 40, 264, 328, 32, 4),          # cut in the short loop
 ])
 @pytest.mark.parametrize("form", ["gather_a", "gather_b", "a_transposed", "b_transposed", "b_kblocked"])
-def test_weight_gradient_loops_at_the_edges(sizes, X, Y, form):
+def test_weight_gradient_loops_at_the_edges(sizes, X, Y, stage, pieces, form):
     # Bound: products of bf16 pairs are exact in fp32, so n of them sum to within n 2^-24 of their
     # absolute sum, and the result is rounded to bf16 once (2^-8 relative).
     from momoe_amd import _hip
@@ -314,6 +328,9 @@ def test_weight_gradient_loops_at_the_edges(sizes, X, Y, form):
         Y = Y // 32 * 32
     N, msum, M = len(sizes), sum(sizes), 1500
     M = max(M, max(sizes))
+    layout = {"a_transposed": 1, "b_transposed": 1, "b_kblocked": 2}.get(form, 0)
+    assert _hip._lib.momoe_wgrad_stage_rows(N, X, Y, msum, layout) == stage
+    assert max(_pieces(_hip._lib, sizes, X, Y, M)) == pieces
     c = [0] + list(torch.tensor(sizes).cumsum(0).tolist())
     cumsums = torch.tensor(c, dtype=torch.int32, device=dev)
     g = torch.Generator(device=dev).manual_seed(21)
@@ -350,6 +367,51 @@ def test_weight_gradient_loops_at_the_edges(sizes, X, Y, form):
             want, size = pa.T @ pb, pa.abs().T @ pb.abs()
             bound = want.abs() * 2.0**-8 + size * (sizes[e] * 2.0**-24 * (1 + 2.0**-8))
             assert torch.all((GW[e].double().cpu() - want).abs() <= bound), f"expert {e} ws={ws}"
+
+
+@pytest.mark.parametrize("sizes,X,Y,pieces", [
+    ([3000, 2600, 64, 0, 3100], 2048, 2304, 1),   # 72 tiles each, 360 items
+    ([9000, 2600, 64, 0, 3100], 2048, 2304, 4),   # one cut by rows
+    ([70, 4000, 4000, 4000], 2304, 2048, 1),      # the first XCD's run starts with short items
+])
+@pytest.mark.parametrize("form", ["a_transposed", "b_kblocked"])
+def test_weight_gradients_in_whole_rounds(sizes, X, Y, pieces, form):
+    """Few experts with thousands of rows and more tiles than workgroups: the XCDs take whole rounds.  Every tile of
+    every expert is written, bounds as above.  (The conditions of WorkItems::whole_rounds, in its units of cost:
+    32 rows, and 4 for an item's stores.)"""
+    from momoe_amd import _hip
+    dev, N, msum, M = "cuda:0", len(sizes), sum(sizes), max(sizes)
+    tiles = -(-X // 256) * -(-Y // 256)
+    assert _hip._lib.momoe_wgrad_stage_rows(N, X, Y, msum, 2) == 64
+    assert max(_pieces(_hip._lib, sizes, X, Y, M)) == pieces
+    items = lambda cut: [(tiles * p, -(-(-(-n // 32)) // p) + 4) for n, p in zip(sizes, cut)]
+    for cut in ([1] * N, _pieces(_hip._lib, sizes, X, Y, M)):
+        share = sum(n * cost for n, cost in items(cut)) // 256
+        assert sum(n for n, _ in items(cut)) > 256 and share >= 8 * N and 8 * max(cost for _, cost in items(cut)) > share
+    c = [0] + list(torch.tensor(sizes).cumsum(0).tolist())
+    cumsums = torch.tensor(c, dtype=torch.int32, device=dev)
+    g = torch.Generator(device=dev).manual_seed(24)
+    A = torch.randn(M if form == "b_kblocked" else msum, X, generator=g, device=dev).to(torch.bfloat16)
+    B = torch.randn(msum if form == "b_kblocked" else M, Y, generator=g, device=dev).to(torch.bfloat16)
+    ids = torch.randint(0, M, (msum,), generator=g, device=dev, dtype=torch.int32)
+    if form == "b_kblocked":
+        blocked = B.reshape(msum, Y // 32, 32).permute(1, 0, 2).contiguous()
+        args, kw, rows_a, rows_b = (A, ids, blocked, None), dict(b_kblocked=True), A[ids.long()], B
+    else:
+        T = torch.zeros(_hip.padded_rows(msum, N), X, device=dev, dtype=torch.bfloat16)
+        for e in range(N):
+            p0 = (c[e] + 31) // 32 * 32 + 32 * e
+            T[p0:p0 + sizes[e]] = A[c[e]:c[e + 1]]
+        grouped = T.reshape(-1, 32, X).permute(0, 2, 1).contiguous()
+        args, kw, rows_a, rows_b = (grouped, None, B, ids), dict(a_transposed=True), A, B[ids.long()]
+    for ws in (None, 0):
+        GW = torch.full((N, X, Y), float("nan"), device=dev, dtype=torch.bfloat16)
+        _hip.wgrad(*args, cumsums, GW, M, msum, workspace_bytes=ws, **kw)
+        for e in range(N):
+            pa, pb = (t[c[e]:c[e + 1]].double() for t in (rows_a, rows_b))
+            want, size = pa.T.contiguous() @ pb, pa.abs().T.contiguous() @ pb.abs()
+            bound = want.abs() * 2.0**-8 + size * (sizes[e] * 2.0**-24 * (1 + 2.0**-8))
+            assert torch.all((GW[e].double() - want).abs() <= bound), f"expert {e} ws={ws}"
 
 
 def _microseconds(launch, launches=20, rounds=5):
@@ -743,6 +805,7 @@ def test_recomputing_gemm_in_the_span_loop(M, D, H, N, K, Ks, skew, row_lo):
     dev = "cuda:0"
     x, W1, _, mask, s, _ = make_layer_inputs(M, D, H, N, K, Ks=Ks, seed=8, skew=skew)
     msum = M * K
+    assert _hip._lib.momoe_recompute_stage_k(msum, N, D, H) == 64
     ib = _hip.index_build(mask.to(dev), K, recompute_table=True)
     idx, c = ib["idx_Msum"], [0] + mask.sum(1).cumsum(0).tolist()
     xb, W1b, sd = x.to(dev).to(torch.bfloat16), W1.to(dev).to(torch.bfloat16), s.to(dev)
