@@ -61,12 +61,13 @@ struct WTile {
 };
 
 constexpr int kBandTiles = 4;
-// Estimated time of an item in units of 32 rows of its main loop; every item has its stores, and in the loop of
-// gemm_span.hpp two stages of 64 at least if it has rows
-constexpr int kStoreCost = 4;
+// Estimated time of an item in units of 32 rows of its main loop; every item has its stores.  In the loop of
+// gemm_span.hpp it has two stages of 64 at least, and items without rows are no part of it (they cost nothing here)
 template <int THREADS>
 __device__ __forceinline__ int item_cost(int ks) {
-  return (THREADS == kSpanThreads && ks > 0 ? max(4, ks + (ks & 1)) : ks) + kStoreCost;
+  constexpr int kStoreCost = 4;
+  if (THREADS != kSpanThreads) return ks + kStoreCost;
+  return ks > 0 ? max(4, ks + (ks & 1)) + kStoreCost : 0;
 }
 constexpr int kMinChunk = 64;     // an expert is never cut into pieces of fewer k-stages
 
@@ -270,7 +271,7 @@ struct WorkItems {
   __device__ __forceinline__ void find_empty(const Plan& pl) {
     for (int e0 = 0; e0 < p.N; e0 += 64) {
       const int e = min(e0 + lane_id(), p.N - 1);
-      some_empty = some_empty || __ballot(pl.cost[e + 1] - pl.cost[e] == (int64_t)tpe * kStoreCost) != 0;
+      some_empty = some_empty || __ballot(pl.cost[e + 1] == pl.cost[e]) != 0;
     }
   }
   // Where a workgroup has few items, runs of equal cost leave rounds of the XCD's workgroups nearly empty: a run
@@ -304,6 +305,10 @@ struct WorkItems {
       for (int i = 0; i < min(64, p.N - e0); ++i) {
         int n = __builtin_amdgcn_readlane(my_items, i);
         const int c = __builtin_amdgcn_readlane(my_cost, i);
+        if (c == 0) {  // no rows
+          first += n;
+          continue;
+        }
         const float inv = 1.0f / (float)c;
         if (left > 0) load += max(0, c - open);
         open = c;
@@ -833,14 +838,15 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
   drop_rows_of_an_overflowed_routing(p);
   const ClockTrace trace(p.clk);
   WorkItems<CUT, kSpanThreads> items(p);
-  // Tiles of experts without rows: stores that nothing waits for, behind the loop.  As two stages of it such a tile
-  // waited for the stores of the tile before it, for the stages' transfers and for its own stores.  Before -> now in
-  // us: X = Y = 1024, 56 of 64 experts empty, 3584 rows in each other 114 -> 99; X = 2048, Y = 1536, 28 of 32 empty,
-  // 4096 rows 184 -> 158.  Stored in front of the loop the zeros held up its first tile (the second of these: 167),
-  // and between its tiles they cost the loop registers (65536 tokens, D = 4096, H = 2048, Wl1 gradient: 14.7 ->
-  // 15.1 ms).
+  // Tiles of experts without rows: stores that nothing waits for, behind the loop, dealt out to all workgroups.  As two
+  // stages of the loop such a tile waited for the stores of the tile before it, for the stages' transfers and for its
+  // own stores; left in the runs of the XCDs, behind the loop, they were stored at the rate of the one or two XCDs that
+  // held them.  First -> second -> now in us: X = 2048, Y = 1536, the last 16 of 32 experts empty, 3000 rows in each
+  // other 300 -> 301 -> 247, 28 empty and 4096 rows 181 -> 154 -> 148; X = Y = 1024, 56 of 64 empty, 3584 rows 117 -> 100 ->
+  // 95; X = Y = 512, every second of 96 empty, 1200 rows 64 -> 65 -> 67.
+  // In front of the loop the zeros held up its first tile, and between its tiles they cost the loop registers (65536
+  // tokens, D = 4096, H = 2048, Wl1 gradient: 14.7 -> 15.1 ms).
   auto no_rows = [](const WTile& t) { return t.rows.re <= t.rows.rb && (!CUT || t.slot < 0); };
-  const WorkItems<CUT, kSpanThreads> all_items = items;
   auto next_tile = [&] {
     WTile t;
     do {
@@ -851,10 +857,15 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
   };
 
   auto zero_tiles = [&] {
-    if (!all_items.some_empty) return;
-    WorkItems<CUT, kSpanThreads> again = all_items;
-    for (WTile t = again.next(); t.valid; t = again.next())
-      if (no_rows(t)) place_tile(p, t), zero_gw_tile(p, t);
+    if (!items.some_empty) return;
+    for (int at = blockIdx.x; at < p.N * items.tpe; at += gridDim.x) {
+      WTile t;
+      t.expert = at / items.tpe;
+      t.q = at - t.expert * items.tpe;
+      if (min(load_uniform(p.cumsums + t.expert + 1), p.msum) > min(load_uniform(p.cumsums + t.expert), p.msum)) continue;
+      place_tile(p, t);
+      zero_gw_tile(p, t);
+    }
   };
 
   WTile c0 = next_tile();

@@ -430,8 +430,8 @@ def _microseconds(launch, launches=20, rounds=5):
 
 @pytest.mark.parametrize("N,held,rows,X,Y", [(64, 8, 3584, 1024, 1024), (32, 4, 4096, 2048, 1536)])
 def test_weight_gradient_of_experts_without_rows_costs_their_zeros(N, held, rows, X, Y):
-    """A launch in which most experts are empty takes as long as that of the others and a fill of the rest (99 us
-    against 83 + 18, 158 against 140 + 27; 114 and 184 with two stages of the loop for each empty tile)."""
+    """A launch in which most experts are empty takes as long as that of the others and a fill of the rest (95 us
+    against 83 + 18, 148 against 140 + 27; 117 and 181 with two stages of the loop for each empty tile)."""
     from momoe_amd import _hip
     dev, msum = "cuda:0", held * rows
     assert _hip._lib.momoe_wgrad_stage_rows(N, X, Y, msum, 2) == 64
