@@ -9,19 +9,21 @@ from momoe_amd import _hip
 ROWS, TRANSPOSED, KBLOCKED = 0, 1, 2
 
 
-# Times in us at 32 and 64 rows a stage, on one MI355X, rows spread as by a router without preferences
+# Times in us at 32 and 64 rows a stage, on one MI355X: rows spread as by a router without preferences | skewed
 @pytest.mark.parametrize("rows_per_expert,N,X,Y,b_layout,stage", [
     (192, 64, 512, 1024, ROWS, 32),        # 39, 42
     (256, 64, 512, 1024, ROWS, 32),        # 44, 46
-    (400, 64, 512, 1024, ROWS, 32),        # 64, 69
+    (280, 64, 1024, 1024, KBLOCKED, 32),   # 68, 72 | 77, 73
+    (320, 96, 256, 512, ROWS, 64),         # 26, 28 | 93, 83
     (448, 64, 512, 1024, ROWS, 64),        # 69, 67
     (192, 32, 768, 2048, ROWS, 32),        # 48, 52
-    (304, 16, 4096, 2048, KBLOCKED, 32),   # 124, 133
     (512, 16, 4096, 2048, KBLOCKED, 64),   # 182, 167
     (192, 64, 512, 512, KBLOCKED, 32),     # 18.9, 20.9
     (192, 64, 2048, 4096, KBLOCKED, 32),   # 361, 381: ten tiles a workgroup and more
+    (200, 128, 2048, 2048, KBLOCKED, 64),  # 402, 378 | 396, 403
     (256, 128, 2048, 2048, KBLOCKED, 64),  # 454, 435
     (192, 128, 1024, 2048, ROWS, 64),      # 215, 205
+    (200, 64, 1024, 2048, ROWS, 64),       # 111, 104 | 110, 109: eight tiles a workgroup
     (192, 64, 2048, 2048, ROWS, 64),       # 214, 199
     (128, 128, 2048, 2048, ROWS, 32),
 ])
