@@ -291,11 +291,12 @@ __global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_bwd_kernel(Lin1Ar
 // rows per expert) 275 -> 267; in one round of tiles 3000, 3072, 1024, 32, 2 112 -> 102; 16000, 1024, 256, 128, 1
 // (125 rows per expert, one round) 34 -> 38; 12000, 256, 128, 32, 4 21.6 -> 23.7.  At the line, D = 1024, H = 512: N = 64,
 // 176 and 200 rows per expert 43 -> 49 and 44 -> 48; N = 32, 320, 400 and 512 rows 35 -> 34, 39 -> 40 and 71 -> 54.
+// At most half a round, whose tiles are cut into pieces (SpanSched), pays off sooner: D = 1152, H = 64, N = 8, 269 rows 27 -> 20.
 inline bool takes_span_recompute(int64_t msum, int64_t n, int64_t h, int64_t d) {
   if (d < WideSpan::AHEAD * kSpan || few_rows_per_expert(msum, n)) return false;
   const double mean = (double)msum / n, tiles = std::ceil(mean / WideSpan::MAX_ROWS);
-  const double rounds = std::max(1.0, n * tiles * (double)cdiv64(h, Lin1BwdSpan::BNH) / persistent_grid());
-  return rounds * d * (0.4 + 0.6 * mean / (tiles * WideSpan::MAX_ROWS)) >= 900;
+  const double rounds = n * tiles * (double)cdiv64(h, Lin1BwdSpan::BNH) / persistent_grid();
+  return std::max(1.0, rounds) * d * (0.4 + 0.6 * mean / (tiles * WideSpan::MAX_ROWS)) >= (rounds > 0.5 ? 900 : 780);
 }
 
 // Tile = up to 320 (256) rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave owns 32 `a`

@@ -89,6 +89,7 @@ def test_loop_of_the_row_tile_gemms(rows_per_expert, N, cols, contraction, span)
     (130, 64, 1024, 512, 32),   # 35, 40
     (512, 32, 1024, 512, 64),   # 71, 54
     (152, 32, 2048, 768, 64),   # 65, 58
+    (269, 8, 1152, 64, 64),     # 27, 20: 16 tiles, cut into pieces
     (512, 128, 2048, 1024, 64),
     (62, 128, 2048, 768, 32),
 ])
