@@ -1100,20 +1100,21 @@ int launch(const WgradArgs& a, bool can_cut, hipStream_t st) {
 }  // namespace span
 
 // Which loop.  Where a workgroup has eight tiles or more (ten with a k-blocked operand) that of gemm_span.hpp from 192 rows
-// per expert on average, with a k-blocked operand and fewer than 128 experts from 256; elsewhere from 288.  Below, an
-// expert is a few stages, the last of which may be half empty, and the eight waves of the other start and store
+// per expert on average, with a k-blocked operand and fewer than 128 experts from 256; where there are no more tiles
+// than workgroups, so that the largest expert decides, from 192; elsewhere from 288.  Below, an expert is a few stages, the last of which may be half empty, and the eight waves of the other start and store
 // sooner; many tiles hide the start and most of the stores.  Between 256 and 400 rows the second line is a compromise:
 // loads that are the same for every expert or spread as by a router without preferences lose up to a tenth, skewed ones,
 // whose large experts hold most of the work, gain as much.  32 rows a stage -> 64 in us, spread | falling as rank^-0.5.
 // Wl2 gradient, 8 tiles a workgroup (D = 2048, H = 1024, N = 64) 200 rows 111 -> 104 | 110 -> 109, 300 132 -> 124 | 134 -> 126,
 // 512 193 -> 169 | 195 -> 176; 16 (N = 128) 200 rows 211 -> 206 | 218 -> 220, 512 374 -> 348 | 384 -> 371; 4 (4096, 2048, 8) 200
 // rows 53 -> 59 | 54 -> 58, 280 65 -> 65 | 65 -> 66, 400 81 -> 77 | 83 -> 73; 1 (512, 256, 96) 200 rows 24 -> 26 | 64 -> 59,
-// 320 26 -> 28 | 93 -> 83, 400 28 -> 30 | 103 -> 81.  Wl1 gradient, 32 tiles (2048, 1024, 128) 200 rows 402 -> 378 | 396 ->
+// 320 26 -> 28 | 93 -> 83, 400 28 -> 30 | 103 -> 81; 96 tiles (128, 256, 96) of 236 rows, falling as rank^-1.8, 166 -> 104.  Wl1 gradient, 32 tiles (2048, 1024, 128) 200 rows 402 -> 378 | 396 ->
 // 403, 240 447 -> 413 | 431 -> 420; (2048, 2048, 64) 192 361 -> 381; 20 (2176, 1152, 64) 200 rows 221 -> 220 | 224 -> 237, 512
 // 417 -> 409 | 402 -> 423; 4 (1024, 512, 64) 176 rows 51 -> 60 | 65 -> 63, 280 68 -> 72 | 77 -> 73, 400 79 -> 83 | 102 -> 96.
 inline bool takes_span_loop(int64_t msum, int64_t n, int64_t x, int64_t y, bool kblocked) {
-  const bool many_tiles = cdiv64(x, BX) * cdiv64(y, BY) * n >= (kblocked ? 10 : 8) * (int64_t)persistent_grid();
-  return msum >= (!many_tiles ? 288 : kblocked && n < 128 ? 256 : 192) * n;
+  const int64_t tiles = cdiv64(x, BX) * cdiv64(y, BY) * n, grid = persistent_grid();
+  const bool many = tiles >= (kblocked ? 10 : 8) * grid;
+  return msum >= (tiles <= grid || (many && (!kblocked || n >= 128)) ? 192 : many ? 256 : 288) * n;
 }
 
 }  // namespace

@@ -14,11 +14,12 @@ ROWS, TRANSPOSED, KBLOCKED = 0, 1, 2
     (192, 64, 512, 1024, ROWS, 32),        # 39, 42
     (256, 64, 512, 1024, ROWS, 32),        # 44, 46
     (280, 64, 1024, 1024, KBLOCKED, 32),   # 68, 72 | 77, 73
-    (320, 96, 256, 512, ROWS, 64),         # 26, 28 | 93, 83
+    (236, 96, 256, 128, ROWS, 64),         # 166, 104 with a load falling as rank^-1.8
+    (200, 96, 256, 512, ROWS, 64),         # 24, 26 | 64, 59: no more tiles than workgroups
     (448, 64, 512, 1024, ROWS, 64),        # 69, 67
     (192, 32, 768, 2048, ROWS, 32),        # 48, 52
     (512, 16, 4096, 2048, KBLOCKED, 64),   # 182, 167
-    (192, 64, 512, 512, KBLOCKED, 32),     # 18.9, 20.9
+    (192, 64, 512, 512, KBLOCKED, 64),     # 18.9, 20.9: no more tiles than workgroups
     (192, 64, 2048, 4096, KBLOCKED, 32),   # 361, 381: ten tiles a workgroup and more
     (200, 128, 2048, 2048, KBLOCKED, 64),  # 402, 378 | 396, 403
     (256, 128, 2048, 2048, KBLOCKED, 64),  # 454, 435

@@ -311,12 +311,12 @@ def _pieces(lib, sizes, X, Y, M):
 
 
 @pytest.mark.parametrize("sizes,X,Y,stage,pieces", [
-    ([0, 1, 33, 64, 65, 130, 1100, 257], 264, 328, 32, 1),  # 206 rows per expert on average, edges in X and Y
-    ([0, 1, 33, 64, 65, 130, 3200, 257], 264, 328, 64, 1),  # the same in the loop of 64 rows a stage
+    ([0, 1, 33, 64, 65, 130, 1100, 257], 264, 328, 64, 1),  # 206 rows per expert on average, edges in X and Y
+    ([0, 1, 33, 64, 65, 130, 900, 257], 264, 328, 32, 1),   # 181: the same in the short loop
     ([2000, 0, 31, 1500], 512, 256, 64, 1),                  # whole tiles
     ([129, 1, 0, 300, 128, 127, 95, 5], 520, 72, 32, 1),     # 98 rows per expert: the short loop
     ([9031, 31, 0, 6000], 264, 328, 64, 4),                  # cut by rows, into pieces of 71 groups of 32
-    ([31, 9031, 0, 6] + [2] * 40, 264, 328, 32, 4),          # cut in the short loop
+    ([31, 9031, 0, 6] + [2] * 50, 264, 328, 32, 4),          # cut in the short loop
 ])
 @pytest.mark.parametrize("form", ["gather_a", "gather_b", "a_transposed", "b_transposed", "b_kblocked"])
 def test_weight_gradient_loops_at_the_edges(sizes, X, Y, stage, pieces, form):
