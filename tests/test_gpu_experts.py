@@ -372,7 +372,7 @@ def test_weight_gradient_loops_at_the_edges(sizes, X, Y, stage, pieces, form):
 @pytest.mark.parametrize("sizes,X,Y,pieces", [
     ([3000, 2600, 64, 0, 3100], 2048, 2304, 1),   # 72 tiles each, 360 items
     ([9000, 2600, 64, 0, 3100], 2048, 2304, 4),   # one cut by rows
-    ([70, 4000, 4000, 4000], 2304, 2048, 1),      # the first XCD's run starts with short items
+    ([70, 0, 4000, 0, 4000, 4000], 2304, 2048, 1),  # short items in front, items without rows between
 ])
 @pytest.mark.parametrize("form", ["a_transposed", "b_kblocked"])
 def test_weight_gradients_in_whole_rounds(sizes, X, Y, pieces, form):
