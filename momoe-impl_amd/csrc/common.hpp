@@ -16,7 +16,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 512;  // every GEMM workgroup is 8 wavefronts of 64: two per SIMD
+constexpr int kThreads = 512;  // of a workgroup of gemm_tile.hpp: 8 wavefronts of 64, two per SIMD (gemm_span.hpp: 4)
 constexpr int kWaves = kThreads / 64;
 constexpr int kWave = 64;
 

@@ -9,8 +9,8 @@
 namespace momoe {
 namespace {
 
-// Both data-gradient GEMMs take WideSpan tiles; launches with few tiles the narrow ones of
-// gemm_tile.hpp (takes_narrow_tiles).
+// Both data-gradient GEMMs take WideSpan tiles (takes_span_tiles).  The rest go to the kernels of gemm_tile.hpp that
+// hold narrow tiles, and wide ones where the table has too many for those (narrow_tiles_fit).
 constexpr int FN = 2;  // of those: 2x4 (4x2) waves, each (32 * FM) rows x 64 columns
 
 struct DhArgs {
@@ -24,9 +24,8 @@ struct DhArgs {
 };
 
 // u = G_y[idx] . Wl2^T: both operands are k-contiguous (k = D).
-template <class G_>
 struct DhSpan {
-  using G = G_;
+  using G = WideSpan;
   static constexpr bool EXCHANGE = false;
   using Rows = SpanGatheredRows<256>;
   using Weights = SpanPitchedRows<G::COLS>;
@@ -55,7 +54,7 @@ struct DhSpan {
 
 __global__ __launch_bounds__(kSpanThreads, 1) void dgrad_h_kernel(DhArgs p) {
   const ClockTrace trace(p.clk);
-  run_span_tiles<DhSpan<WideSpan>>(p, (p.H + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  run_span_tiles<DhSpan>(p, (p.H + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
   trace.finish();
 }
 
@@ -251,9 +250,8 @@ struct DxArgs {
 };
 
 // gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
-template <class G_>
 struct DxSpan {
-  using G = G_;
+  using G = WideSpan;
   static constexpr bool EXCHANGE = false;
   using Rows = SpanBlockedRows<256>;
   using Weights = SpanPitchedRows<G::COLS>;
@@ -282,7 +280,7 @@ struct DxSpan {
 
 __global__ __launch_bounds__(kSpanThreads, 1) void dgrad_x_kernel(DxArgs p) {
   const ClockTrace trace(p.clk);
-  run_span_tiles<DxSpan<WideSpan>>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  run_span_tiles<DxSpan>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
   trace.finish();
 }
 

@@ -31,16 +31,15 @@ struct Lin1Args {
   unsigned long long* clk;
 };
 
-// The forward.  Tile = up to 256 rows x (128 `a` columns + the matching 128 `b` columns), or 64 + 64; a wave's
+// The forward.  Tile = up to 256 rows x (128 `a` columns + the matching 128 `b` columns); a wave's
 // first half of fragments are `a` columns, the second their `b` columns, so the SwiGLU product pairs
 // registers of the same lane.
-template <class G_>
 struct Lin1Span {
-  using G = G_;
+  using G = WideSpan;
   static constexpr bool EXCHANGE = false;
   static constexpr int BNH = G::COLS / 2, WIDTH = 8 * G::FN;  // hidden columns of a tile, of a wave
   using Rows = SpanGatheredRows<256>;
-  using Weights = SpanCols<G::COLS, true>;
+  using Weights = SpanCols<true>;
   using Ids = FetchIds;
   struct Late {};
   const Lin1Args& p;
@@ -122,7 +121,7 @@ __global__ __launch_bounds__(kSpanThreads, 1) void lin1_swiglu_fwd_kernel(Lin1Ar
   const ClockTrace trace(p.clk);
   // without an h output only rows >= ab_lo are wanted: experts entirely below are skipped
   const int first = p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
-  using Prog = Lin1Span<WideSpan>;
+  using Prog = Lin1Span;
   run_span_tiles<Prog>(p, (p.H + Prog::BNH - 1) / Prog::BNH, MOMOE_TILE_ROWS, first);
   trace.finish();
 }
@@ -137,7 +136,7 @@ struct Lin1BwdSpan {
   static constexpr int BNH = G::COLS / 2, WIDTH = 8 * G::FN, HF = G::FN / 2;
   static_assert(BNH == MOMOE_GS_BLOCK && G::WCOLS == 2, "a tile's row sums are one part, from two waves");
   using Rows = SpanGatheredRows<256>;
-  using Weights = SpanCols<G::COLS, true>;
+  using Weights = SpanCols<true>;
   using Stager = SpanStager<WIDTH>;
   struct Ids {
     FetchIds fetch;
@@ -630,12 +629,11 @@ struct Lin2Args {
   unsigned long long* clk;
 };
 
-template <class G_>
 struct Lin2Span {
-  using G = G_;
+  using G = WideSpan;
   static constexpr bool EXCHANGE = false;
   using Rows = SpanBlockedRows<256>;   // rows of h, k-blocked
-  using Weights = SpanCols<G::COLS>;
+  using Weights = SpanCols<>;
   using Ids = RowIds;     // tokens of the rows this wave holds in the accumulators
   using Late = RowScales; // their gate weights
   const Lin2Args& p;
@@ -665,7 +663,7 @@ struct Lin2Span {
 
 __global__ __launch_bounds__(kSpanThreads, 1) void lin2_scale_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
-  run_span_tiles<Lin2Span<WideSpan>>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
+  run_span_tiles<Lin2Span>(p, (p.D + WideSpan::COLS - 1) / WideSpan::COLS, MOMOE_TILE_ROWS);
   trace.finish();
 }
 

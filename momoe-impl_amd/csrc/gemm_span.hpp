@@ -1,8 +1,8 @@
-// Workgroup-level bf16 GEMM for gfx950 (CDNA4): 256 x 256 (256 x 128) fp32 tiles, 64 k-values a stage.
+// Workgroup-level bf16 GEMM for gfx950 (CDNA4): 256 x 256 fp32 tiles, 64 k-values a stage.
 //
 // A workgroup of 4 wavefronts, one per SIMD with the SIMD's whole register file, computes a tile
-// with v_mfma_f32_16x16x32_bf16; each wave owns 128 x 128 (128 x 64) of it in 8 x 8 (8 x 4)
-// accumulators of 4 registers.  One workgroup per CU, persistent.
+// with v_mfma_f32_16x16x32_bf16; each wave owns 128 x 128 of it in 8 x 8 accumulators
+// of 4 registers.  One workgroup per CU, persistent.
 //
 // What bounds such a loop on MI355X is energy: under sustained MFMA load the chip is power-limited and
 // the shader clock falls until the power fits, so time follows what is spent on multiplications,
@@ -23,7 +23,7 @@
 // k-values 1273 -> 4 waves 1229 -> 8 waves with 16 x 16 x 32 1293 -> 4 waves with 16 x 16 x 32 1393.
 //
 // LDS: a ring of stages for each operand, one deeper for the weights, which come from HBM where rows
-// mostly come out of L2: 3 x 32 KiB and 2 x 32 KiB with 256 columns, 4 x 16 and 3 x 32 with 128.
+// mostly come out of L2: 3 x 32 KiB and 2 x 32 KiB.
 //
 // Global memory goes straight to LDS with global_load_lds_dwordx4; every lane chooses its own 16
 // bytes, so the LDS image is swizzled by permuting which piece a lane fetches, and the same freedom
@@ -223,14 +223,13 @@ struct SpanBlockedRows {
 // lanes, lane i supplies the address of columns 4 * (i % 4) .. +3 of k-row i / 4 and receives column
 // i of those 4 k-rows.  The 8 k-rows x 32 bytes of 32 lanes then lie in different banks.
 // PAIRED: the wave's second half of fragments are the columns COLS / 2 further on.
-template <int COLS, bool PAIRED = false>
+template <bool PAIRED = false>
 struct SpanCols {
-  static constexpr int DEP = COLS / 32, FN = COLS / 32;
+  static constexpr int COLS = 256, DEP = COLS / 32, FN = COLS / 32;
   static constexpr int ELEMS = COLS * kSpan;
   static constexpr int PIECES = COLS / 8, RPD = 64 / PIECES;  // pieces of a k-row, k-rows of a deposit
   static constexpr int STEP = RPD * kSpanWaves;                // k-rows of a deposit of all waves
-  static constexpr int PATTERNS = STEP < 16 ? 2 : 1;           // swizzles met by this lane's deposits
-  static_assert(COLS == 256 || COLS == 128, "deposits of 8 or 16 k-rows");
+  static constexpr int PATTERNS = 2;                           // swizzles met by this lane's deposits
   static __device__ __forceinline__ int swz(int k) { return 2 * (k & 3) + 8 * ((k >> 3) & 1); }
   const bf16* base;
   uint32_t off[PATTERNS], pitch;  // bytes
@@ -264,15 +263,14 @@ struct SpanCols {
   static __device__ __forceinline__ bf16x8 frag(const bf16* slot, const Lane& ln, int i, int h) {
     // (pieces 1 to 3 bits up are permuted, so what is added to a column there is an exclusive or)
     const int far = PAIRED && i >= FN / 2 ? COLS / 2 : 0, n = PAIRED ? i % (FN / 2) : i;
-    const int flip = 16 * n + (far < 128 ? far : 0);
-    const bf16* p = (const bf16*)((const char*)slot + (ln.o ^ (2 * flip))) + (far - (flip - 16 * n)) + h * (kHalf * COLS);
+    const bf16* p = (const bf16*)((const char*)slot + (ln.o ^ (32 * n))) + far + h * (kHalf * COLS);
     const bf16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + 4 * COLS);
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   }
 };
 
 // ---- tile geometries --------------------------------------------------------------------------------
-// Waves 2 x 2, each 128 rows and COLS / 2 columns.
+// Waves 2 x 2, each 128 rows and 128 columns.
 struct WideSpan {
   static constexpr int COLS = 256, MAX_ROWS = 256;
   static constexpr int AHEAD = 2;               // stages of rows in LDS; of weights one more
@@ -423,7 +421,7 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
   P prog(args);
   using Rows = typename P::Rows;
   using Weights = typename P::Weights;
-  constexpr int FM = G::FM, FN = G::FN, AHEAD = G::AHEAD;
+  constexpr int FN = G::FN, AHEAD = G::AHEAD;
   constexpr int ROWS_AT = (AHEAD + 1) * Weights::ELEMS;  // the rows' ring lies behind the weights'
   static_assert((ROWS_AT + AHEAD * Rows::ELEMS) * sizeof(bf16) <= kSpanLds, "the rings fit the LDS");
   static_assert(Weights::ELEMS >= kSpanWaves * kStagingElems, "a stage of weights holds the epilogue's staging");

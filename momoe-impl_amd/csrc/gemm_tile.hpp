@@ -705,8 +705,9 @@ inline int persistent_grid() {
   return (cus + 7) / 8 * 8;
 }
 
-// Whether a launch over `cols` output columns takes the kernel that holds NarrowTiles: if with them
-// there is still no more than one tile per CU.  The routing is not known here; its row tiles are taken as
+// Whether a launch over `cols` output columns is one for NarrowTiles: if with them there is still no more than one
+// tile per CU.  Such launches stay out of the loop of gemm_span.hpp and of the read-once kernels; what those decline
+// goes to the kernel that holds NarrowTiles, too, and takes wide ones there.  The routing is not known here; its row tiles are taken as
 // if every expert held a quarter more than its share, and the kernel goes by the table
 // (narrow_tiles_fit).  Beyond one tile per CU the weights' way from HBM sets the pace: dL/dh of 1000
 // tokens over 128 experts with 768 columns takes 112 us in two rounds of wide tiles, 113 in three of
@@ -718,8 +719,8 @@ inline bool takes_narrow_tiles(int64_t msum, int64_t n, int64_t cols) {
 
 // In that kernel: whether the table's tiles in `nb` column blocks of NarrowTiles are at most one per
 // workgroup (two halves of a 320-row one); if not it takes the wide tiles of the table's height.
-// Callers mark the narrow path as the expected one: behind the test it cost a launch 0.1 to 0.5 us less
-// than past the wide path's code.
+// Callers mark the narrow path as the expected one: behind the test it cost a launch of few tiles 0.1 to 0.5 us less
+// than past the wide path's code (launches that take the wide tiles there are tens of us).
 // Forward and step with D = 1024, H = 512, N = 32, K = 4, wide tiles -> narrow ones regardless -> by
 // this rule, us: 1024 tokens, one expert shared (37 tiles x 8) 66 -> 79 -> 67 and 249 -> 265 -> 247;
 // 1300 tokens, load falling as rank^-1.8 (39 x 8 of 320 rows) 70 -> 80 -> 71 and 268 -> 284 -> 270; 700

@@ -636,12 +636,12 @@ static_assert((size_t)(kMaxWgradExperts + 1) * 20 + 512 <= kPlanLds, "prefix sum
 // expert's last one: the M side's zeros meet finite numbers if the expert's are finite.  The stages of a
 // span without rows take row and token 0: the list may hold nothing yet.
 
-// "rows" operand.  LDS [64][256] as SpanCols<256>; wave w deposits k-rows [16 w, 16 w + 16), two a time.  The
+// "rows" operand.  LDS [64][256] as SpanCols; wave w deposits k-rows [16 w, 16 w + 16), two a time.  The
 // ids of gathered rows are wave-uniform and come through scalar loads, 16 at once while all exist.
 // Sources are a wave-uniform base plus a 32-bit byte offset per lane: the matrix for a gathered
 // operand, the span's first row otherwise, so (number of tokens) x (row pitch) must stay below 4 GiB.
 struct RowsOperand {
-  using L = SpanCols<256>;
+  using L = SpanCols<>;
   using Lane = L::Lane;
   static constexpr int DEP = L::DEP, ELEMS = L::ELEMS, ROWS = 2 * DEP;
   typedef int32_t ids_t __attribute__((ext_vector_type(ROWS), aligned(4)));
@@ -706,7 +706,7 @@ struct RowsOperand {
 // feature f of row r at mat[((f / 32) * ld + r) * 32 + f % 32], ld = rows of the matrix (gz, as
 // the SwiGLU backward writes it for dL/dx).  LDS as above; a deposit is k-rows 8 j + 2 w and the next.
 struct BlockedRowsOperand {
-  using L = SpanCols<256>;
+  using L = SpanCols<>;
   using Lane = L::Lane;
   static constexpr int DEP = L::DEP, ELEMS = L::ELEMS;
   const bf16 *mat, *src;
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
       order_fence();
     };
     Span from = c0.rows;  // the span of the stages being requested,
-    int ft = 2, fn = count;  // the one at hand, their number
+    int ft = 2;              // the one at hand
     // Scalar loads share the wait counter of the LDS reads, and the products wait for those at the start of
     // each half: the loads start behind the wait in the middle of a stage, when both operands have used up the
     // last ones, and have half a stage.  The scalar unit issues one instruction in four cycles, and between the
@@ -981,7 +981,6 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
       end = count;  // from here on the next item's stages are requested
       from = c1.rows;
       ft = 0;
-      fn = from.stages();
       A.set_tile(p.a, from, c1.x0, p.X);
       B.set_tile(p.b, from, c1.y0, p.Y);
     }
