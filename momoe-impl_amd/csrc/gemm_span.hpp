@@ -364,8 +364,8 @@ struct SpanFrags {
     unrolled<0, FN + NA>([&](auto R) { read<B, decltype(R)::value, H>(w, a); });
   }
   // The products of register set B; between them the reads of half H (-1: none) of (w, a) into the other set,
-  // and DEP calls of `dep`
-  template <int B, int H, int DEP, class Dep>
+  // and DEP calls of `dep`.  FRESH: the first of a tile, which add to nothing.
+  template <int B, int H, int DEP, bool FRESH = false, class Dep>
   __device__ __forceinline__ void multiply(f32x4 (&acc)[FN][NA > 0 ? NA : 1], const bf16* w, const bf16* a, Dep dep) {
     if constexpr (NM == 0) {
       unrolled<0, DEP>([&](auto D) { dep(D); });
@@ -373,7 +373,7 @@ struct SpanFrags {
       constexpr int NR = H >= 0 ? FN + NA : 0, PER = (2 * NR + NM - 1) / NM;  // reads behind an MFMA: in the first half
       unrolled<0, NM>([&](auto MC) {
         constexpr int m = decltype(MC)::value, j = m / NA, i = (j & 1) ? NA - 1 - m % NA : m % NA;
-        acc[j][i] = mfma16(wf[B][j], af[B][i], acc[j][i]);
+        acc[j][i] = mfma16(wf[B][j], af[B][i], FRESH ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : acc[j][i]);
         unrolled<0, PER>([&](auto R) {
           constexpr int r = m * PER + decltype(R)::value;
           if constexpr (r < NR) read<B ^ 1, r, (H > 0 ? 1 : 0)>(w, a);
@@ -478,10 +478,6 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
     auto tile = [&](auto NAC) {
       constexpr int NA = decltype(NAC)::value;
       f32x4 acc[FN][NA > 0 ? NA : 1];
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int i = 0; i < NA; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       SpanFrags<Rows, Weights, FN, NA> fr(c0.mbase, prog.n_org);
       // the next stage has landed, all but what was requested after it; every wave is done reading this one
       auto turn = [&] {
@@ -492,30 +488,39 @@ __device__ __forceinline__ void run_span_tiles(const Args& args, int nb, int max
       };
       fr.template read_all<0, 0>(at(ring.w), at(ring.a));
       order_fence();
-      int t = 0, end = st.count - AHEAD;
-      while (true) {
-        const int stop = min(end, st.full);
-#pragma unroll 1
-        for (; t < stop; ++t) {
-          const bf16 *wsrc = W.source(k), *asrc = A.source(k);
-          const uint32_t wto = addr + ring.wlast, ato = addr + ring.a;
-          fr.template multiply<0, 1, Weights::DEP>(
-              acc, at(ring.w), at(ring.a), [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
-          turn();
-          fr.template multiply<1, 0, Rows::DEP>(
-              acc, at(ring.wnext), at(ring.anext), [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
-          k = st.after(k);
-          ring.turn();
-        }
-        if (end == st.count) break;
-        k = 0;  // from here on the next tile's stages are requested
-        end = st.count;
+      auto stage = [&](auto FRESH) {
+        const bf16 *wsrc = W.source(k), *asrc = A.source(k);
+        const uint32_t wto = addr + ring.wlast, ato = addr + ring.a;
+        fr.template multiply<0, 1, Weights::DEP, decltype(FRESH)::value>(
+            acc, at(ring.w), at(ring.a), [&](auto D) { W.template deposit<decltype(D)::value>(wsrc, wto); });
+        turn();
+        fr.template multiply<1, 0, Rows::DEP>(
+            acc, at(ring.wnext), at(ring.anext), [&](auto D) { A.template deposit<decltype(D)::value>(asrc, ato); });
+        k = st.after(k);
+        ring.turn();
+      };
+      auto request_next_tile = [&] {
+        k = 0;
         if (c1.valid) {
           prog.setup(c1, g1, A, W);
         } else {
           A.idle();
           W.idle();
         }
+      };
+      // The first stage by itself: its products start from zero, which a loop would have to write to 256 accumulation
+      // registers before them.  In us, 8192 tokens, D = 2048, H = 1024, N = 128, K = 8: x.Wl1 466 -> 462, h.Wl2 270 -> 267,
+      // recomputing GEMM 544 -> 541, dL/dx 451 -> 448, Wl1 gradient 634 -> 622, Wl2 gradient 330 -> 326.
+      if (st.count == AHEAD) request_next_tile();
+      stage(IntC<true>{});
+      int t = 1, end = st.count == AHEAD ? st.count : st.count - AHEAD;
+      while (true) {
+        const int stop = min(end, st.full);
+#pragma unroll 1
+        for (; t < stop; ++t) stage(IntC<false>{});
+        if (end == st.count) break;
+        end = st.count;  // from here on the next tile's stages are requested
+        request_next_tile();
       }
       if (st.tail) {
         const bf16 *wsrc = W.source(k), *asrc = A.source(k);

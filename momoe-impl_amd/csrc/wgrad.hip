@@ -931,10 +931,6 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
     };
     if (behind) request_next();
     TileAcc acc;
-#pragma unroll
-    for (int f = 0; f < FN; ++f)
-#pragma unroll
-      for (int i = 0; i < FM; ++i) acc[f][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     SpanFrags<AOp, BOp, FN, FM> fr(wave_row(), wave_col());
     const bf16 *b = bptr(sb), *a = aptr(sa);
     fr.template read_all<0, 0>(b, a);
@@ -953,36 +949,49 @@ __global__ __launch_bounds__(kSpanThreads, 1) void wgrad_kernel(WgradArgs p) {
     // halves no product runs: with A's loads at a stage's end and some 60 instructions in that place instead
     // of 25, the Wl1 gradient of 65536 tokens (D = 4096, H = 2048, N = 64, K = 8) took 15.2 ms instead of 14.3.
     static_assert(AOp::DEP == BOp::DEP, "prepared together");
+    auto stage = [&](auto FRESH) {
+      const uint32_t bto = bslot(sb == 0 ? 2 : sb - 1), ato = aslot(sa);
+      sb = next3(sb);
+      sa ^= 1;
+      const bf16 *nb = bptr(sb), *na = aptr(sa);
+      B.begin(from, ft);
+      fr.template multiply<0, 1, BOp::DEP, decltype(FRESH)::value>(acc, b, a, [&](auto D) {
+        B.template prepare<decltype(D)::value>();
+        B.template deposit<decltype(D)::value>(bto);
+        A.template prepare<decltype(D)::value>();
+      });
+      turn();
+      request_next();
+      A.begin(from, ft);
+      fr.template multiply<1, 0, AOp::DEP>(acc, nb, na, [&](auto D) { A.template deposit<decltype(D)::value>(ato); });
+      ++ft;
+      b = nb;
+      a = na;
+    };
     int t = 0, end = count - 2;
-    while (true) {
-      const int stop = min(end, real - 1);
-#pragma unroll 1
-      for (; t < stop; ++t) {
-        const uint32_t bto = bslot(sb == 0 ? 2 : sb - 1), ato = aslot(sa);
-        sb = next3(sb);
-        sa ^= 1;
-        const bf16 *nb = bptr(sb), *na = aptr(sa);
-        auto deposit_b = [&](auto D) {
-          B.template prepare<decltype(D)::value>();
-          B.template deposit<decltype(D)::value>(bto);
-          A.template prepare<decltype(D)::value>();
-        };
-        B.begin(from, ft);
-        fr.template multiply<0, 1, BOp::DEP>(acc, b, a, deposit_b);
-        turn();
-        request_next();
-        A.begin(from, ft);
-        fr.template multiply<1, 0, AOp::DEP>(acc, nb, na, [&](auto D) { A.template deposit<decltype(D)::value>(ato); });
-        ++ft;
-        b = nb;
-        a = na;
-      }
-      if (end == count) break;
-      end = count;  // from here on the next item's stages are requested
+    auto request_next_item = [&] {
+      end = count;
       from = c1.rows;
       ft = 0;
       A.set_tile(p.a, from, c1.x0, p.X);
       B.set_tile(p.b, from, c1.y0, p.Y);
+    };
+    if (end == 0) request_next_item();
+    if (real > 1) {  // the first stage by itself: its products start from zero (run_span_tiles)
+      stage(IntC<true>{});
+      t = 1;
+    } else {
+#pragma unroll
+      for (int f = 0; f < FN; ++f)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[f][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    while (true) {
+      const int stop = min(end, real - 1);
+#pragma unroll 1
+      for (; t < stop; ++t) stage(IntC<false>{});
+      if (end == count) break;
+      request_next_item();  // from here on its stages are requested
     }
     // the item's last stage: its k-values past the last row are zeroed on the M side, a half without rows is
     // left out; then, with 64 rows or fewer, a stage without rows
