@@ -87,6 +87,18 @@ __device__ __forceinline__ void store16(void* uniform_base, uint32_t byte_offset
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, valid ? byte_offset : 0xFFFFFFF0u, 0, STREAM ? 2 : 0);
 }
 
+// The same with one bound for all lanes: those whose offset lies at or past `bytes`, a uniform value, store nothing.
+// For a store that many are made of: the comparison costs no instructions.
+template <bool STREAM = false>
+__device__ __forceinline__ void store16_below(void* uniform_base, uint32_t byte_offset, uint32_t bytes, bf16x8 v) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_base, 0, bytes, 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, byte_offset, 0, STREAM ? 2 : 0);
+}
+// how many of a fragment row's 16 rows, from `row` on, are among the first `rows` (a median is taken in vector registers)
+__device__ __forceinline__ uint32_t rows_of_fragment(int row, int rows) {
+  return __builtin_amdgcn_readfirstlane(max(0, min(16, rows - row)));
+}
+
 // the same for 4 bytes
 __device__ __forceinline__ void store4(float* uniform_base, uint32_t byte_offset, bool valid, float v) {
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_base, 0, 0x7FFFFFFF, 0x00027000);
@@ -690,7 +702,11 @@ __device__ __forceinline__ bf16x4 pack_bf16x4(f32x4 v, float s) {
 }
 
 // A wave's accumulators as `rows` rows, from row0, of a row-major matrix of `cols` columns, from column col0; scale(i) is that of
-// the lane's row in fragment row i; lane = fresh_lane()
+// the lane's row in fragment row i; lane = fresh_lane().  Rows behind the last one lie past a bound, a lane without columns
+// names an offset past any.  (With a comparison and two selections for each store instead the vector unit, which all of this is
+// bound by, had a ninth more to do: 8192 tokens, D = 2048, H = 1024, N = 128, K = 8, Wl1 gradient 648 -> 640 us, Wl2 gradient
+// 332 -> 326, h.Wl2 270 -> 268, dL/dx 452 -> 449.  The epilogues of the SwiGLU products gain nothing from it: their bounds differ
+// from store to store, and the scalar registers they take were spilled.)
 template <bool STREAM = false, int FN, int NA, class Scale>
 __device__ __forceinline__ void store_rows(f32x4 (&acc)[FN][NA], bf16* staging, bf16* out, int64_t row0, int rows, int cols,
                                            int col0, int lane, Scale scale) {
@@ -699,13 +715,14 @@ __device__ __forceinline__ void store_rows(f32x4 (&acc)[FN][NA], bf16* staging, 
   bf16* const first = out + row0 * cols + col0;  // uniform
   uint32_t off[Stager::PASSES];
 #pragma unroll
-  for (int p = 0; p < Stager::PASSES; ++p) off[p] = ((uint32_t)stager.row(p) * (uint32_t)cols + stager.col(p)) * 2;
+  for (int p = 0; p < Stager::PASSES; ++p)
+    off[p] = col0 + stager.col(p) < cols ? ((uint32_t)stager.row(p) * (uint32_t)cols + stager.col(p)) * 2 : 0xFFFFFFF0u;
   bf16x8 v[2][Stager::PASSES];
   auto store = [&](int i) {
+    const uint32_t bytes = rows_of_fragment(16 * i, rows) * (uint32_t)cols * 2;
 #pragma unroll
     for (int p = 0; p < Stager::PASSES; ++p)
-      store16<STREAM>(first + (int64_t)(16 * i) * cols, off[p], 16 * i + stager.row(p) < rows && col0 + stager.col(p) < cols,
-              v[i & 1][p]);
+      store16_below<STREAM>(first + (int64_t)(16 * i) * cols, off[p], bytes, v[i & 1][p]);
   };
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
