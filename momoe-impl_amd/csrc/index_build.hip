@@ -399,6 +399,142 @@ __global__ __launch_bounds__(kPanelTokens) void index_tiny_kernel(
   }
 }
 
+// Results of all 64 lanes by the vector unit's lane permutations (quads, rows of 16, then from row to row), as uniform values
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t from_lanes(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v, Op op) {  // op(v, 0) = v
+  v = op(v, from_lanes<0xB1, 0xf>(v));   // quad_perm: lane ^ 1
+  v = op(v, from_lanes<0x4E, 0xf>(v));   // quad_perm: lane ^ 2
+  v = op(v, from_lanes<0x141, 0xf>(v));  // row_half_mirror: the other quad of 8 lanes
+  v = op(v, from_lanes<0x140, 0xf>(v));  // row_mirror: the other half of 16 lanes
+  v = op(v, from_lanes<0x142, 0xa>(v));  // row_bcast15: row 0 -> 1, row 2 -> 3
+  v = op(v, from_lanes<0x143, 0xc>(v));  // row_bcast31: row 1 -> 2, 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The whole index build in one launch for one panel of tokens, at most 256, at most kColumnExperts experts and tiles of at
+// least 256 rows (an expert is one tile): a workgroup per group of 16 experts, a thread per token.  Each reads the
+// whole mask, all of a thread's entries in flight together, so that it knows by itself the pairs and tiles of the groups
+// before its own; a launch that counts first takes longer.  Bound by the latency of the loads and of the exchanges between
+// the waves.  In a graph, us with one fill of 1.6 us, counting and placing -> this: 128 tokens x 8 experts 8.9 -> 7.0,
+// 200 x 64 10.1 -> 8.4; with a second round of loads, 131 x 128 10.2 -> 10.2, and a fourth, 256 x 256, 10.6 -> 14.7: up to 64
+// experts.  The kernel above -> this: 64 x 8 10.4 -> 7.0, 64 x 64 9.0 -> 7.9, 48 x 64 8.2 -> 7.9, 32 x 64 7.1 -> 7.9: from
+// more than kTinyFewExperts tokens on.
+constexpr int kColumnExperts = 64, kTinyFewExperts = 48;
+__global__ __launch_bounds__(kPanelTokens) void index_column_kernel(
+    const int32_t* __restrict__ mask, int64_t sn, int64_t sm, int M, int N, int K, int NG, int64_t* __restrict__ sizes,
+    int32_t* __restrict__ cumsums, int32_t* __restrict__ idx, int32_t* __restrict__ which, int32_t* __restrict__ inv,
+    int32_t* __restrict__ table, int tile_rows, int32_t* __restrict__ table_rc, int32_t* __restrict__ violations) {
+  constexpr int WAVES = kPanelTokens / 64, GROUPS = kColumnExperts / kPanelExperts;
+  __shared__ uint32_t s_held[WAVES][GROUPS / 2];  // experts that hold a token of the wave, two groups a word
+  __shared__ uint32_t s_pairs[WAVES];
+  __shared__ int32_t s_off[kPanelExperts][WAVES];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, g = blockIdx.x, m = t;
+  const int64_t msum = (int64_t)M * K;
+  // a uniform row and the lane's 32-bit offset in it (checked on the host); clamped into the matrix, masked afterwards
+  const uint32_t off = (uint32_t)min(m, M - 1) * (uint32_t)sm * 4;
+  int32_t v[kColumnExperts];
+#pragma unroll
+  for (int e = 0; e < kColumnExperts; ++e) v[e] = *(const int32_t*)((const char*)(mask + (int64_t)min(e, N - 1) * sn) + off);
+  uint32_t b[GROUPS], bits = 0;
+  int k = 0, pairs = 0;  // of the token: pairs in the groups before this one, in all
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) {
+    b[u] = 0;
+#pragma unroll
+    for (int e = 0; e < kPanelExperts; ++e) b[u] |= (v[u * kPanelExperts + e] != 0 ? 1u : 0u) << e;
+    const int left = N - u * kPanelExperts;  // experts there are
+    b[u] &= m < M && left > 0 ? 0xffffu >> (kPanelExperts - min(left, kPanelExperts)) : 0u;
+    const int n = __popc(b[u]);
+    pairs += n;
+    k += u < g ? n : 0;
+    bits = u == g ? b[u] : bits;
+  }
+#pragma unroll
+  for (int u = 0; u < GROUPS; u += 2) {
+    const uint32_t held = wave_reduce(b[u] | b[u + 1] << 16, [](uint32_t x, uint32_t y) { return x | y; });
+    if (lane == 0) s_held[wave][u / 2] = held;
+  }
+  uint64_t ballots[kPanelExperts];
+#pragma unroll
+  for (int q = 0; q < kPanelExperts; ++q) ballots[q] = __ballot((bits >> q) & 1u);
+  // (at most 64 x 64 pairs of a wave's tokens: both sums in one word)
+  const uint32_t sums = wave_reduce((uint32_t)k | (uint32_t)pairs << 16, [](uint32_t x, uint32_t y) { return x + y; });
+  if (lane == 0) {
+    s_pairs[wave] = sums;
+#pragma unroll
+    for (int q = 0; q < kPanelExperts; ++q) s_off[q][wave] = __popcll(ballots[q]);
+  }
+  __syncthreads();
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) base += s_pairs[w] & 0xffff, total += s_pairs[w] >> 16;
+  const bool overflow = (int64_t)total > msum;
+  if (wave == 0) {
+    // lane q: tiles of group q, which are its experts with tokens
+    uint32_t held = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) held |= s_held[w][min(lane, GROUPS - 1) / 2];
+    const int tiles = lane < NG ? __popc((held >> (16 * (lane & 1))) & 0xffff) : 0;
+    const int tiles_to = wave_inclusive_scan(tiles, lane);
+    const int tiles_before = __shfl(tiles_to - tiles, g), all_tiles = __shfl(tiles_to, 63);
+    // lane e: expert e of this group
+    const int i = g * kPanelExperts + lane;
+    const bool mine = lane < kPanelExperts && i < N;
+    int rows = 0;
+    if (mine)
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) rows += s_off[lane][w];
+    int run = base + wave_inclusive_scan(rows, lane) - rows;
+    const uint64_t some = __ballot(rows > 0);
+    if (mine) {
+      const int tile = tiles_before + __popcll(some & ((1ull << lane) - 1));
+      sizes[i] = (int64_t)rows;
+      cumsums[i] = run;
+      if (rows > 0 && !overflow) write_tile_entry(table, table_rc, tile, tile, i, run, rows);
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {  // sorted row of the expert's first token, per wavefront
+        const int n = s_off[lane][w];
+        s_off[lane][w] = run;
+        run += n;
+      }
+    }
+    if (g == NG - 1 && lane == 0) {
+      cumsums[N] = total;
+      if (overflow) atomicAdd(violations, 1);
+      write_tile_header(table, table_rc, overflow ? 0 : all_tiles, tile_rows);
+    }
+  }
+  __syncthreads();
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int q = 0; q < kPanelExperts; ++q) {
+    if ((bits >> q) & 1u) {
+      const int row = s_off[q][wave] + __popcll(ballots[q] & below);
+      if (row < msum) {
+        idx[row] = m;
+        which[row] = k;
+      }
+      if (k < K) inv[(int64_t)m * K + k] = row < msum && !overflow ? row : -1;  // (as index_place_kernel)
+      ++k;
+    }
+  }
+  if (g == NG - 1) {
+    // sorted rows past the last pair (a routing with fewer than M*K pairs): token 0, slot 0
+    for (int64_t r = (int64_t)total + t; r < msum; r += kPanelTokens) {
+      idx[r] = 0;
+      which[r] = 0;
+    }
+    if (m < M && pairs != K) {
+      atomicAdd(violations, 1);
+      for (int kk = pairs; kk < K; ++kk) inv[(int64_t)m * K + kk] = -1;
+    }
+  }
+}
+
 // Passes 2 and 3 in one launch, for N <= kPlaceMaxExperts and N * NC <= kPlaceCounts.  Every
 // workgroup needs the rows of all experts before its panel, i.e. sums over all the counts (at most
 // 64 KiB, from L2): doing that in each of them takes less time than a one-workgroup launch in
@@ -670,13 +806,23 @@ extern "C" int momoe_index_build(const int32_t* mask_NM, int64_t stride_n, int64
   int32_t* part = (int32_t*)workspace;
   int32_t* tokcnt = part + N * NC;
   hipStream_t st = (hipStream_t)stream;
-  if (M <= kTinyTokens && N <= kPanelTokens) {
+  // an expert is one tile; offsets in a row of the mask fit 32 bits
+  const bool one_column = NC == 1 && N <= kColumnExperts && (tile_rows == 0 || tile_rows >= MOMOE_RECOMPUTE_TILE_ROWS) &&
+                          stride_m >= 0 && stride_m < (1 << 20);
+  if (M <= (one_column ? kTinyFewExperts : kTinyTokens) && N <= kPanelTokens) {
     auto kernel = M <= 16 ? index_tiny_kernel<1> : M <= 32 ? index_tiny_kernel<2>
                 : M <= 48 ? index_tiny_kernel<3> : index_tiny_kernel<4>;
     const bool rows_of_int4 = stride_m == 1 && stride_n % 4 == 0 && M % 4 == 0 && ((uintptr_t)mask_NM & 15) == 0;
     kernel<<<1, kPanelTokens, 0, st>>>(mask_NM, stride_n, stride_m, (int)M, (int)N, (int)K, sizes_N,
                                        cumsums_N1, idx_Msum, which_Msum, inv_MK, tile_table,
                                        tile_rows, recompute_table, violations, rows_of_int4);
+    return launch_status();
+  }
+  if (one_column) {
+    // (left to choose, the height is 256: no expert has more rows)
+    index_column_kernel<<<NG, kPanelTokens, 0, st>>>(
+        mask_NM, stride_n, stride_m, (int)M, (int)N, (int)K, NG, sizes_N, cumsums_N1, idx_Msum, which_Msum, inv_MK, tile_table,
+        tile_rows != 0 ? tile_rows : MOMOE_RECOMPUTE_TILE_ROWS, recompute_table, violations);
     return launch_status();
   }
   dim3 grid(NC, NG);

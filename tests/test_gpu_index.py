@@ -171,6 +171,37 @@ def test_strided_mask_single_panel():
     _compare(mask, 3, out)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (49, 64, 4), (48, 64, 4), (49, 65, 4),        # the line to the kernel with one thread per expert
+    (256, 64, 8), (256, 65, 8), (257, 64, 8),     # the most tokens and experts
+    (256, 1, 1), (193, 15, 15), (65, 33, 3), (128, 8, 2),
+])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_one_panel_of_tokens(M, N, K, transposed):
+    from momoe_amd import _hip
+    mask, _ = make_routing(M, N, K, seed=M + N)
+    dev = mask.T.contiguous().to("cuda:0").T if transposed else mask.to("cuda:0")
+    _compare(mask, K, {k: v.cpu() for k, v in _hip.index_build(dev, K, recompute_table=True).items()})
+    out = _hip.index_build(dev, K, tile_rows=_hip.TILE_ROWS)  # a given height
+    _check_table(out["tile_table"].cpu().numpy(), oracle.index_build(mask), _hip.TILE_ROWS)
+    if N <= K:
+        return
+    short = mask.clone()  # the last token lacks an expert, the one before it has none
+    short[:, M - 2] = 0
+    short[int(torch.nonzero(short[:, M - 1])[0]), M - 1] = 0
+    out, o = _run(short, K), oracle.index_build(short)
+    total = M * K - K - 1
+    assert out["violations"].item() == 2 and int(o["cumsums_N"][-1]) == total
+    for k in ("sizes_N", "cumsums_N"):
+        assert np.array_equal(out[k].numpy(), o[k]), k
+    for k in ("idx_Msum", "which_Msum"):
+        assert np.array_equal(out[k].numpy()[:total], o[k]) and np.all(out[k].numpy()[total:] == 0), k
+    assert np.array_equal(out["inv_MK"].numpy(), o["inv_MK"])
+    out = _run(torch.ones(N, M, dtype=torch.int32), K)  # more pairs than rows
+    assert out["violations"].item() >= 1 and np.all(out["inv_MK"].numpy() == -1)
+    assert out["tile_table"][0].item() == 0 and out["recompute_table"][0].item() == 0
+
+
 def test_experts_without_tokens():
     mask = torch.zeros(8, 300, dtype=torch.int32)
     mask[1] = 1
