@@ -269,6 +269,11 @@ int momoe_gs_scatter(const float* gs_part, int64_t nparts, const int32_t* idx_Ms
                      const int32_t* cumsums_N1, float* Gs_NM,
                      int64_t M, int64_t N, int64_t Msum, void* stream);
 
+/* momoe_gs_scatter_tokens: the same as [M,N], element (expert i, token m) at Gs_MN[m * N + i]. */
+int momoe_gs_scatter_tokens(const float* gs_part, int64_t nparts, const int32_t* idx_Msum,
+                            const int32_t* cumsums_N1, float* Gs_MN, int64_t M, int64_t N,
+                            int64_t Msum, void* stream);
+
 /* momoe_dgrad_x replaces the GEMM of lin1_backward_kernel (momoe/momoe.py:662-681):
  *   gxs[r] = bf16( gz[r] @ Wl1[i]^T ), rows kept in sorted order; follow with
  *   momoe_combine to obtain G_x.  gz_blocked as written by the SwiGLU backward entry points.

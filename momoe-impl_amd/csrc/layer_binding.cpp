@@ -316,9 +316,16 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     }
     u.reset();
     if (need_s) {
-      out[4] = empty_f32({N, M}, dev);
-      MOMOE_CALL(momoe_gs_scatter, st, gs_part.data_ptr<float>(), nparts, ib.idx(), ib.cumsums(),
-                 out[4].data_ptr<float>(), M, N, msum);
+      // in the layout of s, where autograd keeps it without a copy
+      if (s.stride(0) == 1 && s.stride(1) == N) {
+        out[4] = empty_f32({M, N}, dev).t();
+        call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part.data_ptr<float>(), nparts,
+             (const int32_t*)ib.idx(), (const int32_t*)ib.cumsums(), out[4].data_ptr<float>(), M, N, msum);
+      } else {
+        out[4] = empty_f32({N, M}, dev);
+        MOMOE_CALL(momoe_gs_scatter, st, gs_part.data_ptr<float>(), nparts, ib.idx(), ib.cumsums(),
+                   out[4].data_ptr<float>(), M, N, msum);
+      }
     }
     gs_part.reset();
 

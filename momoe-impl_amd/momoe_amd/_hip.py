@@ -62,6 +62,7 @@ _SIGNATURES = {
     "momoe_swiglu_bwd_saved": (_int, [_p, _p, _p, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _p, _i64,
                                       _i64, _i64, _i64, _i64, _p]),
     "momoe_gs_scatter": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _p]),
+    "momoe_gs_scatter_tokens": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _p]),
     "momoe_dgrad_x": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "momoe_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "momoe_wgrad_stage_rows": (_int, [_i64, _i64, _i64, _i64, _int]),
@@ -316,6 +317,12 @@ def gs_scatter(gs_part, idx, cumsums, Gs_NM):
     N, M = Gs_NM.shape
     _call("momoe_gs_scatter", _ptr(gs_part), gs_part.shape[0], _ptr(idx), _ptr(cumsums),
                                  _ptr(Gs_NM), M, N, idx.numel(), _stream())
+
+
+def gs_scatter_tokens(gs_part, idx, cumsums, Gs_MN):
+    M, N = Gs_MN.shape
+    _call("momoe_gs_scatter_tokens", _ptr(gs_part), gs_part.shape[0], _ptr(idx), _ptr(cumsums),
+          _ptr(Gs_MN), M, N, idx.numel(), _stream())
 
 
 def dgrad_x(gz, Wl1_ND2H, table, gxs, M):

@@ -8,7 +8,7 @@ import oracle
 from gpu_util import (assert_close, device_layer_inputs, oracle_forward_for_tokens, rel_err,
                       run_device_layer, run_oracle_layer,
                       sampled_parity_on_device_inputs as _sampled_parity_on_device_inputs)
-from helpers import make_layer_inputs
+from helpers import make_layer_inputs, make_routing
 
 pytestmark = pytest.mark.gpu
 
@@ -718,6 +718,43 @@ def test_forward_mode_is_refused(grad):
             layer(dual, mask.to("cuda:0"), s.to("cuda:0"))
         with pytest.raises(RuntimeError):
             moe(dual)
+
+
+@pytest.mark.parametrize("M,N,K,nparts,skew", [
+    (1, 1, 1, 1, None), (63, 15, 4, 2, None), (64, 16, 4, 1, None), (65, 17, 17, 3, None),  # tiles of 64 x 16
+    (256, 1, 1, 1, None), (257, 2, 2, 1, None),    # 256 rows are read without probing
+    (2049, 8, 1, 2, 1.8), (70001, 20, 6, 8, 1.8),  # experts of up to all rows and of none, several probes
+])
+def test_gate_gradient_in_the_layout_of_the_router(M, N, K, nparts, skew):
+    """The same sums as momoe_gs_scatter, element for element, with the experts of a token next to each other."""
+    from momoe_amd import _hip
+    mask, _ = make_routing(M, N, K, seed=M, skew=skew)
+    if M > 2:
+        mask[:, 1] = 0  # a token without experts: the last rows are nobody's
+    ib = _hip.index_build(mask.to("cuda:0"), K)
+    part = torch.randn(nparts, M * K, device="cuda:0")
+    want = torch.full((N, M), 7.0, device="cuda:0")
+    got = torch.full((M, N), 7.0, device="cuda:0")
+    _hip.gs_scatter(part, ib["idx_Msum"], ib["cumsums_N"], want)
+    _hip.gs_scatter_tokens(part, ib["idx_Msum"], ib["cumsums_N"], got)
+    assert torch.equal(got.T, want)
+    # more pairs than rows: nothing but zeros
+    ib = _hip.index_build(torch.ones(N + 1, M, dtype=torch.int32, device="cuda:0"), N)
+    got = torch.full((M, N + 1), 7.0, device="cuda:0")
+    _hip.gs_scatter_tokens(torch.randn(1, M * N, device="cuda:0"), ib["idx_Msum"], ib["cumsums_N"], got)
+    assert not got.any()
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_gate_gradient_has_the_layout_of_the_gate_weights(transposed):
+    x, W1, W2, mask, s, dy = make_layer_inputs(70, 64, 32, 9, 3, seed=4)
+    want = run_device_layer(x, W1, W2, mask, s, dy, 3, 0)["G_s"]
+    import momoe_amd
+    layer = momoe_amd.MoMoE(64, 32, 9, 3, save_percent=0, Wl1_ND2H=W1.to("cuda:0"), Wl2_NHD=W2.to("cuda:0"))
+    s_dev = (s.T.contiguous().to("cuda:0").T if transposed else s.contiguous().to("cuda:0")).requires_grad_()
+    y, _ = layer(x.to("cuda:0", torch.bfloat16)[None], mask.to("cuda:0"), s_dev)
+    y.backward(dy.to("cuda:0", torch.bfloat16)[None])
+    assert s_dev.grad.stride() == s_dev.stride() and torch.equal(s_dev.grad.cpu(), want)
 
 
 @pytest.mark.parametrize("M,D,H,N,K,sp", [
