@@ -354,6 +354,15 @@ int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t gs_stride_
                      const int32_t* mask_NM, int64_t M, int64_t N, int64_t Ks,
                      void* Glogits_MN, void* stream);
 
+/* momoe_gate_wgrad: gradient of the gate weights (in TopKRouterFunction, momoe/topk_router.py:83-145), GWg_DN[d,n] = sum over the tokens of
+ * x_MD[m,d] * Glogits_MN[m,n], bf16 from fp32 sums.  x_MD bf16 with row pitch ldx elements, Glogits_MN bf16 contiguous.
+ * D, N and ldx multiples of 8; x_MD, Glogits_MN and workspace on 16-byte boundaries.
+ * workspace: momoe_gate_wgrad_workspace_bytes(M, D, N) bytes of device memory (-1: sizes that it does not take).
+ */
+int64_t momoe_gate_wgrad_workspace_bytes(int64_t M, int64_t D, int64_t N);
+int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogits_MN, void* GWg_DN,
+                     int64_t M, int64_t D, int64_t N, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* momoe_bias_update (momoe/sample_moe.py:65-67): biases_N[i] += rate * sign(c_avg - sizes_N[i]) in
  * place, fp32; -inf (a shared expert) stays -inf.
  */

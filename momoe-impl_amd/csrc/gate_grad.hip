@@ -1,0 +1,179 @@
+// Gradient of the router's gate weights: G_Wg [D,N] = x^T . G_logits, a contraction over the tokens with few columns.
+//
+// Bound by memory: x is read once for every 128 experts, and that is nearly all there is.  The product has few tiles and a
+// long contraction, so the tokens are split: a workgroup takes 128 columns of x, 128 experts and a range of tokens, and a
+// second launch adds up the fp32 partial products of the ranges.  As many ranges as give every CU a workgroup, of at least 256
+// tokens.  Both launches in a graph, us, with half as many ranges | as they are | twice as many, and the library's product:
+// 8192 tokens, D = 2048, N = 128 25.9 | 20.5 | 25.1, 59.3; 16384, 2048, 64 36.8 | 25.0 | 25.4, 89.9; 32768, 512, 16 22.2 | 18.7 |
+// 21.6, 72.4; 7680, 2176, 64 23.5 | 17.1 | 19.8, 44.8.
+#include <algorithm>
+
+#include "gemm_tile.hpp"
+
+namespace momoe {
+namespace {
+
+constexpr int kTile = 128;           // columns of x, and experts, of a workgroup
+constexpr int kStageRows = 64;       // tokens of a stage
+constexpr int kPitch = kTile + 16;   // elements of a row in LDS: the 4 rows of 16 lanes of a transposing read lie in different banks
+constexpr int kGateThreads = 256;    // 4 wavefronts, 2 x 2, each 64 x 64 of the tile in 4 x 4 accumulators
+constexpr int kPieces = kStageRows * kTile / 8 / kGateThreads;  // 16-byte pieces of an operand's stage per thread
+
+struct GateArgs {
+  const bf16* x;
+  int64_t ldx;
+  const bf16* g;
+  float* part;  // [ranges][D][N]
+  int M, D, N, rows;  // rows: tokens of a range, a multiple of kStageRows
+};
+
+// A thread's pieces of a stage of `cols` columns from `base` (row pitch ld); what does not exist is zero.  Loads are
+// unconditional, rows and columns clamped: under a branch each would be waited for before the next.
+struct StagePieces {
+  bf16x8 v[kPieces];
+  __device__ __forceinline__ void load(const bf16* base, int64_t ld, int cols, int row0, int end) {
+    const int col = (threadIdx.x % (kTile / 8)) * 8;
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q) {
+      const int row = row0 + (int)threadIdx.x / (kTile / 8) + q * (kGateThreads / (kTile / 8));
+      const bf16x8 w = *(const bf16x8*)(base + (int64_t)min(row, end - 1) * ld + min(col, cols - 8));
+      v[q] = row < end && col < cols ? w : bf16x8{};
+    }
+  }
+  __device__ __forceinline__ void put(bf16* lds) const {
+    const int col = (threadIdx.x % (kTile / 8)) * 8;
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q)
+      *(bf16x8*)(lds + ((int)threadIdx.x / (kTile / 8) + q * (kGateThreads / (kTile / 8))) * kPitch + col) = v[q];
+  }
+};
+
+// 16 columns from `col` of k-values 32 h .. +31 of a stage, as a fragment of v_mfma_f32_16x16x32_bf16
+__device__ __forceinline__ bf16x8 stage_frag(const bf16* lds, int col, int h) {
+  const int l = threadIdx.x & 63;
+  const bf16* p = lds + (32 * h + 8 * (l >> 4) + ((l & 15) >> 2)) * kPitch + col + 4 * (l & 3);
+  const bf16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + 4 * kPitch);
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+__global__ __launch_bounds__(kGateThreads, 2) void gate_wgrad_kernel(GateArgs p) {
+  __shared__ __attribute__((aligned(16))) bf16 sx[kStageRows * kPitch], sg[kStageRows * kPitch];
+  const int d0 = blockIdx.x * kTile, n0 = blockIdx.y * kTile;
+  const int begin = blockIdx.z * p.rows, end = min(p.M, begin + p.rows);
+  const int w = wave_id(), d_org = 64 * (w >> 1), n_org = 64 * (w & 1), l = threadIdx.x & 63;
+  const bool some = n0 + n_org < p.N && d0 + d_org < p.D;  // wave-uniform
+  const bf16 *x = p.x + d0, *g = p.g + n0;
+  const int xcols = min(kTile, p.D - d0), gcols = min(kTile, p.N - n0);
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // two stages are on their way while one is multiplied
+  StagePieces px[2], pg[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    px[s].load(x, p.ldx, xcols, begin + s * kStageRows, end);
+    pg[s].load(g, p.N, gcols, begin + s * kStageRows, end);
+  }
+  for (int row = begin; row < end; row += 2 * kStageRows)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int at = row + s * kStageRows;
+      if (at >= end) break;  // uniform
+      px[s].put(sx);
+      pg[s].put(sg);
+      px[s].load(x, p.ldx, xcols, at + 2 * kStageRows, end);
+      pg[s].load(g, p.N, gcols, at + 2 * kStageRows, end);
+      __syncthreads();
+      if (some) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          bf16x8 xf[4], gf[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xf[i] = stage_frag(sx, d_org + 16 * i, h), gf[i] = stage_frag(sg, n_org + 16 * i, h);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gf[j], xf[i], acc[j][i], 0, 0, 0);
+        }
+      }
+      __syncthreads();
+    }
+  if (!some) return;
+  // a lane holds, for one column of x (lane % 16), experts 4 * (lane / 16) .. +3
+  float* const out = p.part + (int64_t)blockIdx.z * p.D * p.N;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int d = d0 + d_org + 16 * i + (l & 15);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + n_org + 16 * j + 4 * (l >> 4);
+      if (d < p.D && n < p.N) *(f32x4*)(out + (int64_t)d * p.N + n) = acc[j][i];
+    }
+  }
+}
+
+// out = sum of the ranges' products, four elements a thread
+__global__ __launch_bounds__(kGateThreads) void gate_wgrad_reduce_kernel(const float* __restrict__ part, int ranges, int64_t quads,
+                                                                        bf16* __restrict__ out) {
+  constexpr int AT_ONCE = 8;
+  const int64_t q = (int64_t)blockIdx.x * kGateThreads + threadIdx.x;
+  if (q >= quads) return;
+  const f32x4* const p = (const f32x4*)part + q;
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int r0 = 0; r0 < ranges; r0 += AT_ONCE) {
+    f32x4 v[AT_ONCE];
+#pragma unroll
+    for (int r = 0; r < AT_ONCE; ++r) v[r] = p[min(r0 + r, ranges - 1) * quads];
+#pragma unroll
+    for (int r = 0; r < AT_ONCE; ++r)
+      if (r0 + r < ranges) sum += v[r];
+  }
+  ((bf16x4*)out)[q] = bf16x4{(bf16)sum[0], (bf16)sum[1], (bf16)sum[2], (bf16)sum[3]};
+}
+
+struct GateSplit {
+  int64_t rows, ranges;
+  GateSplit(int64_t M, int64_t D, int64_t N) {
+    const int64_t tiles = cdiv64(D, kTile) * cdiv64(N, kTile);
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(256 / tiles, cdiv64(M, 4 * kStageRows)));
+    rows = cdiv64(cdiv64(M, want), kStageRows) * kStageRows;
+    ranges = cdiv64(M, rows);
+  }
+};
+
+bool gate_sizes_ok(int64_t M, int64_t D, int64_t N) {
+  return D % 8 == 0 && N % 8 == 0 && D <= (1 << 20) && N <= 4096 && M < (1ll << 31) - 4 * kStageRows && D * N < (1ll << 31);
+}
+
+}  // namespace
+}  // namespace momoe
+
+using namespace momoe;
+
+extern "C" int64_t momoe_gate_wgrad_workspace_bytes(int64_t M, int64_t D, int64_t N) {
+  if (M <= 0 || D <= 0 || N <= 0 || !gate_sizes_ok(M, D, N)) return -1;
+  return GateSplit(M, D, N).ranges * D * N * (int64_t)sizeof(float);
+}
+
+extern "C" int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogits_MN, void* GWg_DN, int64_t M, int64_t D,
+                                int64_t N, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!x_MD || !Glogits_MN || !GWg_DN || !workspace) return MOMOE_ERR_BAD_ARG;
+  if (M <= 0 || D <= 0 || N <= 0 || ldx < D) return MOMOE_ERR_BAD_ARG;
+  if (!gate_sizes_ok(M, D, N) || ldx % 8 != 0) return MOMOE_ERR_UNSUPPORTED;
+  if (((uintptr_t)x_MD & 15) || ((uintptr_t)Glogits_MN & 15) || ((uintptr_t)GWg_DN & 7) || ((uintptr_t)workspace & 15))
+    return MOMOE_ERR_BAD_ARG;
+  const GateSplit split(M, D, N);
+  if (workspace_bytes < split.ranges * D * N * (int64_t)sizeof(float)) return MOMOE_ERR_BAD_ARG;
+  hipStream_t st = (hipStream_t)stream;
+  const GateArgs a{(const bf16*)x_MD, ldx, (const bf16*)Glogits_MN, (float*)workspace, (int)M, (int)D, (int)N, (int)split.rows};
+  const dim3 grid((unsigned)cdiv64(D, kTile), (unsigned)cdiv64(N, kTile), (unsigned)split.ranges);
+  gate_wgrad_kernel<<<grid, kGateThreads, 0, st>>>(a);
+  const int status = launch_status();
+  if (status != MOMOE_OK) return status;
+  const int64_t quads = D * N / 4;
+  gate_wgrad_reduce_kernel<<<(unsigned)cdiv64(quads, kGateThreads), kGateThreads, 0, st>>>((const float*)workspace, (int)split.ranges,
+                                                                                         quads, (bf16*)GWg_DN);
+  return launch_status();
+}

@@ -420,6 +420,21 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
   return r;
 }
 
+// x^T . G_logits [D, N].  The library's product has few tiles and one long contraction for each: below some 1500 tokens it takes as
+// long as the two launches of the kernel (1024 tokens, D = 1024, N = 32 9.3 us against 8.9; 1300 8.6, 9.0), from there on two
+// to four times as long (2000, 1120, 48 19.6 against 9.4; 8192, 2048, 128 59 against 20.6).  Also where autograd records it.
+Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
+  constexpr int64_t kFewTokens = 1536;
+  const int64_t M = x.size(0), D = x.size(1), N = G_logit.size(1);
+  const int64_t bytes = momoe_gate_wgrad_workspace_bytes(M, D, N);
+  const bool rows = x.stride(1) == 1 && x.stride(0) >= D && x.stride(0) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
+  if (M < kFewTokens || bytes < 0 || !rows || at::GradMode::is_enabled()) return at::mm(x.t(), G_logit);
+  const Tensor out = empty_bf16({D, N}, x.device()), ws = empty_f32({bytes / 4}, x.device());
+  MOMOE_CALL(momoe_gate_wgrad, stream_of(x.device()), x.data_ptr(), x.stride(0), G_logit.data_ptr(), out.data_ptr(), M, D, N,
+             ws.data_ptr(), bytes);
+  return out;
+}
+
 struct RouterFn : torch::autograd::Function<RouterFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& Wg, const Tensor& biases,
                                int64_t N, int64_t K, int64_t Ks) {
@@ -458,7 +473,7 @@ struct RouterFn : torch::autograd::Function<RouterFn> {
                  p_sel.data_ptr<float>(), s_MN.data_ptr<float>(), nrm, nrm + M, mask.data_ptr<int32_t>(), M, N,
                  ctx->saved_data["Ks"].toInt(), G_logit.data_ptr());
       if (need_x) G_x = G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
-      if (need_wg) out[1] = at::mm(x.t(), G_logit);
+      if (need_wg) out[1] = gate_gradient(x, G_logit);
     } else if (need_wg) {
       out[1] = at::zeros_like(Wg);
     }

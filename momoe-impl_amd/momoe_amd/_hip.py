@@ -71,6 +71,8 @@ _SIGNATURES = {
                            _i64, _p, _i64, _p]),
     "momoe_router_fwd": (_int, [_p, _int, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]),
     "momoe_router_bwd": (_int, [_p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "momoe_gate_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "momoe_gate_wgrad": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
     "momoe_bias_update": (_int, [_p, ctypes.c_float, ctypes.c_float, _i64, _p, _p]),
 }
 
@@ -382,3 +384,13 @@ def router_bwd(Gs_NM, p_sel_MN, s_MN, Ng_M, Ks_M, mask_NM, Ks):
                                  _ptr(s_MN), _ptr(Ng_M), _ptr(Ks_M), _ptr(mask_NM), M, N, Ks,
                                  _ptr(out), _stream())
     return out
+
+
+def gate_wgrad(x_MD, Glogits_MN, GWg_DN):
+    _need_cuda(x_MD, Glogits_MN, GWg_DN)
+    (M, D), N = x_MD.shape, Glogits_MN.shape[1]
+    assert Glogits_MN.is_contiguous() and GWg_DN.is_contiguous() and x_MD.stride(1) == 1
+    nbytes = _lib.momoe_gate_wgrad_workspace_bytes(M, D, N)
+    ws = torch.empty(max(nbytes, 0), dtype=torch.uint8, device=x_MD.device)
+    _call("momoe_gate_wgrad", _ptr(x_MD), x_MD.stride(0), _ptr(Glogits_MN), _ptr(GWg_DN), M, D, N, _ptr(ws), nbytes,
+          _stream())

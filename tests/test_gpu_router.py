@@ -219,3 +219,44 @@ def test_training_smoke_at_the_reference_size():
     # the routed experts' selection bias moved by at most 210 steps of the update rate
     b = moe.biases_N[:N - Ks]
     assert torch.all(b.abs() <= 210 * 1e-4 + 1e-6) and torch.all(torch.isinf(moe.biases_N[N - Ks:]))
+
+
+@pytest.mark.parametrize("M,D,N", [
+    (1, 8, 8), (64, 128, 128), (65, 136, 136), (255, 120, 16),   # tiles of 128 x 128, stages of 64 tokens
+    (256, 128, 8), (257, 256, 64), (1537, 40, 24), (8200, 2048, 128),  # one range of tokens and several, the last a part
+])
+def test_gate_weight_gradient(M, D, N):
+    from momoe_amd import _hip
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    wide = torch.randn(M, D + 8, generator=g, device="cuda:0").to(torch.bfloat16)
+    gl = torch.randn(M, N, generator=g, device="cuda:0").to(torch.bfloat16)
+    for x in (wide[:, :D].contiguous(), wide[:, :D]):
+        got = torch.full((D, N), 7.0, device="cuda:0", dtype=torch.bfloat16)
+        _hip.gate_wgrad(x, gl, got)
+        xd, gd = x.double(), gl.double()
+        ref, size = xd.T.contiguous() @ gd, xd.abs().T.contiguous() @ gd.abs()
+        # bf16 rounding of the result, and M fp32 additions of products of that size
+        assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + M * 2.0 ** -24 * size).all()
+    # an infinite token stays in its own column of x
+    x = wide[:, :D].contiguous()
+    x[M - 1, 3] = float("inf")
+    _hip.gate_wgrad(x, gl.abs() + 1, got)
+    assert torch.isinf(got[3]).all() and torch.isfinite(torch.cat([got[:3], got[4:]])).all()
+
+
+@pytest.mark.parametrize("M,D,N", [(1535, 64, 16), (1536, 64, 16), (2000, 72, 20), (1600, 96, 24)])
+@pytest.mark.parametrize("pitch", [0, 4, 8])
+def test_gate_weight_gradient_of_the_module(M, D, N, pitch):
+    """Whichever product the module takes, by the tokens, the widths and the layout of x, the gradient is that of
+    the library's, which a backward that is itself recorded takes."""
+    import momoe_amd
+    g = torch.Generator(device="cuda:0").manual_seed(D)
+    r = momoe_amd.TopKRouter(D, N, 4, 0, Wg_DN=torch.randn(D, N, generator=g, device="cuda:0").to(torch.bfloat16) / 8)
+    x = torch.randn(1, M, D + pitch, generator=g, device="cuda:0").to(torch.bfloat16)[..., :D]
+    w = torch.randn(N, M, generator=g, device="cuda:0")
+    grads = []
+    for recorded in (False, True):
+        loss = (r(x, torch.zeros(N, device="cuda:0"))[2] * w).sum()
+        grads.append(torch.autograd.grad(loss, r.Wg_DN, create_graph=recorded)[0].detach().double())
+    assert grads[0].shape == (D, N)
+    assert (grads[0] - grads[1]).abs().max() <= 2.0 ** -7 * grads[1].abs().max()
