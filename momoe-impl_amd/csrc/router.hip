@@ -4,6 +4,8 @@
 // j, j+64, ...), a workgroup per block of consecutive tokens so that the [N, M]
 // tensors (mask, dL/ds) are touched in whole lines.  HBM-bound: a few passes over
 // [M, N] fp32.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace momoe {
@@ -11,15 +13,29 @@ namespace {
 
 constexpr int kMaxCols = 8;  // columns per lane -> N <= 512
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
+// op over the wavefront, in every lane: lanes meet those 32, 16, 8, 4, 2 and 1 apart, by exchanges of the vector unit (through
+// LDS a step is several times as long, and a token has four such chains).  Four apart: eight lanes apart hold the
+// same by then, so the lane four further on in a row of 16 will do.  In us, through LDS -> this: forward 7.4 -> 7.1 (16
+// tokens x 128 experts), backward 7.0 -> 5.8 (1000 x 128), 7.7 -> 6.4 (8192 x 128), 18.5 -> 15.5 (32768 x 96).
+template <class Op>
+__device__ __forceinline__ float wave_all(float v, Op op) {
+  const auto swap = [&](auto pair) { return op(__uint_as_float(pair[0]), __uint_as_float(pair[1])); };
+  v = swap(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  v = swap(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+  const auto lanes = [](auto ctrl, float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v = op(v, lanes(std::integral_constant<int, 0x128>{}, v));  // row_ror:8
+  v = op(v, lanes(std::integral_constant<int, 0x124>{}, v));  // row_ror:4
+  v = op(v, lanes(std::integral_constant<int, 0x4E>{}, v));   // quad_perm: lane ^ 2
+  v = op(v, lanes(std::integral_constant<int, 0xB1>{}, v));   // quad_perm: lane ^ 1
   return v;
 }
+__device__ __forceinline__ float wave_max(float v) {
+  return wave_all(v, [](float a, float b) { return fmaxf(a, b); });
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
-  return v;
+  return wave_all(v, [](float a, float b) { return a + b; });
 }
 
 // The maximum over the wavefront, in every lane, without LDS traffic: lanes exchange within quads
@@ -52,27 +68,30 @@ struct RouterFwdArgs {
   float* ks;
 };
 
-// A workgroup of 16 wavefronts handles kTok consecutive tokens.  The mask is [N, M] (token fastest)
+// A workgroup handles kTok consecutive tokens.  The mask is [N, M] (token fastest)
 // while everything else is per token: the 0/1 flags of the tokens go through LDS and leave as
 // rows of kTok x 4 bytes (written per token they would be N scattered 4-byte stores each).  With
 // 32 tokens, two per wavefront, these are whole 128-byte lines; up to kRouterOneEach tokens, where
 // 16-token workgroups still find a CU each, a wavefront takes one token and the second one's
-// latency is saved.
+// latency is saved.  Up to kRouterSpread tokens a workgroup is four wavefronts with a token each: the vector instructions of
+// the rounds count then, and 16 tokens keep one CU busy where four could share them.  In us, 16 tokens a workgroup -> 4:
+// 16 tokens x 128 experts, K = 8 7.1 -> 5.1, 1000 x 128 7.6 -> 5.8, 2048 x 128 7.8 -> 6.6, 3000 x 64, K = 4 5.0 -> 4.7,
+// 4096 x 64, K = 6 5.0 -> 5.5.
 constexpr int kRouterThreads = 1024;
-constexpr int64_t kRouterOneEach = 256 * 16;
+constexpr int64_t kRouterOneEach = 256 * 16, kRouterSpread = 3072;
 
 // NC = columns held per lane (1, 2, 4 or 8): N <= 64 * NC
-template <int NC, int kTok>
-__global__ __launch_bounds__(kRouterThreads) void router_fwd_kernel(RouterFwdArgs p) {
+template <int NC, int kTok, int THREADS = kRouterThreads>
+__global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
   __shared__ uint8_t flags[64 * NC][kTok];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int N = p.N, Ng = p.N - p.Ks, Kg = p.K - p.Ks;
   const int ncol = (N + 63) >> 6;
   const int m0 = blockIdx.x * kTok;
-  for (int tt = wave; tt < kTok; tt += kRouterThreads / 64) {
+  for (int tt = wave; tt < kTok; tt += THREADS / 64) {
     const int m = m0 + tt;
     if (m >= p.M) break;  // wave-uniform
-    float v[NC], pr[NC], score[NC];
+    float v[NC], pr[NC], score[NC], bias[NC];
     bool sel[NC];
     float mg = -INFINITY, ms = -INFINITY;
     // unconditional loads (column clamped, result masked): loads under a branch would be
@@ -82,6 +101,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_fwd_kernel(RouterFwdArg
       const int jc = min(lane + 64 * min(c, ncol - 1), N - 1);
       v[c] = p.logits_f32 ? ((const float*)p.logits)[(int64_t)m * N + jc]
                           : (float)((const bf16*)p.logits)[(int64_t)m * N + jc];
+      bias[c] = p.bias[jc];
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -113,7 +133,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_fwd_kernel(RouterFwdArg
       score[c] = -INFINITY;
       if (c < ncol && j < N) {
         pr[c] = pr[c] / (j < Ng ? sg : ss);
-        if (j < Ng) score[c] = pr[c] + p.bias[j];
+        if (j < Ng) score[c] = pr[c] + bias[c];
       }
     }
     // top-Kg of score over the routed columns; ties go to the lower column.  A round is bound by
@@ -168,7 +188,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_fwd_kernel(RouterFwdArg
   // mask rows: 32 tokens x 4 bytes per expert
   const int tt = threadIdx.x & (kTok - 1);
   if (m0 + tt < p.M)
-    for (int j = threadIdx.x / kTok; j < N; j += kRouterThreads / kTok)
+    for (int j = threadIdx.x / kTok; j < N; j += THREADS / kTok)
       p.mask[(int64_t)j * p.M + m0 + tt] = flags[j][tt];
 }
 
@@ -292,13 +312,18 @@ extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const flo
   if (N > 64 * kMaxCols || M >= (1ll << 31) - 4) return MOMOE_ERR_UNSUPPORTED;
   RouterFwdArgs a{logits_MN, logits_f32, biases_N, (int)M, (int)N, (int)K, (int)Ks,
                   mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M};
+  hipStream_t st = (hipStream_t)stream;
+  auto by_width = [&](auto one, auto two, auto four, auto eight) { return N <= 64 ? one : N <= 128 ? two : N <= 256 ? four : eight; };
+  if (M <= kRouterSpread) {
+    auto kernel = by_width(router_fwd_kernel<1, 4, 256>, router_fwd_kernel<2, 4, 256>, router_fwd_kernel<4, 4, 256>,
+                           router_fwd_kernel<8, 4, 256>);
+    kernel<<<(unsigned)cdiv64(M, 4), 256, 0, st>>>(a);
+    return launch_status();
+  }
   const bool few = M <= kRouterOneEach;
-  const unsigned grid = (unsigned)cdiv64(M, few ? 16 : 32);
-  auto kernel = N <= 64  ? (few ? router_fwd_kernel<1, 16> : router_fwd_kernel<1, 32>)
-              : N <= 128 ? (few ? router_fwd_kernel<2, 16> : router_fwd_kernel<2, 32>)
-              : N <= 256 ? (few ? router_fwd_kernel<4, 16> : router_fwd_kernel<4, 32>)
-                         : (few ? router_fwd_kernel<8, 16> : router_fwd_kernel<8, 32>);
-  kernel<<<grid, kRouterThreads, 0, (hipStream_t)stream>>>(a);
+  auto kernel = few ? by_width(router_fwd_kernel<1, 16>, router_fwd_kernel<2, 16>, router_fwd_kernel<4, 16>, router_fwd_kernel<8, 16>)
+                    : by_width(router_fwd_kernel<1, 32>, router_fwd_kernel<2, 32>, router_fwd_kernel<4, 32>, router_fwd_kernel<8, 32>);
+  kernel<<<(unsigned)cdiv64(M, few ? 16 : 32), kRouterThreads, 0, st>>>(a);
   return launch_status();
 }
 

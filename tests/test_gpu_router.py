@@ -20,6 +20,8 @@ def _logits(M, N, seed):
     (4097, 130, 6, 2, True),    # one more: two per wavefront, a last block of one token
     (17, 512, 8, 1, True),      # the most experts, a last block of one token
     (64, 8, 8, 0, True),        # every expert is chosen
+    (1, 1, 1, 0, True), (3, 65, 4, 1, True), (5, 129, 4, 0, True), (7, 257, 5, 2, True),  # blocks of four tokens, a part of one
+    (3072, 64, 4, 0, True), (3073, 64, 4, 0, True),  # the most tokens in blocks of four, one more
 ])
 def test_router_forward(M, N, K, Ks, f32):
     from momoe_amd import _hip
