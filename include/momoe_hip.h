@@ -345,6 +345,18 @@ int momoe_router_fwd(const void* logits_MN, int logits_f32, const float* biases_
                      int32_t* mask_NM, float* s_MN, float* p_sel_MN, float* Ng_M, float* Ks_M,
                      void* stream);
 
+/* momoe_gate_router_fwd: momoe_router_fwd of the logits x_MD . Wg_DN (fp32 sums, rounded to bf16), for few tokens.
+ * x_MD bf16 with row pitch ldx elements, Wg_DN bf16 contiguous; D, N and ldx multiples of 8; x_MD, Wg_DN and workspace on
+ * 16-byte boundaries.
+ * workspace: momoe_gate_router_workspace_bytes(M, D, N) bytes of device memory (-1: sizes that it does not take, among them
+ * more tokens than a product that is not split over the contraction handles as fast).
+ */
+int64_t momoe_gate_router_workspace_bytes(int64_t M, int64_t D, int64_t N);
+int momoe_gate_router_fwd(const void* x_MD, int64_t ldx, const void* Wg_DN, const float* biases_N,
+                          int64_t M, int64_t D, int64_t N, int64_t K, int64_t Ks,
+                          int32_t* mask_NM, float* s_MN, float* p_sel_MN, float* Ng_M, float* Ks_M,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
 /* momoe_router_bwd replaces normalize_backward_kernel (momoe/topk_router.py:11-56):
  * gradient w.r.t. the gate logits, bf16 [M,N] row-major.  Gs_NM fp32, element (i,m) at
  * Gs[i*gs_stride_n + m*gs_stride_m]; it is not modified.

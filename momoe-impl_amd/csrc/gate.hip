@@ -8,16 +8,13 @@
 // 21.6, 72.4; 7680, 2176, 64 23.5 | 17.1 | 19.8, 44.8.
 #include <algorithm>
 
-#include "gemm_tile.hpp"
+#include "gate.hpp"
 
 namespace momoe {
 namespace {
 
-constexpr int kTile = 128;           // columns of x, and experts, of a workgroup
-constexpr int kStageRows = 64;       // tokens of a stage
-constexpr int kPitch = kTile + 16;   // elements of a row in LDS: the 4 rows of 16 lanes of a transposing read lie in different banks
-constexpr int kGateThreads = 256;    // 4 wavefronts, 2 x 2, each 64 x 64 of the tile in 4 x 4 accumulators
-constexpr int kPieces = kStageRows * kTile / 8 / kGateThreads;  // 16-byte pieces of an operand's stage per thread
+constexpr int kGateThreads = GateStage::THREADS, kTile = GateStage::COLS, kStageRows = GateStage::ROWS;
+// 4 wavefronts, 2 x 2, each 64 x 64 of the tile in 4 x 4 accumulators
 
 struct GateArgs {
   const bf16* x;
@@ -27,37 +24,8 @@ struct GateArgs {
   int M, D, N, rows;  // rows: tokens of a range, a multiple of kStageRows
 };
 
-// A thread's pieces of a stage of `cols` columns from `base` (row pitch ld); what does not exist is zero.  Loads are
-// unconditional, rows and columns clamped: under a branch each would be waited for before the next.
-struct StagePieces {
-  bf16x8 v[kPieces];
-  __device__ __forceinline__ void load(const bf16* base, int64_t ld, int cols, int row0, int end) {
-    const int col = (threadIdx.x % (kTile / 8)) * 8;
-#pragma unroll
-    for (int q = 0; q < kPieces; ++q) {
-      const int row = row0 + (int)threadIdx.x / (kTile / 8) + q * (kGateThreads / (kTile / 8));
-      const bf16x8 w = *(const bf16x8*)(base + (int64_t)min(row, end - 1) * ld + min(col, cols - 8));
-      v[q] = row < end && col < cols ? w : bf16x8{};
-    }
-  }
-  __device__ __forceinline__ void put(bf16* lds) const {
-    const int col = (threadIdx.x % (kTile / 8)) * 8;
-#pragma unroll
-    for (int q = 0; q < kPieces; ++q)
-      *(bf16x8*)(lds + ((int)threadIdx.x / (kTile / 8) + q * (kGateThreads / (kTile / 8))) * kPitch + col) = v[q];
-  }
-};
-
-// 16 columns from `col` of k-values 32 h .. +31 of a stage, as a fragment of v_mfma_f32_16x16x32_bf16
-__device__ __forceinline__ bf16x8 stage_frag(const bf16* lds, int col, int h) {
-  const int l = threadIdx.x & 63;
-  const bf16* p = lds + (32 * h + 8 * (l >> 4) + ((l & 15) >> 2)) * kPitch + col + 4 * (l & 3);
-  const bf16x4 lo = lds_read_tr4(p), hi = lds_read_tr4(p + 4 * kPitch);
-  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
 __global__ __launch_bounds__(kGateThreads, 2) void gate_wgrad_kernel(GateArgs p) {
-  __shared__ __attribute__((aligned(16))) bf16 sx[kStageRows * kPitch], sg[kStageRows * kPitch];
+  __shared__ __attribute__((aligned(16))) bf16 sx[GateStage::ELEMS], sg[GateStage::ELEMS];
   const int d0 = blockIdx.x * kTile, n0 = blockIdx.y * kTile;
   const int begin = blockIdx.z * p.rows, end = min(p.M, begin + p.rows);
   const int w = wave_id(), d_org = 64 * (w >> 1), n_org = 64 * (w & 1), l = threadIdx.x & 63;
@@ -70,7 +38,7 @@ __global__ __launch_bounds__(kGateThreads, 2) void gate_wgrad_kernel(GateArgs p)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   // two stages are on their way while one is multiplied
-  StagePieces px[2], pg[2];
+  GateStage px[2], pg[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     px[s].load(x, p.ldx, xcols, begin + s * kStageRows, end);
@@ -91,7 +59,7 @@ __global__ __launch_bounds__(kGateThreads, 2) void gate_wgrad_kernel(GateArgs p)
         for (int h = 0; h < 2; ++h) {
           bf16x8 xf[4], gf[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) xf[i] = stage_frag(sx, d_org + 16 * i, h), gf[i] = stage_frag(sg, n_org + 16 * i, h);
+          for (int i = 0; i < 4; ++i) xf[i] = GateStage::frag(sx, d_org + 16 * i, h), gf[i] = GateStage::frag(sg, n_org + 16 * i, h);
 #pragma unroll
           for (int j = 0; j < 4; ++j)
 #pragma unroll

@@ -8,6 +8,7 @@
 // Nothing here synchronises with the device (unless the caller asks for the routing check): every
 // launch is sized from static upper bounds and the routing-dependent tile list lives in device
 // memory.
+#include <ATen/autocast_mode.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -402,33 +403,44 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
   const c10::DeviceGuard guard(dev);
   Routed r;
   r.x_MD = x_BSD.reshape({M, D}).to(dev, at::kBFloat16);
-  // autocast may give the product another type than its operands'; the kernel reads two of them
-  const Tensor logits = at::mm(r.x_MD, Wg).contiguous();
-  if (logits.scalar_type() != at::kBFloat16 && logits.scalar_type() != at::kFloat)
-    throw_python(PyExc_AssertionError, std::string("the gate logits must be bfloat16 or float32, got ") +
-                                           c10::toString(logits.scalar_type()));
-  TORCH_CHECK(logits.size(1) == N, "Wg_DN must have N = ", N, " columns");
   const Tensor bias = biases.to(dev, at::kFloat).contiguous();
   TORCH_CHECK(bias.numel() == N, "biases_N must have N = ", N, " elements");
+  TORCH_CHECK(r.x_MD.size(1) == Wg.size(0) && Wg.size(1) == N, "Wg_DN must be [", D, ", N = ", N, "]");
   r.mask = at::empty({N, M}, at::TensorOptions().dtype(at::kInt).device(dev));
   r.s_MN = empty_f32({M, N}, dev);
   r.p_sel = empty_f32({M, N}, dev);
   r.norms = empty_f32({2, M}, dev);  // per token: sum over the selected, over the shared experts
   float* norms = r.norms.data_ptr<float>();
-  MOMOE_CALL(momoe_router_fwd, stream_of(dev), logits.data_ptr(), logits.scalar_type() == at::kFloat, bias.data_ptr<float>(), M, N, K, Ks,
+  const hipStream_t st = stream_of(dev);
+  // Few tokens: the product in the library's kernel, whose launch alone takes the host 18 us
+  const int64_t ws_bytes = momoe_gate_router_workspace_bytes(M, D, N);
+  const auto aligned = [](const Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  if (ws_bytes >= 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && Wg.is_contiguous() && aligned(Wg) && aligned(r.x_MD) &&
+      r.x_MD.stride(1) == 1 && r.x_MD.stride(0) >= D && r.x_MD.stride(0) % 8 == 0) {
+    const Tensor ws = empty_f32({ws_bytes / 4}, dev);
+    MOMOE_CALL(momoe_gate_router_fwd, st, r.x_MD.data_ptr(), r.x_MD.stride(0), Wg.data_ptr(), bias.data_ptr<float>(), M, D, N, K,
+               Ks, r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M,
+               ws.data_ptr(), ws_bytes);
+    return r;
+  }
+  // autocast may give the product another type than its operands'; the kernel reads two of them
+  const Tensor logits = at::mm(r.x_MD, Wg).contiguous();
+  if (logits.scalar_type() != at::kBFloat16 && logits.scalar_type() != at::kFloat)
+    throw_python(PyExc_AssertionError, std::string("the gate logits must be bfloat16 or float32, got ") +
+                                           c10::toString(logits.scalar_type()));
+  MOMOE_CALL(momoe_router_fwd, st, logits.data_ptr(), logits.scalar_type() == at::kFloat, bias.data_ptr<float>(), M, N, K, Ks,
              r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M);
   return r;
 }
 
-// x^T . G_logits [D, N].  The library's product has few tiles and one long contraction for each: below some 1500 tokens it takes as
-// long as the two launches of the kernel (1024 tokens, D = 1024, N = 32 9.3 us against 8.9; 1300 8.6, 9.0), from there on two
-// to four times as long (2000, 1120, 48 19.6 against 9.4; 8192, 2048, 128 59 against 20.6).  Also where autograd records it.
+// x^T . G_logits [D, N].  (The library's product has few tiles and one long contraction for each, and takes the host 18 us where
+// two launches take 8: 300 tokens, D = 512, N = 64 7.5 us of the GPU against 8.3; 1024, 1024, 32 9.3, 8.9; 2000, 1120, 48 19.6, 9.4;
+// 8192, 2048, 128 59, 20.6.)  The library's where autograd records it.
 Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
-  constexpr int64_t kFewTokens = 1536;
   const int64_t M = x.size(0), D = x.size(1), N = G_logit.size(1);
   const int64_t bytes = momoe_gate_wgrad_workspace_bytes(M, D, N);
   const bool rows = x.stride(1) == 1 && x.stride(0) >= D && x.stride(0) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
-  if (M < kFewTokens || bytes < 0 || !rows || at::GradMode::is_enabled()) return at::mm(x.t(), G_logit);
+  if (bytes < 0 || !rows || at::GradMode::is_enabled()) return at::mm(x.t(), G_logit);
   const Tensor out = empty_bf16({D, N}, x.device()), ws = empty_f32({bytes / 4}, x.device());
   MOMOE_CALL(momoe_gate_wgrad, stream_of(x.device()), x.data_ptr(), x.stride(0), G_logit.data_ptr(), out.data_ptr(), M, D, N,
              ws.data_ptr(), bytes);

@@ -6,7 +6,7 @@
 // [M, N] fp32.
 #include <type_traits>
 
-#include "common.hpp"
+#include "gate.hpp"
 
 namespace momoe {
 namespace {
@@ -56,9 +56,75 @@ __device__ __forceinline__ float wave_max_all(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Gate logits of few tokens: x . Wg split over the contraction, a workgroup for each 128 k-values of 128 experts and 64
+// tokens; the router's kernel adds up the fp32 partial products and rounds the sums to bf16, as a product of its own would.
+// Bound by the latency of one round of loads; with many tokens by the partial sums, so up to kGateMaxTokens.  Product and router in
+// a graph, us, a library product -> this: 1 token, D = 2048, N = 128 10.9 -> 8.9, 16 11.5 -> 9.6, 64 18.0 -> 10.9, 512
+// 12.6 -> 12.6, 1000 21.0 -> 15.1; 33, 1000, 200 27.8 -> 11.7; 1000, 1024, 32 10.1 -> 8.2; 2000, 2048, 64 14.6 -> 15.4; 4096,
+// 2048, 128 23.9 -> 30.4.
+constexpr int64_t kGateMaxTokens = 1024;
+constexpr int kGateTokens = 64, kGateDepth = 2 * GateStage::ROWS;
+
+struct GateFwdArgs {
+  const bf16* x;
+  int64_t ldx;
+  const bf16* wg;
+  float* part;  // [parts][M][N]
+  int M, D, N;
+};
+
+__global__ __launch_bounds__(GateStage::THREADS) void gate_logits_kernel(GateFwdArgs p) {
+  constexpr int FM = kGateTokens / 16, FN = 2;  // fragments of a wavefront: all tokens, 32 experts
+  __shared__ __attribute__((aligned(16))) bf16 sw[2 * GateStage::ELEMS];
+  const int k0 = blockIdx.x * kGateDepth, n0 = blockIdx.y * GateStage::COLS, m0 = blockIdx.z * kGateTokens;
+  const int l = threadIdx.x & 63, n_org = 32 * wave_id();
+  GateStage w[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) w[s].load(p.wg + n0, p.N, min(GateStage::COLS, p.N - n0), k0 + s * GateStage::ROWS, p.D);
+  // k-values 8 * (lane / 16) .. +7 of a token are 16 consecutive bytes; those past the end meet zeros of Wg, so they
+  // have to be finite: zeros, too
+  bf16x8 xf[kGateDepth / 32][FM];
+#pragma unroll
+  for (int h = 0; h < kGateDepth / 32; ++h)
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int k = k0 + 32 * h + 8 * (l >> 4);
+      const bf16x8 v = *(const bf16x8*)(p.x + (int64_t)min(m0 + 16 * i + (l & 15), p.M - 1) * p.ldx + min(k, p.D - 8));
+      xf[h][i] = k < p.D ? v : bf16x8{};
+    }
+  w[0].put(sw);
+  w[1].put(sw + GateStage::ELEMS);
+  __syncthreads();
+  if (n0 + n_org >= p.N) return;  // wave-uniform
+  f32x4 acc[FN][FM];
+#pragma unroll
+  for (int j = 0; j < FN; ++j)
+#pragma unroll
+    for (int i = 0; i < FM; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int h = 0; h < kGateDepth / 32; ++h)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const bf16x8 wf = GateStage::frag(sw + (h / 2) * GateStage::ELEMS, n_org + 16 * j, h % 2);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[h][i], acc[j][i], 0, 0, 0);
+    }
+  // a lane holds, for one token (lane % 16), experts 4 * (lane / 16) .. +3
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + 16 * i + (l & 15);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int n = n0 + n_org + 16 * j + 4 * (l >> 4);
+      if (m < p.M && n < p.N) *(f32x4*)(p.part + ((int64_t)blockIdx.x * p.M + m) * p.N + n) = acc[j][i];
+    }
+  }
+}
+
 struct RouterFwdArgs {
   const void* logits;
   int logits_f32;
+  int parts;  // > 0: `logits` are that many fp32 partial sums [parts][M][N], the logits their sums in bf16
   const float* bias;
   int M, N, K, Ks;
   int32_t* mask;
@@ -99,7 +165,19 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int jc = min(lane + 64 * min(c, ncol - 1), N - 1);
-      v[c] = p.logits_f32 ? ((const float*)p.logits)[(int64_t)m * N + jc]
+      if (p.parts > 0) {
+        constexpr int AT_ONCE = 16;
+        const float* part = (const float*)p.logits + (int64_t)m * N + jc;
+        float sum = 0.0f;
+        for (int q0 = 0; q0 < p.parts; q0 += AT_ONCE) {
+          float t[AT_ONCE];
+#pragma unroll
+          for (int q = 0; q < AT_ONCE; ++q) t[q] = part[(int64_t)min(q0 + q, p.parts - 1) * p.M * N];
+#pragma unroll
+          for (int q = 0; q < AT_ONCE; ++q) sum += q0 + q < p.parts ? t[q] : 0.0f;
+        }
+        v[c] = (float)(bf16)sum;
+      } else v[c] = p.logits_f32 ? ((const float*)p.logits)[(int64_t)m * N + jc]
                           : (float)((const bf16*)p.logits)[(int64_t)m * N + jc];
       bias[c] = p.bias[jc];
     }
@@ -302,17 +380,8 @@ __global__ __launch_bounds__(256) void bias_update_kernel(const int64_t* __restr
 
 using namespace momoe;
 
-extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const float* biases_N,
-                                int64_t M, int64_t N, int64_t K, int64_t Ks, int32_t* mask_NM,
-                                float* s_MN, float* p_sel_MN, float* Ng_M, float* Ks_M,
-                                void* stream) {
-  if (!logits_MN || !biases_N || !mask_NM || !s_MN || !p_sel_MN || !Ng_M || !Ks_M)
-    return MOMOE_ERR_BAD_ARG;
-  if (M <= 0 || N <= 0 || Ks < 0 || K < Ks || Ks > N || K - Ks > N - Ks) return MOMOE_ERR_BAD_ARG;
-  if (N > 64 * kMaxCols || M >= (1ll << 31) - 4) return MOMOE_ERR_UNSUPPORTED;
-  RouterFwdArgs a{logits_MN, logits_f32, biases_N, (int)M, (int)N, (int)K, (int)Ks,
-                  mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M};
-  hipStream_t st = (hipStream_t)stream;
+static int launch_router_fwd(const RouterFwdArgs& a, hipStream_t st) {
+  const int64_t M = a.M, N = a.N;
   auto by_width = [&](auto one, auto two, auto four, auto eight) { return N <= 64 ? one : N <= 128 ? two : N <= 256 ? four : eight; };
   if (M <= kRouterSpread) {
     auto kernel = by_width(router_fwd_kernel<1, 4, 256>, router_fwd_kernel<2, 4, 256>, router_fwd_kernel<4, 4, 256>,
@@ -325,6 +394,47 @@ extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const flo
                     : by_width(router_fwd_kernel<1, 32>, router_fwd_kernel<2, 32>, router_fwd_kernel<4, 32>, router_fwd_kernel<8, 32>);
   kernel<<<(unsigned)cdiv64(M, few ? 16 : 32), kRouterThreads, 0, st>>>(a);
   return launch_status();
+}
+
+static int check_router_fwd(int64_t M, int64_t N, int64_t K, int64_t Ks) {
+  if (M <= 0 || N <= 0 || Ks < 0 || K < Ks || Ks > N || K - Ks > N - Ks) return MOMOE_ERR_BAD_ARG;
+  return N > 64 * kMaxCols || M >= (1ll << 31) - 4 ? MOMOE_ERR_UNSUPPORTED : MOMOE_OK;
+}
+
+extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const float* biases_N,
+                                int64_t M, int64_t N, int64_t K, int64_t Ks, int32_t* mask_NM,
+                                float* s_MN, float* p_sel_MN, float* Ng_M, float* Ks_M,
+                                void* stream) {
+  if (!logits_MN || !biases_N || !mask_NM || !s_MN || !p_sel_MN || !Ng_M || !Ks_M)
+    return MOMOE_ERR_BAD_ARG;
+  const int status = check_router_fwd(M, N, K, Ks);
+  if (status != MOMOE_OK) return status;
+  return launch_router_fwd({logits_MN, logits_f32, 0, biases_N, (int)M, (int)N, (int)K, (int)Ks, mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M},
+                           (hipStream_t)stream);
+}
+
+extern "C" int64_t momoe_gate_router_workspace_bytes(int64_t M, int64_t D, int64_t N) {
+  if (M <= 0 || D <= 0 || N <= 0 || D % 8 != 0 || N % 8 != 0 || N > 64 * kMaxCols || D > (1 << 20) || M > kGateMaxTokens) return -1;
+  return cdiv64(D, kGateDepth) * M * N * (int64_t)sizeof(float);
+}
+
+extern "C" int momoe_gate_router_fwd(const void* x_MD, int64_t ldx, const void* Wg_DN, const float* biases_N, int64_t M, int64_t D,
+                                     int64_t N, int64_t K, int64_t Ks, int32_t* mask_NM, float* s_MN, float* p_sel_MN, float* Ng_M,
+                                     float* Ks_M, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!x_MD || !Wg_DN || !biases_N || !mask_NM || !s_MN || !p_sel_MN || !Ng_M || !Ks_M || !workspace) return MOMOE_ERR_BAD_ARG;
+  const int status = check_router_fwd(M, N, K, Ks);
+  if (status != MOMOE_OK) return status;
+  if (D <= 0 || ldx < D) return MOMOE_ERR_BAD_ARG;
+  const int64_t need = momoe_gate_router_workspace_bytes(M, D, N);
+  if (need < 0 || ldx % 8 != 0) return MOMOE_ERR_UNSUPPORTED;
+  if (workspace_bytes < need || ((uintptr_t)x_MD & 15) || ((uintptr_t)Wg_DN & 15) || ((uintptr_t)workspace & 15)) return MOMOE_ERR_BAD_ARG;
+  hipStream_t st = (hipStream_t)stream;
+  const GateFwdArgs g{(const bf16*)x_MD, ldx, (const bf16*)Wg_DN, (float*)workspace, (int)M, (int)D, (int)N};
+  const dim3 grid((unsigned)cdiv64(D, kGateDepth), (unsigned)cdiv64(N, GateStage::COLS), (unsigned)cdiv64(M, kGateTokens));
+  gate_logits_kernel<<<grid, GateStage::THREADS, 0, st>>>(g);
+  const int launched = launch_status();
+  if (launched != MOMOE_OK) return launched;
+  return launch_router_fwd({workspace, 1, (int)grid.x, biases_N, (int)M, (int)N, (int)K, (int)Ks, mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M}, st);
 }
 
 extern "C" int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t gs_stride_m,

@@ -71,6 +71,8 @@ _SIGNATURES = {
                            _i64, _p, _i64, _p]),
     "momoe_router_fwd": (_int, [_p, _int, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]),
     "momoe_router_bwd": (_int, [_p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "momoe_gate_router_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "momoe_gate_router_fwd": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "momoe_gate_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "momoe_gate_wgrad": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
     "momoe_bias_update": (_int, [_p, ctypes.c_float, ctypes.c_float, _i64, _p, _p]),
@@ -374,6 +376,20 @@ def router_fwd(logits_MN, biases_N, K, Ks):
     _call("momoe_router_fwd", _ptr(logits_MN), int(logits_MN.dtype == torch.float32),
                                  _ptr(biases_N), M, N, K, Ks, _ptr(mask), _ptr(s_MN), _ptr(p_sel),
                                  _ptr(Ng_M), _ptr(Ks_M), _stream())
+    return mask, s_MN, p_sel, Ng_M, Ks_M
+
+
+def gate_router_fwd(x_MD, Wg_DN, biases_N, K, Ks):
+    _need_cuda(x_MD, Wg_DN, biases_N)
+    (M, D), N, dev = x_MD.shape, Wg_DN.shape[1], x_MD.device
+    assert Wg_DN.is_contiguous() and x_MD.stride(1) == 1
+    f32 = lambda *size: torch.empty(size, dtype=torch.float32, device=dev)
+    mask = torch.empty((N, M), dtype=torch.int32, device=dev)
+    s_MN, p_sel, Ng_M, Ks_M = f32(M, N), f32(M, N), f32(M), f32(M)
+    nbytes = _lib.momoe_gate_router_workspace_bytes(M, D, N)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+    _call("momoe_gate_router_fwd", _ptr(x_MD), x_MD.stride(0), _ptr(Wg_DN), _ptr(biases_N), M, D, N, K, Ks, _ptr(mask),
+          _ptr(s_MN), _ptr(p_sel), _ptr(Ng_M), _ptr(Ks_M), _ptr(ws), nbytes, _stream())
     return mask, s_MN, p_sel, Ng_M, Ks_M
 
 

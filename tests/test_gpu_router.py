@@ -262,3 +262,55 @@ def test_gate_weight_gradient_of_the_module(M, D, N, pitch):
         grads.append(torch.autograd.grad(loss, r.Wg_DN, create_graph=recorded)[0].detach().double())
     assert grads[0].shape == (D, N)
     assert (grads[0] - grads[1]).abs().max() <= 2.0 ** -7 * grads[1].abs().max()
+
+
+def _whole_numbers(M, D, N, pitch=0):
+    """x, Wg whose products have the same sum in any order: small whole numbers."""
+    g = torch.Generator().manual_seed(M + D + N)
+    x = torch.randint(-3, 4, (M, D + pitch), generator=g).to("cuda:0", torch.bfloat16)[:, :D]
+    return x, torch.randint(-2, 3, (D, N), generator=g).to("cuda:0", torch.bfloat16)
+
+
+@pytest.mark.parametrize("M,D,N,K,Ks", [
+    (1, 8, 8, 1, 0), (3, 40, 24, 5, 1), (63, 128, 128, 8, 0), (64, 136, 136, 4, 0),  # parts of 128 k-values, blocks of
+    (65, 192, 64, 4, 2), (16, 2048, 128, 8, 0), (130, 1000, 512, 8, 0),              # 128 experts and 64 tokens
+    (1024, 256, 16, 2, 0), (2, 2184, 32, 4, 0),  # the most tokens; 18 parts, two rounds of them
+])
+@pytest.mark.parametrize("pitch", [0, 8])
+def test_router_with_its_product(M, D, N, K, Ks, pitch):
+    from momoe_amd import _hip
+    x, Wg = _whole_numbers(M, D, N, pitch)
+    bias = torch.cat([torch.randn(N - Ks, generator=torch.Generator().manual_seed(1)) * 1e-3, torch.full((Ks,), float("-inf"))]).to("cuda:0")
+    logits = (x.double().cpu() @ Wg.double().cpu()).to("cuda:0", torch.float32).to(torch.bfloat16)
+    want = _hip.router_fwd(logits, bias, K, Ks)
+    for a, b in zip(_hip.gate_router_fwd(x, Wg, bias, K, Ks), want):
+        assert torch.equal(a, b)
+    # a token that is not finite is alone in that
+    x[M // 2, D - 1] = float("inf")
+    got = _hip.gate_router_fwd(x, Wg, bias, K, Ks)
+    rest = torch.arange(M, device="cuda:0") != M // 2
+    assert torch.equal(got[0][:, rest], want[0][:, rest]) and torch.equal(got[1][rest], want[1][rest])
+
+
+def test_sizes_the_router_with_its_product_refuses():
+    from momoe_amd import _hip
+    for M, D, N in [(1025, 64, 8), (4, 20, 8), (4, 64, 12), (4, 64, 520)]:
+        assert _hip._lib.momoe_gate_router_workspace_bytes(M, D, N) == -1
+        with pytest.raises(RuntimeError):
+            _hip.gate_router_fwd(*_whole_numbers(M, D, N), torch.zeros(N, device="cuda:0"), 2, 0)
+
+
+@pytest.mark.parametrize("M,D,N,pitch", [(1024, 64, 8, 0), (1025, 64, 8, 0), (5, 20, 8, 0), (5, 64, 12, 0), (5, 64, 8, 4), (5, 64, 8, 8)])
+def test_module_routes_alike_by_either_product(M, D, N, pitch):
+    import momoe_amd
+    from momoe_amd import _hip
+    x, Wg = _whole_numbers(M, D, N, pitch)
+    bias = torch.zeros(N, device="cuda:0")
+    want = _hip.router_fwd((x.double().cpu() @ Wg.double().cpu()).to("cuda:0", torch.bfloat16), bias, 2, 0)
+    for weight in (Wg, Wg.T.contiguous().T):
+        r = momoe_amd.TopKRouter(D, N, 2, 0, Wg_DN=Wg)
+        r.Wg_DN.data = weight
+        for grad in (False, True):
+            with torch.set_grad_enabled(grad):
+                out = r(x[None], bias)
+            assert torch.equal(out[1], want[0]) and torch.equal(out[2], want[1].T)
