@@ -375,6 +375,13 @@ int64_t momoe_gate_wgrad_workspace_bytes(int64_t M, int64_t D, int64_t N);
 int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogits_MN, void* GWg_DN,
                      int64_t M, int64_t D, int64_t N, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* momoe_gate_dgrad: gradient of the tokens through the gate product (momoe/topk_router.py:83-145), out_MD = Gx_MD +
+ * Glogits_MN . Wg_DN^T, bf16 from fp32 sums; Gx_MD may be NULL (nothing to add) or out_MD.  All contiguous bf16 on 16-byte
+ * boundaries, D and N multiples of 8.
+ */
+int momoe_gate_dgrad(const void* Glogits_MN, const void* Wg_DN, const void* Gx_MD, void* out_MD,
+                     int64_t M, int64_t D, int64_t N, void* stream);
+
 /* momoe_bias_update (momoe/sample_moe.py:65-67): biases_N[i] += rate * sign(c_avg - sizes_N[i]) in
  * place, fp32; -inf (a shared expert) stays -inf.
  */

@@ -1,4 +1,6 @@
-// Gradient of the router's gate weights: G_Wg [D,N] = x^T . G_logits, a contraction over the tokens with few columns.
+// Gradients of the router's gate product.
+//
+// Of the weights: G_Wg [D,N] = x^T . G_logits, a contraction over the tokens with few columns.
 //
 // Bound by memory: x is read once for every 128 experts, and that is nearly all there is.  The product has few tiles and a
 // long contraction, so the tokens are split: a workgroup takes 128 columns of x, 128 experts and a range of tokens, and a
@@ -101,6 +103,67 @@ __global__ __launch_bounds__(kGateThreads) void gate_wgrad_reduce_kernel(const f
   ((bf16x4*)out)[q] = bf16x4{(bf16)sum[0], (bf16)sum[1], (bf16)sum[2], (bf16)sum[3]};
 }
 
+// Of the tokens: out [M,D] = G_x + G_logits . Wg^T, a contraction over the experts.  Bound by memory, G_x in and the sum out;
+// both operands are k-contiguous and small enough for the caches, so fragments are loaded as they are, 64 x 64 a wavefront.
+// A fragment's 16 rows of Wg are those of two runs of columns in turn, so that a lane holds 8 consecutive columns of a token and
+// four lanes store 64 bytes.  In a graph, us, the library's product with its copy of G_x -> this: 128 tokens, D = 128, N = 8 10.3 ->
+// 4.9; 1024, 1024, 32 7.3 -> 4.7; 2000, 1120, 48 14.5 -> 5.0; 8192, 2048, 128 32.7 -> 25.1; 32768, 512, 16 33.7 -> 13.8; 8192, 4096, 96
+// 50.1 -> 31.8.
+struct GateDgradArgs {
+  const bf16 *gl, *wg, *gx;  // gx: nullptr if there is nothing to add
+  bf16* out;
+  int M, D, N;
+};
+
+__global__ __launch_bounds__(kGateThreads, 2) void gate_dgrad_kernel(GateDgradArgs p) {
+  const int l = threadIdx.x & 63, r = l & 15, g = l >> 4, w = wave_id();
+  const int d0 = blockIdx.x * kTile + 64 * (w & 1), m0 = blockIdx.y * kTile + 64 * (w >> 1);
+  if (d0 >= p.D || m0 >= p.M) return;  // wave-uniform
+  // fragment j: column r of it is column 32 (j / 2) + 8 (r / 4) + 4 (j % 2) + r % 4 of the wave's 64
+  const bf16 *grow[4], *wrow[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    grow[i] = p.gl + (int64_t)min(m0 + 16 * i + r, p.M - 1) * p.N;
+    wrow[i] = p.wg + (int64_t)min(d0 + 32 * (i >> 1) + 8 * (r >> 2) + 4 * (i & 1) + (r & 3), p.D - 1) * p.N;
+  }
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int n0 = 0; n0 < p.N; n0 += 32) {
+    const int n = n0 + 8 * g, at = min(n, p.N - 8);
+    bf16x8 gf[4], wf[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gf[i] = *(const bf16x8*)(grow[i] + at), wf[i] = *(const bf16x8*)(wrow[i] + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gf[i] = n < p.N ? gf[i] : bf16x8{}, wf[i] = n < p.N ? wf[i] : bf16x8{};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], gf[i], acc[j][i], 0, 0, 0);
+  }
+  // a lane holds, for token r of fragment i, columns 32 q + 8 g .. +7 in fragments 2 q and 2 q + 1
+  bf16x8 add[4][2];
+  if (p.gx != nullptr) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        add[i][q] = *(const bf16x8*)(p.gx + (int64_t)min(m0 + 16 * i + r, p.M - 1) * p.D + min(d0 + 32 * q + 8 * g, p.D - 8));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16)(acc[2 * q + e / 4][i][e % 4] + (p.gx != nullptr ? (float)add[i][q][e] : 0.0f));
+      const int m = m0 + 16 * i + r, d = d0 + 32 * q + 8 * g;
+      if (m < p.M && d < p.D) *(bf16x8*)(p.out + (int64_t)m * p.D + d) = o;
+    }
+}
+
 struct GateSplit {
   int64_t rows, ranges;
   GateSplit(int64_t M, int64_t D, int64_t N) {
@@ -143,5 +206,17 @@ extern "C" int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogi
   const int64_t quads = D * N / 4;
   gate_wgrad_reduce_kernel<<<(unsigned)cdiv64(quads, kGateThreads), kGateThreads, 0, st>>>((const float*)workspace, (int)split.ranges,
                                                                                          quads, (bf16*)GWg_DN);
+  return launch_status();
+}
+
+extern "C" int momoe_gate_dgrad(const void* Glogits_MN, const void* Wg_DN, const void* Gx_MD, void* out_MD, int64_t M, int64_t D,
+                                int64_t N, void* stream) {
+  if (!Glogits_MN || !Wg_DN || !out_MD || M <= 0 || D <= 0 || N <= 0) return MOMOE_ERR_BAD_ARG;
+  if (!gate_sizes_ok(M, D, N) || cdiv64(M, kTile) > 65535) return MOMOE_ERR_UNSUPPORTED;
+  for (const void* p : {Glogits_MN, Wg_DN, Gx_MD, (const void*)out_MD})
+    if ((uintptr_t)p & 15) return MOMOE_ERR_BAD_ARG;
+  const GateDgradArgs a{(const bf16*)Glogits_MN, (const bf16*)Wg_DN, (const bf16*)Gx_MD, (bf16*)out_MD, (int)M, (int)D, (int)N};
+  const dim3 grid((unsigned)cdiv64(D, kTile), (unsigned)cdiv64(M, kTile));
+  gate_dgrad_kernel<<<grid, kGateThreads, 0, (hipStream_t)stream>>>(a);
   return launch_status();
 }

@@ -440,10 +440,23 @@ Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
   const int64_t M = x.size(0), D = x.size(1), N = G_logit.size(1);
   const int64_t bytes = momoe_gate_wgrad_workspace_bytes(M, D, N);
   const bool rows = x.stride(1) == 1 && x.stride(0) >= D && x.stride(0) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
-  if (bytes < 0 || !rows || at::GradMode::is_enabled()) return at::mm(x.t(), G_logit);
+  if (bytes < 0 || !rows || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA)) return at::mm(x.t(), G_logit);
   const Tensor out = empty_bf16({D, N}, x.device()), ws = empty_f32({bytes / 4}, x.device());
   MOMOE_CALL(momoe_gate_wgrad, stream_of(x.device()), x.data_ptr(), x.stride(0), G_logit.data_ptr(), out.data_ptr(), M, D, N,
              ws.data_ptr(), bytes);
+  return out;
+}
+
+// G_x + G_logits . Wg^T [M, D]; G_x may be undefined.  (The library copies G_x in front of its product.)
+Tensor gate_input_gradient(const Tensor& G_x, const Tensor& G_logit, const Tensor& Wg) {
+  const int64_t M = G_logit.size(0), N = G_logit.size(1), D = Wg.size(0);
+  const auto packed = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0; };
+  if (D % 8 != 0 || N % 8 != 0 || M >= 65535 * 128 || !packed(Wg) || (G_x.defined() && !packed(G_x)) || at::GradMode::is_enabled() ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    return G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
+  const Tensor out = empty_bf16({M, D}, G_logit.device());
+  MOMOE_CALL(momoe_gate_dgrad, stream_of(G_logit.device()), G_logit.data_ptr(), Wg.data_ptr(),
+             G_x.defined() ? (const void*)G_x.data_ptr() : nullptr, out.data_ptr(), M, D, N);
   return out;
 }
 
@@ -484,7 +497,7 @@ struct RouterFn : torch::autograd::Function<RouterFn> {
       MOMOE_CALL(momoe_router_bwd, stream_of(dev), G_s.data_ptr<float>(), G_s.stride(0), G_s.stride(1),
                  p_sel.data_ptr<float>(), s_MN.data_ptr<float>(), nrm, nrm + M, mask.data_ptr<int32_t>(), M, N,
                  ctx->saved_data["Ks"].toInt(), G_logit.data_ptr());
-      if (need_x) G_x = G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
+      if (need_x) G_x = gate_input_gradient(G_x, G_logit, Wg);
       if (need_wg) out[1] = gate_gradient(x, G_logit);
     } else if (need_wg) {
       out[1] = at::zeros_like(Wg);

@@ -58,11 +58,12 @@ __device__ __forceinline__ float wave_max_all(float v) {
 
 // Gate logits of few tokens: x . Wg split over the contraction, a workgroup for each 128 k-values of 128 experts and 64
 // tokens; the router's kernel adds up the fp32 partial products and rounds the sums to bf16, as a product of its own would.
-// Bound by the latency of one round of loads; with many tokens by the partial sums, so up to kGateMaxTokens.  Product and router in
+// Bound by the latency of one round of loads; with many tokens by the partial sums, so up to kGateMaxRows rows of them, and up to
+// kGateMaxTokens, where the host's time for a library product stops to show.  Product and router in
 // a graph, us, a library product -> this: 1 token, D = 2048, N = 128 10.9 -> 8.9, 16 11.5 -> 9.6, 64 18.0 -> 10.9, 512
 // 12.6 -> 12.6, 1000 21.0 -> 15.1; 33, 1000, 200 27.8 -> 11.7; 1000, 1024, 32 10.1 -> 8.2; 2000, 2048, 64 14.6 -> 15.4; 4096,
-// 2048, 128 23.9 -> 30.4.
-constexpr int64_t kGateMaxTokens = 1024;
+// 2048, 128 23.9 -> 30.4; 2048, 1024, 96 17.1 -> 14.6; 1513, 128, 96 9.9 -> 10.4.
+constexpr int64_t kGateMaxTokens = 2048, kGateMaxRows = 16 * 1024;
 constexpr int kGateTokens = 64, kGateDepth = 2 * GateStage::ROWS;
 
 struct GateFwdArgs {
@@ -414,7 +415,9 @@ extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const flo
 }
 
 extern "C" int64_t momoe_gate_router_workspace_bytes(int64_t M, int64_t D, int64_t N) {
-  if (M <= 0 || D <= 0 || N <= 0 || D % 8 != 0 || N % 8 != 0 || N > 64 * kMaxCols || D > (1 << 20) || M > kGateMaxTokens) return -1;
+  if (M <= 0 || D <= 0 || N <= 0 || D % 8 != 0 || N % 8 != 0 || N > 64 * kMaxCols || D > (1 << 20) || M > kGateMaxTokens ||
+      cdiv64(D, kGateDepth) * M > kGateMaxRows)
+    return -1;
   return cdiv64(D, kGateDepth) * M * N * (int64_t)sizeof(float);
 }
 

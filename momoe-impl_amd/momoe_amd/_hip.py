@@ -75,6 +75,7 @@ _SIGNATURES = {
     "momoe_gate_router_fwd": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "momoe_gate_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "momoe_gate_wgrad": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
+    "momoe_gate_dgrad": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "momoe_bias_update": (_int, [_p, ctypes.c_float, ctypes.c_float, _i64, _p, _p]),
 }
 
@@ -410,3 +411,11 @@ def gate_wgrad(x_MD, Glogits_MN, GWg_DN):
     ws = torch.empty(max(nbytes, 0), dtype=torch.uint8, device=x_MD.device)
     _call("momoe_gate_wgrad", _ptr(x_MD), x_MD.stride(0), _ptr(Glogits_MN), _ptr(GWg_DN), M, D, N, _ptr(ws), nbytes,
           _stream())
+
+
+def gate_dgrad(Glogits_MN, Wg_DN, Gx_MD, out_MD):
+    """Gx_MD: None if there is nothing to add."""
+    _need_cuda(Glogits_MN, Wg_DN, Gx_MD, out_MD)
+    (M, N), D = Glogits_MN.shape, Wg_DN.shape[0]
+    assert all(t is None or t.is_contiguous() for t in (Glogits_MN, Wg_DN, Gx_MD, out_MD))
+    _call("momoe_gate_dgrad", _ptr(Glogits_MN), _ptr(Wg_DN), _ptr(Gx_MD), _ptr(out_MD), M, D, N, _stream())

@@ -1,8 +1,8 @@
 """`TopKRouter`: top-k + softmax gate with a selection bias (auxiliary-loss-free load
 balancing) and shared experts, mirroring momoe/topk_router.py:83-173.
 
-The gate matmuls are plain library GEMMs (torch), but for the gradient of the gate weights of many
-tokens; that, the softmax / top-k / renormalise pass and its backward are HIP kernels.
+The gate product of many tokens is a plain library GEMM (torch); that of few tokens, its gradients and the
+softmax / top-k / renormalise pass with its backward are HIP kernels.
 """
 import torch
 import torch.nn as nn

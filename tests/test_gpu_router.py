@@ -246,22 +246,49 @@ def test_gate_weight_gradient(M, D, N):
     assert torch.isinf(got[3]).all() and torch.isfinite(torch.cat([got[:3], got[4:]])).all()
 
 
-@pytest.mark.parametrize("M,D,N", [(1535, 64, 16), (1536, 64, 16), (2000, 72, 20), (1600, 96, 24)])
+@pytest.mark.parametrize("M,D,N", [
+    (1, 8, 8), (64, 64, 32), (127, 128, 40), (129, 136, 136), (300, 264, 512), (8192, 64, 64),  # tiles of 128 x 128, 32 k-values
+])
+@pytest.mark.parametrize("add", [False, True])
+def test_gate_input_gradient(M, D, N, add):
+    from momoe_amd import _hip
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    rnd = lambda *size: torch.randn(*size, generator=g, device="cuda:0").to(torch.bfloat16)
+    gl, Wg, gx = rnd(M, N), rnd(D, N), rnd(M, D)
+    out = torch.full((M, D), 7.0, device="cuda:0", dtype=torch.bfloat16)
+    kept = gx.clone()
+    _hip.gate_dgrad(gl, Wg, gx if add else None, out)
+    assert torch.equal(gx, kept)
+    ref, size = gl.double() @ Wg.double().T.contiguous(), gl.double().abs() @ Wg.double().abs().T.contiguous()
+    if add:
+        ref, size = ref + gx.double(), size + gx.double().abs()
+    # bf16 rounding of the result, and N + 1 fp32 additions of that size
+    assert ((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + (N + 1) * 2.0 ** -24 * size).all()
+    gl[M // 2, N - 1] = float("inf")  # a token that is not finite is alone in that
+    want, rest = out.clone(), torch.arange(M, device="cuda:0") != M // 2
+    _hip.gate_dgrad(gl, Wg, gx if add else None, out)
+    assert torch.equal(out[rest], want[rest]) and not torch.isfinite(out[M // 2]).any()
+
+
+@pytest.mark.parametrize("M,D,N", [(1, 64, 16), (300, 64, 16), (2000, 72, 20), (1600, 96, 24)])
 @pytest.mark.parametrize("pitch", [0, 4, 8])
-def test_gate_weight_gradient_of_the_module(M, D, N, pitch):
-    """Whichever product the module takes, by the tokens, the widths and the layout of x, the gradient is that of
+def test_gate_gradients_of_the_module(M, D, N, pitch):
+    """Whichever product the module takes, by the widths and the layout of x, the gradients are those of
     the library's, which a backward that is itself recorded takes."""
     import momoe_amd
     g = torch.Generator(device="cuda:0").manual_seed(D)
     r = momoe_amd.TopKRouter(D, N, 4, 0, Wg_DN=torch.randn(D, N, generator=g, device="cuda:0").to(torch.bfloat16) / 8)
     x = torch.randn(1, M, D + pitch, generator=g, device="cuda:0").to(torch.bfloat16)[..., :D]
     w = torch.randn(N, M, generator=g, device="cuda:0")
-    grads = []
-    for recorded in (False, True):
-        loss = (r(x, torch.zeros(N, device="cuda:0"))[2] * w).sum()
-        grads.append(torch.autograd.grad(loss, r.Wg_DN, create_graph=recorded)[0].detach().double())
-    assert grads[0].shape == (D, N)
-    assert (grads[0] - grads[1]).abs().max() <= 2.0 ** -7 * grads[1].abs().max()
+    x.requires_grad_()
+    for through in (False, True):  # a gradient of x from elsewhere is added
+        grads = []
+        for recorded in (False, True):
+            out = r(x, torch.zeros(N, device="cuda:0"))
+            loss = (out[2] * w).sum() + (out[0].float().square().sum() if through else 0.0)
+            grads.append([t.detach().double() for t in torch.autograd.grad(loss, (r.Wg_DN, x), create_graph=recorded)])
+        for got, want in zip(*grads):
+            assert got.shape == want.shape and (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
 def _whole_numbers(M, D, N, pitch=0):
@@ -274,7 +301,7 @@ def _whole_numbers(M, D, N, pitch=0):
 @pytest.mark.parametrize("M,D,N,K,Ks", [
     (1, 8, 8, 1, 0), (3, 40, 24, 5, 1), (63, 128, 128, 8, 0), (64, 136, 136, 4, 0),  # parts of 128 k-values, blocks of
     (65, 192, 64, 4, 2), (16, 2048, 128, 8, 0), (130, 1000, 512, 8, 0),              # 128 experts and 64 tokens
-    (1024, 256, 16, 2, 0), (2, 2184, 32, 4, 0),  # the most tokens; 18 parts, two rounds of them
+    (2048, 256, 16, 2, 0), (2, 2184, 32, 4, 0),  # the most tokens; 18 parts, two rounds of them
 ])
 @pytest.mark.parametrize("pitch", [0, 8])
 def test_router_with_its_product(M, D, N, K, Ks, pitch):
@@ -294,13 +321,13 @@ def test_router_with_its_product(M, D, N, K, Ks, pitch):
 
 def test_sizes_the_router_with_its_product_refuses():
     from momoe_amd import _hip
-    for M, D, N in [(1025, 64, 8), (4, 20, 8), (4, 64, 12), (4, 64, 520)]:
+    for M, D, N in [(2049, 64, 8), (1025, 2048, 8), (4, 20, 8), (4, 64, 12), (4, 64, 520)]:
         assert _hip._lib.momoe_gate_router_workspace_bytes(M, D, N) == -1
         with pytest.raises(RuntimeError):
             _hip.gate_router_fwd(*_whole_numbers(M, D, N), torch.zeros(N, device="cuda:0"), 2, 0)
 
 
-@pytest.mark.parametrize("M,D,N,pitch", [(1024, 64, 8, 0), (1025, 64, 8, 0), (5, 20, 8, 0), (5, 64, 12, 0), (5, 64, 8, 4), (5, 64, 8, 8)])
+@pytest.mark.parametrize("M,D,N,pitch", [(2048, 64, 8, 0), (2049, 64, 8, 0), (5, 20, 8, 0), (5, 64, 12, 0), (5, 64, 8, 4), (5, 64, 8, 8)])
 def test_module_routes_alike_by_either_product(M, D, N, pitch):
     import momoe_amd
     from momoe_amd import _hip
