@@ -125,7 +125,7 @@ __global__ __launch_bounds__(GateStage::THREADS) void gate_logits_kernel(GateFwd
 struct RouterFwdArgs {
   const void* logits;
   int logits_f32;
-  int parts;  // > 0: `logits` are that many fp32 partial sums [parts][M][N], the logits their sums in bf16
+  int parts;  // PARTS: `logits` are that many fp32 partial sums [parts][M][N], the logits their sums in bf16
   const float* bias;
   int M, N, K, Ks;
   int32_t* mask;
@@ -146,9 +146,11 @@ struct RouterFwdArgs {
 // 4096 x 64, K = 6 5.0 -> 5.5.
 constexpr int kRouterThreads = 1024;
 constexpr int64_t kRouterOneEach = 256 * 16, kRouterSpread = 3072;
+static_assert(kGateMaxTokens <= kRouterSpread, "partial sums are taken by the workgroups of four tokens");
 
 // NC = columns held per lane (1, 2, 4 or 8): N <= 64 * NC
-template <int NC, int kTok, int THREADS = kRouterThreads>
+// PARTS: the logits are partial sums.
+template <int NC, int kTok, int THREADS = kRouterThreads, bool PARTS = false>
 __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
   __shared__ uint8_t flags[64 * NC][kTok];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -166,7 +168,8 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int jc = min(lane + 64 * min(c, ncol - 1), N - 1);
-      if (p.parts > 0) {
+      bias[c] = p.bias[jc];
+      if constexpr (PARTS) {
         constexpr int AT_ONCE = 16;
         const float* part = (const float*)p.logits + (int64_t)m * N + jc;
         float sum = 0.0f;
@@ -178,9 +181,9 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
           for (int q = 0; q < AT_ONCE; ++q) sum += q0 + q < p.parts ? t[q] : 0.0f;
         }
         v[c] = (float)(bf16)sum;
-      } else v[c] = p.logits_f32 ? ((const float*)p.logits)[(int64_t)m * N + jc]
-                          : (float)((const bf16*)p.logits)[(int64_t)m * N + jc];
-      bias[c] = p.bias[jc];
+      } else {
+        v[c] = p.logits_f32 ? ((const float*)p.logits)[(int64_t)m * N + jc] : (float)((const bf16*)p.logits)[(int64_t)m * N + jc];
+      }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
       }
     }
     mg = wave_max(mg);
-    ms = wave_max(ms);
+    if (p.Ks > 0) ms = wave_max(ms);  // (uniform; nothing to exchange without shared experts)
     float sg = 0.0f, ss = 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
       }
     }
     sg = wave_sum(sg);
-    ss = wave_sum(ss);
+    if (p.Ks > 0) ss = wave_sum(ss);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int j = lane + 64 * c;
@@ -245,7 +248,7 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
       }
     }
     ngsum = wave_sum(ngsum);
-    kssum = wave_sum(kssum);
+    if (p.Ks > 0) kssum = wave_sum(kssum);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int j = lane + 64 * c;
@@ -385,8 +388,10 @@ static int launch_router_fwd(const RouterFwdArgs& a, hipStream_t st) {
   const int64_t M = a.M, N = a.N;
   auto by_width = [&](auto one, auto two, auto four, auto eight) { return N <= 64 ? one : N <= 128 ? two : N <= 256 ? four : eight; };
   if (M <= kRouterSpread) {
-    auto kernel = by_width(router_fwd_kernel<1, 4, 256>, router_fwd_kernel<2, 4, 256>, router_fwd_kernel<4, 4, 256>,
-                           router_fwd_kernel<8, 4, 256>);
+    auto kernel = a.parts > 0 ? by_width(router_fwd_kernel<1, 4, 256, true>, router_fwd_kernel<2, 4, 256, true>,
+                                         router_fwd_kernel<4, 4, 256, true>, router_fwd_kernel<8, 4, 256, true>)
+                              : by_width(router_fwd_kernel<1, 4, 256>, router_fwd_kernel<2, 4, 256>, router_fwd_kernel<4, 4, 256>,
+                                         router_fwd_kernel<8, 4, 256>);
     kernel<<<(unsigned)cdiv64(M, 4), 256, 0, st>>>(a);
     return launch_status();
   }
