@@ -93,6 +93,34 @@ Tensor empty_f32(at::IntArrayRef size, const at::Device& dev) {
   return at::empty(size, at::TensorOptions().dtype(at::kFloat).device(dev));
 }
 
+// Buffers that live no longer than the call: pieces of one allocation where they are few bytes in all, since an
+// allocation takes the host a microsecond and a small call is as long as its host work (in us of the host, a forward of 7 tokens
+// with its router 37.2 -> 34.8, the backward of 128 tokens 88 -> 81); allocations of their own, given back as soon as they are
+// done with, where their size counts.
+class Transients {
+  static constexpr int64_t kSmall = 1 << 20;  // torch's own line between small allocations and large ones
+  const at::Device dev_;
+  Tensor block_;
+  int64_t used_ = 0;
+  static int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
+
+ public:
+  Transients(const at::Device& dev, std::initializer_list<int64_t> sizes) : dev_(dev) {
+    int64_t all = 0;
+    for (int64_t bytes : sizes) all += bytes <= kSmall ? up(bytes) : 2 * kSmall;
+    if (all <= kSmall) block_ = bytes_of(all);
+  }
+  Tensor bytes_of(int64_t bytes) const { return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(dev_)); }
+  // the next of those sizes; `own` holds it if it is an allocation of its own
+  void* take(int64_t bytes, Tensor& own) {
+    if (!block_.defined()) return (own = bytes_of(bytes)).data_ptr();
+    TORCH_INTERNAL_ASSERT(used_ + bytes <= block_.numel());
+    void* const p = (char*)block_.data_ptr() + used_;
+    used_ += up(bytes);
+    return p;
+  }
+};
+
 // A Python exception of the given type, raised when the binding returns
 [[noreturn]] void throw_python(PyObject* type, const std::string& what) {
   py::gil_scoped_acquire gil;
@@ -189,29 +217,33 @@ Forward experts_forward(const Tensor& x_BSD, const Tensor& Wl1, const Tensor& Wl
   const int64_t ws_bytes = momoe_index_workspace_bytes(M, N);
   // only the build itself needs these: its panel counts, the slot of every pair, and the counter
   // of tokens with another number of experts than K, which starts from zero if it is to be read
-  const Tensor scratch = empty_i32(4 + ((msum + 3) & ~(int64_t)3) + (ws_bytes + 3) / 4, dev);
-  int32_t* violations = scratch.data_ptr<int32_t>();
-  if (check) scratch.narrow(0, 0, 4).zero_();
+  const int64_t scratch_bytes = (4 + ((msum + 3) & ~(int64_t)3) + (ws_bytes + 3) / 4) * 4;
+  Transients transients(dev, {scratch_bytes, msum * H * 2, msum * D * 2});
+  Tensor counter, scratch, h_own, ys_own;
+  int32_t* const build = (int32_t*)transients.take(scratch_bytes, scratch);
+  int32_t* violations = build;
+  if (check) {
+    counter = at::zeros({4}, at::TensorOptions().dtype(at::kInt).device(dev));
+    violations = counter.data_ptr<int32_t>();
+  }
   MOMOE_CALL(momoe_index_build, st, mask.data_ptr<int32_t>(), mask.stride(0), mask.stride(1), M, N, K,
-             f.sizes.data_ptr<int64_t>(), ib.cumsums(), ib.idx(), violations + 4, ib.inv(), ib.table(),
-             (int)tile_rows, ib.table_rc(), (void*)(violations + 4 + ((msum + 3) & ~(int64_t)3)), ws_bytes,
+             f.sizes.data_ptr<int64_t>(), ib.cumsums(), ib.idx(), build + 4, ib.inv(), ib.table(),
+             (int)tile_rows, ib.table_rc(), (void*)(build + 4 + ((msum + 3) & ~(int64_t)3)), ws_bytes,
              violations);
 
   if (msave > 0) f.ab_save = empty_bf16({msave, 2 * H}, dev);
-  Tensor ys;
-  {
-    // h in blocks of 32 hidden columns, [H/32][Msum][32]: the layout the down projection reads
-    const Tensor h = empty_bf16({H / 32, msum, 32}, dev);
-    MOMOE_CALL(momoe_lin1_swiglu_fwd, st, f.x.data_ptr(), f.W1.data_ptr(), ib.idx(), ib.table_for(2 * H, D), h.data_ptr(),
-               msave > 0 ? f.ab_save.data_ptr() : nullptr, (int64_t)0, msave, M, D, H, N, msum);
-    ys = empty_bf16({msum, D}, dev);
-    MOMOE_CALL(momoe_lin2_scale_fwd, st, h.data_ptr(), f.W2.data_ptr(), f.s.data_ptr<float>(), f.s.stride(0),
-               f.s.stride(1), ib.idx(), ib.table_for(D, H), ys.data_ptr(), M, D, H, N, msum);
-  }
+  // h in blocks of 32 hidden columns, [H/32][Msum][32]: the layout the down projection reads
+  void* const h = transients.take(msum * H * 2, h_own);
+  MOMOE_CALL(momoe_lin1_swiglu_fwd, st, f.x.data_ptr(), f.W1.data_ptr(), ib.idx(), ib.table_for(2 * H, D), h,
+             msave > 0 ? f.ab_save.data_ptr() : nullptr, (int64_t)0, msave, M, D, H, N, msum);
+  void* const ys = transients.take(msum * D * 2, ys_own);
+  MOMOE_CALL(momoe_lin2_scale_fwd, st, h, f.W2.data_ptr(), f.s.data_ptr<float>(), f.s.stride(0),
+             f.s.stride(1), ib.idx(), ib.table_for(D, H), ys, M, D, H, N, msum);
+  h_own.reset();
   f.y = empty_bf16({B, S, D}, dev);
-  MOMOE_CALL(momoe_combine, st, ys.data_ptr(), ib.inv(), f.y.data_ptr(), M, D, K, msum);
+  MOMOE_CALL(momoe_combine, st, ys, ib.inv(), f.y.data_ptr(), M, D, K, msum);
   if (check) {
-    const int v = scratch.narrow(0, 0, 1).item<int32_t>();
+    const int v = counter.narrow(0, 0, 1).item<int32_t>();
     TORCH_CHECK(v == 0, "mask_NM: ", v, " tokens do not have exactly K = ", K,
                 " experts (or the mask holds more than M*K pairs)");
   }
@@ -285,22 +317,30 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     const Tensor Gy = grads[0].reshape({M, D}).to(dev, at::kBFloat16).contiguous();
 
     // dL/dh before the gate weight, in sorted order
-    Tensor u = empty_bf16({msum, H}, dev);
-    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u.data_ptr(), M, D, H, N,
-               msum);
+    const int64_t u_bytes = msum * H * 2, gz_bytes = 2 * u_bytes, hst_bytes = momoe_padded_rows(msum, N) * H * 2;
+    const int64_t nparts = momoe_gs_parts(H, N, msum), parts_bytes = nparts * msum * 4, gxs_bytes = need_x ? msum * D * 2 : 0;
+    // scratch for the weight gradients of experts with many rows: what the library can use, but no
+    // more than u occupied (just freed, so the peak does not move)
+    auto scratch_bytes = [&](bool need, int64_t X, int64_t Y) {
+      return need ? std::min(u_bytes, momoe_wgrad_workspace_bytes(N, X, Y, msum)) : 0;
+    };
+    const int64_t ws2_bytes = scratch_bytes(need_w2, H, D), ws1_bytes = scratch_bytes(need_w1, D, 2 * H);
+    Transients transients(dev, {u_bytes, gz_bytes, hst_bytes, parts_bytes, ws2_bytes, ws1_bytes, gxs_bytes});
+    Tensor u_own, gz_own, hst_own, parts_own;
+    void* const u = transients.take(u_bytes, u_own);
+    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u, M, D, H, N, msum);
     // SwiGLU backward: rows with saved a|b read them; the others recompute a|b = x.Wl1 and consume
     // them straight from the GEMM's accumulators.
     // G_a|G_b in blocks of 32 columns, [2H/32][Msum][32]: the layout dL/dx contracts over
-    const Tensor gz = empty_bf16({2 * H / 32, msum, 32}, dev);
+    void* const gz = transients.take(gz_bytes, gz_own);
     // s*h in groups of 32 padded sorted rows, feature-major inside a group: the layout the Wl2
     // gradient reads fastest
-    Tensor hst = empty_bf16({momoe_padded_rows(msum, N) / 32, H, 32}, dev);
-    const int64_t nparts = momoe_gs_parts(H, N, msum);
-    Tensor gs_part = empty_f32({nparts, msum}, dev);
+    void* const hst = transients.take(hst_bytes, hst_own);
+    float* const gs_part = (float*)transients.take(parts_bytes, parts_own);
     if (msave > 0)
-      MOMOE_CALL(momoe_swiglu_bwd_saved, st, ab_save.data_ptr(), u.data_ptr(), s.data_ptr<float>(), s.stride(0),
-                 s.stride(1), ib.idx(), ib.cumsums(), msave, gz.data_ptr(), hst.data_ptr(), H,
-                 gs_part.data_ptr<float>(), nparts, M, H, N, msum);
+      MOMOE_CALL(momoe_swiglu_bwd_saved, st, ab_save.data_ptr(), u, s.data_ptr<float>(), s.stride(0),
+                 s.stride(1), ib.idx(), ib.cumsums(), msave, gz, hst, H,
+                 gs_part, nparts, M, H, N, msum);
     if (msave < msum) {
       // the recomputing GEMM takes no taller tiles: a table of its own where another height was given
       Tensor own;
@@ -312,51 +352,47 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
         table_rc = own.data_ptr<int32_t>();
       }
       call("momoe_lin1_swiglu_bwd", st, momoe_lin1_swiglu_bwd_parts, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc,
-           u.data_ptr(), s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz.data_ptr(), hst.data_ptr(), H,
-           gs_part.data_ptr<float>(), nparts, M, D, H, N, msum);
+           u, s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz, hst, H,
+           gs_part, nparts, M, D, H, N, msum);
     }
-    u.reset();
+    u_own.reset();
     if (need_s) {
       // in the layout of s, where autograd keeps it without a copy
       if (s.stride(0) == 1 && s.stride(1) == N) {
         out[4] = empty_f32({M, N}, dev).t();
-        call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part.data_ptr<float>(), nparts,
+        call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part, nparts,
              (const int32_t*)ib.idx(), (const int32_t*)ib.cumsums(), out[4].data_ptr<float>(), M, N, msum);
       } else {
         out[4] = empty_f32({N, M}, dev);
-        MOMOE_CALL(momoe_gs_scatter, st, gs_part.data_ptr<float>(), nparts, ib.idx(), ib.cumsums(),
+        MOMOE_CALL(momoe_gs_scatter, st, gs_part, nparts, ib.idx(), ib.cumsums(),
                    out[4].data_ptr<float>(), M, N, msum);
       }
     }
-    gs_part.reset();
+    parts_own.reset();
 
-    // scratch for the weight gradients of experts with many rows: what the library can use, but no
-    // more than u occupied (just freed, so the peak does not move)
-    auto workspace = [&](int64_t X, int64_t Y, int64_t& bytes) {
-      bytes = std::min(msum * H * 2, momoe_wgrad_workspace_bytes(N, X, Y, msum));
-      return bytes > 0 ? at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(dev)) : Tensor();
-    };
-    int64_t ws_bytes = 0;
     if (need_w2) {
       out[2] = at::empty_like(W2);
-      const Tensor ws = workspace(H, D, ws_bytes);
-      MOMOE_CALL(momoe_wgrad, st, hst.data_ptr(), H, MOMOE_LAYOUT_TRANSPOSED, (const int32_t*)nullptr, Gy.data_ptr(),
+      Tensor ws_own;
+      void* const ws = ws2_bytes > 0 ? transients.take(ws2_bytes, ws_own) : nullptr;
+      MOMOE_CALL(momoe_wgrad, st, hst, H, MOMOE_LAYOUT_TRANSPOSED, (const int32_t*)nullptr, Gy.data_ptr(),
                  D, MOMOE_LAYOUT_ROWS, (const int32_t*)ib.idx(), ib.cumsums(), out[2].data_ptr(), M, N, H, D, msum,
-                 ws.defined() ? ws.data_ptr() : nullptr, ws_bytes);
+                 ws, ws2_bytes);
     }
-    hst.reset();
+    hst_own.reset();
     if (need_w1) {
       out[1] = at::empty_like(W1);
-      const Tensor ws = workspace(D, 2 * H, ws_bytes);
-      MOMOE_CALL(momoe_wgrad, st, x.data_ptr(), D, MOMOE_LAYOUT_ROWS, (const int32_t*)ib.idx(), gz.data_ptr(), msum,
+      Tensor ws_own;
+      void* const ws = ws1_bytes > 0 ? transients.take(ws1_bytes, ws_own) : nullptr;
+      MOMOE_CALL(momoe_wgrad, st, x.data_ptr(), D, MOMOE_LAYOUT_ROWS, (const int32_t*)ib.idx(), gz, msum,
                  MOMOE_LAYOUT_KBLOCKED, (const int32_t*)nullptr, ib.cumsums(), out[1].data_ptr(), M, N, D, 2 * H, msum,
-                 ws.defined() ? ws.data_ptr() : nullptr, ws_bytes);
+                 ws, ws1_bytes);
     }
     if (need_x) {
-      const Tensor gxs = empty_bf16({msum, D}, dev);
-      MOMOE_CALL(momoe_dgrad_x, st, gz.data_ptr(), W1.data_ptr(), ib.table_for(D, 2 * H), gxs.data_ptr(), M, D, H, N, msum);
+      Tensor gxs_own;
+      void* const gxs = transients.take(gxs_bytes, gxs_own);
+      MOMOE_CALL(momoe_dgrad_x, st, gz, W1.data_ptr(), ib.table_for(D, 2 * H), gxs, M, D, H, N, msum);
       Tensor Gx = empty_bf16({B, S, D}, dev);
-      MOMOE_CALL(momoe_combine, st, gxs.data_ptr(), ib.inv(), Gx.data_ptr(), M, D, K, msum);
+      MOMOE_CALL(momoe_combine, st, gxs, ib.inv(), Gx.data_ptr(), M, D, K, msum);
       out[0] = gdev == dev ? Gx : Gx.to(gdev);
     }
     return out;
