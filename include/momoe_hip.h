@@ -282,6 +282,18 @@ int momoe_dgrad_x(const void* gz_blocked, const void* Wl1_ND2H, const int32_t* t
                   void* gxs_MsumD, int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum,
                   void* stream);
 
+/* momoe_backward_tail: momoe_wgrad of both weights (Wl2 from hsT and the gathered Gy, Wl1 from the gathered x and gz) and
+ * momoe_dgrad_x in one launch, with the arguments that those take, and momoe_gs_scatter_tokens unless Gs_MN is NULL; every pointer to
+ * bf16 data on a 16-byte boundary.  For small
+ * calls: momoe_backward_tail_fits says (1 or 0), from the sizes alone, whether it takes them.
+ */
+int momoe_backward_tail_fits(int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum);
+int momoe_backward_tail(const void* hsT_GH32, int64_t ld_hsT, const void* Gy_MD, const void* x_MD,
+                        const void* gz_blocked, const void* Wl1_ND2H, const int32_t* idx_Msum,
+                        const int32_t* cumsums_N1, const int32_t* tile_table, void* GW2_NHD, void* GW1_ND2H,
+                        void* gxs_MsumD, const float* gs_part, int64_t nparts, float* Gs_MN,
+                        int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum, void* stream);
+
 /* momoe_wgrad replaces weights_update_kernel (momoe/momoe.py:356-412):
  *   GW[i][x][y] = bf16( sum over sorted rows r of expert i of A(r, x) * B(r, y) ).
  * Each operand comes in one of two layouts:

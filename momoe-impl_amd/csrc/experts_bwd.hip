@@ -4,7 +4,9 @@
 // gradient into [N, M].
 #include <algorithm>
 
+#include "dgrad_x.hpp"
 #include "gemm_span.hpp"
+#include "gs_tokens.hpp"
 
 namespace momoe {
 namespace {
@@ -239,16 +241,6 @@ __global__ __launch_bounds__(256) void swiglu_bwd_saved_kernel(SavedArgs p) {
     for (int q = gridDim.y + (t & 7); q < p.nparts; q += 8) p.gs_part[(int64_t)q * p.msum + r] = 0.0f;
 }
 
-struct DxArgs {
-  const bf16* gz;
-  const bf16* w1;
-  const int32_t* table;
-  bf16* gxs;
-  int D, H;
-  int64_t msum;
-  unsigned long long* clk;
-};
-
 // gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
 struct DxSpan {
   using G = WideSpan;
@@ -284,74 +276,7 @@ __global__ __launch_bounds__(kSpanThreads, 1) void dgrad_x_kernel(DxArgs p) {
   trace.finish();
 }
 
-// gxs = gz . Wl1^T: contraction over the 2H contiguous columns of both operands.
-template <class G>
-struct DxProg {
-  static constexpr int FM = G::FM, BN = G::COLS;
-  static constexpr bool MAY_ONCE = false;
-  using BlockedA = RBlockedDma<G::AROWS>;  // sorted rows of the k-blocked gz
-  using RowsB = RDma<BN>;                  // weight rows, k-contiguous
-  using Ring = StageRing<BlockedA, RowsB, G::STAGES>;
-  struct Prep {};
-  const DxArgs& p;
-  const int ktiles, wn;
-
-  __device__ __forceinline__ void gather(const TileCoord&, Prep&) const {}
-  __device__ __forceinline__ void late(const TileCoord&, Prep&) const {}
-  __device__ __forceinline__ void setup(const TileCoord& t, const Prep&, BlockedA& A, RowsB& B) const {
-    const int D = p.D, H2 = 2 * p.H;
-    const bf16* w = p.w1 + (int64_t)t.expert * D * H2;
-    const int d0 = t.tn * BN;
-    A.init(p.gz, p.msum, t.row0, t.rows);
-    B.init(w, [&](int r, int) { return (uint32_t)min(d0 + r, D - 1) * (uint32_t)(2 * H2); });
-  }
-  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x16 (&acc)[FN][FM], const Prep&, bf16* epi) const {
-    const int D = p.D;
-    const RowStager<2> stager(epi);
-    const int d0 = tc.tn * BN + wn * 64;  // first output column of this wave
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      if (i >= tc.na) break;
-#pragma unroll
-      for (int f = 0; f < FN; ++f)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          stager.put(f, q, pack_bf16x4(acc[f][i][4 * q], acc[f][i][4 * q + 1],
-                                       acc[f][i][4 * q + 2], acc[f][i][4 * q + 3]));
-      stager.flush([&](int row, int col) -> bf16* {
-        const int rl = (tc.mbase + 32 * i) + row;
-        if (rl >= tc.rows || d0 + col >= D) return nullptr;
-        return p.gxs + ((int64_t)tc.row0 + rl) * D + d0 + col;
-      });
-    }
-  }
-};
-
-template <class G, class Sched = TileSched>
-__device__ __forceinline__ void dgrad_x_tiles(const DxArgs& p) {
-  using Prog = DxProg<G>;
-  typename Prog::Ring ring(dyn_lds());
-  Sched sched(p.table, (p.D + G::COLS - 1) / G::COLS, MOMOE_TILE_ROWS);
-  const int wn = wave_id() % G::WCOLS;
-  const int n_org[FN] = {wn * 64, wn * 64 + 32};
-  Prog prog{p, (2 * p.H) / kBK, wn};
-  run_row_tiles<Prog::FM, FN>(prog, sched, ring, n_org);
-}
-
-__device__ __forceinline__ void dgrad_x_by_table(const DxArgs& p) {
-  if (TileSched::tile_rows_of(p.table) > StdTiles::MAX_ROWS) dgrad_x_tiles<TallTiles>(p);
-  else dgrad_x_tiles<StdTiles>(p);
-}
-__global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) {
-  const ClockTrace trace(p.clk);
-  if (__builtin_expect(narrow_tiles_fit(p.table, (p.D + NarrowTiles::COLS - 1) / NarrowTiles::COLS), 1))
-    dgrad_x_tiles<NarrowTiles, OneGeometrySched<NarrowTiles>>(p);
-  else
-    dgrad_x_by_table(p);
-  trace.finish();
-}
-constexpr size_t kDxLds = std::max(DxProg<TallTiles>::Ring::BYTES, DxProg<StdTiles>::Ring::BYTES);
-constexpr size_t kDxNarrowLds = std::max(DxProg<NarrowTiles>::Ring::BYTES, kDxLds);
+__global__ __launch_bounds__(kThreads, 2) void dgrad_x_narrow_kernel(DxArgs p) { dgrad_x_short(p); }
 
 // dL/ds [N][M] from the partial row sums in sorted order.  One workgroup per (expert, kGsTokens
 // tokens) writes its piece whole, zeros included, through LDS: every line of the matrix is stored
@@ -390,59 +315,9 @@ __global__ __launch_bounds__(256) void gs_scatter_kernel(const float* __restrict
   for (int m = m0 + t; m < m1; m += 256) gs[(int64_t)expert * M + m] = piece[m - m0];
 }
 
-// The same with the experts of a token next to each other, as a router that works on [tokens, experts] hands them over: dL/ds in
-// the layout of s needs no copy.  A workgroup writes a tile of 64 tokens x 16 experts whole, half a wavefront an expert.
-// Bound by latency, a chain of prefix sum -> token of a row -> its partial sums: an expert of up to 256 rows is read
-// as it is, a larger one probed at 32 places at a time until that many are left, and partial sums are loaded eight at
-// a time.  In us, the kernel above and the copy behind it -> this: 1024 tokens x 32 experts of 128 rows 9.1 -> 4.3, 8192 x 128
-// of 512 18.5 -> 9.1, 16384 x 64, four of them with every token, 55 -> 10; 128 x 8 5.9 -> 2.8.
-constexpr int kGsTileTokens = 64, kGsTileExperts = 16, kGsLanes = 32;
-
-__global__ __launch_bounds__(kGsLanes * kGsTileExperts) void gs_scatter_tokens_kernel(
-    const float* __restrict__ part, int nparts, const int32_t* __restrict__ idx, const int32_t* __restrict__ cumsums,
-    float* __restrict__ gs, int M, int N, int64_t msum) {
-  constexpr int THREADS = kGsLanes * kGsTileExperts, ROUNDS = 8, AT_ONCE = 8;
-  __shared__ float tile[kGsTileTokens][kGsTileExperts + 1];
-  const int t = threadIdx.x, e = t / kGsLanes, s = t % kGsLanes, e0 = blockIdx.y * kGsTileExperts, expert = min(e0 + e, N - 1);
-  const int m0 = blockIdx.x * kGsTileTokens, m1 = min(M, m0 + kGsTileTokens);
-  const int limit = cumsums[N] > msum ? 0 : (int)msum;  // as above
-  const int c0 = min(cumsums[expert], limit), rows = e0 + e < N ? min(cumsums[expert + 1], limit) - c0 : 0;
-  for (int i = t; i < kGsTileTokens * (kGsTileExperts + 1); i += THREADS) (&tile[0][0])[i] = 0.0f;
-  int lo = 0, hi = rows;  // the rows of the tile's tokens, 64 at most, lie in [lo, hi)
-  for (int probes = 0; probes < 6 && __any(hi - lo > ROUNDS * kGsLanes); ++probes) {
-    const int step = (hi - lo + kGsLanes - 1) / kGsLanes, probe = lo + (s + 1) * step - 1;
-    const bool is = step > 0 && probe < hi;
-    const int m = is ? idx[c0 + probe] : m1;
-    const int below = __popc((uint32_t)(__ballot(is && m < m0) >> (t & 32)));
-    const int before_end = __popc((uint32_t)(__ballot(is && m < m1) >> (t & 32)));
-    hi = min(hi, lo + (before_end + 1) * step);
-    lo += below * step;
-  }
-  __syncthreads();
-  for (; lo < hi; lo += ROUNDS * kGsLanes) {  // (once, if no token is listed twice)
-    int m[ROUNDS];
-#pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) m[j] = idx[c0 + min(lo + s + j * kGsLanes, hi - 1)];
-#pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) {
-      const int r = lo + s + j * kGsLanes;
-      if (r >= hi || m[j] < m0 || m[j] >= m1) continue;
-      float v = 0.0f;
-      for (int q0 = 0; q0 < nparts; q0 += AT_ONCE) {
-        float p[AT_ONCE];
-#pragma unroll
-        for (int q = 0; q < AT_ONCE; ++q) p[q] = part[(int64_t)min(q0 + q, nparts - 1) * msum + c0 + r];
-#pragma unroll
-        for (int q = 0; q < AT_ONCE; ++q) v += q0 + q < nparts ? p[q] : 0.0f;
-      }
-      tile[m[j] - m0][e] = v;
-    }
-  }
-  __syncthreads();
-  for (int i = t; i < kGsTileTokens * kGsTileExperts; i += THREADS) {
-    const int m = m0 + i / kGsTileExperts, x = i % kGsTileExperts;
-    if (m < M && e0 + x < N) gs[(int64_t)m * N + e0 + x] = tile[i / kGsTileExperts][x];
-  }
+__global__ __launch_bounds__(kGsThreads) void gs_scatter_tokens_kernel(GsTokensArgs p) {
+  __shared__ GsTile tile;
+  gs_scatter_tokens(p, blockIdx.x, blockIdx.y, tile);
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -528,8 +403,8 @@ extern "C" int momoe_gs_scatter_tokens(const float* gs_part, int64_t nparts, con
   const int64_t across = cdiv64(N, kGsTileExperts);
   if (Msum >= (1ll << 31) || M >= (1ll << 31) - kGsTileTokens || across > 65535) return MOMOE_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)cdiv64(M, kGsTileTokens), (unsigned)across);
-  gs_scatter_tokens_kernel<<<grid, kGsLanes * kGsTileExperts, 0, (hipStream_t)stream>>>(
-      gs_part, (int)nparts, idx_Msum, cumsums_N1, Gs_MN, (int)M, (int)N, Msum);
+  gs_scatter_tokens_kernel<<<grid, kGsThreads, 0, (hipStream_t)stream>>>(
+      {gs_part, (int)nparts, idx_Msum, cumsums_N1, Gs_MN, (int)M, (int)N, Msum});
   return launch_status();
 }
 

@@ -324,7 +324,9 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     auto scratch_bytes = [&](bool need, int64_t X, int64_t Y) {
       return need ? std::min(u_bytes, momoe_wgrad_workspace_bytes(N, X, Y, msum)) : 0;
     };
-    const int64_t ws2_bytes = scratch_bytes(need_w2, H, D), ws1_bytes = scratch_bytes(need_w1, D, 2 * H);
+    // small: both weight gradients and dL/dx in one launch
+    const bool tail = need_w1 && need_w2 && need_x && momoe_backward_tail_fits(M, D, H, N, msum) != 0;
+    const int64_t ws2_bytes = scratch_bytes(need_w2 && !tail, H, D), ws1_bytes = scratch_bytes(need_w1 && !tail, D, 2 * H);
     Transients transients(dev, {u_bytes, gz_bytes, hst_bytes, parts_bytes, ws2_bytes, ws1_bytes, gxs_bytes});
     Tensor u_own, gz_own, hst_own, parts_own;
     void* const u = transients.take(u_bytes, u_own);
@@ -356,11 +358,13 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
            gs_part, nparts, M, D, H, N, msum);
     }
     u_own.reset();
+    float* gs_tail = nullptr;
     if (need_s) {
       // in the layout of s, where autograd keeps it without a copy
       if (s.stride(0) == 1 && s.stride(1) == N) {
         out[4] = empty_f32({M, N}, dev).t();
-        call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part, nparts,
+        if (tail) gs_tail = out[4].data_ptr<float>();
+        else call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part, nparts,
              (const int32_t*)ib.idx(), (const int32_t*)ib.cumsums(), out[4].data_ptr<float>(), M, N, msum);
       } else {
         out[4] = empty_f32({N, M}, dev);
@@ -368,10 +372,19 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                    out[4].data_ptr<float>(), M, N, msum);
       }
     }
-    parts_own.reset();
+    if (!tail) parts_own.reset();
 
-    if (need_w2) {
-      out[2] = at::empty_like(W2);
+    if (need_w2) out[2] = at::empty_like(W2);
+    if (need_w1 && tail) out[1] = at::empty_like(W1);
+    Tensor gxs_own;
+    void* gxs = nullptr;
+    if (tail) {
+      gxs = transients.take(gxs_bytes, gxs_own);
+      MOMOE_CALL(momoe_backward_tail, st, hst, H, Gy.data_ptr(), x.data_ptr(), gz, W1.data_ptr(), (const int32_t*)ib.idx(),
+                 (const int32_t*)ib.cumsums(), (const int32_t*)ib.table_for(D, 2 * H), out[2].data_ptr(), out[1].data_ptr(), gxs,
+                 (const float*)gs_part, nparts, gs_tail, M, D, H, N, msum);
+    }
+    if (need_w2 && !tail) {
       Tensor ws_own;
       void* const ws = ws2_bytes > 0 ? transients.take(ws2_bytes, ws_own) : nullptr;
       MOMOE_CALL(momoe_wgrad, st, hst, H, MOMOE_LAYOUT_TRANSPOSED, (const int32_t*)nullptr, Gy.data_ptr(),
@@ -379,7 +392,7 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                  ws, ws2_bytes);
     }
     hst_own.reset();
-    if (need_w1) {
+    if (need_w1 && !tail) {
       out[1] = at::empty_like(W1);
       Tensor ws_own;
       void* const ws = ws1_bytes > 0 ? transients.take(ws1_bytes, ws_own) : nullptr;
@@ -388,9 +401,10 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                  ws, ws1_bytes);
     }
     if (need_x) {
-      Tensor gxs_own;
-      void* const gxs = transients.take(gxs_bytes, gxs_own);
-      MOMOE_CALL(momoe_dgrad_x, st, gz, W1.data_ptr(), ib.table_for(D, 2 * H), gxs, M, D, H, N, msum);
+      if (!tail) {
+        gxs = transients.take(gxs_bytes, gxs_own);
+        MOMOE_CALL(momoe_dgrad_x, st, gz, W1.data_ptr(), ib.table_for(D, 2 * H), gxs, M, D, H, N, msum);
+      }
       Tensor Gx = empty_bf16({B, S, D}, dev);
       MOMOE_CALL(momoe_combine, st, gxs, ib.inv(), Gx.data_ptr(), M, D, K, msum);
       out[0] = gdev == dev ? Gx : Gx.to(gdev);

@@ -13,7 +13,9 @@
 // (takes_span_loop).  The k-values past the expert's last row are zeroed in registers on the M side.
 #include <algorithm>
 
+#include "dgrad_x.hpp"
 #include "gemm_span.hpp"
+#include "gs_tokens.hpp"
 
 namespace momoe {
 namespace {
@@ -70,6 +72,7 @@ __device__ __forceinline__ int item_cost(int ks) {
   return ks > 0 ? max(4, ks + (ks & 1)) + kStoreCost : 0;
 }
 constexpr int kMinChunk = 64;     // an expert is never cut into pieces of fewer k-stages
+constexpr int64_t kTailBytes = 64 << 20;  // momoe_backward_tail_fits
 
 // How one expert's rows are dealt out: `splits` equal pieces of `chunk` k-stages (the last
 // may be shorter).  An expert is cut once it holds at least 2*kc stages, so a piece has
@@ -492,7 +495,7 @@ __device__ __forceinline__ f32x4* partial_piece(float* ws, int slot, int i, int 
 }
 
 template <bool CUT, class AOp, class BOp, int FM, int FN>
-__global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(WgradArgs p) {
+__device__ __forceinline__ void wgrad_tiles(WgradArgs p) {
   drop_rows_of_an_overflowed_routing(p);
   using Ring = StageRing<AOp, BOp, kStages>;
   static_assert(Ring::BYTES == kRingBytes, "ring size assumed by the launch");
@@ -563,6 +566,34 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(WgradArgs p) {
     tc = nx;
   }
   trace.finish();
+}
+
+template <bool CUT, class AOp, class BOp, int FM, int FN>
+__global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(WgradArgs p) {
+  wgrad_tiles<CUT, AOp, BOp, FM, FN>(p);
+}
+
+// The end of a small call's backward, three products that do not need each other and dL/ds, in one launch: the workgroups of a
+// part start on the CUs that the part before it leaves, where a launch would wait for its last tile and then find its work.  The
+// longest first.  A step in us, four launches -> one: 128 tokens, D = 128, H = 64, N = 8, K = 2, which is bound by the host's launches,
+// 111 -> 95; 1024 tokens, D = 1024, H = 512, N = 32, K = 4 159 -> 152.
+struct TailArgs {
+  WgradArgs w1, w2;
+  DxArgs dx;
+  GsTokensArgs gs;  // gs.gs == nullptr: not wanted
+};
+__global__ __launch_bounds__(kThreads, 2) void backward_tail_kernel(TailArgs p) {
+  if (blockIdx.y == 0) wgrad_tiles<false, RowsOperand, BlockedRowsOperand, 4, 2>(p.w1);
+  else if (blockIdx.y == 1) dgrad_x_short(p.dx);
+  else if (blockIdx.y == 2) wgrad_tiles<false, TransposedOperand, RowsOperand, 4, 2>(p.w2);
+  else if (p.gs.gs != nullptr) {
+    static_assert(kGsThreads == kThreads, "the same workgroups");
+    const int across = (p.gs.M + kGsTileTokens - 1) / kGsTileTokens, tiles = across * ((p.gs.N + kGsTileExperts - 1) / kGsTileExperts);
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+      gs_scatter_tokens(p.gs, t % across, t / across, *(GsTile*)dyn_lds());
+      __syncthreads();
+    }
+  }
 }
 
 // Adds up the partial tiles of the experts that wgrad_kernel cut into pieces and stores the
@@ -1212,4 +1243,42 @@ extern "C" int momoe_wgrad(const void* A, int64_t lda, int a_layout, const int32
   if (bt) return tile::launch<tile::RowsOperand, tile::TransposedOperand, 2, 4>(a, can_cut, st);
   if (bk) return tile::launch<tile::RowsOperand, tile::BlockedRowsOperand, 4, 2>(a, can_cut, st);
   return tile::launch<tile::RowsOperand, tile::RowsOperand, 4, 2>(a, can_cut, st);
+}
+
+extern "C" int momoe_backward_tail_fits(int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum) {
+  if (M <= 0 || D <= 0 || H <= 0 || N <= 0 || Msum <= 0 || D % kBK != 0 || H % kBK != 0 || N > kMaxWgradExperts) return 0;
+  // no expert can be long enough to be cut, and what the three products read and write besides the weights is little: it is
+  // all there at once
+  if (M >= 2 * kMinChunk * kBK || D > (1 << 20) || H > (1 << 19)) return 0;
+  const int64_t bytes = (Msum * (2 * H + D) + momoe_padded_rows(Msum, N) * H) * (int64_t)sizeof(bf16);
+  if (bytes > kTailBytes || D * H * 4 >= (1ll << 32) || cdiv64(D, BX) * cdiv64(2 * H, BY) * N >= (1ll << 31)) return 0;
+  return !takes_span_loop(Msum, N, D, 2 * H, true) && !takes_span_loop(Msum, N, H, D, false) && !takes_span_tiles(Msum, N, D, 2 * H);
+}
+
+extern "C" int momoe_backward_tail(const void* hsT_GH32, int64_t ld_hsT, const void* Gy_MD, const void* x_MD,
+                                   const void* gz_blocked, const void* Wl1_ND2H, const int32_t* idx_Msum,
+                                   const int32_t* cumsums_N1, const int32_t* tile_table, void* GW2_NHD, void* GW1_ND2H,
+                                   void* gxs_MsumD, const float* gs_part, int64_t nparts, float* Gs_MN, int64_t M, int64_t D,
+                                   int64_t H, int64_t N, int64_t Msum, void* stream) {
+  for (const void* p : {hsT_GH32, Gy_MD, x_MD, gz_blocked, Wl1_ND2H, (const void*)GW2_NHD, (const void*)GW1_ND2H, (const void*)gxs_MsumD})
+    if (!p || ((uintptr_t)p & 15)) return MOMOE_ERR_BAD_ARG;
+  if (!idx_Msum || !cumsums_N1 || !tile_table || ld_hsT < H || ld_hsT % 8 != 0) return MOMOE_ERR_BAD_ARG;
+  if (Gs_MN != nullptr && (!gs_part || nparts <= 0)) return MOMOE_ERR_BAD_ARG;
+  if (!momoe_backward_tail_fits(M, D, H, N, Msum)) return MOMOE_ERR_UNSUPPORTED;
+  auto weight = [&](const void* a, int64_t lda, const int32_t* ga, const void* b, int64_t ldb, const int32_t* gb, void* gw, int64_t X,
+                    int64_t Y) {
+    return WgradArgs{(const bf16*)a, lda, ga, (const bf16*)b, ldb, gb, cumsums_N1, (bf16*)gw, nullptr, 0x7fffffff, (int)N, (int)X,
+                     (int)Y, (int)cdiv64(X, BX), (int)cdiv64(Y, BY), (int)Msum, clock_trace_buffer()};
+  };
+  const tile::TailArgs a{weight(x_MD, D, idx_Msum, gz_blocked, Msum, nullptr, GW1_ND2H, D, 2 * H),
+                         weight(hsT_GH32, ld_hsT, nullptr, Gy_MD, D, idx_Msum, GW2_NHD, H, D),
+                         {(const bf16*)gz_blocked, (const bf16*)Wl1_ND2H, tile_table, (bf16*)gxs_MsumD, (int)D, (int)H, Msum,
+                          clock_trace_buffer()},
+                         {gs_part, (int)nparts, idx_Msum, cumsums_N1, Gs_MN, (int)M, (int)N, Msum}};
+  constexpr size_t lds = std::max(tile::kWgradLds, kDxNarrowLds);
+  static LdsLimit once;
+  if (!allow_lds(tile::backward_tail_kernel, lds, once)) return MOMOE_ERR_LAUNCH;
+  // (as many workgroups in a row as a launch has, a multiple of 8: a part's are on the XCDs that they take themselves to be on)
+  tile::backward_tail_kernel<<<dim3(persistent_grid(), Gs_MN != nullptr ? 4 : 3), kThreads, lds, (hipStream_t)stream>>>(a);
+  return launch_status();
 }

@@ -75,6 +75,9 @@ _SIGNATURES = {
     "momoe_gate_router_fwd": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "momoe_gate_wgrad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "momoe_gate_wgrad": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
+    "momoe_backward_tail_fits": (_int, [_i64] * 5),
+    "momoe_backward_tail": (_int, [_p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64,
+                                   _p]),
     "momoe_gate_dgrad": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "momoe_bias_update": (_int, [_p, ctypes.c_float, ctypes.c_float, _i64, _p, _p]),
 }
@@ -361,6 +364,14 @@ def wgrad(A, a_gather, B, b_gather, cumsums, GW_NXY, M, Msum, workspace_bytes=No
     _call("momoe_wgrad", _ptr(A), lda, int(a_transposed), _ptr(a_gather), _ptr(B),
           ldb, 2 if b_kblocked else int(b_transposed), _ptr(b_gather), _ptr(cumsums), _ptr(GW_NXY), M, N, X, Y,
           Msum, _ptr(ws), workspace_bytes, _stream())
+
+
+def backward_tail(hsT, Gy_MD, x_MD, gz, Wl1_ND2H, idx, cumsums, table, GW2_NHD, GW1_ND2H, gxs, gs_part=None, Gs_MN=None):
+    _need_cuda(hsT, Gy_MD, x_MD, gz, Wl1_ND2H)
+    (M, D), (N, H, _) = x_MD.shape, GW2_NHD.shape
+    _call("momoe_backward_tail", _ptr(hsT), hsT.shape[1], _ptr(Gy_MD), _ptr(x_MD), _ptr(gz), _ptr(Wl1_ND2H), _ptr(idx),
+          _ptr(cumsums), _ptr(table), _ptr(GW2_NHD), _ptr(GW1_ND2H), _ptr(gxs), _ptr(gs_part),
+          0 if gs_part is None else gs_part.shape[0], _ptr(Gs_MN), M, D, H, N, idx.numel(), _stream())
 
 
 # ---------------------------------------------------------------- router

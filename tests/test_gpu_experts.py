@@ -720,6 +720,58 @@ def test_forward_mode_is_refused(grad):
             moe(dual)
 
 
+@pytest.mark.parametrize("M,D,H,N,K,skew", [
+    (1, 32, 32, 1, 1, None), (128, 128, 64, 8, 2, None), (300, 352, 288, 9, 3, 1.8),  # a tile each, tiles cut off, few rows
+    (4095, 64, 32, 70, 3, 1.8), (1000, 1056, 544, 16, 1, None),   # the most tokens; more tiles than workgroups
+])
+@pytest.mark.parametrize("overflow", [False, True])
+def test_tail_of_a_small_backward(M, D, H, N, K, skew, overflow):
+    """The three products in one launch are those of the three launches, bit for bit."""
+    from momoe_amd import _hip
+    dev, msum = "cuda:0", M * K
+    assert _hip._lib.momoe_backward_tail_fits(M, D, H, N, msum) == 1
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=2, skew=skew)
+    if overflow:
+        if N == K:
+            return
+        mask = torch.ones_like(mask)  # more pairs than rows: no rows for anyone, the gradients are zeros
+    elif N > 2:
+        mask[N // 2] = 0  # an expert without tokens
+    rnd = lambda *size: torch.randn(*size, generator=torch.Generator(device=dev).manual_seed(5), device=dev).to(torch.bfloat16)
+    new = lambda *size: torch.full(size, 7, device=dev, dtype=torch.bfloat16)
+    x, Gy, W1 = (t.to(dev, torch.bfloat16) for t in (x, dy, W1))
+    ib = _hip.index_build(mask.to(dev), K)
+    idx, cumsums, table = (ib[k] for k in ("idx_Msum", "cumsums_N", "tile_table"))
+    gz, hsT = rnd(2 * H // 32, msum, 32), rnd(_hip.padded_rows(msum, N) // 32, H, 32)
+    GW1, GW2, gxs = new(N, D, 2 * H), new(N, H, D), new(msum, D)
+    part = torch.randn(3, msum, device=dev)
+    Gs, wantGs = torch.full((M, N), 7.0, device=dev), torch.full((M, N), 7.0, device=dev)
+    _hip.backward_tail(hsT, Gy, x, gz, W1, idx, cumsums, table, GW2, GW1, gxs, part, Gs)
+    _hip.gs_scatter_tokens(part, idx, cumsums, wantGs)
+    want1, want2, wantx = new(N, D, 2 * H), new(N, H, D), new(msum, D)
+    _hip.wgrad(hsT, None, Gy, idx, cumsums, want2, M, msum, workspace_bytes=0, a_transposed=True)
+    _hip.wgrad(x, idx, gz, None, cumsums, want1, M, msum, workspace_bytes=0, b_kblocked=True)
+    _hip.dgrad_x(gz, W1, table, wantx, M)
+    results = ((GW1, want1), (GW2, want2), (gxs, wantx), (Gs, wantGs))
+    assert all(torch.equal(a, b) for a, b in results)
+    for a, _ in results:
+        a.fill_(7)  # (what there are no rows for stays as it was)
+    _hip.backward_tail(hsT, Gy, x, gz, W1, idx, cumsums, table, GW2, GW1, gxs)  # without dL/ds
+    assert (Gs == 7).all() and all(torch.equal(a, b) for a, b in results[:3])
+
+
+def test_calls_that_are_too_large_for_the_tail():
+    from momoe_amd import _hip
+    fits = _hip._lib.momoe_backward_tail_fits
+    assert fits(4096, 64, 32, 70, 4096 * 3) == 0         # an expert may be cut
+    assert fits(1024, 1024, 512, 32, 4096) == 1 and fits(1024, 8192, 4096, 32, 4096) == 0  # 64 MiB of rows
+    assert fits(2048, 512, 256, 16, 8192) == 0           # the loop of 64 rows a stage
+    assert fits(128, 100, 64, 8, 256) == 0
+    z = torch.zeros(16, device="cuda:0", dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        _hip._call("momoe_backward_tail", *[z.data_ptr() if i != 1 else 64 for i in range(12)], None, 0, None, 128, 100, 64, 8, 256, _hip._stream())
+
+
 @pytest.mark.parametrize("M,N,K,nparts,skew", [
     (1, 1, 1, 1, None), (63, 15, 4, 2, None), (64, 16, 4, 1, None), (65, 17, 17, 3, None),  # tiles of 64 x 16
     (256, 1, 1, 1, None), (257, 2, 2, 1, None),    # 256 rows are read without probing
