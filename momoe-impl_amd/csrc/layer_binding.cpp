@@ -501,7 +501,7 @@ Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
 Tensor gate_input_gradient(const Tensor& G_x, const Tensor& G_logit, const Tensor& Wg) {
   const int64_t M = G_logit.size(0), N = G_logit.size(1), D = Wg.size(0);
   const auto packed = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0; };
-  if (D % 8 != 0 || N % 8 != 0 || M >= 65535 * 128 || !packed(Wg) || (G_x.defined() && !packed(G_x)) || at::GradMode::is_enabled() ||
+  if (momoe_gate_wgrad_workspace_bytes(M, D, N) < 0 || M >= 65535 * 128 || !packed(Wg) || (G_x.defined() && !packed(G_x)) || at::GradMode::is_enabled() ||
       at::autocast::is_autocast_enabled(at::kCUDA))
     return G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
   const Tensor out = empty_bf16({M, D}, G_logit.device());

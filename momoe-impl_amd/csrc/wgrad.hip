@@ -1249,7 +1249,7 @@ extern "C" int momoe_backward_tail_fits(int64_t M, int64_t D, int64_t H, int64_t
   if (M <= 0 || D <= 0 || H <= 0 || N <= 0 || Msum <= 0 || D % kBK != 0 || H % kBK != 0 || N > kMaxWgradExperts) return 0;
   // no expert can be long enough to be cut, and what the three products read and write besides the weights is little: it is
   // all there at once
-  if (M >= 2 * kMinChunk * kBK || D > (1 << 20) || H > (1 << 19)) return 0;
+  if (M >= 2 * kMinChunk * kBK || Msum < M || D > (1 << 20) || H > (1 << 19)) return 0;
   const int64_t bytes = (Msum * (2 * H + D) + momoe_padded_rows(Msum, N) * H) * (int64_t)sizeof(bf16);
   if (bytes > kTailBytes || D * H * 4 >= (1ll << 32) || cdiv64(D, BX) * cdiv64(2 * H, BY) * N >= (1ll << 31)) return 0;
   return !takes_span_loop(Msum, N, D, 2 * H, true) && !takes_span_loop(Msum, N, H, D, false) && !takes_span_tiles(Msum, N, D, 2 * H);

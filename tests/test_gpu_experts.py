@@ -767,6 +767,7 @@ def test_calls_that_are_too_large_for_the_tail():
     assert fits(1024, 1024, 512, 32, 4096) == 1 and fits(1024, 8192, 4096, 32, 4096) == 0  # 64 MiB of rows
     assert fits(2048, 512, 256, 16, 8192) == 0           # the loop of 64 rows a stage
     assert fits(128, 100, 64, 8, 256) == 0
+    assert fits(4000, 1 << 20, 32, 1, 1) == 0            # gathered rows are addressed with 32 bits
     z = torch.zeros(16, device="cuda:0", dtype=torch.bfloat16)
     with pytest.raises(RuntimeError):
         _hip._call("momoe_backward_tail", *[z.data_ptr() if i != 1 else 64 for i in range(12)], None, 0, None, 128, 100, 64, 8, 256, _hip._stream())

@@ -341,3 +341,14 @@ def test_module_routes_alike_by_either_product(M, D, N, pitch):
             with torch.set_grad_enabled(grad):
                 out = r(x[None], bias)
             assert torch.equal(out[1], want[0]) and torch.equal(out[2], want[1].T)
+
+
+def test_gate_gradients_of_widths_that_the_kernels_refuse():
+    import momoe_amd
+    D, N = (1 << 20) + 8, 8
+    x, Wg = _whole_numbers(3, D, N)
+    r = momoe_amd.TopKRouter(D, N, 2, 0, Wg_DN=Wg)
+    x.requires_grad_()
+    out = r(x[None], torch.zeros(N, device="cuda:0"))
+    out[2].square().sum().backward()
+    assert x.grad.shape == x.shape and r.Wg_DN.grad.shape == Wg.shape
