@@ -455,31 +455,37 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
   const c10::DeviceGuard guard(dev);
   Routed r;
   r.x_MD = x_BSD.reshape({M, D}).to(dev, at::kBFloat16);
+  // Few tokens: the product in the library's kernel, whose launch alone takes the host 18 us
+  const int64_t ws_bytes = momoe_gate_router_workspace_bytes(M, D, N);
+  const auto aligned = [](const Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  const bool own = ws_bytes >= 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && Wg.dim() == 2 && Wg.size(0) == D &&
+                   Wg.size(1) == N && Wg.is_contiguous() && aligned(Wg) && aligned(r.x_MD) && r.x_MD.stride(1) == 1 &&
+                   r.x_MD.stride(0) >= D && r.x_MD.stride(0) % 8 == 0;
+  // Other products come first of all: the GPU has work while the host allocates
+  Tensor logits;
+  if (!own) {
+    // autocast may give the product another type than its operands'; the kernel reads two of them
+    logits = at::mm(r.x_MD, Wg).contiguous();
+    if (logits.scalar_type() != at::kBFloat16 && logits.scalar_type() != at::kFloat)
+      throw_python(PyExc_AssertionError, std::string("the gate logits must be bfloat16 or float32, got ") +
+                                             c10::toString(logits.scalar_type()));
+    TORCH_CHECK(logits.size(1) == N, "Wg_DN must have N = ", N, " columns");
+  }
   const Tensor bias = biases.to(dev, at::kFloat).contiguous();
   TORCH_CHECK(bias.numel() == N, "biases_N must have N = ", N, " elements");
-  TORCH_CHECK(r.x_MD.size(1) == Wg.size(0) && Wg.size(1) == N, "Wg_DN must be [", D, ", N = ", N, "]");
   r.mask = at::empty({N, M}, at::TensorOptions().dtype(at::kInt).device(dev));
   r.s_MN = empty_f32({M, N}, dev);
   r.p_sel = empty_f32({M, N}, dev);
   r.norms = empty_f32({2, M}, dev);  // per token: sum over the selected, over the shared experts
   float* norms = r.norms.data_ptr<float>();
   const hipStream_t st = stream_of(dev);
-  // Few tokens: the product in the library's kernel, whose launch alone takes the host 18 us
-  const int64_t ws_bytes = momoe_gate_router_workspace_bytes(M, D, N);
-  const auto aligned = [](const Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
-  if (ws_bytes >= 0 && !at::autocast::is_autocast_enabled(at::kCUDA) && Wg.is_contiguous() && aligned(Wg) && aligned(r.x_MD) &&
-      r.x_MD.stride(1) == 1 && r.x_MD.stride(0) >= D && r.x_MD.stride(0) % 8 == 0) {
+  if (own) {
     const Tensor ws = empty_f32({ws_bytes / 4}, dev);
     MOMOE_CALL(momoe_gate_router_fwd, st, r.x_MD.data_ptr(), r.x_MD.stride(0), Wg.data_ptr(), bias.data_ptr<float>(), M, D, N, K,
                Ks, r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M,
                ws.data_ptr(), ws_bytes);
     return r;
   }
-  // autocast may give the product another type than its operands'; the kernel reads two of them
-  const Tensor logits = at::mm(r.x_MD, Wg).contiguous();
-  if (logits.scalar_type() != at::kBFloat16 && logits.scalar_type() != at::kFloat)
-    throw_python(PyExc_AssertionError, std::string("the gate logits must be bfloat16 or float32, got ") +
-                                           c10::toString(logits.scalar_type()));
   MOMOE_CALL(momoe_router_fwd, st, logits.data_ptr(), logits.scalar_type() == at::kFloat, bias.data_ptr<float>(), M, N, K, Ks,
              r.mask.data_ptr<int32_t>(), r.s_MN.data_ptr<float>(), r.p_sel.data_ptr<float>(), norms, norms + M);
   return r;

@@ -343,6 +343,27 @@ def test_module_routes_alike_by_either_product(M, D, N, pitch):
             assert torch.equal(out[1], want[0]) and torch.equal(out[2], want[1].T)
 
 
+def test_the_product_of_many_tokens_comes_before_what_the_host_allocates():
+    """The GPU has the product to work on while the host goes on with the call."""
+    import momoe_amd
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Recorded(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    names = []
+    x, Wg = _whole_numbers(3000, 64, 8)
+    r, bias = momoe_amd.TopKRouter(64, 8, 2, 0, Wg_DN=Wg), torch.zeros(8, device="cuda:0")
+    with torch.no_grad(), Recorded():
+        r(x[None], bias)
+    assert "mm" in names and "empty" in names and names.index("mm") < names.index("empty")
+    r.Wg_DN.data = Wg.flatten()  # what is no matrix is refused as the product refuses it
+    with pytest.raises(RuntimeError):
+        r(x[None, :5], bias)
+
+
 def test_gate_gradients_of_widths_that_the_kernels_refuse():
     import momoe_amd
     D, N = (1 << 20) + 8, 8
