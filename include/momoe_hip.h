@@ -361,7 +361,7 @@ int momoe_router_fwd(const void* logits_MN, int logits_f32, const float* biases_
  * x_MD bf16 with row pitch ldx elements, Wg_DN bf16 contiguous; D, N and ldx multiples of 8; x_MD, Wg_DN and workspace on
  * 16-byte boundaries.
  * workspace: momoe_gate_router_workspace_bytes(M, D, N) bytes of device memory (-1: sizes that it does not take, among them
- * more tokens than a product that is not split over the contraction handles as fast).
+ * more tokens or partial sums than a product that is not split over the contraction handles as fast).
  */
 int64_t momoe_gate_router_workspace_bytes(int64_t M, int64_t D, int64_t N);
 int momoe_gate_router_fwd(const void* x_MD, int64_t ldx, const void* Wg_DN, const float* biases_N,

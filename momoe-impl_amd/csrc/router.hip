@@ -58,12 +58,15 @@ __device__ __forceinline__ float wave_max_all(float v) {
 
 // Gate logits of few tokens: x . Wg split over the contraction, a workgroup for each 128 k-values of 128 experts and 64
 // tokens; the router's kernel adds up the fp32 partial products and rounds the sums to bf16, as a product of its own would.
-// Bound by the latency of one round of loads; with many tokens by the partial sums, so up to kGateMaxRows rows of them, and up to
-// kGateMaxTokens, where the host's time for a library product stops to show.  Product and router in
-// a graph, us, a library product -> this: 1 token, D = 2048, N = 128 10.9 -> 8.9, 16 11.5 -> 9.6, 64 18.0 -> 10.9, 512
-// 12.6 -> 12.6, 1000 21.0 -> 15.1; 33, 1000, 200 27.8 -> 11.7; 1000, 1024, 32 10.1 -> 8.2; 2000, 2048, 64 14.6 -> 15.4; 4096,
-// 2048, 128 23.9 -> 30.4; 2048, 1024, 96 17.1 -> 14.6; 1513, 128, 96 9.9 -> 10.4.
-constexpr int64_t kGateMaxTokens = 2048, kGateMaxRows = 16 * 1024;
+// Bound by the latency of one round of loads; with many tokens by the partial sums, so up to kGateMaxRows rows and kGateMaxSums
+// of them (8 MiB), and up to kGateMaxTokens, where the host's time for a library product stops to show.  Product and router in
+// a graph, us, a library product -> this: 1 token, D = 2048, N = 128 10.3 -> 8.2, 16 10.7 -> 8.8, 64 17.4 -> 9.9, 512
+// 11.7 -> 12.0, 1000 20.5 -> 14.3; 1000, 1024, 128 15.6 -> 12.2; 2048, 1024, 128 15.9 -> 14.9; 2048, 512, 16 8.0 -> 8.5;
+// 2048, 128, 128 10.7 -> 11.7; 512, 1024, 256 15.2 -> 15.0; 256, 1024, 512 19.3 -> 20.8.  Whole calls, H = 64, K = 4, forward | forward and backward,
+// below the line: 2000, 512, 256 52.2 -> 50.8 | 201 -> 174; 512, 2048, 256 81.7 -> 79.8 | 283 -> 273; 256, 2048, 512 171.9 -> 167.8 |
+// 511 -> 503; above it: 2000, 1024, 256 67.6 -> 72.3 | 220 -> 216; 1000, 2048, 256 85.1 -> 88.6 | 291 -> 285; 2000, 1024, 512
+// 131.4 -> 143.1 | 380 -> 379.  Past the tokens and rows, in a graph: 2000, 2048, 64 14.6 -> 15.4; 4096, 2048, 128 23.9 -> 30.4.
+constexpr int64_t kGateMaxTokens = 2048, kGateMaxRows = 16 * 1024, kGateMaxSums = kGateMaxRows * 128;
 constexpr int kGateTokens = 64, kGateDepth = 2 * GateStage::ROWS;
 
 struct GateFwdArgs {
@@ -421,7 +424,7 @@ extern "C" int momoe_router_fwd(const void* logits_MN, int logits_f32, const flo
 
 extern "C" int64_t momoe_gate_router_workspace_bytes(int64_t M, int64_t D, int64_t N) {
   if (M <= 0 || D <= 0 || N <= 0 || D % 8 != 0 || N % 8 != 0 || N > 64 * kMaxCols || D > (1 << 20) || M > kGateMaxTokens ||
-      cdiv64(D, kGateDepth) * M > kGateMaxRows)
+      cdiv64(D, kGateDepth) * M > kGateMaxRows || cdiv64(D, kGateDepth) * M * N > kGateMaxSums)
     return -1;
   return cdiv64(D, kGateDepth) * M * N * (int64_t)sizeof(float);
 }

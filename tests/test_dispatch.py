@@ -100,3 +100,14 @@ def test_loop_of_the_recomputing_gemm(rows_per_expert, N, D, H, stage):
 
 def test_no_recomputing_launch():
     assert _hip._lib.momoe_recompute_stage_k(0, 8, 64, 64) == 0
+
+
+# (times of either side beside the constants, csrc/router.hip)
+@pytest.mark.parametrize("M,D,N,own", [
+    (1024, 2048, 128, True), (1025, 2048, 128, False), (2048, 1024, 128, True), (2049, 128, 8, False),  # rows of partial sums, tokens
+    (1024, 1024, 256, True), (1025, 1024, 256, False), (1000, 2048, 256, False), (2048, 128, 256, True),  # partial sums
+    (512, 1024, 512, True), (513, 1024, 512, False), (2000, 1024, 512, False), (1, 8192, 512, True),
+])
+def test_tokens_of_the_router_with_its_product(M, D, N, own):
+    parts = -(-D // 128)
+    assert _hip._lib.momoe_gate_router_workspace_bytes(M, D, N) == (parts * M * N * 4 if own else -1)
