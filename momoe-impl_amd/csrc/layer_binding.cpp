@@ -505,11 +505,16 @@ Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
   return out;
 }
 
-// G_x + G_logits . Wg^T [M, D]; G_x may be undefined.  (The library copies G_x in front of its product.)
+// G_x + G_logits . Wg^T [M, D]; G_x may be undefined.  (The library copies G_x in front of its product, and takes the host 14 us
+// more.)  The own kernel reloads both operands for every 32 experts and waits for each: with more than 128 experts it takes
+// products of up to 2^31 terms.  In a graph, us, the library's -> own: 8192 tokens, D = 2048, N = 128 32.4 -> 26.1; 32768, 4096, 128
+// 232 -> 198; 1000, 1024, 256 9.9 -> 12.3; 8192, 1024, 256 25.8 -> 22.9; 4096, 1024, 512 20.4 -> 20.8; 1000, 2048, 512 14.2 -> 19.7; past
+// the line 4096, 2048, 512 29.7 -> 36.6; 8192, 2048, 256 35.3 -> 39.7; 32768, 4096, 512 299 -> 511.
 Tensor gate_input_gradient(const Tensor& G_x, const Tensor& G_logit, const Tensor& Wg) {
   const int64_t M = G_logit.size(0), N = G_logit.size(1), D = Wg.size(0);
   const auto packed = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0; };
-  if (momoe_gate_wgrad_workspace_bytes(M, D, N) < 0 || M >= 65535 * 128 || !packed(Wg) || (G_x.defined() && !packed(G_x)) || at::GradMode::is_enabled() ||
+  const bool sizes = momoe_gate_wgrad_workspace_bytes(M, D, N) >= 0 && M < 65535 * 128 && (N <= 128 || M * D * N <= (1ll << 31));
+  if (!sizes || !packed(Wg) || (G_x.defined() && !packed(G_x)) || at::GradMode::is_enabled() ||
       at::autocast::is_autocast_enabled(at::kCUDA))
     return G_x.defined() ? at::addmm(G_x, G_logit, Wg.t()) : at::mm(G_logit, Wg.t());
   const Tensor out = empty_bf16({M, D}, G_logit.device());

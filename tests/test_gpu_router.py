@@ -291,6 +291,35 @@ def test_gate_gradients_of_the_module(M, D, N, pitch):
             assert got.shape == want.shape and (got - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
+def _gate_backward(M, D, N):
+    """The entry points that a backward of the router calls, and its gradients next to the library's."""
+    import momoe_amd
+    from momoe_amd import _hip
+    g = torch.Generator(device="cuda:0").manual_seed(D)
+    r = momoe_amd.TopKRouter(D, N, 4, 0, Wg_DN=torch.randn(D, N, generator=g, device="cuda:0").to(torch.bfloat16) / D ** 0.5)
+    x = torch.randn(1, M, D, generator=g, device="cuda:0").to(torch.bfloat16).requires_grad_()
+    w = torch.randn(M, N, generator=g, device="cuda:0").T
+
+    def grads(recorded):
+        out = r(x, torch.zeros(N, device="cuda:0"))
+        return torch.autograd.grad((out[2], out[0]), (r.Wg_DN, x), (w, x.detach()), create_graph=recorded)
+
+    want = grads(True)  # (a backward that is itself recorded takes the library's products)
+    with _hip.kernel_timer() as kt:
+        got = grads(False)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and (a.double() - b.double()).abs().max() <= 2.0 ** -7 * b.double().abs().max()
+    return [n for n, _ in kt.durations_ms()]
+
+
+@pytest.mark.parametrize("M,D,N,own", [
+    (5000, 8192, 128, True), (64, 512, 256, True), (4096, 1024, 512, True), (2048, 4096, 256, True),
+    (2049, 4096, 256, False), (4097, 1024, 512, False),  # more than 128 experts and 2^31 terms
+])
+def test_which_product_takes_the_gradient_of_the_tokens(M, D, N, own):
+    assert ("momoe_gate_dgrad" in _gate_backward(M, D, N)) == own
+
+
 def _whole_numbers(M, D, N, pitch=0):
     """x, Wg whose products have the same sum in any order: small whole numbers."""
     g = torch.Generator().manual_seed(M + D + N)
