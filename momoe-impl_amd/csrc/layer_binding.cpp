@@ -492,13 +492,18 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
 }
 
 // x^T . G_logits [D, N].  (The library's product has few tiles and one long contraction for each, and takes the host 18 us where
-// two launches take 8: 300 tokens, D = 512, N = 64 7.5 us of the GPU against 8.3; 1024, 1024, 32 9.3, 8.9; 2000, 1120, 48 19.6, 9.4;
-// 8192, 2048, 128 59, 20.6.)  The library's where autograd records it.
+// two launches take 8: 300 tokens, D = 512, N = 64 9.0 us of the GPU against 9.6; 1024, 1024, 32 9.3, 8.9; 2000, 1120, 48 19.6, 9.4;
+// 8192, 2048, 128 60, 22.)  The own kernel's partial sums are D * N at the least, written and read for each range of tokens:
+// it takes more than 2^18 results only from a token for 1024 of them on, and up to 2^20, where the library's tiles
+// fill the chip.  Us, 300 tokens, D = 2048, N = 128 10.3, 11.6; 1000, 2048, 256 14.7, 15.9; 4096, 2048, 256 29.9, 21.3;
+// 4096, 2048, 512 31.3, 30.3; past the line 300, 2048, 256 9.2, 12.8; 1000, 2048, 512 15.4, 21.9; 4096, 4096, 512 38.5, 47.1; 8192, 8192, 512
+// 91, 147 (though 32768, 4096, 512 302, 276).  And the library's where autograd records it.
 Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
   const int64_t M = x.size(0), D = x.size(1), N = G_logit.size(1);
   const int64_t bytes = momoe_gate_wgrad_workspace_bytes(M, D, N);
+  const bool sizes = bytes >= 0 && (D * N <= 1 << 18 || (D * N <= 1 << 20 && D * N <= 1024 * M));
   const bool rows = x.stride(1) == 1 && x.stride(0) >= D && x.stride(0) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0;
-  if (bytes < 0 || !rows || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA)) return at::mm(x.t(), G_logit);
+  if (!sizes || !rows || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA)) return at::mm(x.t(), G_logit);
   const Tensor out = empty_bf16({D, N}, x.device()), ws = empty_f32({bytes / 4}, x.device());
   MOMOE_CALL(momoe_gate_wgrad, stream_of(x.device()), x.data_ptr(), x.stride(0), G_logit.data_ptr(), out.data_ptr(), M, D, N,
              ws.data_ptr(), bytes);

@@ -320,6 +320,15 @@ def test_which_product_takes_the_gradient_of_the_tokens(M, D, N, own):
     assert ("momoe_gate_dgrad" in _gate_backward(M, D, N)) == own
 
 
+@pytest.mark.parametrize("M,D,N,own", [
+    (1, 2048, 128, True), (1, 2056, 128, False),                              # up to 2^18 results: any number of tokens
+    (512, 2048, 256, True), (511, 2048, 256, False), (1024, 2048, 512, True),  # more: by tokens
+    (4200, 4096, 264, False),                                                # more than 2^20
+])
+def test_which_product_takes_the_gradient_of_the_gate_weights(M, D, N, own):
+    assert ("momoe_gate_wgrad" in _gate_backward(M, D, N)) == own
+
+
 def _whole_numbers(M, D, N, pitch=0):
     """x, Wg whose products have the same sum in any order: small whole numbers."""
     g = torch.Generator().manual_seed(M + D + N)
