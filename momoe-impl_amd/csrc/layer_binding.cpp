@@ -365,9 +365,11 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
       // in the layout of s, where autograd keeps it without a copy
       if (s.stride(0) == 1 && s.stride(1) == N) {
         out[4] = empty_f32({M, N}, dev).t();
-        if (tail) gs_tail = out[4].data_ptr<float>();
-        else call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part, nparts,
-             (const int32_t*)ib.idx(), (const int32_t*)ib.cumsums(), out[4].data_ptr<float>(), M, N, msum);
+        if (tail)
+          gs_tail = out[4].data_ptr<float>();
+        else
+          call("momoe_gs_scatter", st, momoe_gs_scatter_tokens, gs_part, nparts, (const int32_t*)ib.idx(),
+               (const int32_t*)ib.cumsums(), out[4].data_ptr<float>(), M, N, msum);
       } else {
         out[4] = empty_f32({N, M}, dev);
         MOMOE_CALL(momoe_gs_scatter, st, gs_part, nparts, ib.idx(), ib.cumsums(),
@@ -375,7 +377,9 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
       }
     }
     if (!tail) parts_own.reset();
-
+    // (what the joined launch reads and writes is all there at once: the peak is the weight gradients, gz, s*h, the partial sums and
+    // gxs, where one launch after the other has dL/dx in the place of s*h: 11.6 MiB more at 700 tokens, D = 2048, H = 768, N = 128,
+    // K = 8, and always less than the 64 MiB of momoe_backward_tail_fits)
     if (need_w2) out[2] = at::empty_like(W2);
     if (need_w1 && tail) out[1] = at::empty_like(W1);
     Tensor gxs_own;
@@ -385,6 +389,8 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
       MOMOE_CALL(momoe_backward_tail, st, hst, H, Gy.data_ptr(), x.data_ptr(), gz, W1.data_ptr(), (const int32_t*)ib.idx(),
                  (const int32_t*)ib.cumsums(), (const int32_t*)ib.table_for(D, 2 * H), out[2].data_ptr(), out[1].data_ptr(), gxs,
                  (const float*)gs_part, nparts, gs_tail, M, D, H, N, msum);
+      parts_own.reset();
+      gz_own.reset();
     }
     if (need_w2 && !tail) {
       Tensor ws_own;

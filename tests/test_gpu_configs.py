@@ -115,6 +115,36 @@ def test_memory_contract_at_the_headline_layer(M, D, H, N, K):
     assert held[100] <= msum * (2 * H + D) * 2 + 1 * MiB
 
 
+@pytest.mark.parametrize("M,D,H,N,K", [
+    (700, 2048, 768, 128, 8),   # 52 of the 64 MiB that the joined launch takes: s*h counts
+    (3000, 2048, 128, 16, 1),   # dL/dx is more than s*h and the partial sums
+])
+def test_memory_of_a_small_backward(M, D, H, N, K):
+    """The launch that ends a small backward has the weight gradients, gz, s*h, the partial dL/ds and gxs next to each other; the
+    combine behind it the weight gradients, gxs and dL/dx only."""
+    import momoe_amd
+    from momoe_amd import _hip
+    dev, msum = "cuda:0", M * K
+    assert _hip._lib.momoe_backward_tail_fits(M, D, H, N, msum) == 1
+    x, dy, W1, W2, mask, s = device_layer_inputs(M, D, H, N, K)
+    layer = momoe_amd.MoMoE(D, H, N, K, Wl1_ND2H=W1, Wl2_NHD=W2)
+    x = x.reshape(1, M, D).requires_grad_()
+    s = s.T.contiguous().to(dev).T.requires_grad_()
+    y, _ = layer(x, mask.to(dev), s)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(dy.reshape(1, M, D))
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated() - base
+    gz, gxs, Gx, weights = msum * 4 * H, msum * 2 * D, M * 2 * D, 6 * D * H * N
+    hs, parts = _hip.padded_rows(msum, N) * 2 * H, _hip._lib.momoe_gs_parts(H, N, msum) * msum * 4
+    print(f"[memory] backward of {M} tokens: {peak / MiB:.2f} MiB, {(peak - weights) / MiB:.2f} without the weight gradients")
+    # dL/ds in either, and 512 bytes that the allocator may add to each of at most eight buffers
+    assert peak <= weights + 4 * M * N + gxs + max(gz + hs + parts, Gx) + 8 * 512
+
+
+
 @pytest.mark.parametrize("sp", [0, 100])
 def test_tokens_with_fewer_than_k_experts(sp):
     # The layer's precondition is exactly K experts per token (momoe/momoe.py:831).  With fewer,
