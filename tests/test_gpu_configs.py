@@ -132,16 +132,17 @@ def test_memory_of_a_small_backward(M, D, H, N, K):
     s = s.T.contiguous().to(dev).T.requires_grad_()
     y, _ = layer(x, mask.to(dev), s)
     torch.cuda.synchronize()
-    base = torch.cuda.memory_allocated()
+    # bytes asked for: what the allocator adds depends on the blocks it has
+    asked = lambda which: torch.cuda.memory_stats()["requested_bytes.all." + which]
+    base = asked("current")
     torch.cuda.reset_peak_memory_stats()
     y.backward(dy.reshape(1, M, D))
     torch.cuda.synchronize()
-    peak = torch.cuda.max_memory_allocated() - base
+    peak = asked("peak") - base
     gz, gxs, Gx, weights = msum * 4 * H, msum * 2 * D, M * 2 * D, 6 * D * H * N
     hs, parts = _hip.padded_rows(msum, N) * 2 * H, _hip._lib.momoe_gs_parts(H, N, msum) * msum * 4
     print(f"[memory] backward of {M} tokens: {peak / MiB:.2f} MiB, {(peak - weights) / MiB:.2f} without the weight gradients")
-    # dL/ds in either, and 512 bytes that the allocator may add to each of at most eight buffers
-    assert peak <= weights + 4 * M * N + gxs + max(gz + hs + parts, Gx) + 8 * 512
+    assert peak <= weights + 4 * M * N + gxs + max(gz + hs + parts, Gx)  # (dL/ds in either)
 
 
 
