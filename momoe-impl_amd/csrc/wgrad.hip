@@ -72,7 +72,12 @@ __device__ __forceinline__ int item_cost(int ks) {
   return ks > 0 ? max(4, ks + (ks & 1)) + kStoreCost : 0;
 }
 constexpr int kMinChunk = 64;     // an expert is never cut into pieces of fewer k-stages
-constexpr int64_t kTailBytes = 64 << 20;  // momoe_backward_tail_fits
+// momoe_backward_tail_fits: what gz, gxs and s*h may take together, a bound on memory: one launch was the faster one in each of
+// 37 calls of 0.2 to 63 MiB and up to 4095 tokens, with even loads, loads that fall as rank^-0.5 and rank^-1.8 and shared experts.  A
+// step near the line, us, four launches -> one: 4095 tokens, D = 512, H = 2048, N = 64, K = 1 (60 MiB) rank^-1.8 361 -> 282; 4095, 4096,
+// 1024, 16, 1 (57) even 626 -> 599, rank^-1.8 766 -> 645; 700, 2048, 768, 128, 8 (52) 912 -> 893, 677 -> 641; 1500, 1024, 512,
+// 64, 8 (61), two of them shared, 407 -> 337; 300, 4096, 1408, 128, 8 (49) rank^-0.5 3040 -> 2955.
+constexpr int64_t kTailBytes = 64 << 20;
 
 // How one expert's rows are dealt out: `splits` equal pieces of `chunk` k-stages (the last
 // may be shorter).  An expert is cut once it holds at least 2*kc stages, so a piece has
@@ -574,19 +579,25 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(WgradArgs p) {
 }
 
 // The end of a small call's backward, three products that do not need each other and dL/ds, in one launch: the workgroups of a
-// part start on the CUs that the part before it leaves, where a launch would wait for its last tile and then find its work.  The
-// longest first.  A step in us, four launches -> one: 128 tokens, D = 128, H = 64, N = 8, K = 2, which is bound by the host's launches,
-// 111 -> 95; 1024 tokens, D = 1024, H = 512, N = 32, K = 4 159 -> 152.
+// part start on the CUs that the part before it leaves, where a launch would wait for its last tile and then find its work.  In the
+// order that launches of their own would have, the longer weight gradient first: dL/dx between the two took weights that do
+// not fit the last-level cache past the time of four launches.  A step in us, four launches | dL/dx second | as it is:
+// 1500 tokens, D = 2048, H = 512, N = 96, K = 4 517 | 529 | 515; 64, 4096, 1408, 128, 8 2715 | 2754 | 2682; 1024, 1024, 512, 128, 8
+// 347 | 352 | 341; 1024, 1024, 512, 32, 4 153 | 142 | 142; 128, 128, 64, 8, 2, bound by the host's launches, 117 | 108 | 108; loads that fall as
+// rank^-1.8 4095, 1024, 512, 64, 2 373 | 273 | 241; 3000, 2048, 1408, 128, 1 716 | 634 | 666; 1500, 2048, 512, 96, 4 417 | 372 | 377.
 struct TailArgs {
   WgradArgs w1, w2;
   DxArgs dx;
   GsTokensArgs gs;  // gs.gs == nullptr: not wanted
 };
 __global__ __launch_bounds__(kThreads, 2) void backward_tail_kernel(TailArgs p) {
-  if (blockIdx.y == 0) wgrad_tiles<false, RowsOperand, BlockedRowsOperand, 4, 2>(p.w1);
-  else if (blockIdx.y == 1) dgrad_x_short(p.dx);
-  else if (blockIdx.y == 2) wgrad_tiles<false, TransposedOperand, RowsOperand, 4, 2>(p.w2);
-  else if (p.gs.gs != nullptr) {
+  if (blockIdx.y == 0) {
+    wgrad_tiles<false, RowsOperand, BlockedRowsOperand, 4, 2>(p.w1);
+  } else if (blockIdx.y == 1) {
+    wgrad_tiles<false, TransposedOperand, RowsOperand, 4, 2>(p.w2);
+  } else if (blockIdx.y == 2) {
+    dgrad_x_short(p.dx);
+  } else if (p.gs.gs != nullptr) {
     static_assert(kGsThreads == kThreads, "the same workgroups");
     const int across = (p.gs.M + kGsTileTokens - 1) / kGsTileTokens, tiles = across * ((p.gs.N + kGsTileExperts - 1) / kGsTileExperts);
     for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
