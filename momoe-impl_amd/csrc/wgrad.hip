@@ -74,8 +74,8 @@ __device__ __forceinline__ int item_cost(int ks) {
 constexpr int kMinChunk = 64;     // an expert is never cut into pieces of fewer k-stages
 // momoe_backward_tail_fits: what gz, gxs and s*h may take together, a bound on memory: one launch was the faster one in each of
 // 37 calls of 0.2 to 63 MiB and up to 4095 tokens, with even loads, loads that fall as rank^-0.5 and rank^-1.8 and shared experts.  A
-// step near the line, us, four launches -> one: 4095 tokens, D = 512, H = 2048, N = 64, K = 1 (60 MiB) rank^-1.8 361 -> 282; 4095, 4096,
-// 1024, 16, 1 (57) even 626 -> 599, rank^-1.8 766 -> 645; 700, 2048, 768, 128, 8 (52) 912 -> 893, 677 -> 641; 1500, 1024, 512,
+// step near the line, us, four launches -> one: 4095 tokens, D = 512, H = 2048, N = 64, K = 1 (60 MiB) rank^-1.8 361 -> 282; 4095,
+// 4096, 1024, 16, 1 (57) even 626 -> 599, rank^-1.8 766 -> 645; 700, 2048, 768, 128, 8 (52) 912 -> 893, 677 -> 641; 1500, 1024, 512,
 // 64, 8 (61), two of them shared, 407 -> 337; 300, 4096, 1408, 128, 8 (49) rank^-0.5 3040 -> 2955.
 constexpr int64_t kTailBytes = 64 << 20;
 
@@ -579,24 +579,28 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(WgradArgs p) {
 }
 
 // The end of a small call's backward, three products that do not need each other and dL/ds, in one launch: the workgroups of a
-// part start on the CUs that the part before it leaves, where a launch would wait for its last tile and then find its work.  In the
-// order that launches of their own would have, the longer weight gradient first: dL/dx between the two took weights that do
-// not fit the last-level cache past the time of four launches.  A step in us, four launches | dL/dx second | as it is:
-// 1500 tokens, D = 2048, H = 512, N = 96, K = 4 517 | 529 | 515; 64, 4096, 1408, 128, 8 2715 | 2754 | 2682; 1024, 1024, 512, 128, 8
-// 347 | 352 | 341; 1024, 1024, 512, 32, 4 153 | 142 | 142; 128, 128, 64, 8, 2, bound by the host's launches, 117 | 108 | 108; loads that fall as
-// rank^-1.8 4095, 1024, 512, 64, 2 373 | 273 | 241; 3000, 2048, 1408, 128, 1 716 | 634 | 666; 1500, 2048, 512, 96, 4 417 | 372 | 377.
+// part start on the CUs that the part before it leaves, where a launch would wait for its last tile and then find its work.
+// The Wl1 gradient first, the longest; then dL/dx, whose few long tiles would end the launch late, or behind both weight gradients
+// where the weights, or their gradients, do not fit the last-level cache (kBeyondCache): between them it took even loads
+// past the time of four launches.  A step in us, four launches | dL/dx second | last: 1024 tokens, D = 1024, H = 512, N = 32, K = 4
+// 153 | 142 | 142; 307, 512, 1728, 32, 6 186 | 163 | 170; 868, 256, 1152, 128, 6, two of them shared, 320 | 271 | 280; 128, 128, 64, 8,
+// 2, bound by the host's launches, 117 | 108 | 108; past the line 1500, 2048, 512, 96, 4 517 | 529 | 515; 64, 4096, 1408, 128, 8
+// 2715 | 2754 | 2682; 1024, 1024, 512, 128, 8 347 | 352 | 341; 195, 1792, 2016, 64, 6 949 | 962 | 924; and, loads that fall as
+// rank^-1.8, 700, 2048, 768, 128, 8 677 | 668 | 641; 1500, 2048, 512, 96, 4 417 | 372 | 377; 3000, 2048, 1408, 128, 1 716 | 634 | 666.
+constexpr unsigned kTailParts = 4;
 struct TailArgs {
   WgradArgs w1, w2;
   DxArgs dx;
   GsTokensArgs gs;  // gs.gs == nullptr: not wanted
+  unsigned dx_part;
 };
 __global__ __launch_bounds__(kThreads, 2) void backward_tail_kernel(TailArgs p) {
   if (blockIdx.y == 0) {
     wgrad_tiles<false, RowsOperand, BlockedRowsOperand, 4, 2>(p.w1);
-  } else if (blockIdx.y == 1) {
-    wgrad_tiles<false, TransposedOperand, RowsOperand, 4, 2>(p.w2);
-  } else if (blockIdx.y == 2) {
+  } else if (blockIdx.y == p.dx_part) {
     dgrad_x_short(p.dx);
+  } else if (blockIdx.y < kTailParts - 1) {
+    wgrad_tiles<false, TransposedOperand, RowsOperand, 4, 2>(p.w2);
   } else if (p.gs.gs != nullptr) {
     static_assert(kGsThreads == kThreads, "the same workgroups");
     const int across = (p.gs.M + kGsTileTokens - 1) / kGsTileTokens, tiles = across * ((p.gs.N + kGsTileExperts - 1) / kGsTileExperts);
@@ -1271,7 +1275,8 @@ extern "C" int momoe_backward_tail(const void* hsT_GH32, int64_t ld_hsT, const v
                                    const int32_t* cumsums_N1, const int32_t* tile_table, void* GW2_NHD, void* GW1_ND2H,
                                    void* gxs_MsumD, const float* gs_part, int64_t nparts, float* Gs_MN, int64_t M, int64_t D,
                                    int64_t H, int64_t N, int64_t Msum, void* stream) {
-  for (const void* p : {hsT_GH32, Gy_MD, x_MD, gz_blocked, Wl1_ND2H, (const void*)GW2_NHD, (const void*)GW1_ND2H, (const void*)gxs_MsumD})
+  for (const void* p : {hsT_GH32, Gy_MD, x_MD, gz_blocked, Wl1_ND2H, (const void*)GW2_NHD, (const void*)GW1_ND2H,
+                        (const void*)gxs_MsumD})
     if (!p || ((uintptr_t)p & 15)) return MOMOE_ERR_BAD_ARG;
   if (!idx_Msum || !cumsums_N1 || !tile_table || ld_hsT < H || ld_hsT % 8 != 0) return MOMOE_ERR_BAD_ARG;
   if (Gs_MN != nullptr && (!gs_part || nparts <= 0)) return MOMOE_ERR_BAD_ARG;
@@ -1285,11 +1290,13 @@ extern "C" int momoe_backward_tail(const void* hsT_GH32, int64_t ld_hsT, const v
                          weight(hsT_GH32, ld_hsT, nullptr, Gy_MD, D, idx_Msum, GW2_NHD, H, D),
                          {(const bf16*)gz_blocked, (const bf16*)Wl1_ND2H, tile_table, (bf16*)gxs_MsumD, (int)D, (int)H, Msum,
                           clock_trace_buffer()},
-                         {gs_part, (int)nparts, idx_Msum, cumsums_N1, Gs_MN, (int)M, (int)N, Msum}};
+                         {gs_part, (int)nparts, idx_Msum, cumsums_N1, Gs_MN, (int)M, (int)N, Msum},
+                         3 * D * H * N * (int64_t)sizeof(bf16) >= kBeyondCache ? 2u : 1u};
   constexpr size_t lds = std::max(tile::kWgradLds, kDxNarrowLds);
   static LdsLimit once;
   if (!allow_lds(tile::backward_tail_kernel, lds, once)) return MOMOE_ERR_LAUNCH;
   // (as many workgroups in a row as a launch has, a multiple of 8: a part's are on the XCDs that they take themselves to be on)
-  tile::backward_tail_kernel<<<dim3(persistent_grid(), Gs_MN != nullptr ? 4 : 3), kThreads, lds, (hipStream_t)stream>>>(a);
+  const dim3 grid(persistent_grid(), tile::kTailParts - (Gs_MN != nullptr ? 0 : 1));
+  tile::backward_tail_kernel<<<grid, kThreads, lds, (hipStream_t)stream>>>(a);
   return launch_status();
 }
