@@ -723,6 +723,7 @@ def test_forward_mode_is_refused(grad):
 @pytest.mark.parametrize("M,D,H,N,K,skew", [
     (1, 32, 32, 1, 1, None), (128, 128, 64, 8, 2, None), (300, 352, 288, 9, 3, 1.8),  # a tile each, tiles cut off, few rows
     (4095, 64, 32, 70, 3, 1.8), (1000, 1056, 544, 16, 1, None),   # the most tokens; more tiles than workgroups
+    (64, 1056, 544, 80, 3, None),  # weights past the last-level cache: dL/dx behind both weight gradients
 ])
 @pytest.mark.parametrize("overflow", [False, True])
 def test_tail_of_a_small_backward(M, D, H, N, K, skew, overflow):
@@ -733,7 +734,7 @@ def test_tail_of_a_small_backward(M, D, H, N, K, skew, overflow):
     x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=2, skew=skew)
     if overflow:
         if N == K:
-            return
+            pytest.skip("a token cannot have more than all experts")
         mask = torch.ones_like(mask)  # more pairs than rows: no rows for anyone, the gradients are zeros
     elif N > 2:
         mask[N // 2] = 0  # an expert without tokens
