@@ -404,10 +404,18 @@ def test_the_product_of_many_tokens_comes_before_what_the_host_allocates():
 
 def test_gate_gradients_of_widths_that_the_kernels_refuse():
     import momoe_amd
-    D, N = (1 << 20) + 8, 8
-    x, Wg = _whole_numbers(3, D, N)
-    r = momoe_amd.TopKRouter(D, N, 2, 0, Wg_DN=Wg)
-    x.requires_grad_()
-    out = r(x[None], torch.zeros(N, device="cuda:0"))
-    out[2].square().sum().backward()
-    assert x.grad.shape == x.shape and r.Wg_DN.grad.shape == Wg.shape
+    from momoe_amd import _hip
+    M, D, N, K = 3, (1 << 20) + 8, 8, 2
+    x, Wg = _whole_numbers(M, D, N)
+    r = momoe_amd.TopKRouter(D, N, K, 0, Wg_DN=Wg)
+    w = torch.randn(M, N, generator=torch.Generator(device="cuda:0").manual_seed(3), device="cuda:0").T
+    xg = x[None].clone().requires_grad_()
+    out = r(xg, torch.zeros(N, device="cuda:0"))
+    GW, Gx = torch.autograd.grad((out[2], out[0]), (r.Wg_DN, xg), (w, x[None]))
+    mask, s, p_sel, Ng, Ks = _hip.router_fwd(torch.mm(x, Wg), torch.zeros(N, device="cuda:0"), K, 0)
+    assert torch.equal(out[1], mask) and torch.equal(out[2], s.T)
+    G, xd, Wd = _hip.router_bwd(w, p_sel, s, Ng, Ks, mask, 0).double(), x.double(), Wg.double()
+    # one rounding to bf16 (2^-8), and of the sums in fp32
+    for got, want, terms in ((GW, xd.T @ G, xd.T.abs() @ G.abs()), (Gx[0], xd + G @ Wd.T, xd.abs() + G.abs() @ Wd.T.abs())):
+        assert got.shape == want.shape and ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * terms).all()
+
