@@ -96,9 +96,9 @@ Tensor empty_f32(at::IntArrayRef size, const at::Device& dev) {
 // Buffers that live no longer than the call: pieces of one allocation where they are few bytes in all, since an
 // allocation takes the host a microsecond and a small call is as long as its host work (in us of the host, a forward of 7 tokens
 // with its router 37.2 -> 34.8, the backward of 128 tokens 88 -> 81); allocations of their own, given back as soon as they are
-// done with, where their size counts.  Of a backward up to torch's own line between small allocations and large ones; a
-// forward of more than a quarter of that is no longer bound by its host, and runs faster where y takes the place of h, which
-// has just been written: 400 tokens, D = 384, H = 128, N = 64, K = 2 (0.83 MB) in one allocation 25.1 us, in several 24.8.
+// done with, where their size counts.  The line is torch's own between small allocations and large ones; forwards in a row below
+// it, us, in several -> in one: 7 tokens, D = 256, H = 128, N = 16, K = 2 19.8 -> 18.2; 128, 512, 128, 32, 2 21.9 -> 21.6; 150, 512, 128, 48, 4
+// 22.3 -> 22.1; 300, 512, 256, 16, 2 25.9 -> 25.4; 200, 256, 256, 96, 4 26.7 -> 26.6; 400, 384, 128, 64, 2 24.2 -> 24.1.
 class Transients {
   const at::Device dev_;
   Tensor block_;
@@ -106,11 +106,11 @@ class Transients {
   static int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
 
  public:
-  static constexpr int64_t kForward = 1 << 18, kBackward = 1 << 20;
-  Transients(const at::Device& dev, int64_t most, std::initializer_list<int64_t> sizes) : dev_(dev) {
+  Transients(const at::Device& dev, std::initializer_list<int64_t> sizes) : dev_(dev) {
+    constexpr int64_t kMost = 1 << 20;
     int64_t all = 0;
-    for (int64_t bytes : sizes) all += bytes <= most ? up(bytes) : 2 * most;
-    if (all <= most) block_ = bytes_of(all);
+    for (int64_t bytes : sizes) all += bytes <= kMost ? up(bytes) : 2 * kMost;
+    if (all <= kMost) block_ = bytes_of(all);
   }
   Tensor bytes_of(int64_t bytes) const { return at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(dev_)); }
   // the next of those sizes; `own` holds it if it is an allocation of its own
@@ -220,7 +220,7 @@ Forward experts_forward(const Tensor& x_BSD, const Tensor& Wl1, const Tensor& Wl
   // only the build itself needs these: its panel counts, the slot of every pair, and the counter
   // of tokens with another number of experts than K, which starts from zero if it is to be read
   const int64_t scratch_bytes = (4 + ((msum + 3) & ~(int64_t)3) + (ws_bytes + 3) / 4) * 4;
-  Transients transients(dev, Transients::kForward, {scratch_bytes, msum * H * 2, msum * D * 2});
+  Transients transients(dev, {scratch_bytes, msum * H * 2, msum * D * 2});
   Tensor counter, scratch, h_own, ys_own;
   int32_t* const build = (int32_t*)transients.take(scratch_bytes, scratch);
   int32_t* violations = build;
@@ -329,7 +329,7 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     // small: both weight gradients and dL/dx in one launch
     const bool tail = need_w1 && need_w2 && need_x && momoe_backward_tail_fits(M, D, H, N, msum) != 0;
     const int64_t ws2_bytes = scratch_bytes(need_w2 && !tail, H, D), ws1_bytes = scratch_bytes(need_w1 && !tail, D, 2 * H);
-    Transients transients(dev, Transients::kBackward, {u_bytes, gz_bytes, hst_bytes, parts_bytes, ws2_bytes, ws1_bytes, gxs_bytes});
+    Transients transients(dev, {u_bytes, gz_bytes, hst_bytes, parts_bytes, ws2_bytes, ws1_bytes, gxs_bytes});
     Tensor u_own, gz_own, hst_own, parts_own;
     void* const u = transients.take(u_bytes, u_own);
     MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u, M, D, H, N, msum);
@@ -502,8 +502,8 @@ Routed router_forward(const Tensor& x_BSD, const Tensor& Wg, const Tensor& biase
 // 8192, 2048, 128 60, 22.)  The own kernel's partial sums are D * N at the least, written and read for each range of tokens:
 // it takes more than 2^18 results only from a token for 1024 of them on, and up to 2^20, where the library's tiles
 // fill the chip.  Us, 300 tokens, D = 2048, N = 128 10.3, 11.6; 1000, 2048, 256 14.7, 15.9; 4096, 2048, 256 29.9, 21.3;
-// 4096, 2048, 512 31.3, 30.3; past the line 300, 2048, 256 9.2, 12.8; 1000, 2048, 512 15.4, 21.9; 4096, 4096, 512 38.5, 47.1; 8192, 8192, 512
-// 91, 147 (though 32768, 4096, 512 302, 276).  And the library's where autograd records it.
+// 4096, 2048, 512 31.3, 30.3; past the line 300, 2048, 256 9.2, 12.8; 1000, 2048, 512 15.4, 21.9; 4096, 4096, 512 38.5, 47.1; 8192,
+// 8192, 512 91, 147 (though 32768, 4096, 512 302, 276).  And the library's where autograd records it.
 Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
   const int64_t M = x.size(0), D = x.size(1), N = G_logit.size(1);
   const int64_t bytes = momoe_gate_wgrad_workspace_bytes(M, D, N);
@@ -519,8 +519,8 @@ Tensor gate_gradient(const Tensor& x, const Tensor& G_logit) {
 // G_x + G_logits . Wg^T [M, D]; G_x may be undefined.  (The library copies G_x in front of its product, and takes the host 14 us
 // more.)  The own kernel reloads both operands for every 32 experts and waits for each: with more than 128 experts it takes
 // products of up to 2^31 terms.  In a graph, us, the library's -> own: 8192 tokens, D = 2048, N = 128 32.4 -> 26.1; 32768, 4096, 128
-// 232 -> 198; 1000, 1024, 256 9.9 -> 12.3; 8192, 1024, 256 25.8 -> 22.9; 4096, 1024, 512 20.4 -> 20.8; 1000, 2048, 512 14.2 -> 19.7; past
-// the line 4096, 2048, 512 29.7 -> 36.6; 8192, 2048, 256 35.3 -> 39.7; 32768, 4096, 512 299 -> 511.
+// 232 -> 198; 1000, 1024, 256 9.9 -> 12.3; 8192, 1024, 256 25.8 -> 22.9; 4096, 1024, 512 20.4 -> 20.8; 1000, 2048, 512 14.2 -> 19.7;
+// past the line 4096, 2048, 512 29.7 -> 36.6; 8192, 2048, 256 35.3 -> 39.7; 32768, 4096, 512 299 -> 511.
 Tensor gate_input_gradient(const Tensor& G_x, const Tensor& G_logit, const Tensor& Wg) {
   const int64_t M = G_logit.size(0), N = G_logit.size(1), D = Wg.size(0);
   const auto packed = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0; };
