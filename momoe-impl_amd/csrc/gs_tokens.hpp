@@ -7,7 +7,8 @@ namespace momoe {
 namespace {
 
 // dL/ds [M][N] from the partial row sums in sorted order, the experts of a token next to each other, as a router that works on
-// [tokens, experts] hands the gate weights over: a gradient in their layout needs no copy.  A workgroup writes a tile of 64 tokens x 16 experts whole, half a wavefront an expert.
+// [tokens, experts] hands the gate weights over: a gradient in their layout needs no copy.  A workgroup writes a tile of
+// 64 tokens x 16 experts whole, half a wavefront an expert.
 // Bound by latency, a chain of prefix sum -> token of a row -> its partial sums: an expert of up to 256 rows is read
 // as it is, a larger one probed at 32 places at a time until that many are left, and partial sums are loaded eight at
 // a time.  In us, a scatter to [N][M] and the copy behind it -> this: 1024 tokens x 32 experts of 128 rows 9.1 -> 4.3, 8192 x 128
@@ -30,7 +31,8 @@ __device__ __forceinline__ void gs_scatter_tokens(const GsTokensArgs& p, int bx,
   constexpr int THREADS = kGsThreads, ROUNDS = 8, AT_ONCE = 8;
   const int t = threadIdx.x, e = t / kGsLanes, s = t % kGsLanes, e0 = by * kGsTileExperts, expert = min(e0 + e, p.N - 1);
   const int m0 = bx * kGsTileTokens, m1 = min(p.M, m0 + kGsTileTokens);
-  const int limit = p.cumsums[p.N] > p.msum ? 0 : (int)p.msum;  // more pairs than rows: the routing was refused (empty tile table), dL/ds is zero
+  // more pairs than rows: the routing was refused (empty tile table), dL/ds is zero
+  const int limit = p.cumsums[p.N] > p.msum ? 0 : (int)p.msum;
   const int c0 = min(p.cumsums[expert], limit), rows = e0 + e < p.N ? min(p.cumsums[expert + 1], limit) - c0 : 0;
   for (int i = t; i < kGsTileTokens * (kGsTileExperts + 1); i += THREADS) (&tile[0][0])[i] = 0.0f;
   int lo = 0, hi = rows;  // the rows of the tile's tokens, 64 at most, lie in [lo, hi)

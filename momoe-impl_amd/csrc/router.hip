@@ -2,8 +2,8 @@
 // part of the forward (everything after the gate GEMM) and the backward through
 // renormalisation and softmax.  One wavefront per token (lane j holds columns
 // j, j+64, ...), a workgroup per block of consecutive tokens so that the [N, M]
-// tensors (mask, dL/ds) are touched in whole lines.  HBM-bound: a few passes over
-// [M, N] fp32.
+// tensors (mask, dL/ds) are touched in whole lines where that counts.  HBM-bound: a few
+// passes over [M, N] fp32.
 #include <type_traits>
 
 #include "gate.hpp"
@@ -62,8 +62,8 @@ __device__ __forceinline__ float wave_max_all(float v) {
 // of them (8 MiB), and up to kGateMaxTokens, where the host's time for a library product stops to show.  Product and router in
 // a graph, us, a library product -> this: 1 token, D = 2048, N = 128 10.3 -> 8.2, 16 10.7 -> 8.8, 64 17.4 -> 9.9, 512
 // 11.7 -> 12.0, 1000 20.5 -> 14.3; 1000, 1024, 128 15.6 -> 12.2; 2048, 1024, 128 15.9 -> 14.9; 2048, 512, 16 8.0 -> 8.5;
-// 2048, 128, 128 10.7 -> 11.7; 512, 1024, 256 15.2 -> 15.0; 256, 1024, 512 19.3 -> 20.8.  Whole calls, H = 64, K = 4, forward | forward and backward,
-// below the line: 2000, 512, 256 52.2 -> 50.8 | 201 -> 174; 512, 2048, 256 81.7 -> 79.8 | 283 -> 273; 256, 2048, 512 171.9 -> 167.8 |
+// 2048, 128, 128 10.7 -> 11.7; 512, 1024, 256 15.2 -> 15.0; 256, 1024, 512 19.3 -> 20.8.  Whole calls, H = 64, K = 4,
+// forward | forward and backward, below the line: 2000, 512, 256 52.2 -> 50.8 | 201 -> 174; 512, 2048, 256 81.7 -> 79.8 | 283 -> 273; 256, 2048, 512 171.9 -> 167.8 |
 // 511 -> 503; above it: 2000, 1024, 256 67.6 -> 72.3 | 220 -> 216; 1000, 2048, 256 85.1 -> 88.6 | 291 -> 285; 2000, 1024, 512
 // 131.4 -> 143.1 | 380 -> 379.  Past the tokens and rows, in a graph: 2000, 2048, 64 14.6 -> 15.4; 4096, 2048, 128 23.9 -> 30.4.
 constexpr int64_t kGateMaxTokens = 2048, kGateMaxRows = 16 * 1024, kGateMaxSums = kGateMaxRows * 128;
@@ -144,7 +144,8 @@ struct RouterFwdArgs {
 // 32 tokens, two per wavefront, these are whole 128-byte lines; up to kRouterOneEach tokens, where
 // 16-token workgroups still find a CU each, a wavefront takes one token and the second one's
 // latency is saved.  Up to kRouterSpread tokens a workgroup is four wavefronts with a token each: the vector instructions of
-// the rounds count then, and 16 tokens keep one CU busy where four could share them.  In us, 16 tokens a workgroup -> 4:
+// the rounds count then, and 16 tokens keep one CU busy where four could share them; the mask leaves in pieces of 16 bytes, an
+// eighth of a line, which its size at that many tokens (1.5 MiB of 128 experts) allows.  In us, 16 tokens a workgroup -> 4:
 // 16 tokens x 128 experts, K = 8 7.1 -> 5.1, 1000 x 128 7.6 -> 5.8, 2048 x 128 7.8 -> 6.6, 3000 x 64, K = 4 5.0 -> 4.7,
 // 4096 x 64, K = 6 5.0 -> 5.5.
 constexpr int kRouterThreads = 1024;
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(THREADS) void router_fwd_kernel(RouterFwdArgs p) {
     }
   }
   __syncthreads();
-  // mask rows: 32 tokens x 4 bytes per expert
+  // mask rows: kTok tokens x 4 bytes per expert
   const int tt = threadIdx.x & (kTok - 1);
   if (m0 + tt < p.M)
     for (int j = threadIdx.x / kTok; j < N; j += THREADS / kTok)
@@ -438,14 +439,16 @@ extern "C" int momoe_gate_router_fwd(const void* x_MD, int64_t ldx, const void* 
   if (D <= 0 || ldx < D) return MOMOE_ERR_BAD_ARG;
   const int64_t need = momoe_gate_router_workspace_bytes(M, D, N);
   if (need < 0 || ldx % 8 != 0) return MOMOE_ERR_UNSUPPORTED;
-  if (workspace_bytes < need || ((uintptr_t)x_MD & 15) || ((uintptr_t)Wg_DN & 15) || ((uintptr_t)workspace & 15)) return MOMOE_ERR_BAD_ARG;
+  if (workspace_bytes < need || ((uintptr_t)x_MD & 15) || ((uintptr_t)Wg_DN & 15) || ((uintptr_t)workspace & 15))
+    return MOMOE_ERR_BAD_ARG;
   hipStream_t st = (hipStream_t)stream;
   const GateFwdArgs g{(const bf16*)x_MD, ldx, (const bf16*)Wg_DN, (float*)workspace, (int)M, (int)D, (int)N};
   const dim3 grid((unsigned)cdiv64(D, kGateDepth), (unsigned)cdiv64(N, GateStage::COLS), (unsigned)cdiv64(M, kGateTokens));
   gate_logits_kernel<<<grid, GateStage::THREADS, 0, st>>>(g);
   const int launched = launch_status();
   if (launched != MOMOE_OK) return launched;
-  return launch_router_fwd({workspace, 1, (int)grid.x, biases_N, (int)M, (int)N, (int)K, (int)Ks, mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M}, st);
+  return launch_router_fwd({workspace, 1, (int)grid.x, biases_N, (int)M, (int)N, (int)K, (int)Ks, mask_NM, s_MN, p_sel_MN, Ng_M, Ks_M},
+                           st);
 }
 
 extern "C" int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t gs_stride_m,
