@@ -76,7 +76,7 @@ constexpr int kMinChunk = 64;     // an expert is never cut into pieces of fewer
 // 37 calls of 0.2 to 63 MiB and up to 4095 tokens, with even loads, loads that fall as rank^-0.5 and rank^-1.8 and shared experts.  A
 // step near the line, us, four launches -> one: 4095 tokens, D = 512, H = 2048, N = 64, K = 1 (60 MiB) rank^-1.8 361 -> 282; 4095,
 // 4096, 1024, 16, 1 (57) even 626 -> 599, rank^-1.8 766 -> 645; 700, 2048, 768, 128, 8 (52) 912 -> 893, 677 -> 641; 1500, 1024, 512,
-// 64, 8 (61), two of them shared, 407 -> 337; 300, 4096, 1408, 128, 8 (49) rank^-0.5 3040 -> 2955.
+// 64, 8 (61), two of them shared, 407 -> 356; 300, 4096, 1408, 128, 8 (49) rank^-0.5 3040 -> 2955.
 constexpr int64_t kTailBytes = 64 << 20;
 
 // How one expert's rows are dealt out: `splits` equal pieces of `chunk` k-stages (the last
