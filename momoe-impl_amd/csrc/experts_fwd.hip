@@ -588,29 +588,38 @@ int launch_lin1_narrow(const Lin1Args& a, hipStream_t st) {
   return launch_status();
 }
 
-// The few-row tiles (FewRows): its own operands and loop, the epilogue of the narrow ones.
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p) {
-  using Prog = Lin1Prog<false, FewRows::G>;
+// The few-row tiles (FewRows): 32 `a` columns and their 32 `b` columns.
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p, int last_entry) {
+  constexpr int BNH = FewRows::G::COLS / 2;
   const ClockTrace trace(p.clk);
   bf16* lds = dyn_lds();
   const int first_tile = p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
-  TileSched sched(p.table, (p.H + Prog::BNH - 1) / Prog::BNH, MOMOE_TILE_ROWS, first_tile);
-  const int n_org[FN] = {0, Prog::BNH};
-  const Prog prog{p, 0, 0};
+  FewRows::Sched sched(p.table, (p.H + BNH - 1) / BNH, first_tile, last_entry);
   const int D = p.D, H = p.H;
   FewRows op;
   for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
     const TileCoord t = FewRows::piece(left);
-    op.rows(p.x, FewRows::BK, D, [&](int row, int piece) {
-      return (uint32_t)p.idx[t.row0 + min(row, t.rows - 1)] * (uint32_t)(2 * D) + piece * 16;
-    });
-    const int j0 = t.tn * Prog::BNH;
+    const FewRows::Tokens tokens(p.idx + t.row0, t.rows);
+    const int j0 = t.tn * BNH;
     op.weights(p.w1 + (int64_t)t.expert * D * 2 * H, D,
-               [&](int c) { return (c / Prog::BNH) * H + min(j0 + (c % Prog::BNH), H - 8); }, 2 * H);
-    f32x16 acc[FN][1];
+               [&](int c) { return (c / BNH) * H + min(j0 + (c % BNH), H - 8); }, 2 * H);
     __builtin_amdgcn_s_barrier();  // the previous tile's partial sums have been read
-    op.multiply(acc, lds, D, n_org);
-    if (wave_id() == 0) prog.epilogue_fwd(t, acc, FewRows::staging(lds));
+    op.request_weights(lds, D);
+    op.rows(p.x, FewRows::BK, D, [&](int, int piece) { return tokens.mine() * (uint32_t)(2 * D) + piece * 16; });
+    f32x4 sum[FN];
+    op.multiply(sum, lds, D, [] {});
+    const int col = j0 + FewRows::column();
+    const int64_t r = t.row0 + acc_row();
+    if (FewRows::stores() && acc_row() < t.rows) {
+      const f32x4 a = sum[0], b = sum[1];
+      if (p.h)  // k-blocked: the tile's columns are one block
+        store_bf16x4(p.h + ((int64_t)(j0 >> 5) * p.msum + r) * 32 + FewRows::column(), a[0] * b[0] * sigmoidf_fast(b[0]),
+                     a[1] * b[1] * sigmoidf_fast(b[1]), a[2] * b[2] * sigmoidf_fast(b[2]), a[3] * b[3] * sigmoidf_fast(b[3]));
+      if (p.ab && r >= p.ab_lo && r < p.ab_hi) {
+        store_bf16x4(p.ab + r * 2 * H + col, a[0], a[1], a[2], a[3]);
+        store_bf16x4(p.ab + r * 2 * H + H + col, b[0], b[1], b[2], b[3]);
+      }
+    }
     wait_lgkm0();
   }
   trace.finish();
@@ -763,31 +772,63 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args
 }
 constexpr size_t kLin2NarrowLds = std::max(Lin2Prog<NarrowTiles>::kLds, kLin2Lds<StdTiles>);
 
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
-  using Prog = Lin2Prog<FewRows::G>;
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p, int last_entry) {
   const ClockTrace trace(p.clk);
   bf16* lds = dyn_lds();
-  TileSched sched(p.table, (p.D + FewRows::G::COLS - 1) / FewRows::G::COLS, MOMOE_TILE_ROWS);
-  const int n_org[FN] = {0, 32};
-  const Prog prog{p, 0, 0};
+  FewRows::Sched sched(p.table, (p.D + FewRows::G::COLS - 1) / FewRows::G::COLS, 0, last_entry);
   const int D = p.D, H = p.H;
   FewRows op;
   for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
     const TileCoord t = FewRows::piece(left);
-    Prog::Prep prep;
-    prog.gather(t, prep);
+    // The gate weights of the rows come through the scalar unit, too: a chain of two loads, each waited for a step later; most
+    // tiles have no more rows than the first of them
+    constexpr int kAtOnce = 8;
+    const int32_t* const idx = p.idx + t.row0;
+    const float* const s = p.s + (int64_t)t.expert * p.ssn;
+    int32_t tok[kAtOnce];
+    float sv[kAtOnce], mine = 0.0f;
+    auto load_tokens = [&](int r0) {
+#pragma unroll
+      for (int i = 0; i < kAtOnce; ++i) tok[i] = load_uniform(idx + min(r0 + i, t.rows - 1));
+    };
+    auto load_gate_weights = [&] {
+#pragma unroll
+      for (int i = 0; i < kAtOnce; ++i) sv[i] = load_uniform(s + (int64_t)tok[i] * p.ssm);
+    };
+    auto keep_mine = [&](int r0) {
+#pragma unroll
+      for (int i = 0; i < kAtOnce; ++i) mine = acc_row() == r0 + i ? sv[i] : mine;
+    };
+    load_tokens(0);
+    const int d0 = t.tn * FewRows::G::COLS;
+    op.weights(p.w2 + (int64_t)t.expert * H * D, H, [&](int c) { return min(d0 + c, D - 8); }, D);
+    __builtin_amdgcn_s_barrier();  // the previous tile's partial sums have been read
+    op.request_weights(lds, H);
     // h is k-blocked: a stage is four blocks of 32 k-values
     const uint32_t block = (uint32_t)p.msum * (kBK * 2);
     op.rows(p.h + (int64_t)t.row0 * kBK, 4 * p.msum * kBK, H, [&](int row, int piece) {
       return (uint32_t)min(row, t.rows - 1) * (kBK * 2) + (piece >> 2) * block + (piece & 3) * 16;
     });
-    const int d0 = t.tn * FewRows::G::COLS;
-    op.weights(p.w2 + (int64_t)t.expert * H * D, H, [&](int c) { return min(d0 + c, D - 8); }, D);
-    prog.late(t, prep);
-    f32x16 acc[FN][1];
-    __builtin_amdgcn_s_barrier();  // the previous tile's partial sums have been read
-    op.multiply(acc, lds, H, n_org);
-    if (wave_id() == 0) prog.epilogue(t, acc, prep, FewRows::staging(lds));
+    f32x4 sum[FN];
+    op.multiply(sum, lds, H, [&] {
+      if (FewRows::stores())
+        for (int r0 = kAtOnce; r0 < t.rows; r0 += kAtOnce) {
+          load_gate_weights();
+          keep_mine(r0 - kAtOnce);
+          load_tokens(r0);
+        }
+      load_gate_weights();
+    });
+    keep_mine((t.rows - 1) / kAtOnce * kAtOnce);
+    if (FewRows::stores() && acc_row() < t.rows) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int col = d0 + 32 * j + FewRows::column();
+        if (col < D)
+          store_bf16x4(p.ys + (int64_t)(t.row0 + acc_row()) * D + col, sum[j][0] * mine, sum[j][1] * mine, sum[j][2] * mine,
+                       sum[j][3] * mine);
+      }
+    }
     wait_lgkm0();
   }
   trace.finish();
@@ -863,7 +904,7 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
   if (takes_few_rows_tiles(M, Msum, N, 2 * H)) {
     static LdsLimit few;
     if (!allow_lds(lin1_swiglu_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
-    lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
+    lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a, (int)std::min(N, Msum) - 1);
     return launch_status();
   }
   if (takes_span_tiles(Msum, N, 2 * H, D)) {
@@ -949,7 +990,7 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
   if (takes_few_rows_tiles(M, Msum, N, D)) {
     static LdsLimit few;
     if (!allow_lds(lin2_scale_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
-    lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
+    lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a, (int)std::min(N, Msum) - 1);
     return launch_status();
   }
   if (takes_span_tiles(Msum, N, D, H)) {

@@ -121,9 +121,10 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 first, bf16x8 second, f32x16 c) 
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(first, second, c, 0, 0, 0);
 }
 
-// uniform (scalar-unit) load of an int32 that no kernel writes while this one runs
-__device__ __forceinline__ int32_t load_uniform(const int32_t* p) {
-  return *(const int32_t __attribute__((address_space(4)))*)p;
+// uniform (scalar-unit) load of an int32 or float that no kernel writes while this one runs
+template <class T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+  return *(const T __attribute__((address_space(4)))*)p;
 }
 
 // ---- k-contiguous operand -------------------------------------------------------------
@@ -909,17 +910,24 @@ struct RowStager {
 // the chain table -> row ids -> rows are most of both).  64 x 128 tiles with half the k-values a
 // stage took 14.8 and 9.8.  With more than one tile per CU the gap between two tiles, in which
 // nothing is on the way, would cost what the CUs gain.
+// A third of such a launch lies before its first and behind its last transfer: the table, the row ids, the rows and
+// gate weights are a chain of loads, and the slices' sums meet.  So the first weights are requested as soon as the expert is known, what
+// the rows need goes through the scalar unit meanwhile, and four waves share the sums and the stores, where one had
+// 56 reads to make one after the other (1.5 us of either launch).  Cold weights, us, one token of the above: x.Wl1 16.1 -> 14.9, h.Wl2
+// 10.0 -> 9.0, the forward 31.9 -> 29.6; 20 tokens, D = 2048, H = 1024, N = 8, K = 1 36.2 -> 33.2; 32, 1024, 512, 8, 2 27.0 -> 25.2; 4, 4096,
+// 1408, 8, 2, all of it the stream, 67.7 -> 67.9.  What is left of x.Wl1 at one token: 2.7 us until all is requested, 6.6 of the
+// stream (the last workgroup 8.9), 1.1 for sums and stores, the launch.
 struct FewRows {
   static constexpr int ROWS = 32, BK = 128, STAGES = 5;
-  using G = RowTileGeometry<1, 4, 8>;  // 64 columns and the accumulators of one wave, for the epilogues
+  using G = RowTileGeometry<1, 4, 8>;  // 64 columns and the accumulators of one wave
   using W = TLayoutT<G::COLS>;         // its swizzle and fragment reads hold for 128 k-rows as for 32
   static constexpr int FN = G::FN;
   static constexpr int A_ELEMS = ROWS * BK, W_ELEMS = BK * G::COLS, STAGE = A_ELEMS + W_ELEMS;
   static constexpr int WCH = W_ELEMS / (kChunkElems * kWaves), LOADS = 1 + WCH;  // deposits per wave
   static_assert(G::FM == 1 && G::COLS == 64 && BK == 16 * kWaves && A_ELEMS == kChunkElems * kWaves && WCH == 2,
                 "a wave's share of a stage");
-  static constexpr size_t BYTES = (size_t)STAGES * STAGE * sizeof(bf16) + kStageBytesPerWave;
-  static_assert((kWaves - 1) * FN * 1024 * sizeof(float) <= (size_t)STAGES * STAGE * sizeof(bf16),
+  static constexpr size_t BYTES = (size_t)STAGES * STAGE * sizeof(bf16);
+  static_assert(kWaves * FN * 1024 * sizeof(float) <= (size_t)STAGES * STAGE * sizeof(bf16),
                 "the partial sums fit where the stages were");
 
   const bf16 *abase, *wbase;   // wave-uniform
@@ -952,27 +960,52 @@ struct FewRows {
       wtail[j] = (uint32_t)((col + (int64_t)(krow < K % BK ? krow : krow & 31) * ld) * 2);
     }
   }
-  __device__ __forceinline__ void issue(int kt, int K, uint32_t stage) const {
-    const int w = wave_id();
-    const bool tail = kt * BK + BK > K;  // uniform
-    dma16(abase + kt * astride, tail ? atail : aoff, stage + w * (kChunkElems * 2));
+  static __device__ __forceinline__ bool is_tail(int kt, int K) { return kt * BK + BK > K; }  // uniform
+  __device__ __forceinline__ void issue_rows(int kt, int K, uint32_t stage) const {
+    dma16(abase + kt * astride, is_tail(kt, K) ? atail : aoff, stage + wave_id() * (kChunkElems * 2));
+  }
+  __device__ __forceinline__ void issue_weights(int kt, int K, uint32_t stage) const {
 #pragma unroll
     for (int j = 0; j < WCH; ++j)
-      dma16(wbase + kt * wstride, tail ? wtail[j] : woff[j],
-            stage + A_ELEMS * 2 + (w * WCH + j) * (kChunkElems * 2));
+      dma16(wbase + kt * wstride, is_tail(kt, K) ? wtail[j] : woff[j],
+            stage + A_ELEMS * 2 + (wave_id() * WCH + j) * (kChunkElems * 2));
   }
-  // acc of wave 0 = the tile's sums over K (a multiple of 32) k-values; the other waves' acc is left
-  // undefined.  Every wave must be done with `lds` on entry; on return wave 0 may still be reading
-  // it.  n_org: {0, 32}.
-  __device__ __forceinline__ void multiply(f32x16 (&acc)[FN][1], bf16* lds, int K, const int (&n_org)[FN]) const {
+  __device__ __forceinline__ void issue(int kt, int K, uint32_t stage) const {
+    issue_rows(kt, K, stage);
+    issue_weights(kt, K, stage);
+  }
+  // Weights of the first two stages, before anything is known of the rows: what a CU can have on the way
+  // at once.  Every wave must be done with `lds`.
+  __device__ __forceinline__ void request_weights(bf16* lds, int K) const {
+    const uint32_t addr = lds_address(lds);
+    issue_weights(0, K, addr);
+    if (K > BK) issue_weights(1, K, addr + STAGE * 2);
+  }
+  // sum[j] of the waves that store = the tile's sums over K (a multiple of 32) k-values, columns 32 j + column() .. +3.  Behind
+  // request_weights(); on return they may still be reading `lds`.  hook(): what else is to be loaded, through the
+  // scalar unit, once the first stages are on their way.
+  template <class Hook>
+  __device__ __forceinline__ void multiply(f32x4 (&sum)[FN], bf16* lds, int K, Hook hook) const {
     const int slice = wave_id(), l = threadIdx.x & 63;
+    f32x16 acc[FN][1];
     const int ktiles = (K + BK - 1) / BK;
     const uint32_t addr = lds_address(lds);
     zero_acc<1, FN>(acc);
-    for (int s = 0; s < min(STAGES - 1, ktiles); ++s) issue(s, K, addr + s * (STAGE * 2));
+    issue_rows(0, K, addr);
+    if (ktiles > 1) issue_rows(1, K, addr + STAGE * 2);
+    for (int s = 2; s < min(STAGES - 1, ktiles); ++s) issue(s, K, addr + s * (STAGE * 2));
+    hook();
     int cur = 0, next = STAGES - 1;  // buffers of stage kt and of the stage to request
     for (int kt = 0; kt < ktiles; ++kt) {
-      wait_stage<LOADS, STAGES>(kt, ktiles);
+      if (kt == 0) {  // behind the rows of stage 0 are those of stage 1, whose weights were first, and two whole stages
+        static_assert(STAGES == 5, "as many stages ahead");
+        if (ktiles > 3) wait_vmcnt<3 * LOADS - WCH>();
+        else if (ktiles > 2) wait_vmcnt<2 * LOADS - WCH>();
+        else if (ktiles > 1) wait_vmcnt<LOADS - WCH>();
+        else wait_vmcnt<0>();
+      } else {
+        wait_stage<LOADS, STAGES>(kt, ktiles);
+      }
       wait_lgkm0();  // this wave's reads of stage kt-1, whose buffer is requested into next
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
@@ -982,36 +1015,32 @@ struct FewRows {
         const int row = l & 31, piece = (2 * slice + (l >> 5)) ^ (row & 15);
         const bf16x8 af = *(const bf16x8*)(sa + row * BK + piece * 8);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[j][0] = mfma32(W::frag(sa + A_ELEMS, n_org[j], slice), af, acc[j][0]);
+        for (int j = 0; j < FN; ++j) acc[j][0] = mfma32(W::frag(sa + A_ELEMS, 32 * j, slice), af, acc[j][0]);
       }
       cur = cur + 1 == STAGES ? 0 : cur + 1;
       next = next + 1 == STAGES ? 0 : next + 1;
     }
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();  // the last stage has been read: partial sums take its place
-    auto at = [&](int sl, int j, int q) { return (f32x4*)lds + ((sl - 1) * FN + j) * 256 + q * 64 + l; };
-    if (slice > 0) {
+    auto at = [&](int sl, int j, int q) { return (f32x4*)lds + (sl * FN + j) * 256 + q * 64 + l; };
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *at(slice, j, q) = f32x4{acc[j][0][4 * q], acc[j][0][4 * q + 1], acc[j][0][4 * q + 2], acc[j][0][4 * q + 3]};
-    }
+      for (int q = 0; q < 4; ++q)
+        *at(slice, j, q) = f32x4{acc[j][0][4 * q], acc[j][0][4 * q + 1], acc[j][0][4 * q + 2], acc[j][0][4 * q + 3]};
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();
-    if (slice > 0) return;
+    if (!stores()) return;
 #pragma unroll
-    for (int sl = 1; sl < kWaves; ++sl)
+    for (int j = 0; j < FN; ++j) {
+      sum[j] = *at(0, j, slice);
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 v = *at(sl, j, q);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[j][0][4 * q + r] += v[r];
-        }
+      for (int sl = 1; sl < kWaves; ++sl) sum[j] += *at(sl, j, slice);
+    }
   }
-  static __device__ __forceinline__ bf16* staging(bf16* lds) { return lds + STAGES * STAGE; }
+  // Wave q < 4 adds up and stores quad q of both fragments: its lanes hold column() .. +3 of row acc_row()
+  static __device__ __forceinline__ bool stores() { return wave_id() < 4; }
+  static __device__ __forceinline__ int column() { return acc_col(wave_id()); }
 
   // A tile of the table is worked on in pieces of ROWS rows: one for a mask of at most ROWS tokens,
   // more if the caller's index lists a token several times for an expert.  t holds the rows left.
@@ -1021,12 +1050,66 @@ struct FewRows {
     t.na = 1;
     return t;
   }
-  static __device__ __forceinline__ TileCoord following(TileSched& sched, TileCoord t) {
+  template <class Sched>
+  static __device__ __forceinline__ TileCoord following(Sched& sched, TileCoord t) {
     if (t.rows <= ROWS) return sched.next();
     t.row0 += ROWS;
     t.rows -= ROWS;
     return t;
   }
+
+  // Tiles in the table's order, the columns fastest: the place of a workgroup's first entry does not depend on
+  // the table's header, and the two are loaded at once.  `last`: no entry of a mask's table lies further on.
+  // Two tiles in a row go to one XCD: 32 columns of each half of Wl1 are half a line, and on two XCDs, whose L2s
+  // each fetch the line, x.Wl1 took 20 us instead of 15 (four or eight in a row 0 to 0.6 more than two).
+  struct Sched : TileSched {
+    Raw head;
+    static constexpr int kTogether = 2;
+    static __device__ __forceinline__ int place() {
+      const int b = blockIdx.x, group = 8 * kTogether, in = b % group;
+      return gridDim.x % group != 0 ? b : b - in + in % 8 * kTogether + in / 8;
+    }
+    static __device__ __forceinline__ Raw at(const int* table, int q, int row_tile) {
+      const int __attribute__((address_space(4)))* e = (const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * row_tile);
+      return Raw{q, e[0], e[1], e[2], e[3], true};
+    }
+    __device__ __forceinline__ Sched(const int* table_, int nb_, int first_row_tile, int last)
+        : TileSched(table_, nb_, MOMOE_TILE_ROWS, first_row_tile),
+          head(at(table_, first_row_tile * nb_ + place(), min(first_row_tile + place() / nb_, last))) {
+      xcd = 0;
+      pos = place();
+      stride = gridDim.x;
+      limit = total - begin;
+    }
+    __device__ __forceinline__ TileCoord next() {
+      Raw r = head;
+      r.any = pos < limit;
+      pos += stride;
+      if (pos < limit) head = entry(pos, true);
+      if (!r.any || r.mi > bm) return resolve(r);
+      TileCoord t = {};  // the only tile of its expert, as nearly all are: without the divisions
+      t.expert = r.expert;
+      t.row0 = r.rstart;
+      t.rows = r.mi;
+      t.tn = r.q - r.first * nb;
+      t.valid = true;
+      return t;
+    }
+  };
+
+  // Tokens of the four rows that a wave's lanes fetch, through the scalar unit: its loads do not stand in line
+  // behind the transfers of the weights, whose way they would be waited for
+  struct Tokens {
+    int32_t v[4];
+    __device__ __forceinline__ Tokens(const int32_t* idx, int rows) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = load_uniform(idx + min(4 * wave_id() + i, rows - 1));
+    }
+    __device__ __forceinline__ uint32_t mine() const {
+      const int i = (threadIdx.x & 63) >> 4;
+      return (uint32_t)(i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3]);
+    }
+  };
 };
 
 // Whether a forward GEMM over `cols` output columns takes FewRows tiles.  More rows than tokens x

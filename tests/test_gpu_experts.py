@@ -192,6 +192,25 @@ def test_tiles_of_few_rows(M, D, H, N, K, Ks, sp):
     _check_all(dev, run_oracle_layer(x, W1, W2, mask, s, dy))
 
 
+@pytest.mark.parametrize("M", [7, 8, 9, 16, 17, 25, 32])
+def test_gate_weights_of_few_rows(M):
+    """Every expert holds every token: h.Wl2 takes the gate weights eight rows at a time, in either layout of s."""
+    D, H, N = 160, 96, 3
+    x, W1, W2, mask, s, _ = make_layer_inputs(M, D, H, N, N, seed=M, wstd=0.2)  # (outputs of some units)
+    b = lambda t: t.to("cuda:0", torch.bfloat16)
+    import momoe_amd
+    layer = momoe_amd.MoMoE(D, H, N, N, Wl1_ND2H=b(W1), Wl2_NHD=b(W2))
+    f = lambda t: t.to(torch.bfloat16).float()
+    want = torch.zeros(M, D)
+    for i in range(N):
+        ab = f(x) @ f(W1)[i]
+        want += s[i][:, None] * (f(ab[:, :H] * torch.nn.functional.silu(ab[:, H:])) @ f(W2)[i])
+    for s_dev in (s.contiguous().to("cuda:0"), s.T.contiguous().to("cuda:0").T):
+        with torch.no_grad():
+            y, _ = layer(b(x).reshape(1, M, D), mask.to("cuda:0"), s_dev)
+        assert_close(y.reshape(M, D), want, "y")
+
+
 @pytest.mark.parametrize("rows", [32, 256, 320])
 @pytest.mark.parametrize("sizes", [[33, 0, 1, 64, 2, 0, 0, 0], [0, 0, 250, 0, 0, 0, 0, 0], [0, 700, 5, 0, 0, 31, 0, 0]])
 def test_index_that_repeats_tokens(sizes, rows):
