@@ -274,6 +274,17 @@ int momoe_gs_scatter_tokens(const float* gs_part, int64_t nparts, const int32_t*
                             const int32_t* cumsums_N1, float* Gs_MN, int64_t M, int64_t N,
                             int64_t Msum, void* stream);
 
+/* momoe_dgrad_h_lin1_bwd: momoe_dgrad_h and, with row_lo = 0, momoe_lin1_swiglu_bwd_parts in one launch; the
+ * arguments are theirs, nparts = momoe_gs_parts, the results the same bits; u_MsumH is scratch, not always written.  For launches of few tiles, as
+ * momoe_dgrad_h_lin1_bwd_fits says (1 or 0) from the sizes alone.
+ */
+int momoe_dgrad_h_lin1_bwd_fits(int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum);
+int momoe_dgrad_h_lin1_bwd(const void* Gy_MD, const void* Wl2_NHD, const void* x_MD, const void* Wl1_ND2H,
+                           const int32_t* idx_Msum, const int32_t* tile_table, const float* s_NM,
+                           int64_t s_stride_n, int64_t s_stride_m, void* u_MsumH, void* gz_blocked,
+                           void* hsT_GH32, int64_t ld_hsT, float* gs_part, int64_t nparts, int64_t M, int64_t D,
+                           int64_t H, int64_t N, int64_t Msum, void* stream);
+
 /* momoe_dgrad_x replaces the GEMM of lin1_backward_kernel (momoe/momoe.py:662-681):
  *   gxs[r] = bf16( gz[r] @ Wl1[i]^T ), rows kept in sorted order; follow with
  *   momoe_combine to obtain G_x.  gz_blocked as written by the SwiGLU backward entry points.

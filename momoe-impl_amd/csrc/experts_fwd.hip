@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "dgrad_h.hpp"
 #include "gemm_span.hpp"
 
 namespace momoe {
@@ -29,6 +30,9 @@ struct Lin1Args {
   float* gs_part;
   int64_t msum;
   unsigned long long* clk;
+  // where u is made on the way (Lin1DhProg): G_y and Wl2
+  const bf16* gy = nullptr;
+  const bf16* w2 = nullptr;
 };
 
 // The forward.  Tile = up to 256 rows x (128 `a` columns + the matching 128 `b` columns); a wave's
@@ -348,8 +352,16 @@ struct Lin1Prog {
   }
   // epi: store staging; in the backward also the row-sum exchange
   __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x16 (&acc)[FN][FM], const Prep& g, bf16* epi) const {
-    if (BWD) epilogue_bwd(tc, acc, g, epi);
-    else epilogue_fwd(tc, acc, epi);
+    if (BWD) {
+      const int H = p.H, j0 = tc.tn * BNH + wn * 32;
+      epilogue_bwd(tc, acc, g, epi, [&](int i, bf16x4 (&uq)[4]) {
+        const int64_t r = (int64_t)tc.row0 + min((tc.mbase + 32 * i) + acc_row(), tc.rows - 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) uq[q] = *(const bf16x4*)(p.u + r * H + min(j0 + acc_col(q), H - 4));
+      });
+    } else {
+      epilogue_fwd(tc, acc, epi);
+    }
   }
 
   __device__ __forceinline__ void epilogue_fwd(const TileCoord& tc, f32x16 (&acc)[FN][FM], bf16* epi) const {
@@ -406,17 +418,14 @@ struct Lin1Prog {
 
   // SwiGLU backward on the recomputed a|b (momoe/momoe.py:421-535): with u = dL/dh before the
   // gate weight s,  G_a = s u b sig(b),  G_b = s u a sig(b) (1 + b (1 - sig(b))),
-  // hs = s a b sig(b),  and the partial row sum of u a b sig(b) over this tile's columns.
-  __device__ __forceinline__ void epilogue_bwd(const TileCoord& tc, f32x16 (&acc)[FN][FM], const Prep& g, bf16* epi) const {
+  // hs = s a b sig(b),  and the partial row sum of u a b sig(b) over this tile's columns.  load_u(i, uq): the lane's u in
+  // fragment row i.
+  template <int NF, class LoadU>
+  __device__ __forceinline__ void epilogue_bwd(const TileCoord& tc, f32x16 (&acc)[NF][FM], const Prep& g, bf16* epi, LoadU load_u) const {
     const int H = p.H;
     RowStager<1> stager(epi);
     float* red = (float*)epi;  // [column waves][BM]
     const int j0 = tc.tn * BNH + wn * 32;  // first hidden column of this wave
-    auto load_u = [&](int i, bf16x4 (&uq)[4]) {
-      const int64_t r = (int64_t)tc.row0 + min((tc.mbase + 32 * i) + acc_row(), tc.rows - 1);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) uq[q] = *(const bf16x4*)(p.u + r * H + min(j0 + acc_col(q), H - 4));
-    };
     RowStager<1> stager1(epi, 1);
     // Rows below the save boundary are not this kernel's: the boundary is moved down to a
     // multiple of 32 rows from the expert's first row (tiles start at such multiples), so that
@@ -587,6 +596,66 @@ int launch_lin1_narrow(const Lin1Args& a, hipStream_t st) {
   lin1_swiglu_narrow_kernel<BWD><<<persistent_grid(), kThreads, bytes, st>>>(a);
   return launch_status();
 }
+
+// The same with dL/dh made on the way, for few tiles: u = G_y[idx] . Wl2^T contracts over D like a|b, for the same
+// tokens, so both products share a main loop, and u of the tile's 64 hidden columns is rounded as momoe_dgrad_h would store it,
+// but stays in registers.  A launch of few tiles is bound by what lies before its first and behind its last stage (5 us) and by the
+// way of a stage from the L2, not by products: of two launches, the first with as many tiles as half of the second's, one is left, with
+// 44 KiB a stage where each had 24, three stages (all that fit the LDS).  Two launches -> one, a step in us: 1024 tokens, D =
+// 1024, H = 512, N = 32, K = 4 146 -> 140 (18.5 + 22.9 -> 33.7 of the GPU's); 700 of that kind, falling as rank^-1.8, 158 -> 152; 200, 2048, 768,
+// 16, 2 182 -> 178; 3000, 256, 256, 16, 1 105 -> 102; 128, 128, 64, 8, 2, bound by the host, 96 -> 94; wide tiles: 1600, 1024, 512, 32, 4,
+// rank^-0.5, 244 -> 234; 800, 2048, 1024, 16, 4 311 -> 304.  Up to 2560 k-values: past the line a CU's share is long
+// and the launch saved is little: D = 4096, H = 2048, N = 8, K = 4, 110 tokens 327 -> 329, 170 364 -> 359, 400 604 -> 609; D = 3072, 256 tokens
+// 340 -> 333, 400 497 -> 502; D = 2560, H = 960, N = 16, K = 6, 300 tokens 274 -> 270.  And up to one and a half row tiles per expert:
+// 600, 2048, 768, 8, 4 (300 rows) 214 -> 206; past it 2048, 512, 256, 16, 4 126 -> 122 and 4000, 256, 128, 16, 2 114 -> 117, no more
+// than the runs of one side differ by.
+struct Lin1DhProg : Lin1Prog<true, NarrowTiles> {
+  using Base = Lin1Prog<true, NarrowTiles>;
+  using RowsOp = TwoRowsDma<NarrowTiles::AROWS>;
+  using WeightOp = ColsAndRowsDma<NarrowTiles::COLS>;
+  static_assert(WeightOp::ROWS == BNH, "the rows of Wl2 are those of the tile's hidden columns");
+  using Ring = StageRing<RowsOp, WeightOp, 3>;
+  static constexpr int NF = 3;  // column fragments: a, b, u
+  __device__ __forceinline__ void setup(const TileCoord& t, const Prep& g, RowsOp& A, WeightOp& B) const {
+    const int D = p.D, H = p.H, j0 = t.tn * BNH;
+    A.init(p.x, p.gy, [&](int, int j) { return (uint32_t)g.tok[j] * (uint32_t)(2 * D); });
+    B.t.init(p.w1 + (int64_t)t.expert * D * 2 * H, [&](int c) { return (c / BNH) * H + min(j0 + (c % BNH), H - 8); }, 2 * H);
+    B.init_rows(p.w2 + (int64_t)t.expert * H * D, [&](int r) { return (uint32_t)min(j0 + r, H - 1) * (uint32_t)(2 * D); });
+  }
+  __device__ __forceinline__ void epilogue(const TileCoord& tc, f32x16 (&acc)[NF][FM], const Prep& g, bf16* epi) const {
+    epilogue_bwd(tc, acc, g, epi, [&](int i, bf16x4 (&uq)[4]) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        uq[q] = pack_bf16x4(acc[2][i][4 * q], acc[2][i][4 * q + 1], acc[2][i][4 * q + 2], acc[2][i][4 * q + 3]);
+    });
+  }
+};
+// Where the table holds more tiles than those, the tiles are wide ones, which have no registers for u.  It goes
+// through memory there, but not past the workgroup: its 128 hidden columns of a row tile are a tile of either loop,
+// dealt out alike, so a workgroup first makes u for all tiles that it will read it for.
+__global__ __launch_bounds__(kThreads, 2) void lin1_dh_narrow_kernel(Lin1Args p) {
+  const ClockTrace trace(p.clk);
+  using Prog = Lin1DhProg;
+  const int nb = (p.H + Prog::BNH - 1) / Prog::BNH;
+  if (__builtin_expect(narrow_tiles_fit(p.table, nb), 1)) {
+    typename Prog::Ring ring(dyn_lds());
+    TileSchedT<NarrowTiles::WROWS> sched(p.table, nb, Prog::BM);
+    const int wn = wave_id() % NarrowTiles::WCOLS;
+    const int n_org[Prog::NF] = {wn * 32, Prog::BNH + wn * 32, wn * 32};
+    Prog prog{{p, p.D / kBK, wn}};
+    run_row_tiles<Prog::FM, Prog::NF>(prog, sched, ring, n_org);
+  } else {
+    using Wide = Lin1Prog<true, StdTilesHalfParts>;
+    static_assert(Wide::BNH == NarrowTiles::COLS && Wide::BM == NarrowTiles::MAX_ROWS, "the same tiles");
+    dgrad_h_tiles<NarrowTiles, TileSchedT<NarrowTiles::WROWS>>(
+        DhArgs{p.gy, p.w2, p.idx, p.table, const_cast<bf16*>(p.u), p.D, p.H, nullptr}, Wide::BM);
+    __syncthreads();  // u has been stored, the ring has been read
+    lin1_swiglu_tiles<true, StdTilesHalfParts>(p);
+  }
+  trace.finish();
+}
+constexpr size_t kLin1DhLds =
+    std::max({Lin1DhProg::Ring::BYTES, DhProg<NarrowTiles>::Ring::BYTES, Lin1Prog<true, StdTilesHalfParts>::kLds});
 
 // The few-row tiles (FewRows): 32 `a` columns and their 32 `b` columns.
 __global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p, int last_entry) {
@@ -972,6 +1041,36 @@ extern "C" int momoe_lin1_swiglu_bwd_parts(const void* x_MD, const void* Wl1_ND2
     return launch_span(lin1_swiglu_bwd_kernel, a, span, (hipStream_t)stream);
   }
   return launch_lin1<true, StdTiles>(a, (hipStream_t)stream);
+}
+
+extern "C" int momoe_dgrad_h_lin1_bwd_fits(int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum) {
+  return check_dims(M, D, H, N, Msum) == MOMOE_OK && takes_narrow_tiles(Msum, N, 2 * H) && D < 3072 &&
+         2 * Msum <= 3 * N * StdTiles::MAX_ROWS;
+}
+
+extern "C" int momoe_dgrad_h_lin1_bwd(const void* Gy_MD, const void* Wl2_NHD, const void* x_MD, const void* Wl1_ND2H,
+                                      const int32_t* idx_Msum, const int32_t* tile_table, const float* s_NM, int64_t s_stride_n,
+                                      int64_t s_stride_m, void* u_MsumH, void* gz_blocked, void* hsT_GH32, int64_t ld_hsT,
+                                      float* gs_part, int64_t nparts, int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum,
+                                      void* stream) {
+  if (!Gy_MD || !Wl2_NHD || !x_MD || !Wl1_ND2H || !idx_Msum || !tile_table || !s_NM || !u_MsumH || !gz_blocked || !hsT_GH32 ||
+      !gs_part)
+    return MOMOE_ERR_BAD_ARG;
+  for (const void* q : {Gy_MD, Wl2_NHD, x_MD, Wl1_ND2H, (const void*)u_MsumH, (const void*)gz_blocked, (const void*)hsT_GH32})
+    if (!aligned16(q)) return MOMOE_ERR_BAD_ARG;
+  if (ld_hsT < H || ld_hsT % 8 != 0) return MOMOE_ERR_BAD_ARG;
+  const int st = check_dims(M, D, H, N, Msum);
+  if (st != MOMOE_OK) return st;
+  if (!momoe_dgrad_h_lin1_bwd_fits(M, D, H, N, Msum)) return MOMOE_ERR_UNSUPPORTED;
+  if (nparts != cdiv64(H, MOMOE_GS_BLOCK / 2)) return MOMOE_ERR_BAD_ARG;
+  const Lin1Args a{(const bf16*)x_MD, (const bf16*)Wl1_ND2H, idx_Msum, tile_table, nullptr, nullptr,
+                   0, Msum, (int)D, (int)H, (const bf16*)u_MsumH, s_NM, s_stride_n, s_stride_m,
+                   (bf16*)gz_blocked, (bf16*)hsT_GH32, ld_hsT, gs_part, Msum, clock_trace_buffer(),
+                   (const bf16*)Gy_MD, (const bf16*)Wl2_NHD};
+  static LdsLimit lds;
+  if (!allow_lds(lin1_dh_narrow_kernel, kLin1DhLds, lds)) return MOMOE_ERR_LAUNCH;
+  lin1_dh_narrow_kernel<<<persistent_grid(), kThreads, kLin1DhLds, (hipStream_t)stream>>>(a);
+  return launch_status();
 }
 
 extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, const float* s_NM,

@@ -293,6 +293,70 @@ struct TDmaT {
 
 using TDma = TDmaT<256>;
 
+// Two row operands of the same tokens, for two products in one main loop (k-contiguous, equal pitches)
+template <int ROWS>
+struct TwoRowsDma {
+  using R = RDma<ROWS>;
+  static constexpr int NCH = 2 * R::NCH;
+  static constexpr int LDS_ELEMS = 2 * R::LDS_ELEMS;
+  R r;
+  const bf16* second;  // wave-uniform
+  template <class RowOff>
+  __device__ __forceinline__ void init(const bf16* first_, const bf16* second_, RowOff rowoff) {
+    r.init(first_, rowoff);
+    second = second_;
+  }
+  __device__ __forceinline__ void issue(int kt, uint32_t stage) {
+    const int w = wave_id();
+    const bf16 *b = r.base + kt * kBK, *c = second + kt * kBK;
+#pragma unroll
+    for (int j = 0; j < R::NCH; ++j) dma16(b, r.off[j], stage + (j * kWaves + w) * (kChunkElems * 2));
+#pragma unroll
+    for (int j = 0; j < R::NCH; ++j)
+      dma16(c, r.off[j], stage + R::LDS_ELEMS * 2 + (j * kWaves + w) * (kChunkElems * 2));
+  }
+  template <int S>
+  __device__ __forceinline__ void issue_head(uint32_t stage) { issue(S, stage); }
+  static __device__ __forceinline__ bf16x8 frag(const bf16* stage, int r0, int kk) { return R::frag(stage, r0, kk); }
+  static __device__ __forceinline__ bf16x8 frag_second(const bf16* stage, int r0, int kk) {
+    return R::frag(stage + R::LDS_ELEMS, r0, kk);
+  }
+};
+// Their weights: a k-strided operand for the first, 64 k-contiguous rows, half a deposit of each wave, for the second
+template <int COLS>
+struct ColsAndRowsDma {
+  using T = TDmaT<COLS>;
+  using R = RDma<16 * kWaves>;
+  static constexpr int ROWS = 8 * kWaves;
+  static constexpr int NCH = T::NCH + 1;
+  static constexpr int LDS_ELEMS = T::LDS_ELEMS + ROWS * kBK;
+  T t;
+  const bf16* rows;  // wave-uniform
+  uint32_t off;
+  // row r (< ROWS) of the second's weights starts at (char*)rows_ + rowoff(r)
+  template <class RowOff>
+  __device__ __forceinline__ void init_rows(const bf16* rows_, RowOff rowoff) {
+    const int l = threadIdx.x & 31, row = wave_id() * 8 + (l >> 2);
+    rows = rows_;
+    off = rowoff(row) + ((l & 3) ^ ((row >> 2) & 3)) * 16;
+  }
+  __device__ __forceinline__ void issue(int kt, uint32_t stage) {
+    t.issue(kt, stage);
+    if ((threadIdx.x & 63) < 32) dma16(rows + kt * kBK, off, stage + T::LDS_ELEMS * 2 + wave_id() * kChunkElems);
+  }
+  template <int S>
+  __device__ __forceinline__ void issue_head(uint32_t stage) { issue(S, stage); }
+  static __device__ __forceinline__ bf16x8 frag(const bf16* stage, int c0, int kk) { return T::frag(stage, c0, kk); }
+  static __device__ __forceinline__ bf16x8 frag_second(const bf16* stage, int r0, int kk) {
+    return R::frag(stage + T::LDS_ELEMS, r0, kk);
+  }
+};
+// Whether a row operand is two: the last column fragment is then that of the second product
+template <class Op>
+inline constexpr bool kTwoProducts = false;
+template <int ROWS>
+inline constexpr bool kTwoProducts<TwoRowsDma<ROWS>> = true;
+
 // Such an operand within a tile whose choice is known: no branch in the main loop.
 template <class Op, bool ONCE>
 struct KnownOnce {
@@ -517,7 +581,8 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
   static_assert(kKSteps == 2, "written for 2 k-steps per stage");
   static_assert(NA >= 0 && NA <= FM, "active fragment rows");
   constexpr int LOADS = AOp::NCH + BOp::NCH;
-  bf16x8 af[2][FM], bf[2][FN];
+  constexpr int kSecond = kTwoProducts<AOp> ? FN - 1 : FN;  // column fragments of the first product
+  bf16x8 af[2][FM], bf[2][FN], af_second[2][kTwoProducts<AOp> ? FM : 1];
   auto load_frags = [&](int kt, int kk) {
     if (NA == 0) return;
     const bf16* la = ring.buf(kt);
@@ -525,13 +590,22 @@ __device__ __forceinline__ void gemm_mainloop(AOp& A, BOp& B, f32x16 (&acc)[FN][
 #pragma unroll
     for (int i = 0; i < NA; ++i) af[kk][i] = AOp::frag(la, m_org[i], kk);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) bf[kk][j] = BOp::frag(lb, n_org[j], kk);
+    for (int j = 0; j < kSecond; ++j) bf[kk][j] = BOp::frag(lb, n_org[j], kk);
+    if constexpr (kTwoProducts<AOp>) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) af_second[kk][i] = AOp::frag_second(la, m_org[i], kk);
+      bf[kk][kSecond] = BOp::frag_second(lb, n_org[kSecond], kk);
+    }
   };
   auto multiply = [&](int kk) {
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < kSecond; ++j)
 #pragma unroll
       for (int i = 0; i < NA; ++i) acc[j][i] = mfma32(bf[kk][j], af[kk][i], acc[j][i]);
+    if constexpr (kTwoProducts<AOp>) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) acc[kSecond][i] = mfma32(bf[kk][kSecond], af_second[kk][i], acc[kSecond][i]);
+    }
   };
   // The scheduling fences keep the compiler from hoisting fragment reads across k-steps.
   auto fence = [] { __builtin_amdgcn_sched_barrier(0); };

@@ -319,6 +319,8 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     const Tensor Gy = grads[0].reshape({M, D}).to(dev, at::kBFloat16).contiguous();
 
     // dL/dh before the gate weight, in sorted order
+    // few tiles and no row saved: made on the way by the launch that needs it
+    const bool joined = msave == 0 && momoe_dgrad_h_lin1_bwd_fits(M, D, H, N, msum) != 0;
     const int64_t u_bytes = msum * H * 2, gz_bytes = 2 * u_bytes, hst_bytes = momoe_padded_rows(msum, N) * H * 2;
     const int64_t nparts = momoe_gs_parts(H, N, msum), parts_bytes = nparts * msum * 4, gxs_bytes = need_x ? msum * D * 2 : 0;
     // scratch for the weight gradients of experts with many rows: what the library can use, but no
@@ -332,7 +334,7 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
     Transients transients(dev, {u_bytes, gz_bytes, hst_bytes, parts_bytes, ws2_bytes, ws1_bytes, gxs_bytes});
     Tensor u_own, gz_own, hst_own, parts_own;
     void* const u = transients.take(u_bytes, u_own);
-    MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u, M, D, H, N, msum);
+    if (!joined) MOMOE_CALL(momoe_dgrad_h, st, Gy.data_ptr(), W2.data_ptr(), ib.idx(), ib.table_for(H, D), u, M, D, H, N, msum);
     // SwiGLU backward: rows with saved a|b read them; the others recompute a|b = x.Wl1 and consume
     // them straight from the GEMM's accumulators.
     // G_a|G_b in blocks of 32 columns, [2H/32][Msum][32]: the layout dL/dx contracts over
@@ -355,7 +357,11 @@ struct ExpertsFn : torch::autograd::Function<ExpertsFn> {
                    own.data_ptr<int32_t>());
         table_rc = own.data_ptr<int32_t>();
       }
-      call("momoe_lin1_swiglu_bwd", st, momoe_lin1_swiglu_bwd_parts, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc,
+      if (joined)
+        MOMOE_CALL(momoe_dgrad_h_lin1_bwd, st, Gy.data_ptr(), W2.data_ptr(), x.data_ptr(), W1.data_ptr(), (const int32_t*)ib.idx(),
+                   table_rc, (const float*)s.data_ptr<float>(), s.stride(0), s.stride(1), u, gz, hst, H, gs_part, nparts, M, D, H, N, msum);
+      else
+        call("momoe_lin1_swiglu_bwd", st, momoe_lin1_swiglu_bwd_parts, x.data_ptr(), W1.data_ptr(), ib.idx(), table_rc,
            u, s.data_ptr<float>(), s.stride(0), s.stride(1), msave, gz, hst, H,
            gs_part, nparts, M, D, H, N, msum);
     }

@@ -59,6 +59,9 @@ _SIGNATURES = {
     "momoe_gs_parts": (_i64, [_i64, _i64, _i64]),
     "momoe_lin1_swiglu_bwd_parts": (_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64, _p,
                                            _i64, _i64, _i64, _i64, _i64, _i64, _p]),
+    "momoe_dgrad_h_lin1_bwd_fits": (_int, [_i64] * 5),
+    "momoe_dgrad_h_lin1_bwd": (_int, [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _i64, _p, _i64,
+                                      _i64, _i64, _i64, _i64, _i64, _p]),
     "momoe_swiglu_bwd_saved": (_int, [_p, _p, _p, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _p, _i64,
                                       _i64, _i64, _i64, _i64, _p]),
     "momoe_gs_scatter": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _p]),
@@ -310,6 +313,15 @@ def lin1_swiglu_bwd(x_MD, Wl1_ND2H, idx, table, u, s_NM, row_lo, gz, hsT, gs_par
     _call("momoe_lin1_swiglu_bwd", _ptr(x_MD), _ptr(Wl1_ND2H), _ptr(idx), _ptr(table), _ptr(u),
           _ptr(s_NM), s_NM.stride(0), s_NM.stride(1), row_lo, _ptr(gz), _ptr(hsT), hsT.shape[1],
           _ptr(gs_part), M, D, H2 // 2, N, idx.numel(), _stream())
+
+
+def dgrad_h_lin1_bwd(Gy_MD, Wl2_NHD, x_MD, Wl1_ND2H, idx, table, s_NM, u, gz, hsT, gs_part):
+    _need_cuda(Gy_MD, x_MD, Wl1_ND2H)
+    M, D = x_MD.shape
+    N, H = Wl2_NHD.shape[:2]
+    _call("momoe_dgrad_h_lin1_bwd", _ptr(Gy_MD), _ptr(Wl2_NHD), _ptr(x_MD), _ptr(Wl1_ND2H), _ptr(idx), _ptr(table),
+          _ptr(s_NM), s_NM.stride(0), s_NM.stride(1), _ptr(u), _ptr(gz), _ptr(hsT), hsT.shape[1], _ptr(gs_part),
+          gs_part.shape[0], M, D, H, N, idx.numel(), _stream())
 
 
 def swiglu_bwd_saved(ab_save, u, s_NM, idx, cumsums, Msave, gz, hsT, gs_part):

@@ -740,6 +740,38 @@ def test_forward_mode_is_refused(grad):
 
 
 @pytest.mark.parametrize("M,D,H,N,K,skew", [
+    (1, 32, 32, 1, 1, None), (128, 64, 96, 8, 2, None), (300, 96, 160, 9, 3, 1.8),  # one to three stages, a half column block
+    (257, 416, 64, 3, 3, None), (1024, 1024, 512, 32, 4, None),  # a second tile of one row; one tile per CU
+    (800, 160, 2048, 8, 2, 1.8),                                 # more tiles than CUs: u goes through memory
+])
+@pytest.mark.parametrize("overflow", [False, True])
+def test_dgrad_h_on_the_way_to_the_swiglu_backward(M, D, H, N, K, skew, overflow):
+    """The two products in one launch are those of the two launches, bit for bit."""
+    from momoe_amd import _hip
+    dev, msum = "cuda:0", M * K
+    assert _hip._lib.momoe_dgrad_h_lin1_bwd_fits(M, D, H, N, msum) == 1
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=3, skew=skew)
+    if overflow:
+        if N == K:
+            pytest.skip("a token cannot have more than all experts")
+        mask = torch.ones_like(mask)  # more pairs than rows: nothing is written
+    x, Gy, W1, W2 = (t.to(dev, torch.bfloat16) for t in (x, dy, W1, W2))
+    s = s.to(dev)
+    ib = _hip.index_build(mask.to(dev), K, tile_rows=_hip.RECOMPUTE_TILE_ROWS)
+    idx, table = ib["idx_Msum"], ib["tile_table"]
+    nparts = _hip._lib.momoe_gs_parts(H, N, msum)
+    new = lambda *size: torch.full(size, 7, device=dev, dtype=torch.bfloat16)
+    outs = lambda: (new(2 * H // 32, msum, 32), new(_hip.padded_rows(msum, N) // 32, H, 32), torch.full((nparts, msum), 7.0, device=dev))
+    u, want, got = new(msum, H), outs(), outs()
+    _hip.dgrad_h(Gy, W2, idx, table, u)
+    p = lambda t: t.data_ptr()
+    _hip._call("momoe_lin1_swiglu_bwd_parts", p(x), p(W1), p(idx), p(table), p(u), p(s), s.stride(0), s.stride(1), 0, p(want[0]),
+               p(want[1]), H, p(want[2]), nparts, M, D, H, N, msum, _hip._stream())
+    _hip.dgrad_h_lin1_bwd(Gy, W2, x, W1, idx, table, s, new(msum, H), *got)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("M,D,H,N,K,skew", [
     (1, 32, 32, 1, 1, None), (128, 128, 64, 8, 2, None), (300, 352, 288, 9, 3, 1.8),  # a tile each, tiles cut off, few rows
     (4095, 64, 32, 70, 3, 1.8), (1000, 1056, 544, 16, 1, None),   # the most tokens; more tiles than workgroups
     (64, 1056, 544, 80, 3, None),  # weights past the last-level cache: dL/dx behind both weight gradients
