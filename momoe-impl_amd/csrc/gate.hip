@@ -8,6 +8,8 @@
 // for every 256 tokens begun.  Both launches in a graph, us, with half as many ranges | as they are | twice as many, and the library's product:
 // 8192 tokens, D = 2048, N = 128 25.9 | 20.5 | 25.1, 59.3; 16384, 2048, 64 36.8 | 25.0 | 25.4, 89.9; 32768, 512, 16 22.2 | 18.7 |
 // 21.6, 72.4; 7680, 2176, 64 23.5 | 17.1 | 19.8, 44.8.
+// One range, up to 256 tokens, is all of the product: no second launch, which such a call, bound by the host, waits for.  Steps with
+// their router, us, two launches -> one: 64 tokens, D = 256, N = 16 178.0 -> 171.9; 200, 1024, 32 186.0 -> 179.6.
 #include <algorithm>
 
 #include "gate.hpp"
@@ -23,6 +25,7 @@ struct GateArgs {
   int64_t ldx;
   const bf16* g;
   float* part;  // [ranges][D][N]
+  bf16* out;    // [D][N] where one range is all: it is stored rounded, and nothing is left to add up
   int M, D, N, rows;  // rows: tokens of a range, a multiple of kStageRows
 };
 
@@ -79,7 +82,10 @@ __global__ __launch_bounds__(kGateThreads, 2) void gate_wgrad_kernel(GateArgs p)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + n_org + 16 * j + 4 * (l >> 4);
-      if (d < p.D && n < p.N) *(f32x4*)(out + (int64_t)d * p.N + n) = acc[j][i];
+      if (d >= p.D || n >= p.N) continue;
+      const f32x4 v = acc[j][i];
+      if (p.out) store_bf16x4(p.out + (int64_t)d * p.N + n, v[0] + 0.0f, v[1] + 0.0f, v[2] + 0.0f, v[3] + 0.0f);
+      else *(f32x4*)(out + (int64_t)d * p.N + n) = v;
     }
   }
 }
@@ -200,11 +206,12 @@ extern "C" int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogi
   const GateSplit split(M, D, N);
   if (workspace_bytes < split.ranges * D * N * (int64_t)sizeof(float)) return MOMOE_ERR_BAD_ARG;
   hipStream_t st = (hipStream_t)stream;
-  const GateArgs a{(const bf16*)x_MD, ldx, (const bf16*)Glogits_MN, (float*)workspace, (int)M, (int)D, (int)N, (int)split.rows};
+  const GateArgs a{(const bf16*)x_MD, ldx, (const bf16*)Glogits_MN, (float*)workspace,
+                   split.ranges == 1 ? (bf16*)GWg_DN : nullptr, (int)M, (int)D, (int)N, (int)split.rows};
   const dim3 grid((unsigned)cdiv64(D, kTile), (unsigned)cdiv64(N, kTile), (unsigned)split.ranges);
   gate_wgrad_kernel<<<grid, kGateThreads, 0, st>>>(a);
   const int status = launch_status();
-  if (status != MOMOE_OK) return status;
+  if (status != MOMOE_OK || split.ranges == 1) return status;
   const int64_t quads = D * N / 4;
   gate_wgrad_reduce_kernel<<<(unsigned)cdiv64(quads, kGateThreads), kGateThreads, 0, st>>>((const float*)workspace, (int)split.ranges,
                                                                                          quads, (bf16*)GWg_DN);
