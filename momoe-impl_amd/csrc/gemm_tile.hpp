@@ -357,7 +357,7 @@ inline constexpr bool kTwoProducts = false;
 template <int ROWS>
 inline constexpr bool kTwoProducts<TwoRowsDma<ROWS>> = true;
 
-// Such an operand within a tile whose choice is known: no branch in the main loop.
+// A TDmaT within a tile whose choice of the hint is known: no branch in the main loop.
 template <class Op, bool ONCE>
 struct KnownOnce {
   static constexpr int NCH = Op::NCH, LDS_ELEMS = Op::LDS_ELEMS;
