@@ -1133,7 +1133,8 @@ struct FewRows {
   }
 
   // Tiles in the table's order, the columns fastest: the place of a workgroup's first entry does not depend on
-  // the table's header, and the two are loaded at once.  `last`: no entry of a mask's table lies further on.
+  // the table's header, and the two are loaded at once.  `last`: no entry of a mask's table lies further on, and the table has
+  // room for it.  A list that repeats tokens may have more entries: those are loaded behind the header, by a branch that no mask takes.
   // Two tiles in a row go to one XCD: 32 columns of each half of Wl1 are half a line, and on two XCDs, whose L2s
   // each fetch the line, x.Wl1 took 20 us instead of 15 (four or eight in a row 0 to 0.6 more than two).
   struct Sched : TileSched {
@@ -1154,6 +1155,7 @@ struct FewRows {
       pos = place();
       stride = gridDim.x;
       limit = total - begin;
+      if (__builtin_expect(first_row_tile + pos / nb > last && pos < limit, 0)) head = entry(pos, true);
     }
     __device__ __forceinline__ TileCoord next() {
       Raw r = head;

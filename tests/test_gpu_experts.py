@@ -241,6 +241,52 @@ def test_index_that_repeats_tokens(sizes, rows):
         assert_close(ys[r], (got_h[r] @ f(W2)[i]) * s[i, tok][:, None], f"rows of expert {i}")
 
 
+@pytest.mark.parametrize("sizes,rows,H", [
+    ([100] + [1] * 7, 32, 96),      # 11 entries, three column blocks in either GEMM
+    ([250, 1] + [0] * 6, 32, 96),   # the one entry too many is another expert's than the one before it
+    ([33] * 7 + [1], 32, 768),      # 15 entries in 24 column blocks: more tiles than workgroups
+    ([257] + [1] * 15, 256, 256),   # 17 entries
+    ([700] + [1] * 31, 256, 96), ([700] + [1] * 31, 320, 96),
+])
+def test_more_tiles_than_experts_of_few_rows(sizes, rows, H):
+    """At most 32 tokens and an index that repeats them: a table of more entries than experts.  Nothing is written behind the results."""
+    from momoe_amd import _hip
+    M, D, N, msum, dev = 32, 160, len(sizes), sum(sizes), "cuda:0"
+    assert msum <= M * N and sum(-(-n // rows) for n in sizes) > min(N, msum) and N * -(-2 * H // 64) <= 256  # what such launches take
+    x, W1, W2, _, s, _ = make_layer_inputs(M, D, H, N, 2, seed=17)
+    cumsums = torch.zeros(N + 1, dtype=torch.int32)
+    cumsums[1:] = torch.cumsum(torch.tensor(sizes), 0)
+    idx = torch.randint(0, M, (msum,), generator=torch.Generator().manual_seed(2), dtype=torch.int32)
+    s = torch.rand(N, M, generator=torch.Generator().manual_seed(3))
+    b = lambda t: t.to(dev, torch.bfloat16)
+    table = _hip.tile_table_build(cumsums.to(dev), 1, msum, rows)
+    owned = []
+
+    def guarded(*size):  # as many elements again behind the result
+        n = torch.Size(size).numel()
+        owned.append((torch.full((2 * n,), 7.0, device=dev, dtype=torch.bfloat16), n))
+        return owned[-1][0][:n].view(size)
+
+    h, ys, ab = guarded(H // 32, msum, 32), guarded(msum, D), guarded(msum, 2 * H)
+    lo = sizes[0]  # rows of the first expert are not saved, and its tiles left out
+    _hip.lin1_swiglu_fwd(b(x), b(W1), idx.to(dev), table, h, None, 0, 0)
+    _hip.lin1_swiglu_fwd(b(x), b(W1), idx.to(dev), table, None, ab, lo, msum)
+    _hip.lin2_scale_fwd(h, b(W2), s.to(dev), idx.to(dev), table, ys, M)
+    assert all(bool((t[n:] == 7.0).all()) for t, n in owned) and bool((ab[:lo] == 7.0).all())
+    f = lambda t: t.to(torch.bfloat16).float()
+    got_h = h.permute(1, 0, 2).reshape(msum, H).float().cpu()
+    for i in range(N):
+        r = slice(int(cumsums[i]), int(cumsums[i + 1]))
+        if sizes[i] == 0:
+            continue
+        tok = idx[r].long()
+        want = f(x)[tok] @ f(W1)[i]
+        assert_close(got_h[r], want[:, :H] * torch.nn.functional.silu(want[:, H:]), f"h of expert {i}")
+        assert_close(ys[r], (got_h[r] @ f(W2)[i]) * s[i, tok][:, None], f"rows of expert {i}")
+        if i > 0:
+            assert_close(ab[r], want, f"a|b of expert {i}")
+
+
 @pytest.mark.parametrize("gather_a", [True, False])
 def test_weight_gradient_of_cut_experts(gather_a):
     # experts of 20000 / 3 / 0 / 5000 rows: the first is contracted in pieces that meet in the
