@@ -604,9 +604,13 @@ int launch_lin1_narrow(const Lin1Args& a, hipStream_t st) {
 // 44 KiB a stage where each had 24, three stages (all that fit the LDS).  Two launches -> one, a step in us: 1024 tokens, D =
 // 1024, H = 512, N = 32, K = 4 146 -> 140 (18.5 + 22.9 -> 33.7 of the GPU's); 700 of that kind, falling as rank^-1.8, 158 -> 152; 200, 2048, 768,
 // 16, 2 182 -> 178; 3000, 256, 256, 16, 1 105 -> 102; 128, 128, 64, 8, 2, bound by the host, 96 -> 94; wide tiles: 1600, 1024, 512, 32, 4,
-// rank^-0.5, 244 -> 234; 800, 2048, 1024, 16, 4 311 -> 304.  Up to 2560 k-values: past the line a CU's share is long
-// and the launch saved is little: D = 4096, H = 2048, N = 8, K = 4, 110 tokens 327 -> 329, 170 364 -> 359, 400 604 -> 609; D = 3072, 256 tokens
-// 340 -> 333, 400 497 -> 502; D = 2560, H = 960, N = 16, K = 6, 300 tokens 274 -> 270.  And up to one and a half row tiles per expert:
+// rank^-0.5, 244 -> 234; 800, 2048, 1024, 16, 4 311 -> 304.  Below 3072 k-values: the longer a CU's share, the less the launch
+// saved is of it.  H = 2048, N = 8, K = 4, 110 | 256 | 400 tokens, the last falling as rank^-0.5: D = 2592 236 -> 227 | 305 -> 295 | 436 ->
+// 440, 2816 257 -> 252 | 326 -> 319 | 480 -> 481, 3040 279 -> 276 | 351 -> 345 | 508 -> 514; 400, 3040, 960, 16, 6 364 -> 361; from the line on
+// D = 3072, 256 tokens 340 -> 333, 400 497 -> 502; 4096, 110 tokens 327 -> 329, 170 364 -> 359, 400 604 -> 609.  What loses there, and
+// 1 % below (2048, 400 tokens 321 -> 324), are tiles a few too many for narrow ones: 144 wide ones leave half of the CUs
+// idle in either form, which the host cannot know; other such loads gain (800, 2560, 1024, 16, 4, rank^-1.8 436 -> 416; 1500, 2816, 512, 32, 4
+// 501 -> 478).  And up to one and a half row tiles per expert:
 // 600, 2048, 768, 8, 4 (300 rows) 214 -> 206; past it 2048, 512, 256, 16, 4 126 -> 122 and 4000, 256, 128, 16, 2 114 -> 117, no more
 // than the runs of one side differ by.
 struct Lin1DhProg : Lin1Prog<true, NarrowTiles> {
