@@ -392,7 +392,8 @@ int momoe_router_bwd(const float* Gs_NM, int64_t gs_stride_n, int64_t gs_stride_
 /* momoe_gate_wgrad: gradient of the gate weights (in TopKRouterFunction, momoe/topk_router.py:83-145), GWg_DN[d,n] = sum over the tokens of
  * x_MD[m,d] * Glogits_MN[m,n], bf16 from fp32 sums.  x_MD bf16 with row pitch ldx elements, Glogits_MN bf16 contiguous.
  * D, N and ldx multiples of 8; x_MD, Glogits_MN and workspace on 16-byte boundaries.
- * workspace: momoe_gate_wgrad_workspace_bytes(M, D, N) bytes of device memory (-1: sizes that it does not take).
+ * workspace: momoe_gate_wgrad_workspace_bytes(M, D, N) bytes of device memory (-1: sizes that it does not take); scratch, not
+ * always written, but demanded for all sizes.
  */
 int64_t momoe_gate_wgrad_workspace_bytes(int64_t M, int64_t D, int64_t N);
 int momoe_gate_wgrad(const void* x_MD, int64_t ldx, const void* Glogits_MN, void* GWg_DN,

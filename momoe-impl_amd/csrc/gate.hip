@@ -8,8 +8,9 @@
 // for every 256 tokens begun.  Both launches in a graph, us, with half as many ranges | as they are | twice as many, and the library's product:
 // 8192 tokens, D = 2048, N = 128 25.9 | 20.5 | 25.1, 59.3; 16384, 2048, 64 36.8 | 25.0 | 25.4, 89.9; 32768, 512, 16 22.2 | 18.7 |
 // 21.6, 72.4; 7680, 2176, 64 23.5 | 17.1 | 19.8, 44.8.
-// One range, up to 256 tokens, is all of the product: no second launch, which such a call, bound by the host, waits for.  Steps with
-// their router, us, two launches -> one: 64 tokens, D = 256, N = 16 178.0 -> 171.9; 200, 1024, 32 186.0 -> 179.6.
+// One range (of up to 256 tokens, or of any number in more than 128 tiles) is all of the product: no partial sums, which leaves the
+// workspace as it is, and no second launch, which a call of few tokens, bound by the host, waits for.  Steps with their
+// router, us, two launches -> one: 64 tokens, D = 256, N = 16 178.0 -> 171.9; 200, 1024, 32 186.0 -> 179.6.
 #include <algorithm>
 
 #include "gate.hpp"

@@ -246,6 +246,15 @@ def test_gate_weight_gradient(M, D, N):
     assert torch.isinf(got[3]).all() and torch.isfinite(torch.cat([got[:3], got[4:]])).all()
 
 
+def test_gate_weight_gradient_in_many_tiles():
+    """130 tiles: one range, though of more tokens than a range has elsewhere."""
+    from momoe_amd import _hip
+    M, D, N = 600, 16520, 8
+    ranges = lambda D: _hip._lib.momoe_gate_wgrad_workspace_bytes(M, D, N) // (D * N * 4)
+    assert ranges(D) == 1 and ranges(8256) == 3
+    test_gate_weight_gradient(M, D, N)
+
+
 @pytest.mark.parametrize("M,D,N", [
     (1, 8, 8), (64, 64, 32), (127, 128, 40), (129, 136, 136), (300, 264, 512), (8192, 64, 64),  # tiles of 128 x 128, 32 k-values
 ])
