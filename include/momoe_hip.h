@@ -39,8 +39,8 @@ extern "C" {
  * (momoe_index_build, momoe_tile_table_build).  momoe_lin1_swiglu_fwd, momoe_lin2_scale_fwd,
  * momoe_dgrad_h and momoe_dgrad_x take tables of any height up to MOMOE_TILE_ROWS and any list of
  * tokens per expert; which of their tile shapes a launch takes follows from its sizes and, on the device,
- * from the table (its height, its number of tiles, whether a tile is its expert's only one).  momoe_lin1_swiglu_bwd takes heights up to MOMOE_RECOMPUTE_TILE_ROWS (its epilogue
- * leaves no registers for a taller tile).  A kernel given a table of a greater height than it
+ * from the table (its height, its number of tiles, whether a tile is its expert's only one).  momoe_lin1_swiglu_bwd and
+ * momoe_dgrad_h_lin1_bwd take heights up to MOMOE_RECOMPUTE_TILE_ROWS (their epilogue leaves no registers for a taller tile).  A kernel given a table of a greater height than it
  * takes returns without writing anything.
  * tile_rows = 0 in momoe_index_build lets the library choose between the two heights from the
  * routing itself, on the device: taller tiles when they save enough passes over the experts'
@@ -275,8 +275,9 @@ int momoe_gs_scatter_tokens(const float* gs_part, int64_t nparts, const int32_t*
                             int64_t Msum, void* stream);
 
 /* momoe_dgrad_h_lin1_bwd: momoe_dgrad_h and, with row_lo = 0, momoe_lin1_swiglu_bwd_parts in one launch; the
- * arguments are theirs, nparts = momoe_gs_parts, the results the same bits; u_MsumH is scratch, not always written.  For launches of few tiles, as
- * momoe_dgrad_h_lin1_bwd_fits says (1 or 0) from the sizes alone.
+ * arguments are theirs, the table one that the latter takes, nparts = momoe_gs_parts, the results the same bits; u_MsumH (on a
+ * 16-byte boundary) is scratch, not always written.  For launches of few tiles, as momoe_dgrad_h_lin1_bwd_fits says (1 or 0)
+ * from the sizes alone; other sizes: MOMOE_ERR_UNSUPPORTED.
  */
 int momoe_dgrad_h_lin1_bwd_fits(int64_t M, int64_t D, int64_t H, int64_t N, int64_t Msum);
 int momoe_dgrad_h_lin1_bwd(const void* Gy_MD, const void* Wl2_NHD, const void* x_MD, const void* Wl1_ND2H,

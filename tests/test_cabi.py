@@ -78,6 +78,30 @@ def test_parts_of_the_gate_gradient(lib, H, N, msum, parts):
                                                    i64(256), i64(64), i64(H), i64(N), i64(msum), p(0)) == 1
 
 
+def test_refusals_of_the_joined_backward_launch(lib):
+    """All before any launch."""
+    i64, p = ctypes.c_int64, ctypes.c_void_p
+    good = dict(Gy=4096, W2=4096, x=4096, W1=4096, idx=4096, table=4096, s=4096, sn=1, sm=1, u=4096, gz=4096, hst=4096, ld=64, gs=4096,
+                nparts=1, M=256, D=64, H=64, N=8, msum=512)
+    pointers = ("Gy", "W2", "x", "W1", "idx", "table", "s", "u", "gz", "hst", "gs")
+
+    def status(**changed):
+        a = {**good, **changed}
+        return lib.momoe_dgrad_h_lin1_bwd(*[(p if k in pointers else i64)(v) for k, v in a.items()], p(0))
+
+    fits = lambda **c: lib.momoe_dgrad_h_lin1_bwd_fits(*[i64({**good, **c}[k]) for k in ("M", "D", "H", "N", "msum")])
+    assert fits() == 1
+    assert all(status(**{k: 0}) == 1 for k in pointers)
+    assert all(status(**{k: 4096 + 8}) == 1 for k in ("Gy", "W2", "x", "W1", "u", "gz", "hst"))
+    assert status(ld=56) == status(ld=68) == 1
+    assert status(M=0) == status(msum=0) == 1 and fits(M=0) == 0
+    assert all(status(nparts=n) == 1 for n in (0, 2, -1))
+    # the lines: 3072 k-values, one and a half row tiles per expert, one tile per CU; and widths that no kernel takes
+    assert fits(D=3040) == 1 and fits(msum=3072) == 1
+    for c in (dict(D=3072), dict(msum=3073), dict(H=4096, ld=4096, nparts=64), dict(D=48)):
+        assert fits(**c) == 0 and status(**c) == 2, c
+
+
 def test_host_modules_refuse_cpu_tensors():
     import torch
     import momoe_amd

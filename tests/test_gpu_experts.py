@@ -817,6 +817,20 @@ def test_dgrad_h_on_the_way_to_the_swiglu_backward(M, D, H, N, K, skew, overflow
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("M,D,H,N,K,skew", [(300, 96, 160, 9, 3, 1.8), (800, 160, 2048, 8, 2, 1.8)])  # u in registers, through memory
+def test_tables_that_the_joined_launch_does_not_take(M, D, H, N, K, skew):
+    from momoe_amd import _hip
+    dev, msum = "cuda:0", M * K
+    x, W1, W2, mask, s, dy = make_layer_inputs(M, D, H, N, K, seed=3, skew=skew)
+    x, Gy, W1, W2 = (t.to(dev, torch.bfloat16) for t in (x, dy, W1, W2))
+    ib = _hip.index_build(mask.to(dev), K, tile_rows=_hip.TILE_ROWS)
+    full = lambda *size, dt=torch.bfloat16: torch.full(size, 7.0, device=dev, dtype=dt)
+    outs = (full(msum, H), full(2 * H // 32, msum, 32), full(_hip.padded_rows(msum, N) // 32, H, 32),
+            full(_hip._lib.momoe_gs_parts(H, N, msum), msum, dt=torch.float32))
+    _hip.dgrad_h_lin1_bwd(Gy, W2, x, W1, ib["idx_Msum"], ib["tile_table"], s.to(dev), *outs)
+    assert all(bool((t == 7.0).all()) for t in outs)  # tiles too tall: nothing is written
+
+
 @pytest.mark.parametrize("M,D,H,N,K,skew", [
     (1, 32, 32, 1, 1, None), (128, 128, 64, 8, 2, None), (300, 352, 288, 9, 3, 1.8),  # a tile each, tiles cut off, few rows
     (4095, 64, 32, 70, 3, 1.8), (1000, 1056, 544, 16, 1, None),   # the most tokens; more tiles than workgroups
