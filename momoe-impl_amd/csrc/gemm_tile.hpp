@@ -1120,8 +1120,6 @@ struct FewRows {
   // more if the caller's index lists a token several times for an expert.  t holds the rows left.
   static __device__ __forceinline__ TileCoord piece(TileCoord t) {
     t.rows = min(t.rows, ROWS);
-    t.mbase = 0;
-    t.na = 1;
     return t;
   }
   template <class Sched>
