@@ -662,12 +662,12 @@ constexpr size_t kLin1DhLds =
     std::max({Lin1DhProg::Ring::BYTES, DhProg<NarrowTiles>::Ring::BYTES, Lin1Prog<true, StdTilesHalfParts>::kLds});
 
 // The few-row tiles (FewRows): 32 `a` columns and their 32 `b` columns.
-__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p, int last_entry) {
+__global__ __launch_bounds__(kThreads, 2) void lin1_swiglu_few_rows_kernel(Lin1Args p) {
   constexpr int BNH = FewRows::G::COLS / 2;
   const ClockTrace trace(p.clk);
   bf16* lds = dyn_lds();
   const int first_tile = p.h == nullptr && p.ab_lo > 0 ? TileSched::expert_tile_of_row(p.table, p.ab_lo) : 0;
-  FewRows::Sched sched(p.table, (p.H + BNH - 1) / BNH, first_tile, last_entry);
+  FewRows::Sched sched(p.table, (p.H + BNH - 1) / BNH, first_tile);
   const int D = p.D, H = p.H;
   FewRows op;
   for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
@@ -845,10 +845,10 @@ __global__ __launch_bounds__(kThreads, 2) void lin2_scale_narrow_kernel(Lin2Args
 }
 constexpr size_t kLin2NarrowLds = std::max(Lin2Prog<NarrowTiles>::kLds, kLin2Lds<StdTiles>);
 
-__global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p, int last_entry) {
+__global__ __launch_bounds__(kThreads, 2) void lin2_scale_few_rows_kernel(Lin2Args p) {
   const ClockTrace trace(p.clk);
   bf16* lds = dyn_lds();
-  FewRows::Sched sched(p.table, (p.D + FewRows::G::COLS - 1) / FewRows::G::COLS, 0, last_entry);
+  FewRows::Sched sched(p.table, (p.D + FewRows::G::COLS - 1) / FewRows::G::COLS, 0);
   const int D = p.D, H = p.H;
   FewRows op;
   for (TileCoord left = sched.next(); left.valid; left = FewRows::following(sched, left)) {
@@ -977,7 +977,7 @@ extern "C" int momoe_lin1_swiglu_fwd(const void* x_MD, const void* Wl1_ND2H,
   if (takes_few_rows_tiles(M, Msum, N, 2 * H)) {
     static LdsLimit few;
     if (!allow_lds(lin1_swiglu_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
-    lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a, (int)std::min(N, Msum) - 1);
+    lin1_swiglu_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
   if (takes_span_tiles(Msum, N, 2 * H, D)) {
@@ -1093,7 +1093,7 @@ extern "C" int momoe_lin2_scale_fwd(const void* h_blocked, const void* Wl2_NHD, 
   if (takes_few_rows_tiles(M, Msum, N, D)) {
     static LdsLimit few;
     if (!allow_lds(lin2_scale_few_rows_kernel, FewRows::BYTES, few)) return MOMOE_ERR_LAUNCH;
-    lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a, (int)std::min(N, Msum) - 1);
+    lin2_scale_few_rows_kernel<<<persistent_grid(), kThreads, FewRows::BYTES, (hipStream_t)stream>>>(a);
     return launch_status();
   }
   if (takes_span_tiles(Msum, N, D, H)) {

@@ -1130,9 +1130,9 @@ struct FewRows {
     return t;
   }
 
-  // Tiles in the table's order, the columns fastest: the place of a workgroup's first entry does not depend on
-  // the table's header, and the two are loaded at once.  `last`: no entry of a mask's table lies further on, and the table has
-  // room for it.  A list that repeats tokens may have more entries: those are loaded behind the header, by a branch that no mask takes.
+  // Tiles in the table's order, the columns fastest; the next tile's entry is loaded while the present one is worked on.  (The first
+  // one's beside the table's header, from a place bounded by what a mask's table holds, is no faster: 28.0 us at one token in
+  // either form; the table of a list that repeats tokens goes past any such bound.)
   // Two tiles in a row go to one XCD: 32 columns of each half of Wl1 are half a line, and on two XCDs, whose L2s
   // each fetch the line, x.Wl1 took 20 us instead of 15 (four or eight in a row 0 to 0.6 more than two).
   struct Sched : TileSched {
@@ -1142,18 +1142,13 @@ struct FewRows {
       const int b = blockIdx.x, group = 8 * kTogether, in = b % group;
       return gridDim.x % group != 0 ? b : b - in + in % 8 * kTogether + in / 8;
     }
-    static __device__ __forceinline__ Raw at(const int* table, int q, int row_tile) {
-      const int __attribute__((address_space(4)))* e = (const int __attribute__((address_space(4)))*)(table + kTileHeader + 4 * row_tile);
-      return Raw{q, e[0], e[1], e[2], e[3], true};
-    }
-    __device__ __forceinline__ Sched(const int* table_, int nb_, int first_row_tile, int last)
-        : TileSched(table_, nb_, MOMOE_TILE_ROWS, first_row_tile),
-          head(at(table_, first_row_tile * nb_ + place(), min(first_row_tile + place() / nb_, last))) {
+    __device__ __forceinline__ Sched(const int* table_, int nb_, int first_row_tile)
+        : TileSched(table_, nb_, MOMOE_TILE_ROWS, first_row_tile) {
       xcd = 0;
       pos = place();
       stride = gridDim.x;
       limit = total - begin;
-      if (__builtin_expect(first_row_tile + pos / nb > last && pos < limit, 0)) head = entry(pos, true);
+      head = entry(pos, pos < limit);
     }
     __device__ __forceinline__ TileCoord next() {
       Raw r = head;
